@@ -1285,19 +1285,46 @@ __global__ void k_bnd_coef_st(int n, const int* __restrict__ list, const double*
     A[(size_t)i * 288 + g * 36 + t * 9 + m] = s < 27 ? ST[st_index(node >> 6, node & 63, s * 9 + m)] : 0.0;
 }
 
+// Tagged entries of the boundary iterate: a 32-bit half of a component with
+// the number of updates it has seen, in one 64-bit word (FP32: 3 words per
+// node, FP64: 6), read and written as relaxed 64-bit atomics.  The value and
+// its tag travel together, so a reader needs no barrier and no fence.
+using TagWord = unsigned long long;
+__device__ __forceinline__ TagWord tag_word(unsigned half, unsigned tag) { return ((TagWord)tag << 32) | half; }
+__device__ __forceinline__ TagWord tag_load(const TagWord* p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void tag_store(TagWord* p, TagWord v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// words per component
+template <class T>
+struct TagPack {
+  static constexpr int W = sizeof(T) / 4;
+  __device__ static __forceinline__ void put(TagWord* p, float v, unsigned tag) {
+    tag_store(p, tag_word(__float_as_uint(v), tag));
+  }
+  __device__ static __forceinline__ void put(TagWord* p, double v, unsigned tag) {
+    const TagWord b = (TagWord)__double_as_longlong(v);
+    tag_store(p, tag_word((unsigned)b, tag));
+    tag_store(p + 1, tag_word((unsigned)(b >> 32), tag));
+  }
+  __device__ static __forceinline__ void get(const TagWord* w, float& v) { v = __uint_as_float((unsigned)w[0]); }
+  __device__ static __forceinline__ void get(const TagWord* w, double& v) {
+    v = __longlong_as_double((long long)((w[1] << 32) | (w[0] & 0xffffffffull)));
+  }
+};
+
 // b~_i = b_i - sum over spokes to nodes outside the boundary set (bt is
-// padded to 4 entries per node).  With `ub` given it also copies the
-// boundary iterate to ub ([3][n+1], zero sentinel at n) and clears the grid
-// barrier counter `ctr` of the single-launch phase; with `xmap` given it
-// writes the dense map's input [u_B (3n), b~ (3n)].
+// padded to 4 entries per node).  With `tu` given it also writes the
+// boundary iterate as tagged entries, tag 0 (k_bnd_flow); with `xmap` given
+// the dense map's input [u_B (3n), b~ (3n)].
 template <class T>
 __global__ void __launch_bounds__(256) k_bnd_rhs(int n, const int* __restrict__ list, const int* __restrict__ bslot,
                                                  const T* __restrict__ A, const T* __restrict__ u,
-                                                 const T* __restrict__ b, T* __restrict__ bt, T* __restrict__ ub = nullptr,
-                                                 unsigned* __restrict__ ctr = nullptr, T* __restrict__ xmap = nullptr) {
+                                                 const T* __restrict__ b, T* __restrict__ bt,
+                                                 TagWord* __restrict__ tu = nullptr, T* __restrict__ xmap = nullptr) {
   const int i = blockIdx.x * 32 + (threadIdx.x >> 3), g = threadIdx.x & 7;
-  if (ub && blockIdx.x == 0 && threadIdx.x < 3) ub[threadIdx.x * (n + 1) + n] = T(0);
-  if (ctr && blockIdx.x == 0 && threadIdx.x == 0) *ctr = 0u;
   const bool live = i < n;
   // the node's own b and u go out with the neighbour loads below
   const int node = live ? list[i] : 0, blk = node >> 6, l = node & 63;
@@ -1334,9 +1361,9 @@ __global__ void __launch_bounds__(256) k_bnd_rhs(int n, const int* __restrict__ 
     bt[i * 4 + 1] = bn[1] - a1;
     bt[i * 4 + 2] = bn[2] - a2;
     bt[i * 4 + 3] = T(0);
-    if (ub)
+    if (tu)
 #pragma unroll
-      for (int c = 0; c < 3; ++c) ub[c * (n + 1) + i] = un[c];
+      for (int c = 0; c < 3; ++c) TagPack<T>::put(tu + ((size_t)i * 3 + c) * TagPack<T>::W, un[c], 0u);
     if (xmap) {
 #pragma unroll
       for (int c = 0; c < 3; ++c) xmap[3 * i + c] = un[c];
@@ -1839,174 +1866,159 @@ __global__ void __launch_bounds__(B0_THREADS) k_bnd0_sweeps(int n, BndOff L, Col
   }
 }
 
-// Level-0 boundary phase over several CUs: one launch of G <= 32
-// workgroups (all resident at once), each of 8 waves; wave I computes cell
-// corner I's row for 64 nodes of a colour, the corner rows meet in LDS and
-// wave 0 updates the nodes.  The boundary iterate lives in `ub` ([3][n+1],
-// entry n a zero sentinel, filled by k_bnd_rhs); colour steps are separated
-// by a grid barrier.  Each node's update in the last sweep also goes to u.
-// A barrier wait longer than `limit` wall-clock ticks sets coop[1] and ends
-// the kernel, so every wave exits whatever happens.
-static constexpr int BC_THREADS = 512;
-static constexpr int BC_MAX_WG = 32;
-// per-lane tables of one node group: the corner's modulus and node indices,
-// and (wave 0) b~, the inverse self block, the node and its flags
+// Boundary phase by data flow over many CUs: one launch of G one-wave
+// workgroups (all resident at once).  A wave updates 8 nodes of a colour at
+// a time, an octet of lanes per node, lane g adding spokes g, g+8, g+16, g+24
+// from the stored coefficient rows; its groups follow in the order of the
+// colour steps.  No barrier separates the steps: the iterate lives in tagged
+// entries (`tu`, filled by k_bnd_rhs with tag 0), a node's update number k
+// carries tag k, and a node waits until each of its set neighbours carries
+// the tag that the sequential order gives it: sweep + 1 for colours earlier
+// in the sweep, sweep for its own and later ones.  A neighbour cannot run
+// ahead of that tag, because its next update waits for this node's (the
+// coupling is symmetric), so no entry is overwritten before it is read.
+// Waits are on earlier steps only; one longer than `limit` wall-clock ticks
+// sets the error word and ends the wave, so every wave exits.
+// Bound by the latency of one cross-XCD store-to-load hop per colour step; the
+// coefficients of the next group are loaded before the wait.  A phase of 24
+// steps takes 41 us at 405 nodes and 49 us at 21125 (FP32), 58 us at 2400
+// (FP64); steps separated by grid barriers (release add, poll, acquire fence,
+// reload) took 61, 99 and 103 us.
+static constexpr int BF_MAX_WG = 1024;
 template <class T>
-struct CoopFetch {
-  T e, r[3], di[6];
-  int cw[4];
-  int node, i;
+struct FlowFetch {
+  BndFetch<T> f;
+  T di[6];
+  int node, c, sw;
   uint8_t fl;
-  bool live;
 };
 template <class T>
-__global__ void __launch_bounds__(BC_THREADS) k_bnd0_coop(int n, BndOff L, ColourOrder ord, int sweeps,
-                                                          const int* __restrict__ list,
-                                                          const uint8_t* __restrict__ flags,
-                                                          const T* __restrict__ bE,
-                                                          const int16_t* __restrict__ cnode,
-                                                          const T* __restrict__ bD, const T* __restrict__ bt, T dx,
-                                                          T* ub, T* __restrict__ u, unsigned* coop,
-                                                          unsigned long long limit) {
-  __shared__ T P[8][3][64];
-  __shared__ int bad;
-  const int n1 = n + 1;
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int I = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int G = gridDim.x;
-  const int steps = sweeps * 8;
-  unsigned* ctr = coop;
-  int* err = reinterpret_cast<int*>(coop + 1);
-  // everything but the iterate: loaded ahead, the next step's first group
-  // while the grid barrier is pending
-  auto fetch = [&](CoopFetch<T>& F, int st, int q) {
-    const int c = ord.at(st & 7), o0 = L.off[c], nc = L.off[c + 1] - o0;
-    const int j = q * 64 + lane;
-    F.live = j < nc;
-    F.i = o0 + (F.live ? j : 0);
-    F.e = T(0);
-    F.cw[0] = F.cw[1] = F.cw[2] = F.cw[3] = -1;
-    if (F.live) {
-      F.e = bE[I * n + F.i];
-      const int4 a = *reinterpret_cast<const int4*>(cnode + ((size_t)I * n + F.i) * 8);
-      F.cw[0] = a.x;
-      F.cw[1] = a.y;
-      F.cw[2] = a.z;
-      F.cw[3] = a.w;
+__global__ void __launch_bounds__(64) k_bnd_flow(BndOff L, ColourOrder ord, ColourOrder pos, int sweeps,
+                                                 const int* __restrict__ list, const int* __restrict__ bci,
+                                                 const T* __restrict__ A, const uint8_t* __restrict__ flags,
+                                                 const T* __restrict__ bt, TagWord* tu, T* __restrict__ u, int* err,
+                                                 unsigned long long limit) {
+  constexpr int W = TagPack<T>::W, NW = 3 * W;
+  const int lane = threadIdx.x, oct = lane >> 3, g = lane & 7;
+  const int G = gridDim.x, steps = sweeps * 8;
+  // colour offset of each of the lane's spokes
+  int par[4];
+#pragma unroll
+  for (int t = 0; t < 4; ++t) {
+    const int s = g + 8 * t;
+    par[t] = ((s / 9 != 1) << 2) | (((s / 3) % 3 != 1) << 1) | (s % 3 != 1);
+  }
+  // next group (st, q) at or after (st, q), st = steps at the end
+  auto seek = [&](int& st, int& q) {
+    while (st < steps) {
+      const int c = ord.at(st & 7);
+      if (q * 8 < L.off[c + 1] - L.off[c]) return;
+      ++st;
+      q = blockIdx.x;
     }
-#pragma unroll
-    for (int v = 0; v < 3; ++v) F.r[v] = T(0);
-#pragma unroll
-    for (int v = 0; v < 6; ++v) F.di[v] = T(0);
+  };
+  auto fetch = [&](FlowFetch<T>& F, int st, int q) {
+    const int c = ord.at(st & 7), i = L.off[c] + q * 8 + oct;
+    bnd_fetch<T>(F.f, i, i < L.off[c + 1], g, bci, A, bt);
+    F.c = c;
+    F.sw = st >> 3;
     F.node = 0;
     F.fl = 0;
-    if (I == 0 && F.live) {
-#pragma unroll
-      for (int v = 0; v < 3; ++v) F.r[v] = bt[F.i * 4 + v];
-#pragma unroll
-      for (int v = 0; v < 6; ++v) F.di[v] = bD[F.i * 8 + v];
-      F.node = list[F.i];
+    if (g == 5 && F.f.live) {
+      F.node = list[i];
       F.fl = flags[F.node];
     }
   };
-  CoopFetch<T> F;
-  fetch(F, 0, blockIdx.x);
-  for (int st = 0; st < steps; ++st) {
-    const int c = ord.at(st & 7);
-    const bool last = st >= steps - 8;
-    const int nc = L.off[c + 1] - L.off[c];
-    for (int q = blockIdx.x; q * 64 < nc; q += G) {
-      if (q != (int)blockIdx.x) fetch(F, st, q);
-      T a0 = 0, a1 = 0, a2 = 0, x[3];
-#pragma unroll
-      for (int J = 0; J < 8; ++J) {
-        const int wv = F.cw[J >> 1];
-        int k = (J & 1) ? (wv >> 16) : (int)(short)(wv & 0xffff);
-        k = k < 0 ? n : k;
-        const T v0 = ub[k], v1 = ub[n1 + k], v2 = ub[2 * n1 + k];
-        if (J == 0) {  // for corner 0, node 0 of the cell is the node itself
-          x[0] = v0;
-          x[1] = v1;
-          x[2] = v2;
-        }
-        const int kb = (I * 8 + J) * 9;
-        a0 = fmaT(KT<T>::k(kb + 0), v0, a0);
-        a0 = fmaT(KT<T>::k(kb + 1), v1, a0);
-        a0 = fmaT(KT<T>::k(kb + 2), v2, a0);
-        a1 = fmaT(KT<T>::k(kb + 3), v0, a1);
-        a1 = fmaT(KT<T>::k(kb + 4), v1, a1);
-        a1 = fmaT(KT<T>::k(kb + 5), v2, a1);
-        a2 = fmaT(KT<T>::k(kb + 6), v0, a2);
-        a2 = fmaT(KT<T>::k(kb + 7), v1, a2);
-        a2 = fmaT(KT<T>::k(kb + 8), v2, a2);
-      }
-      P[I][0][lane] = F.e * a0;
-      P[I][1][lane] = F.e * a1;
-      P[I][2][lane] = F.e * a2;
-      __syncthreads();
-      if (I == 0 && F.live) {
-        const int i = F.i;
-        T f[3];
-#pragma unroll
-        for (int v = 0; v < 3; ++v) {
-          T acc = 0;
-#pragma unroll
-          for (int cc = 0; cc < 8; ++cc) acc += P[cc][v][lane];
-          f[v] = dx * acc;
-        }
-        const uint8_t fl = F.fl;
-        if (fl & 1) {
-          const T r0 = F.r[0] - f[0], r1 = F.r[1] - f[1], r2 = F.r[2] - f[2];
-          const T u0 = x[0] + F.di[0] * r0 + F.di[3] * r1 + F.di[4] * r2;
-          const T u1 = x[1] + F.di[3] * r0 + F.di[1] * r1 + F.di[5] * r2;
-          const T u2 = x[2] + F.di[4] * r0 + F.di[5] * r1 + F.di[2] * r2;
-          x[0] = (fl & 2) ? T(0) : u0;
-          x[1] = (fl & 4) ? T(0) : u1;
-          x[2] = (fl & 8) ? T(0) : u2;
-        } else {
-#pragma unroll
-          for (int v = 0; v < 3; ++v)
-            if (fl & (2 << v)) x[v] = T(0);
-        }
-#pragma unroll
-        for (int v = 0; v < 3; ++v) ub[v * n1 + i] = x[v];
-        if (last) {
-          const int blk = F.node >> 6, l = F.node & 63;
-#pragma unroll
-          for (int v = 0; v < 3; ++v) u[vidx(blk, v, l)] = x[v];
-        }
-      }
-      __syncthreads();  // P is reused by the next group
+  // the inverse self block, before the wait
+  auto invert = [&](FlowFetch<T>& F) {
+    if (g == 5) {
+      F.di[0] = F.f.m[9]; F.di[1] = F.f.m[13]; F.di[2] = F.f.m[17];
+      F.di[3] = F.f.m[10]; F.di[4] = F.f.m[11]; F.di[5] = F.f.m[14];
+      dirichlet_inverse(F.di, F.fl);
     }
-    if (st + 1 == steps) break;
-    // Grid barrier.  Thread 0 (of wave 0, the only wave that stores to
-    // global memory) publishes the step with a release add, the workgroup
-    // then loads the next step's tables, and thread 0 waits for all G
-    // arrivals; a wait longer than `limit` wall-clock ticks sets the error
-    // word and ends the kernel, so every wave exits.
-    const unsigned target = (unsigned)(G * (st + 1));
-    __syncthreads();
-    if (tid == 0) __hip_atomic_fetch_add(ctr, 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
-    fetch(F, st + 1, blockIdx.x);
-    if (tid == 0) {
-      int b = 0;
-      const unsigned long long t0 = wall_clock64();
-      // relaxed polls (an acquire load would invalidate the L2 at every
-      // poll), then one acquire fence for the data the other workgroups
-      // published with their release add
-      while (__hip_atomic_load(ctr, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < target) {
-        if (wall_clock64() - t0 > limit) {
-          __hip_atomic_fetch_or(err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-          b = 1;
-          break;
-        }
-        __builtin_amdgcn_s_sleep(1);
+  };
+  auto update = [&](const FlowFetch<T>& F) -> bool {
+    T x[4][3];
+    unsigned long long t0 = 0;
+    for (bool first = true;; first = false) {
+      bool ok = true;
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        const int j = F.f.j[t];
+        const unsigned need = (unsigned)F.sw + (pos.at(F.c ^ par[t]) < pos.at(F.c) ? 1u : 0u);
+        TagWord w[NW];
+#pragma unroll
+        for (int k = 0; k < NW; ++k) w[k] = j >= 0 ? tag_load(tu + (size_t)j * NW + k) : tag_word(0u, need);
+#pragma unroll
+        for (int k = 0; k < NW; ++k) ok = ok && (unsigned)(w[k] >> 32) >= need;
+#pragma unroll
+        for (int v = 0; v < 3; ++v) TagPack<T>::get(w + v * W, x[t][v]);
       }
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-      bad = b;
+      if (__all(ok)) break;
+      if (first) t0 = wall_clock64();
+      else if (wall_clock64() - t0 > limit) {
+        if (lane == 0) __hip_atomic_fetch_or(err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        return false;
+      }
     }
-    __syncthreads();
-    if (bad) return;
+    T a0 = 0, a1 = 0, a2 = 0;
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      const T* m = F.f.m + t * 9;
+      a0 = fmaT(m[0], x[t][0], a0);
+      a0 = fmaT(m[1], x[t][1], a0);
+      a0 = fmaT(m[2], x[t][2], a0);
+      a1 = fmaT(m[3], x[t][0], a1);
+      a1 = fmaT(m[4], x[t][1], a1);
+      a1 = fmaT(m[5], x[t][2], a1);
+      a2 = fmaT(m[6], x[t][0], a2);
+      a2 = fmaT(m[7], x[t][1], a2);
+      a2 = fmaT(m[8], x[t][2], a2);
+    }
+    a0 = octet_sum(a0);
+    a1 = octet_sum(a1);
+    a2 = octet_sum(a2);
+    if (g == 5 && F.f.live) {  // spoke 13 = (g 5, t 1) is the node itself
+      T n0 = x[1][0], n1 = x[1][1], n2 = x[1][2];
+      if (F.fl & 1) {
+        const T r0 = F.f.r[0] - a0, r1 = F.f.r[1] - a1, r2 = F.f.r[2] - a2;
+        n0 += F.di[0] * r0 + F.di[3] * r1 + F.di[4] * r2;
+        n1 += F.di[3] * r0 + F.di[1] * r1 + F.di[5] * r2;
+        n2 += F.di[4] * r0 + F.di[5] * r1 + F.di[2] * r2;
+      }
+      if (F.fl & 2) n0 = T(0);
+      if (F.fl & 4) n1 = T(0);
+      if (F.fl & 8) n2 = T(0);
+      TagWord* p = tu + (size_t)F.f.i * NW;
+      const unsigned tag = (unsigned)F.sw + 1u;
+      TagPack<T>::put(p, n0, tag);
+      TagPack<T>::put(p + W, n1, tag);
+      TagPack<T>::put(p + 2 * W, n2, tag);
+      if (F.sw + 1 == sweeps) {
+        const int blk = F.node >> 6, l = F.node & 63;
+        u[vidx(blk, 0, l)] = n0;
+        u[vidx(blk, 1, l)] = n1;
+        u[vidx(blk, 2, l)] = n2;
+      }
+    }
+    return true;
+  };
+  int st = 0, q = blockIdx.x;
+  seek(st, q);
+  if (st >= steps) return;
+  FlowFetch<T> X, Y;
+  fetch(X, st, q);
+  for (;;) {
+    invert(X);
+    q += G;
+    seek(st, q);
+    if (st < steps) fetch(Y, st, q);
+    if (!update(X) || st >= steps) return;
+    invert(Y);
+    q += G;
+    seek(st, q);
+    if (st < steps) fetch(X, st, q);
+    if (!update(Y) || st >= steps) return;
   }
 }
 
@@ -2790,12 +2802,12 @@ static BndLists bnd_lists(const LevelDev& L) {
 // a boundary phase runs in one workgroup while no colour list is longer than this
 static constexpr int kFusedBoundaryMax = 4096;
 // SPG_BOUNDARY_PATH selects the boundary smoother for tests: 0 (default)
-// automatic (level 0: the cooperative matrix-free phase, else one launch per
-// colour step; explicit levels: the dense map, else the LDS coefficient-row
-// system), 1 the single-workgroup global-memory kernel, 2 one launch per
+// automatic (level 0: the data-flow phase, else one launch per colour step;
+// explicit levels: the dense map, else the LDS coefficient-row system), 1 the
+// single-workgroup global-memory kernel, 2 one launch per
 // colour step, 3 the coefficient-row LDS system also on level 0, 4 the
-// matrix-free single-workgroup level-0 phase, 5 the cooperative level-0
-// phase (automatic on the explicit levels).
+// matrix-free single-workgroup level-0 phase, 5 the data-flow level-0 phase
+// (automatic on the explicit levels).
 static int boundary_path() {
   const char* e = std::getenv("SPG_BOUNDARY_PATH");
   return e ? std::atoi(e) : 0;
@@ -2864,23 +2876,21 @@ static bool launch_bnd0_phase(hipStream_t st, const LevelDev& L, T dx, T* u, con
                                                L.b0node, bD, bt, dx, u);
   return true;
 }
-// level-0 boundary phase as one launch over several CUs; false if the
-// tables are absent or a cooperative launch is refused (the caller then runs
-// another path; `loud` reports a refused launch on stderr).  SPG_COOP_WG
-// caps the workgroup count (tests use it to make a workgroup take several
-// node groups per colour step).
+// boundary phase by data flow (k_bnd_flow); false if the level has no tables
+// for it or a cooperative launch is refused (the caller then runs another
+// path; `loud` reports a refused launch on stderr).  SPG_COOP_WG caps the
+// workgroup count (tests use it to make a wave take several node groups per
+// colour step).
 template <class T>
-static bool launch_bnd0_coop(hipStream_t st, const LevelDev& L, T dx, T* u, const T* b, int sweeps, bool forward,
-                             bool loud) {
+static bool launch_bnd_flow(hipStream_t st, const LevelDev& L, T* u, const T* b, int sweeps, bool level0, bool forward,
+                            bool loud) {
   const int n = L.bnd_off[8];
   const T* A = BndPtr<T>::A(L);
   T* bt = BndPtr<T>::bt(L);
-  const T* bE = Bnd0Ptr<T>::E(L);
-  const T* bD = Bnd0Ptr<T>::D(L);
-  if (!A || !bt || !bE || !bD || !L.b0node || !L.bslot || !L.b0ub || !L.coop) return false;
+  if (!A || !bt || !L.bci || !L.bslot || !L.btag || !L.coop || L.coop_off) return false;
   int groups = 1;
-  for (int c = 0; c < 8; ++c) groups = std::max(groups, (L.bnd_off[c + 1] - L.bnd_off[c] + 63) / 64);
-  int G = std::min(groups, BC_MAX_WG);
+  for (int c = 0; c < 8; ++c) groups = std::max(groups, (L.bnd_off[c + 1] - L.bnd_off[c] + 7) / 8);
+  int G = std::min(groups, BF_MAX_WG);
   if (const char* e = std::getenv("SPG_COOP_WG"))
     if (std::atoi(e) > 0) G = std::min(G, std::atoi(e));
   static const unsigned long long wait_50ms = [] {
@@ -2890,34 +2900,33 @@ static bool launch_bnd0_coop(hipStream_t st, const LevelDev& L, T dx, T* u, cons
     return (unsigned long long)khz * 50;
   }();
   // SPG_COOP_LIMIT_TICKS shortens the wait (tests force the time-out path)
-  unsigned long long limit = wait_50ms;
+  unsigned long long lim = wait_50ms;
   if (const char* e = std::getenv("SPG_COOP_LIMIT_TICKS"))
-    if (std::atoll(e) > 0) limit = (unsigned long long)std::atoll(e);
-  T* ub = reinterpret_cast<T*>(L.b0ub);
-  k_bnd_rhs<T><<<(n + 31) / 32, 256, 0, st>>>(n, L.bnd, L.bslot, A, u, b, bt, ub, L.coop);
+    if (std::atoll(e) > 0) lim = (unsigned long long)std::atoll(e);
+  TagWord* tu = static_cast<TagWord*>(L.btag);
+  k_bnd_rhs<T><<<(n + 31) / 32, 256, 0, st>>>(n, L.bnd, L.bslot, A, u, b, bt, tu);
   BndOff o;
   for (int c = 0; c < 9; ++c) o.off[c] = L.bnd_off[c];
-  ColourOrder ord = colour_order(true, forward);
-  const int16_t* cn = L.b0node;
+  ColourOrder ord = colour_order(level0, forward), pos{0};
+  for (int i = 0; i < 8; ++i) pos.v |= (unsigned)i << (4 * ord.at(i));
   const int* list = L.bnd;
+  const int* bci = L.bci;
   const uint8_t* flags = L.flags;
-  unsigned* coop = L.coop;
-  unsigned long long lim = limit;
-  int nn = n, sw = sweeps;
+  int* err = reinterpret_cast<int*>(L.coop + 1);
+  int sw = sweeps;
   // An ordinary launch by default: the solver's stream runs one kernel at a
-  // time, so the G <= 32 small workgroups all start at once on the empty
-  // device (256 CUs).  The cooperative launch API guarantees that even
-  // while other streams fill the device, but costs about 40 us per phase
-  // (256^3 shell: phase 96 vs 115 us, mixed solve 40.2 vs 42.9 ms);
-  // SPG_COOP_LAUNCH=1 selects it.  Either way a barrier wait ends after
-  // `limit` and is reported.
+  // time, so the one-wave workgroups (at most 1024: 4 per CU) all start at
+  // once on the empty device.  The cooperative launch API guarantees that
+  // even while other streams fill the device, but costs about 40 us per
+  // phase; SPG_COOP_LAUNCH=1 selects it.  Either way a wait ends after the
+  // limit and is reported.
   const char* cl = std::getenv("SPG_COOP_LAUNCH");
   if (!(cl && std::atoi(cl) == 1)) {
-    k_bnd0_coop<T><<<G, BC_THREADS, 0, st>>>(nn, o, ord, sw, list, flags, bE, cn, bD, bt, dx, ub, u, coop, lim);
+    k_bnd_flow<T><<<G, 64, 0, st>>>(o, ord, pos, sw, list, bci, A, flags, bt, tu, u, err, lim);
     return true;
   }
-  void* args[] = {&nn, &o, &ord, &sw, &list, &flags, &bE, &cn, &bD, &bt, &dx, &ub, &u, &coop, &lim};
-  const hipError_t e = hipLaunchCooperativeKernel((const void*)k_bnd0_coop<T>, dim3(G), dim3(BC_THREADS), args, 0, st);
+  void* args[] = {&o, &ord, &pos, &sw, &list, &bci, &A, &flags, &bt, &tu, &u, &err, &lim};
+  const hipError_t e = hipLaunchCooperativeKernel((const void*)k_bnd_flow<T>, dim3(G), dim3(64), args, 0, st);
   if (e == hipSuccess) return true;
   (void)hipGetLastError();
   if (loud)
@@ -3028,13 +3037,13 @@ void launch_gs0_boundary(hipStream_t st, const LevelDev& L, const T* E, T dx, T*
                          bool forward) {
   if (sweeps <= 0 || L.bnd_off[8] == 0) return;
   int path = boundary_path();
-  // Automatic choice, from measurement on the 256^3 shell (3655 boundary
-  // nodes, 3 sweeps), FP32 / FP64 per phase: cooperative launch 123 / 136
-  // us, per-colour list launches 145 / 168 us, single workgroup 154 / 235
-  // us (one CU's VALU work).  The lists remain for sets beyond the int16
-  // node tables and for a refused cooperative launch.
+  // Automatic choice, FP32 per phase of 3 sweeps on the 256^3 shell (3655
+  // boundary nodes): data flow 45 us, grid barriers between the steps 87 us,
+  // per-colour list launches 145 us, single workgroup 154 us (one CU's VALU
+  // work).  The lists remain for a refused cooperative launch and after a
+  // time-out.
   if (path == 0 || path == 5) {
-    if (!L.coop_off && launch_bnd0_coop<T>(st, L, dx, u, b, sweeps, forward, path == 5)) return;
+    if (launch_bnd_flow<T>(st, L, u, b, sweeps, true, forward, path == 5)) return;
     path = 2;
   }
   if (path == 4 && launch_bnd0_phase<T>(st, L, dx, u, b, sweeps, forward)) return;
@@ -3087,7 +3096,7 @@ void launch_st_boundary(hipStream_t st, const LevelDev& L, const T* ST, T* u, co
     // two launches: b~ and the map input, then the map with the result
     // written to u (the separate gather / scatter kernels cost two launch
     // gaps per phase)
-    k_bnd_rhs<T><<<(n + 31) / 32, 256, 0, st>>>(n, L.bnd, L.bslot, BndPtr<T>::A(L), u, b, bt, nullptr, nullptr, x);
+    k_bnd_rhs<T><<<(n + 31) / 32, 256, 0, st>>>(n, L.bnd, L.bslot, BndPtr<T>::A(L), u, b, bt, nullptr, x);
     k_bmap_gemv<T><<<(3 * n + 3) / 4, 256, 0, st>>>(3 * n, Kp, M, x, x + Kp, L.bnd, u);
     return;
   }

@@ -48,11 +48,11 @@ struct LevelDev {
   const double* b0E64 = nullptr;
   const float* b0D32 = nullptr;
   const double* b0D64 = nullptr;
-  // cooperative level-0 phase: boundary iterate [3*(n+1)] (8-byte entries,
-  // either precision) and {barrier counter, error word}
-  void* b0ub = nullptr;
+  // data-flow boundary phase: tagged iterate [n*6] 64-bit words (either
+  // precision) and {unused, error word}
+  void* btag = nullptr;
   unsigned* coop = nullptr;
-  int coop_off = 0;  // 1 after a barrier time-out: the list launches take over
+  int coop_off = 0;  // 1 after a wait timed out: the list launches take over
   // explicit levels: dense maps [G H] of one boundary phase (forward,
   // backward colour order) for `bmap_sweeps` sweeps, and their vector
   // scratch ([6n] input then [3n] output)

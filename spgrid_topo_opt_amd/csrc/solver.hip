@@ -183,7 +183,7 @@ void Solver::check_coop() {
     HIPCHK(hipMemsetAsync(static_cast<unsigned*>(lv_[0].coop.p) + 1, 0, sizeof(unsigned), st_));
     HIPCHK(hipStreamSynchronize(st_));
     throw SpgError(SPG_E_HIP,
-                   "level-0 boundary phase: grid barrier wait timed out (workgroups not resident together; "
+                   "level-0 boundary phase: a wait timed out (workgroups not resident together; "
                    "SPG_COOP_LAUNCH=1 uses the cooperative launch API, SPG_BOUNDARY_PATH=2 per-colour launches)");
   }
 }
@@ -220,6 +220,13 @@ void Solver::upload_layout() {
       R.bA32.alloc(bnd.size() * 288 * 4);
       R.bt64.alloc(bnd.size() * 4 * 8);
       R.bt32.alloc(bnd.size() * 4 * 4);
+      if (l == 0) {
+        R.btag.alloc(bnd.size() * 6 * 8);
+        R.coop.alloc(2 * sizeof(unsigned));
+        HIPCHK(hipMemset(R.coop.p, 0, 2 * sizeof(unsigned)));
+        R.d.btag = R.btag.p;
+        R.d.coop = R.coop.as<unsigned>();
+      }
     }
     if (!D.bnd_cslot.empty()) {
       upload(R.b0cslot, D.bnd_cslot);
@@ -233,11 +240,6 @@ void Solver::upload_layout() {
       R.d.b0E32 = R.b0E32.as<float>();
       R.d.b0D64 = R.b0D64.as<double>();
       R.d.b0D32 = R.b0D32.as<float>();
-      R.b0ub.alloc((bnd.size() + 1) * 3 * 8);
-      R.coop.alloc(2 * sizeof(unsigned));
-      HIPCHK(hipMemset(R.coop.p, 0, 2 * sizeof(unsigned)));
-      R.d.b0ub = R.b0ub.p;
-      R.d.coop = R.coop.as<unsigned>();
     }
     R.d.bci = R.bci.as<int>();
     R.d.bslot = R.bslot.as<int>();
