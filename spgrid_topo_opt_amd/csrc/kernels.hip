@@ -1884,7 +1884,9 @@ __global__ void __launch_bounds__(B0_THREADS) k_bnd0_sweeps(int n, BndOff L, Col
 // steps takes 41 us at 405 nodes and 49 us at 21125 (FP32), 58 us at 2400
 // (FP64); steps separated by grid barriers (release add, poll, acquire fence,
 // reload) took 61, 99 and 103 us.
-static constexpr int BF_MAX_WG = 1024;
+// The FP64 kernel's 256 registers leave one wave per SIMD: 512 one-wave
+// workgroups are half of what the 256 CUs hold at once.
+static constexpr int BF_MAX_WG = 512;
 template <class T>
 struct FlowFetch {
   BndFetch<T> f;
@@ -2915,7 +2917,7 @@ static bool launch_bnd_flow(hipStream_t st, const LevelDev& L, T* u, const T* b,
   int* err = reinterpret_cast<int*>(L.coop + 1);
   int sw = sweeps;
   // An ordinary launch by default: the solver's stream runs one kernel at a
-  // time, so the one-wave workgroups (at most 1024: 4 per CU) all start at
+  // time, so the one-wave workgroups (at most 512: 2 per CU) all start at
   // once on the empty device.  The cooperative launch API guarantees that
   // even while other streams fill the device, but costs about 40 us per
   // phase; SPG_COOP_LAUNCH=1 selects it.  Either way a wait ends after the
