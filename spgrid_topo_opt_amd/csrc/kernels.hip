@@ -1317,13 +1317,12 @@ struct TagPack {
 
 // b~_i = b_i - sum over spokes to nodes outside the boundary set (bt is
 // padded to 4 entries per node).  With `tu` given it also writes the
-// boundary iterate as tagged entries, tag 0 (k_bnd_flow); with `xmap` given
-// the dense map's input [u_B (3n), b~ (3n)].
+// boundary iterate as tagged entries, tag 0 (k_bnd_flow).
 template <class T>
 __global__ void __launch_bounds__(256) k_bnd_rhs(int n, const int* __restrict__ list, const int* __restrict__ bslot,
                                                  const T* __restrict__ A, const T* __restrict__ u,
                                                  const T* __restrict__ b, T* __restrict__ bt,
-                                                 TagWord* __restrict__ tu = nullptr, T* __restrict__ xmap = nullptr) {
+                                                 TagWord* __restrict__ tu = nullptr) {
   const int i = blockIdx.x * 32 + (threadIdx.x >> 3), g = threadIdx.x & 7;
   const bool live = i < n;
   // the node's own b and u go out with the neighbour loads below
@@ -1364,13 +1363,57 @@ __global__ void __launch_bounds__(256) k_bnd_rhs(int n, const int* __restrict__ 
     if (tu)
 #pragma unroll
       for (int c = 0; c < 3; ++c) TagPack<T>::put(tu + ((size_t)i * 3 + c) * TagPack<T>::W, un[c], 0u);
-    if (xmap) {
+  }
+}
+
+// Residual of the boundary equations, the input of the dense map: free
+// components b - A u over all neighbours (`ball`: slot of spoke g + 8t at
+// [i*32 + g*4 + t], in or outside the set, -1 absent), Dirichlet components
+// -u (their equation is u = 0), components of inactive nodes 0.
+template <class T>
+__global__ void __launch_bounds__(256) k_bnd_res(int n, const int* __restrict__ list, const int* __restrict__ ball,
+                                                 const T* __restrict__ A, const uint8_t* __restrict__ flags,
+                                                 const T* __restrict__ u, const T* __restrict__ b,
+                                                 T* __restrict__ x) {
+  const int i = blockIdx.x * 32 + (threadIdx.x >> 3), g = threadIdx.x & 7;
+  const bool live = i < n;
+  const int node = live ? list[i] : 0, blk = node >> 6, l = node & 63;
+  T bn[3] = {T(0), T(0), T(0)}, un[3] = {T(0), T(0), T(0)};
+  uint8_t fl = 0;
+  if (g == 0 && live) {
+    fl = flags[node];
 #pragma unroll
-      for (int c = 0; c < 3; ++c) xmap[3 * i + c] = un[c];
-      xmap[3 * n + 3 * i + 0] = bn[0] - a0;
-      xmap[3 * n + 3 * i + 1] = bn[1] - a1;
-      xmap[3 * n + 3 * i + 2] = bn[2] - a2;
+    for (int c = 0; c < 3; ++c) {
+      bn[c] = b[vidx(blk, c, l)];
+      un[c] = u[vidx(blk, c, l)];
     }
+  }
+  T a0 = 0, a1 = 0, a2 = 0;
+#pragma unroll
+  for (int t = 0; t < 4; ++t) {
+    const int sl = live ? ball[i * 32 + g * 4 + t] : -1;
+    if (sl >= 0) {
+      const T x0 = u[vidx(sl >> 6, 0, sl & 63)], x1 = u[vidx(sl >> 6, 1, sl & 63)], x2 = u[vidx(sl >> 6, 2, sl & 63)];
+      const T* M = A + (size_t)i * 288 + g * 36 + t * 9;
+      a0 = fmaT(M[0], x0, a0);
+      a0 = fmaT(M[1], x1, a0);
+      a0 = fmaT(M[2], x2, a0);
+      a1 = fmaT(M[3], x0, a1);
+      a1 = fmaT(M[4], x1, a1);
+      a1 = fmaT(M[5], x2, a1);
+      a2 = fmaT(M[6], x0, a2);
+      a2 = fmaT(M[7], x1, a2);
+      a2 = fmaT(M[8], x2, a2);
+    }
+  }
+  a0 = octet_sum(a0);
+  a1 = octet_sum(a1);
+  a2 = octet_sum(a2);
+  if (g == 0 && live) {
+    const bool act = fl & 1;
+    x[3 * i + 0] = (fl & 2) ? -un[0] : (act ? bn[0] - a0 : T(0));
+    x[3 * i + 1] = (fl & 4) ? -un[1] : (act ? bn[1] - a1 : T(0));
+    x[3 * i + 2] = (fl & 8) ? -un[2] : (act ? bn[2] - a2 : T(0));
   }
 }
 
@@ -1571,80 +1614,102 @@ __global__ void __launch_bounds__(NT) k_bnd_sweeps(int n, BndOff L, ColourOrder 
   }
 }
 
-// Dense map [G H] of a boundary phase, u_B <- G u_B + H b~ (row-major,
-// 3n x 6n with rows padded to bmap_stride(n), entry index node*3 + component).  Column-parallel: the phase is
-// run on all unit vectors at once, lane = column (columns j < 3n start from
-// u_B = e_j with b~ = 0, columns 3n + j from u_B = 0 with b~ = e_j), so
-// every node row and its coefficients are wave-uniform.  The 16 waves of a
-// workgroup share 64 columns and split the nodes of each colour; the
-// matrix itself holds the iterate (nodes of one colour do not couple).
-constexpr int BM_WAVES = 16;
-__global__ void __launch_bounds__(64 * BM_WAVES) k_bmap_build(int n, BndOff L, ColourOrder ord, int sweeps,
-                                                            const int* __restrict__ list,
-                                                            const int* __restrict__ bci,
-                                                            const double* __restrict__ A,
-                                                            const uint8_t* __restrict__ flags,
-                                                            double* __restrict__ M) {
-  const int64_t K = bmap_stride(n);  // row stride; columns >= 6n stay zero
-  const int col = blockIdx.x * 64 + (threadIdx.x & 63);
-  const bool live = col < 6 * n;
-  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int rows = 3 * n;
-  double* Mc = M + col;
-  if (live)
-    for (int r = w; r < rows; r += BM_WAVES) Mc[(int64_t)r * K] = (col == r) ? 1.0 : 0.0;
-  const int hj = col - rows;  // right-hand-side unit index of an H column
+// Dense map M of a boundary phase.  The phase is a stationary iteration that
+// leaves the exact solution unchanged, so u_B <- u_B + M r with r the residual
+// of the boundary equations (k_bnd_res) and M the phase's answer to unit
+// right-hand sides from u_B = 0 (row-major, 3n x 3n with rows padded to
+// bmap_stride(n), entry index node*3 + component; a Dirichlet component's
+// equation is u = its right-hand side).  Half the entries of the form
+// u_B <- G u_B + H b~.
+// A workgroup runs the phase on NC unit vectors at once, their iterate in LDS
+// ([3n][NC]): an octet of lanes per node, lane g adding spokes g, g+8, g+16,
+// g+24 for all NC columns from one read of its coefficients.  Bound by
+// streaming the coefficient rows (2.3 KB a node and sweep) from L2 into every
+// workgroup, so NC is the most columns the LDS holds.  blockIdx.y: 0 forward,
+// 1 backward map.
+constexpr int BM_THREADS = 1024;
+template <int NC>
+__global__ void __launch_bounds__(BM_THREADS) k_bmap_build(int n, BndOff L, ColourOrder ord0, ColourOrder ord1,
+                                                           int sweeps, const int* __restrict__ list,
+                                                           const int* __restrict__ bci, const double* __restrict__ A,
+                                                           const uint8_t* __restrict__ flags, double* __restrict__ M0,
+                                                           double* __restrict__ M1, float* __restrict__ F0,
+                                                           float* __restrict__ F1) {
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+  double* U = reinterpret_cast<double*>(smem_raw);  // [3n][NC]
+  const ColourOrder ord = blockIdx.y ? ord1 : ord0;
+  double* M = blockIdx.y ? M1 : M0;
+  float* F = blockIdx.y ? F1 : F0;
+  const int rows = 3 * n, col0 = blockIdx.x * NC;
+  const int oct = threadIdx.x >> 3, g = threadIdx.x & 7;
+  for (int e = threadIdx.x; e < rows * NC; e += BM_THREADS) U[e] = 0.0;
   for (int sw = 0; sw < sweeps; ++sw)
     for (int k = 0; k < 8; ++k) {
-      __syncthreads();
       const int c = ord.at(k);
-      for (int i = L.off[c] + w; i < L.off[c + 1]; i += BM_WAVES) {
+      __syncthreads();
+      for (int i = L.off[c] + oct; i < L.off[c + 1]; i += BM_THREADS / 8) {
+        BndFetch<double> X;
+        bnd_fetch<double>(X, i, true, g, bci, A, nullptr);
+        double a[3][NC];
+#pragma unroll
+        for (int q = 0; q < NC; ++q) a[0][q] = a[1][q] = a[2][q] = 0.0;
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+          const int j = X.j[t];
+          if (j < 0) continue;
+          const double* m = X.m + t * 9;
+          const double* u = U + 3 * j * NC;
+#pragma unroll
+          for (int q = 0; q < NC; ++q) {
+            const double x = u[q], y = u[NC + q], z = u[2 * NC + q];
+            a[0][q] = fmaT(m[0], x, fmaT(m[1], y, fmaT(m[2], z, a[0][q])));
+            a[1][q] = fmaT(m[3], x, fmaT(m[4], y, fmaT(m[5], z, a[1][q])));
+            a[2][q] = fmaT(m[6], x, fmaT(m[7], y, fmaT(m[8], z, a[2][q])));
+          }
+        }
+#pragma unroll
+        for (int v = 0; v < 3; ++v)
+#pragma unroll
+          for (int q = 0; q < NC; ++q) a[v][q] = octet_sum(a[v][q]);
+        if (g != 5) continue;  // spoke 13 = (g 5, t 1): the self block
         const uint8_t fl = flags[list[i]];
-        double* Ui = Mc + (int64_t)(3 * i) * K;
-        if (!live) continue;
-        if (fl & 1) {
-          const double* Ai = A + (size_t)i * 288;
-          const int* Ji = bci + (size_t)i * 32;
-          double a0 = 0, a1 = 0, a2 = 0;
+        double d[6] = {X.m[9], X.m[13], X.m[17], X.m[10], X.m[11], X.m[14]};
+        if (fl & 1) dirichlet_inverse(d, fl);
+        double* u = U + 3 * i * NC;
 #pragma unroll
-          for (int g = 0; g < 8; ++g)
-#pragma unroll
-            for (int t = 0; t < 4; ++t) {
-              const int j = Ji[g * 4 + t];
-              if (j < 0) continue;
-              const double* m = Ai + g * 36 + t * 9;
-              const double* Uj = Mc + (int64_t)(3 * j) * K;
-              const double x = Uj[0], y = Uj[K], z = Uj[2 * K];
-              a0 = fmaT(m[0], x, fmaT(m[1], y, fmaT(m[2], z, a0)));
-              a1 = fmaT(m[3], x, fmaT(m[4], y, fmaT(m[5], z, a1)));
-              a2 = fmaT(m[6], x, fmaT(m[7], y, fmaT(m[8], z, a2)));
-            }
-          // self block: spoke 13 = (g 5, t 1)
-          const double* m = Ai + 5 * 36 + 9;
-          double d[6] = {m[0], m[4], m[8], m[1], m[2], m[5]};
-          dirichlet_inverse(d, fl);
-          const double r0 = (hj == 3 * i ? 1.0 : 0.0) - a0;
-          const double r1 = (hj == 3 * i + 1 ? 1.0 : 0.0) - a1;
-          const double r2 = (hj == 3 * i + 2 ? 1.0 : 0.0) - a2;
-          const double u0 = Ui[0] + d[0] * r0 + d[3] * r1 + d[4] * r2;
-          const double u1 = Ui[K] + d[3] * r0 + d[1] * r1 + d[5] * r2;
-          const double u2 = Ui[2 * K] + d[4] * r0 + d[5] * r1 + d[2] * r2;
-          Ui[0] = (fl & 2) ? 0.0 : u0;
-          Ui[K] = (fl & 4) ? 0.0 : u1;
-          Ui[2 * K] = (fl & 8) ? 0.0 : u2;
-        } else {
-          if (fl & 2) Ui[0] = 0.0;
-          if (fl & 4) Ui[K] = 0.0;
-          if (fl & 8) Ui[2 * K] = 0.0;
+        for (int q = 0; q < NC; ++q) {
+          // the column's unit right-hand side at this node
+          const int h = col0 + q - 3 * i;
+          const double e0 = h == 0 ? 1.0 : 0.0, e1 = h == 1 ? 1.0 : 0.0, e2 = h == 2 ? 1.0 : 0.0;
+          double u0 = u[q], u1 = u[NC + q], u2 = u[2 * NC + q];
+          if (fl & 1) {
+            const double r0 = e0 - a[0][q], r1 = e1 - a[1][q], r2 = e2 - a[2][q];
+            u0 += d[0] * r0 + d[3] * r1 + d[4] * r2;
+            u1 += d[3] * r0 + d[1] * r1 + d[5] * r2;
+            u2 += d[4] * r0 + d[5] * r1 + d[2] * r2;
+          }
+          u[q] = (fl & 2) ? e0 : u0;
+          u[NC + q] = (fl & 4) ? e1 : u1;
+          u[2 * NC + q] = (fl & 8) ? e2 : u2;
         }
       }
     }
+  __syncthreads();
+  const int64_t K = bmap_stride(n);
+  for (int e = threadIdx.x; e < rows * NC; e += BM_THREADS) {
+    const int r = e / NC, col = col0 + e % NC;
+    if (col >= rows) continue;  // the padding columns stay zero
+    M[r * K + col] = U[e];
+    F[r * K + col] = (float)U[e];
+  }
 }
 
-// Dense boundary map apply: x = [u_B; b~] (node-major), y = [G H] x.  Rows
-// are padded to a multiple of 64 entries (zeros), one wavefront per row
-// streams it with 16-byte loads, four in flight per lane, and reduces in a
-// fixed order.
+// Dense boundary map apply: u_B += M x, x the residual of the boundary
+// equations (node-major).  Rows are padded to a multiple of 64 entries
+// (zeros), one wavefront per row streams it with 16-byte loads, four in flight
+// per lane, and reduces in a fixed order.  A Dirichlet row holds a single 1,
+// so its component ends at u - u = 0.  Bound by streaming M from HBM or the
+// memory-side cache.
 template <class T>
 __device__ __forceinline__ T dot4(const typename Vec4<T>::type& a, const typename Vec4<T>::type& b, T acc);
 template <>
@@ -1655,12 +1720,10 @@ template <>
 __device__ __forceinline__ double dot4<double>(const double2& a, const double2& b, double acc) {
   return fma(a.y, b.y, fma(a.x, b.x, acc));
 }
-// y = M x, one wavefront per row; with `list` given, row 3i+c goes straight
-// to u at boundary node list[i], component c
+// row 3i+c belongs to boundary node list[i], component c
 template <class T>
 __global__ void __launch_bounds__(256) k_bmap_gemv(int rows, int Kp, const T* __restrict__ M, const T* __restrict__ x,
-                                                   T* __restrict__ y, const int* __restrict__ list = nullptr,
-                                                   T* __restrict__ u = nullptr) {
+                                                   const int* __restrict__ list, T* __restrict__ u) {
   using V = typename Vec4<T>::type;
   constexpr int PER = 16 / sizeof(T);
   const int r = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
@@ -1682,12 +1745,8 @@ __global__ void __launch_bounds__(256) k_bmap_gemv(int rows, int Kp, const T* __
 #pragma unroll
   for (int o = 32; o >= 1; o >>= 1) acc += __shfl_xor(acc, o);
   if (lane == 0) {
-    if (list) {
-      const int i = r / 3, c = r - 3 * i, node = list[i];
-      u[vidx(node >> 6, c, node & 63)] = acc;
-    } else {
-      y[r] = acc;
-    }
+    const int i = r / 3, c = r - 3 * i, node = list[i];
+    u[vidx(node >> 6, c, node & 63)] += acc;
   }
 }
 // ------------------------------------- level-0 matrix-free boundary phase
@@ -2804,9 +2863,9 @@ static BndLists bnd_lists(const LevelDev& L) {
 // a boundary phase runs in one workgroup while no colour list is longer than this
 static constexpr int kFusedBoundaryMax = 4096;
 // SPG_BOUNDARY_PATH selects the boundary smoother for tests: 0 (default)
-// automatic (level 0: the data-flow phase, else one launch per colour step;
-// explicit levels: the dense map, else the LDS coefficient-row system), 1 the
-// single-workgroup global-memory kernel, 2 one launch per
+// automatic (small sets the dense map, larger ones the data-flow phase; if that
+// is off, level 0 one launch per colour step, explicit levels the LDS
+// coefficient-row system), 1 the single-workgroup global-memory kernel, 2 one launch per
 // colour step, 3 the coefficient-row LDS system also on level 0, 4 the
 // matrix-free single-workgroup level-0 phase, 5 the data-flow level-0 phase
 // (automatic on the explicit levels).
@@ -2936,6 +2995,31 @@ static bool launch_bnd_flow(hipStream_t st, const LevelDev& L, T* u, const T* b,
                hipGetErrorString(e));
   return false;
 }
+template <class T>
+struct BmapPtr;
+template <>
+struct BmapPtr<float> {
+  static const float* M(const LevelDev& L, bool fwd) { return L.bmap32[fwd ? 0 : 1]; }
+  static float* x(const LevelDev& L) { return L.bmx32; }
+};
+template <>
+struct BmapPtr<double> {
+  static const double* M(const LevelDev& L, bool fwd) { return L.bmap64[fwd ? 0 : 1]; }
+  static double* x(const LevelDev& L) { return L.bmx64; }
+};
+// the boundary phase as its dense map; false if the level has none for this
+// precision and sweep count.  Two launches: the residual, then the map with
+// the result added to u.
+template <class T>
+static bool launch_bnd_map(hipStream_t st, const LevelDev& L, T* u, const T* b, int sweeps, bool forward) {
+  const T* M = BmapPtr<T>::M(L, forward);
+  if (!M || sweeps != L.bmap_sweeps) return false;
+  const int n = L.bnd_off[8];
+  T* x = BmapPtr<T>::x(L);  // zero past 3n
+  k_bnd_res<T><<<(n + 31) / 32, 256, 0, st>>>(n, L.bnd, L.ball, BndPtr<T>::A(L), L.flags, u, b, x);
+  k_bmap_gemv<T><<<(3 * n + 3) / 4, 256, 0, st>>>(3 * n, (int)bmap_stride(n), M, x, L.bnd, u);
+  return true;
+}
 void launch_bnd0_setup(hipStream_t st, const LevelDev& L, const int* cslot, const double* E, double dx, double* bE,
                        double* bD) {
   const int n = L.bnd_off[8];
@@ -2945,13 +3029,27 @@ void launch_bnd_coef0(hipStream_t st, const LevelDev& L, const double* E, double
   const int n = L.bnd_off[8];
   if (n > 0) k_bnd_coef0<<<nblk((int64_t)n * 32), TPB, 0, st>>>(n, L.bnd, L.nbr, E, dx, A);
 }
-void launch_bmap_build(hipStream_t st, const LevelDev& L, int sweeps, bool forward, double* M) {
+template <int NC>
+static void launch_bmap_build_nc(hipStream_t st, const LevelDev& L, int sweeps, bool level0, double* const M[2],
+                                 float* const F[2]) {
   const int n = L.bnd_off[8];
-  if (n == 0) return;
   BndOff o;
   for (int c = 0; c < 9; ++c) o.off[c] = L.bnd_off[c];
-  k_bmap_build<<<(6 * n + 63) / 64, 64 * BM_WAVES, 0, st>>>(n, o, colour_order(false, forward), sweeps, L.bnd, L.bci,
-                                                           L.bA64, L.flags, M);
+  (void)hipFuncSetAttribute((const void*)k_bmap_build<NC>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kMaxLds);
+  k_bmap_build<NC><<<dim3((3 * n + NC - 1) / NC, 2), BM_THREADS, (size_t)3 * n * NC * 8, st>>>(
+      n, o, colour_order(level0, true), colour_order(level0, false), sweeps, L.bnd, L.bci, L.bA64, L.flags, M[0], M[1],
+      F[0], F[1]);
+}
+int bmap_max_nodes() { return (int)(kMaxLds / 24); }
+void launch_bmap_build(hipStream_t st, const LevelDev& L, int sweeps, bool level0, double* const M[2],
+                       float* const F[2]) {
+  const int n = L.bnd_off[8];
+  if (n == 0) return;
+  const size_t col = (size_t)3 * n * 8;
+  if (8 * col <= kMaxLds) launch_bmap_build_nc<8>(st, L, sweeps, level0, M, F);
+  else if (4 * col <= kMaxLds) launch_bmap_build_nc<4>(st, L, sweeps, level0, M, F);
+  else if (2 * col <= kMaxLds) launch_bmap_build_nc<2>(st, L, sweeps, level0, M, F);
+  else launch_bmap_build_nc<1>(st, L, sweeps, level0, M, F);
 }
 void launch_bnd_coef_st(hipStream_t st, const LevelDev& L, const double* ST, double* A) {
   const int n = L.bnd_off[8];
@@ -3039,11 +3137,12 @@ void launch_gs0_boundary(hipStream_t st, const LevelDev& L, const T* E, T dx, T*
                          bool forward) {
   if (sweeps <= 0 || L.bnd_off[8] == 0) return;
   int path = boundary_path();
-  // Automatic choice, FP32 per phase of 3 sweeps on the 256^3 shell (3655
+  // Automatic choice beyond the dense map (solver.hip has that line), FP32 per phase of 3 sweeps on the 256^3 shell (3655
   // boundary nodes): data flow 45 us, grid barriers between the steps 87 us,
   // per-colour list launches 145 us, single workgroup 154 us (one CU's VALU
   // work).  The lists remain for a refused cooperative launch and after a
   // time-out.
+  if (path == 0 && launch_bnd_map<T>(st, L, u, b, sweeps, forward)) return;
   if (path == 0 || path == 5) {
     if (launch_bnd_flow<T>(st, L, u, b, sweeps, true, forward, path == 5)) return;
     path = 2;
@@ -3074,34 +3173,12 @@ void launch_st_gs(hipStream_t st, const LevelDev& L, const T* ST, T* u, const T*
   k_st_colour<T, 0><<<nwg, 64 * GS_WAVES, 0, st>>>(L.nb, colour, L.nbr, L.flags, ST, u, b, nullptr);
 }
 template <class T>
-struct BmapPtr;
-template <>
-struct BmapPtr<float> {
-  static const float* M(const LevelDev& L, bool fwd) { return L.bmap32[fwd ? 0 : 1]; }
-  static float* x(const LevelDev& L) { return L.bmx32; }
-};
-template <>
-struct BmapPtr<double> {
-  static const double* M(const LevelDev& L, bool fwd) { return L.bmap64[fwd ? 0 : 1]; }
-  static double* x(const LevelDev& L) { return L.bmx64; }
-};
-template <class T>
 void launch_st_boundary(hipStream_t st, const LevelDev& L, const T* ST, T* u, const T* b, int sweeps, bool forward) {
   if (sweeps <= 0 || L.bnd_off[8] == 0) return;
   const int path = boundary_path() == 5 ? 0 : boundary_path();  // 5 selects a level-0 phase only
-  const T* M = BmapPtr<T>::M(L, forward);
-  if (path == 0 && M && sweeps == L.bmap_sweeps) {
-    const int n = L.bnd_off[8];
-    const int Kp = (int)bmap_stride(n);
-    T* x = BmapPtr<T>::x(L);  // [Kp] input (zero past 6n), then [3n] output behind it
-    T* bt = BndPtr<T>::bt(L);
-    // two launches: b~ and the map input, then the map with the result
-    // written to u (the separate gather / scatter kernels cost two launch
-    // gaps per phase)
-    k_bnd_rhs<T><<<(n + 31) / 32, 256, 0, st>>>(n, L.bnd, L.bslot, BndPtr<T>::A(L), u, b, bt, nullptr, x);
-    k_bmap_gemv<T><<<(3 * n + 3) / 4, 256, 0, st>>>(3 * n, Kp, M, x, x + Kp, L.bnd, u);
-    return;
-  }
+  if (path == 0 && launch_bnd_map<T>(st, L, u, b, sweeps, forward)) return;
+  // sets too large for a dense map: data flow; after a time-out one workgroup
+  if (path == 0 && launch_bnd_flow<T>(st, L, u, b, sweeps, false, forward, false)) return;
   if (path == 0 && launch_bnd_phase<T>(st, L, u, b, sweeps, false, forward)) return;
   const ColourOrder ord = colour_order(false, forward);
   if (path != 2 && L.bnd_max <= kFusedBoundaryMax) {

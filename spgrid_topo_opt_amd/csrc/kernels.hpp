@@ -53,9 +53,10 @@ struct LevelDev {
   void* btag = nullptr;
   unsigned* coop = nullptr;
   int coop_off = 0;  // 1 after a wait timed out: the list launches take over
-  // explicit levels: dense maps [G H] of one boundary phase (forward,
-  // backward colour order) for `bmap_sweeps` sweeps, and their vector
-  // scratch ([6n] input then [3n] output)
+  // slots of all neighbours of the boundary nodes ([n*32], in or outside the
+  // set), and dense maps of one boundary phase (forward, backward colour
+  // order) for `bmap_sweeps` sweeps with their input ([bmap_stride(n)])
+  const int* ball = nullptr;
   const float* bmap32[2] = {nullptr, nullptr};
   const double* bmap64[2] = {nullptr, nullptr};
   float* bmx32 = nullptr;
@@ -190,11 +191,14 @@ void launch_bnd_coef0(hipStream_t st, const LevelDev& L, const double* E, double
 void launch_bnd0_setup(hipStream_t st, const LevelDev& L, const int* cslot, const double* E, double dx, double* bE,
                        double* bD);
 void launch_bnd_coef_st(hipStream_t st, const LevelDev& L, const double* ST, double* A);
-// row stride of the dense boundary map of an n-node boundary set: 6n padded to 64
-__host__ __device__ inline int64_t bmap_stride(int n) { return ((int64_t)6 * n + 63) / 64 * 64; }
-// dense FP64 map [G H] (3n x 6n, row-major, stride bmap_stride(n)) of a boundary
-// phase on an explicit level; the padding columns must hold zeros
-void launch_bmap_build(hipStream_t st, const LevelDev& L, int sweeps, bool forward, double* M);
+// row stride of the dense boundary map of an n-node boundary set: 3n padded to 64
+__host__ __device__ inline int64_t bmap_stride(int n) { return ((int64_t)3 * n + 63) / 64 * 64; }
+// dense maps (3n x 3n, row-major, stride bmap_stride(n)) of a boundary phase,
+// [0] forward and [1] backward, in FP64 and rounded to FP32, for at most
+// bmap_max_nodes() nodes; the padding columns must hold zeros
+int bmap_max_nodes();
+void launch_bmap_build(hipStream_t st, const LevelDev& L, int sweeps, bool level0, double* const M[2],
+                       float* const F[2]);
 // bottom
 void launch_dense_assemble(hipStream_t st, const LevelDev& L, const double* ST, const int* var_of, int64_t n,
                            double* A);

@@ -32,9 +32,13 @@ static double now_s() {
   return std::chrono::duration<double>(std::chrono::steady_clock::now().time_since_epoch()).count();
 }
 
-// boundary phases of explicit levels with at most this many unknowns run as
-// one dense map (2 maps x 3n x 6n entries in FP64 and FP32)
-static constexpr int kMaxDenseBoundary = 6144;
+// Boundary phases over at most this many nodes run as one dense map (2 maps x
+// 3n x 3n entries in FP64 and FP32).  Level-0 phase by map / by data flow, FP32
+// and FP64: 7.6 / 45 and 8.5 / 62 us at 405 nodes, 9.8 / 47 and 17 / 62 at 1425,
+// 18 / 46 and 30 / 61 at 2400, 25 / 46 and 42 / 62 at 3000.  A density update
+// builds both maps: 0.2, 1.0, 1.9 and 5.9 ms, which a solve of 25 V-cycles (4
+// phases each) earns back up to about here.
+static constexpr int kMaxDenseBoundary = 2560;
 // pcg() result: a level-0 boundary phase reported a barrier time-out; the
 // pass is repeated with the per-colour list launches
 static constexpr int kCoopRetry = -100;
@@ -221,11 +225,13 @@ void Solver::upload_layout() {
       R.bt64.alloc(bnd.size() * 4 * 8);
       R.bt32.alloc(bnd.size() * 4 * 4);
       if (l == 0) {
-        R.btag.alloc(bnd.size() * 6 * 8);
         R.coop.alloc(2 * sizeof(unsigned));
         HIPCHK(hipMemset(R.coop.p, 0, 2 * sizeof(unsigned)));
+      }
+      if (l == 0 || bnd.size() > (size_t)kMaxDenseBoundary) {
+        R.btag.alloc(bnd.size() * 6 * 8);
         R.d.btag = R.btag.p;
-        R.d.coop = R.coop.as<unsigned>();
+        R.d.coop = lv_[0].coop.as<unsigned>();  // one error word for every level
       }
     }
     if (!D.bnd_cslot.empty()) {
@@ -491,23 +497,30 @@ void Solver::build_boundary_rows() {
     else if (lay_.lv[l].is_explicit) launch_bnd_coef_st(st_, R.d, R.st64.as<double>(), R.bA64.as<double>());
     else continue;
     launch_cast_d2f(st_, R.bA64.as<double>(), R.bA32.as<float>(), (int64_t)n * 288);
-    // small boundary sets of explicit levels: each phase becomes one dense map
-    if (l > 0 && lay_.lv[l].is_explicit && 3 * n <= kMaxDenseBoundary && cfg_.boundary_iters > 0) {
+    // small boundary sets: each phase becomes one dense map
+    if (n <= kMaxDenseBoundary && cfg_.boundary_iters > 0) {
       const size_t entries = (size_t)3 * n * bmap_stride(n);
-      for (int d = 0; d < 2; ++d) {
+      for (int d = 0; d < 2; ++d)
         if (!R.bmap64[d].p) {
-          // padding columns stay zero: the build writes columns < 6n only
+          // padding columns stay zero: the build writes columns < 3n only
           R.bmap64[d].alloc(entries * 8);
           R.bmap32[d].alloc(entries * 4);
           HIPCHK(hipMemsetAsync(R.bmap64[d].p, 0, entries * 8, st_));
+          HIPCHK(hipMemsetAsync(R.bmap32[d].p, 0, entries * 4, st_));
+          R.d.bmap64[d] = R.bmap64[d].as<double>();
+          R.d.bmap32[d] = R.bmap32[d].as<float>();
         }
-        launch_bmap_build(st_, R.d, cfg_.boundary_iters, d == 0, R.bmap64[d].as<double>());
-        launch_cast_d2f(st_, R.bmap64[d].as<double>(), R.bmap32[d].as<float>(), (int64_t)entries);
-        R.d.bmap64[d] = R.bmap64[d].as<double>();
-        R.d.bmap32[d] = R.bmap32[d].as<float>();
-      }
+      double* const M[2] = {R.bmap64[0].as<double>(), R.bmap64[1].as<double>()};
+      float* const F[2] = {R.bmap32[0].as<float>(), R.bmap32[1].as<float>()};
+      launch_bmap_build(st_, R.d, cfg_.boundary_iters, l == 0, M, F);
       if (!R.bmx64.p) {
-        const size_t nx = (size_t)bmap_stride(n) + 3 * n;
+        const size_t nx = (size_t)bmap_stride(n);
+        const LevelDesc& D = lay_.lv[l];
+        std::vector<int32_t> list, all(D.bnd_ci.size());
+        for (int c = 0; c < 8; ++c) list.insert(list.end(), D.bnd_list[c].begin(), D.bnd_list[c].end());
+        for (size_t e = 0; e < all.size(); ++e) all[e] = D.bnd_ci[e] >= 0 ? list[D.bnd_ci[e]] : D.bnd_slot[e];
+        upload(R.ball, all);
+        R.d.ball = R.ball.as<int>();
         R.bmx64.alloc(nx * 8);
         R.bmx32.alloc(nx * 4);
         HIPCHK(hipMemsetAsync(R.bmx64.p, 0, nx * 8, st_));
@@ -917,7 +930,7 @@ int Solver::pcg(T* x, T* r, double tol, int maxit, int* iters, double* last_nrm)
       // the caller repeat the pass.
       HIPCHK(hipMemsetAsync(lv_[0].coop.as<unsigned>() + 1, 0, sizeof(unsigned), st_));
       sync();
-      lv_[0].d.coop_off = 1;
+      for (LevelRT& R : lv_) R.d.coop_off = 1;
       std::fprintf(stderr,
                    "spgrid_topo_opt_amd: level-0 boundary phase barrier timed out (workgroups not resident "
                    "together); continuing with per-colour launches\n");

@@ -333,6 +333,30 @@ def test_boundary_phase_multi_sweep(blocky, path, monkeypatch):
                 assert rel(got, want) < tol, (lv, fwd, prec)
 
 
+@pytest.mark.parametrize("level,shape", [(0, (12, 8, 8)), (0, (12, 22, 21)), (0, (12, 22, 22)), (2, (24, 92, 92))])
+def test_dense_map_and_data_flow_match_step_by_step(level, shape, monkeypatch):
+    """the automatic boundary phase (level-0 sets of 405 and 2530 nodes: dense
+    map, 2645 nodes and an explicit-level set of 2880: data flow) against the
+    colour steps one after the other, from an iterate that is not zero at the
+    Dirichlet components; FP64 to 1e-11, FP32 to 1e-4 relative (sums of up to
+    7590 products in another order)"""
+    s = _lib.Solver(W.box(*shape, seed=4, mg_levels=4 if level else 3))
+    gx, gf = s.level_nodes(level)
+    rng = np.random.default_rng(31)
+    u = rng.standard_normal((len(gx), 3)) * 1e-3
+    u[(gf & 1) == 0] = 0
+    b = rng.standard_normal((len(gx), 3))
+    for fwd in (True, False):
+        for prec, tol in ((1, 1e-11), (0, 1e-4)):
+            monkeypatch.setenv("SPG_BOUNDARY_PATH", "2" if level == 0 else "1")
+            want = s.kernel(_lib.OP_GS_BOUNDARY, level, u, b, precision=prec, forward=fwd, sweeps=3)
+            monkeypatch.delenv("SPG_BOUNDARY_PATH")
+            got = s.kernel(_lib.OP_GS_BOUNDARY, level, u, b, precision=prec, forward=fwd, sweeps=3)
+            assert rel(got, want) < tol, (fwd, prec)
+            assert np.abs(got - u).max() > 0
+    s.close()
+
+
 @pytest.mark.parametrize("prec,tol", [(1, 1e-13), (0, 1e-6)])
 def test_restriction_and_prolongation(blocky, prec, tol):
     P = blocky
