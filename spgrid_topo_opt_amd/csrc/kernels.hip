@@ -2649,20 +2649,11 @@ __global__ void k_density_update(int64_t n, const int* __restrict__ slot, const 
 
 // -------------------------------------------------------------- sensitivity
 // s_e = a_e^T K0 u_e over the 8 nodes of the cell at this slot
-// (objective/minimal_compliance.cpp:86-146; K0 without dx)
-__global__ void __launch_bounds__(TPB) k_sensitivity(int nb, const int* __restrict__ nbr, const double* __restrict__ rho,
-                                                     const double* __restrict__ u, const double* __restrict__ a,
-                                                     double penalty, double emin, double* __restrict__ dc,
-                                                     double* __restrict__ objcell) {
-  const int gid = blockIdx.x * blockDim.x + threadIdx.x;
-  if (gid >= nb * 64) return;
-  const int blk = gid >> 6, l = gid & 63;
-  const double d = rho[gid];
-  if (!(d > 0.0)) {
-    dc[gid] = 0.0;
-    if (objcell) objcell[gid] = 0.0;
-    return;
-  }
+// (objective/minimal_compliance.cpp:86-146; K0 without dx).  With `part` each
+// workgroup also writes the sum of its cells' objective terms, reduced as a
+// tree in a fixed order; bound by reading u (and a) once through the caches.
+__device__ __forceinline__ double cell_sensitivity(const int* __restrict__ nbr, const double* __restrict__ u,
+                                                   const double* __restrict__ a, int blk, int l) {
   const int li = l >> 4, lj = (l >> 2) & 3, lk = l & 3;
   const Ring R = make_ring(nbr, blk, li, lj, lk);
   double ue[24], ae[24];
@@ -2687,8 +2678,28 @@ __global__ void __launch_bounds__(TPB) k_sensitivity(int nb, const int* __restri
         const int kb = ((I * 8 + J) * 3 + v) * 3;
         s += ae[3 * I + v] * (cK0d[kb] * ue[3 * J] + cK0d[kb + 1] * ue[3 * J + 1] + cK0d[kb + 2] * ue[3 * J + 2]);
       }
-  dc[gid] = -(s * pow(d, penalty - 1.0) * penalty * (1.0 - emin));
-  if (objcell) objcell[gid] = s * (emin + pow(d, penalty) * (1.0 - emin));
+  return s;
+}
+__global__ void __launch_bounds__(TPB) k_sensitivity(int nb, const int* __restrict__ nbr, const double* __restrict__ rho,
+                                                     const double* __restrict__ u, const double* __restrict__ a,
+                                                     double penalty, double emin, double* __restrict__ dc,
+                                                     double* __restrict__ part) {
+  static_assert(TPB == RED_T, "block_reduce sums RED_T threads");
+  const int gid = blockIdx.x * blockDim.x + threadIdx.x;
+  double obj = 0.0;
+  if (gid < nb * 64) {
+    const double d = rho[gid];
+    double g = 0.0;
+    if (d > 0.0) {
+      const double s = cell_sensitivity(nbr, u, a, gid >> 6, gid & 63);
+      g = -(s * pow(d, penalty - 1.0) * penalty * (1.0 - emin));
+      if (part) obj = s * (emin + pow(d, penalty) * (1.0 - emin));
+    }
+    dc[gid] = g;
+  }
+  if (!part) return;
+  obj = block_reduce<0>(obj);
+  if (threadIdx.x == 0) part[blockIdx.x] = obj;
 }
 
 // -------------------------------------------------------- input-order maps
@@ -3325,8 +3336,13 @@ void launch_symv(hipStream_t st, int nT, const T* tiles, const T* x, T* part, T*
   k_symv_reduce<T><<<nblk((int64_t)nT * 64), TPB, 0, st>>>(nT * 64, S, (int64_t)nT * 64, part, y);
 }
 void launch_sensitivity(hipStream_t st, const LevelDev& L, const double* rho, const double* u, const double* a,
-                        double penalty, double emin, double* dc, double* objcell) {
-  k_sensitivity<<<nblk((int64_t)L.nb * 64), TPB, 0, st>>>(L.nb, L.nbr, rho, u, a, penalty, emin, dc, objcell);
+                        double penalty, double emin, double* dc, double* bpart, double* part, double* obj) {
+  const unsigned n = nblk((int64_t)L.nb * 64);
+  k_sensitivity<<<n, TPB, 0, st>>>(L.nb, L.nbr, rho, u, a, penalty, emin, dc, obj ? bpart : nullptr);
+  if (!obj) return;
+  const unsigned g = red_grid(n);
+  k_sum_part<<<g, RED_T, 0, st>>>(bpart, n, part);
+  k_final<0><<<1, RED_T, 0, st>>>(part, (int)g, obj);
 }
 void launch_scatter_input_vec(hipStream_t st, const int* in_slot, int64_t nin, const double* in3, double* v) {
   if (nin > 0) k_scatter_input_vec<<<nblk(nin), TPB, 0, st>>>(in_slot, nin, in3, v);

@@ -222,9 +222,11 @@ void launch_pack_sym_tiles(hipStream_t st, const double* A, int64_t nv, int nT, 
 int symv_splits(int nT);
 template <class T>
 void launch_symv(hipStream_t st, int nT, const T* tiles, const T* x, T* part, T* y);
-// sensitivity: per level-0 slot (cell): dc = -p rho^(p-1)(1-Emin) a_e^T K0 u_e ; obj partials
+// sensitivity: per level-0 slot (cell): dc = -p rho^(p-1)(1-Emin) a_e^T K0 u_e,
+// and with `obj` given *obj = the objective (deterministic sum; `bpart` holds
+// apply_dot_partials(nb) doubles, `part` reduce_partials)
 void launch_sensitivity(hipStream_t st, const LevelDev& L, const double* rho, const double* u, const double* a,
-                        double penalty, double emin, double* dc, double* objcell);
+                        double penalty, double emin, double* dc, double* bpart, double* part, double* obj);
 // gather / scatter between input-block order and level-0 slots
 void launch_scatter_input_vec(hipStream_t st, const int* in_slot, int64_t nin, const double* in3, double* v);
 void launch_gather_input_vec(hipStream_t st, const int* in_slot, int64_t nin, const double* v, double* out3);

@@ -1117,13 +1117,11 @@ int Solver::solve_adjoint(const spg_solve_params& prm, const double* g_in3, doub
   launch_zero<double>(st_, tmp_.as<double>(), n);
   launch_scatter_input_vec(st_, in_slot_.as<int>(), nin, g_in3, tmp_.as<double>());
   launch_project<double>(st_, R0.d, tmp_.as<double>(), true);
-  // lambda with homogeneous Dirichlet data; reuse z64 as its storage
-  launch_zero<double>(st_, z64_.as<double>(), n);
-  DBuf lam;
-  lam.alloc(n * 8);
-  launch_zero<double>(st_, lam.as<double>(), n);
-  const int rc = solve_rhs(prm, lam.as<double>(), tmp_.as<double>(), info, false);
-  launch_gather_input_vec(st_, in_slot_.as<int>(), nin, lam.as<double>(), lam_in3);
+  // lambda with homogeneous Dirichlet data
+  if (!lam_.p) lam_.alloc(n * 8);
+  launch_zero<double>(st_, lam_.as<double>(), n);
+  const int rc = solve_rhs(prm, lam_.as<double>(), tmp_.as<double>(), info, false);
+  launch_gather_input_vec(st_, in_slot_.as<int>(), nin, lam_.as<double>(), lam_in3);
   sync();
   return rc;
 }
@@ -1175,17 +1173,15 @@ void Solver::displacement_in3(double* dev) const {
 double Solver::sensitivity(const double* u_in3_dev, const double* lam_in3_dev, double* dc_in_dev) {
   activate();
   const LevelRT& R0 = lv_[0];
-  const int64_t nslot = (int64_t)R0.d.nb * 64;
   const int64_t nin = lay_.nin_blocks * 64;
-  DBuf dc, obj, uu;
-  dc.alloc(nslot * 8);
-  obj.alloc(nslot * 8);
+  // the FP64 PCG vectors are free between solves: x64 takes the scattered u,
+  // q64 the sensitivities
+  double* dc = q64_.as<double>();
   const double* u = u_.as<double>();
   if (u_in3_dev) {
-    uu.alloc(R0.n3 * 8);
-    launch_zero<double>(st_, uu.as<double>(), R0.n3);
-    launch_scatter_input_vec(st_, in_slot_.as<int>(), nin, u_in3_dev, uu.as<double>());
-    u = uu.as<double>();
+    launch_zero<double>(st_, x64_.as<double>(), R0.n3);
+    launch_scatter_input_vec(st_, in_slot_.as<int>(), nin, u_in3_dev, x64_.as<double>());
+    u = x64_.as<double>();
   }
   const double* a = u;
   if (lam_in3_dev) {
@@ -1193,19 +1189,14 @@ double Solver::sensitivity(const double* u_in3_dev, const double* lam_in3_dev, d
     launch_scatter_input_vec(st_, in_slot_.as<int>(), nin, lam_in3_dev, tmp_.as<double>());
     a = tmp_.as<double>();
   }
-  launch_sensitivity(st_, R0.d, rho_.as<double>(), u, a, cfg_.penalty, cfg_.min_stiffness, dc.as<double>(),
-                     lam_in3_dev ? nullptr : obj.as<double>());
-  launch_gather_input_scalar(st_, in_slot_.as<int>(), nin, dc.as<double>(), dc_in_dev);
-  double objective = 0.0;
-  if (!lam_in3_dev) {
-    // ordered FP64 sum of the per-cell objective terms on the host
-    std::vector<double> h(nslot);
-    HIPCHK(hipMemcpyAsync(h.data(), obj.p, nslot * 8, hipMemcpyDeviceToHost, st_));
-    sync();
-    for (double v : h) objective += v;
-  }
+  double* part = part_.as<double>();
+  double* obj = lam_in3_dev ? nullptr : part + reduce_partials(0);
+  launch_sensitivity(st_, R0.d, rho_.as<double>(), u, a, cfg_.penalty, cfg_.min_stiffness, dc, apart_.as<double>(),
+                     part, obj);
+  launch_gather_input_scalar(st_, in_slot_.as<int>(), nin, dc, dc_in_dev);
+  if (obj) return read_scalar(obj);
   sync();
-  return objective;
+  return 0.0;
 }
 
 // ----------------------------------------------------------- kernel hooks

@@ -160,6 +160,7 @@ class Solver {
   // PCG / outer vectors (level 0)
   DBuf x32_, rr32_, s32_, q32_, z32_, x64_, rr64_, s64_, q64_, z64_;
   DBuf u_, f_, res_, tmp_;
+  DBuf lam_;  // adjoint solution, allocated by the first adjoint solve
   DBuf scal_, part_, pinned_;
   DBuf apart_;  // per-workgroup partials of the fused operator apply + dot
   DBuf fcm_, bcm_;  // level-0 flags and b in colour-major order (either precision)
