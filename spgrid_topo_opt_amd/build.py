@@ -13,7 +13,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 ROOT = os.path.dirname(HERE)
 LIB = os.path.join(HERE, "libspgrid_topo_opt_amd.so")
-SOURCES = ["layout.cpp", "kernels.hip", "solver.hip", "capi.hip", "opt_kernels.hip", "bottom_nd.hip"]
+SOURCES = ["layout.cpp", "kernels.hip", "solver.hip", "capi.hip", "opt_kernels.hip", "bottom_nd.hip", "sweep.hip"]
 ARCH = os.environ.get("SPG_OFFLOAD_ARCH", "gfx950")
 
 
@@ -57,7 +57,7 @@ def build(verbose: bool = False, jobs: int = 4) -> str:
         raise RuntimeError("HIP build failed:\n" + msg)
     tmp = LIB + ".tmp"
     link = [cc, "-shared", f"--offload-arch={ARCH}", "-fPIC", "-o", tmp] + objs + [
-        "-L/opt/rocm/lib", "-lrocsolver", "-lrocblas", "-pthread", "-Wl,-rpath,/opt/rocm/lib"]
+        "-L/opt/rocm/lib", "-lrocblas", "-pthread", "-Wl,-rpath,/opt/rocm/lib"]
     if verbose:
         print(" ".join(link), flush=True)
     r = subprocess.run(link, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)

@@ -13,19 +13,18 @@
 //   symbolic   one front per separator (and per leaf box): its pivots are
 //              eliminated together, its boundary is the set of later nodes
 //              coupled to its subtree (host, once per topology).
-//   numeric    per front, in postorder: assemble the stencil entries and the
-//              children's update matrices, partial Cholesky (rocSOLVER
-//              potrf, rocBLAS trsm and syrk), then the explicit inverse
-//              M = L11^-1 (trtri) and G = L21 M (trmm) for the solve.
-//   solve      forward (deepest fronts first): y_P = M w_P and
-//              u = w_B - G w_P, with w the front's right-hand side plus its
-//              children's update vectors; backward (root first):
-//              x_P = M^T y_P - G^T x_B.  Every step is a GEMV over a stored
-//              row-major copy, one wavefront per row, one launch per tree
-//              depth; sums run in a fixed order, so a solve is deterministic.
+//   numeric    all fronts of a tree depth together, deepest first: the stencil
+//              entries and the children's update matrices in packed 64x64
+//              tiles (pivots padded to whole tiles with ones on the diagonal),
+//              then the block sweep of the pivots (sweep.hip), which leaves
+//              -A11^-1, G = A21 A11^-1 and the update matrix in place.
+//   solve      forward (deepest fronts first): u = w_B - G w_P, with w the
+//              front's right-hand side plus its children's update vectors;
+//              backward (root first): x_P = A11^-1 w_P - G^T x_B.  One launch
+//              per tree depth and direction, a workgroup per tile row; each
+//              gathers the vectors it needs, and sums run in a fixed order, so
+//              a solve is deterministic.
 #include <hip/hip_runtime.h>
-#include <rocblas/rocblas.h>
-#include <rocsolver/rocsolver.h>
 
 #include <algorithm>
 #include <climits>
@@ -51,127 +50,165 @@ constexpr int kLeafNodes = 64;  // a box of at most this many nodes is one front
     hipError_t e_ = (x);                                                                      \
     if (e_ != hipSuccess) throw std::runtime_error(std::string(#x) + ": " + hipGetErrorString(e_)); \
   } while (0)
-#define NDRB(x)                                                                                       \
-  do {                                                                                                \
-    rocblas_status s_ = (x);                                                                          \
-    if (s_ != rocblas_status_success)                                                                 \
-      throw std::runtime_error(std::string(#x) + ": rocblas status " + std::to_string((int)s_));     \
-  } while (0)
 
 // ------------------------------------------------------------------ kernels
-// Stencil entries of one front: entry e = (slot of pivot node i, spoke s,
-// local dof of i, local dof of neighbour j); F(j*, i*) = st(i, s) (the
-// transpose of row i's block, by symmetry), F column-major with leading
-// dimension m.
-__global__ void k_nd_assemble(int n, const int4* __restrict__ ent, const double* __restrict__ ST, int m,
-                              double* __restrict__ F) {
-  const int g = blockIdx.x * blockDim.x + threadIdx.x;
+// a front's local dof (pivots, then boundary) in its padded tile matrix
+__device__ __forceinline__ int padded(int f, int p, int tp) { return f < p ? f : tp * 64 + (f - p); }
+
+// add (or set) an entry of the lower triangle, r >= c; diagonal tiles are whole
+__device__ __forceinline__ void add_entry(double* __restrict__ m, int r, int c, double v) {
+  const int R = r >> 6, C = c >> 6;
+  double* t = m + tile_at(R, C) * 4096;
+  t[(r & 63) * 64 + (c & 63)] += v;
+  if (R == C && r != c) t[(c & 63) * 64 + (r & 63)] += v;
+}
+
+// ones on the diagonal of the padded pivots
+__global__ void k_nd_pad(const NdFrontDev* __restrict__ fr, double* __restrict__ tiles) {
+  const NdFrontDev F = fr[blockIdx.x];
+  const int r = F.p + threadIdx.x;
+  if (r < F.tp * 64) tiles[(F.t_off + tile_at(r >> 6, r >> 6)) * 4096 + (r & 63) * 65] = 1.0;
+}
+
+// Stencil entries of all fronts: entry e = (slot of pivot node i, spoke s,
+// local dof of i, local dof of neighbour j) of front of[e]; F(j*, i*) =
+// st(i, s) (the transpose of row i's block, by symmetry).
+__global__ void k_nd_assemble(int64_t n, const int4* __restrict__ ent, const int* __restrict__ of,
+                              const NdFrontDev* __restrict__ fr, const double* __restrict__ ST,
+                              double* __restrict__ tiles) {
+  const int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (g >= n * 9) return;
   const int4 e = ent[g / 9];
-  const int v = (g % 9) / 3, w = g % 3;
-  const int blk = e.x >> 6, l = e.x & 63;
-  F[(int64_t)(e.w + w) + (int64_t)(e.z + v) * m] = ST[st_index(blk, l, e.y * 9 + v * 3 + w)];
+  const NdFrontDev F = fr[of[g / 9]];
+  const int v = (int)(g % 9) / 3, w = (int)(g % 9) % 3;
+  if (e.w + w < e.z + v) return;  // above the diagonal of a node's own block
+  add_entry(tiles + F.t_off * 4096, padded(e.w + w, F.p, F.tp), e.z + v, ST[st_index(e.x >> 6, e.x & 63, e.y * 9 + v * 3 + w)]);
 }
 
-// F(map[a], map[b]) += U(a, b) over the lower triangle of a child's update
-// matrix U (b x b, column-major)
-__global__ void k_nd_extend_add(int b, const double* __restrict__ U, const int* __restrict__ map, int m,
-                                double* __restrict__ F) {
-  const int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (g >= (int64_t)b * b) return;
-  const int a = (int)(g % b), c = (int)(g / b);
-  if (a < c) return;
-  F[(int64_t)map[a] + (int64_t)map[c] * m] += U[g];
-}
-
-// The solve's copies of one front: MF (m x p, row-major) = [M; G] and
-// MB (p x m, row-major) = [M^T G^T].  M is the lower triangle of F's leading
-// p x p block, G (b x p, column-major) sits in T.
-__global__ void k_nd_pack(int p, int b, int m, const double* __restrict__ F, const double* __restrict__ T,
-                          double* __restrict__ MF, double* __restrict__ MB) {
-  const int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (g >= (int64_t)m * p) return;
-  const int r = (int)(g / p), j = (int)(g % p);  // MF[r][j]
-  double v;
-  if (r < p) v = r >= j ? F[(int64_t)r + (int64_t)j * m] : 0.0;
-  else v = T[(int64_t)(r - p) + (int64_t)j * b];
-  MF[g] = v;
-  MB[(int64_t)j * m + r] = v;
-}
-
-// forward gather: w[f] = (f < p ? b[pos0 + f] : 0) + sum of the children's
-// update entries mapped to f
-__global__ void k_nd_fgather(int n, const int2* __restrict__ item, const NdFrontDev* __restrict__ fr,
-                             const int64_t* __restrict__ gptr, const int64_t* __restrict__ gidx,
-                             const double* __restrict__ b, const double* __restrict__ ustore,
-                             double* __restrict__ w) {
-  const int g = blockIdx.x * blockDim.x + threadIdx.x;
-  if (g >= n) return;
-  const int2 it = item[g];
-  const NdFrontDev F = fr[it.x];
-  const int f = it.y;
-  double v = f < F.p ? b[F.dof0 + f] : 0.0;
-  const int64_t k0 = gptr[F.g_off + f], k1 = gptr[F.g_off + f + 1];
-  for (int64_t k = k0; k < k1; ++k) v += ustore[gidx[k]];
-  w[F.w_off + f] = v;
-}
-
-__device__ __forceinline__ double wave_sum(double s) {
-  for (int o = 32; o > 0; o >>= 1) s += __shfl_down(s, o, 64);
-  return s;
-}
-
-// forward GEMV, one wavefront per row r of a front: rows r < p give
-// y = M w_P (lower triangle), rows r >= p the update u = w_B - G w_P
-__global__ void __launch_bounds__(256) k_nd_fgemv(int n, const int2* __restrict__ item,
-                                                  const NdFrontDev* __restrict__ fr, const double* __restrict__ MF,
-                                                  const double* __restrict__ w, double* __restrict__ y,
-                                                  double* __restrict__ ustore) {
-  const int row = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
-  if (row >= n) return;
-  const int2 it = item[row];
-  const NdFrontDev F = fr[it.x];
-  const int r = it.y;
-  const int len = r < F.p ? r + 1 : F.p;
-  const double* A = MF + F.mf_off + (int64_t)r * F.p;
-  const double* x = w + F.w_off;
-  double s = 0.0;
-  for (int j = lane; j < len; j += 64) s += A[j] * x[j];
-  s = wave_sum(s);
-  if (lane == 0) {
-    if (r < F.p) y[F.dof0 + r] = s;
-    else ustore[F.u_off + (r - F.p)] = x[r] - s;
+// a child's update matrix added to its parent's entries; blockIdx.y: child of
+// the list, blockIdx.x: tile of its update matrix (children of one parent run
+// in separate launches)
+__global__ void __launch_bounds__(256) k_nd_extend_add(const int* __restrict__ child, const NdFrontDev* __restrict__ fr,
+                                                       const int* __restrict__ emap, double* __restrict__ tiles) {
+  const NdFrontDev C = fr[child[blockIdx.y]];
+  const int64_t e = blockIdx.x;
+  if (e >= tile_at(C.tb, 0)) return;
+  int R = (int)((sqrt(8.0 * (double)e + 1.0) - 1.0) * 0.5);
+  while (tile_at(R + 1, 0) <= e) ++R;
+  while (tile_at(R, 0) > e) --R;
+  const int S = (int)(e - tile_at(R, 0));
+  const NdFrontDev P = fr[C.parent];
+  const double* u = tiles + (C.t_off + tile_at(C.tp + R, C.tp + S)) * 4096;
+  const int* map = emap + C.emap_off;
+  double* m = tiles + P.t_off * 4096;
+  for (int q = threadIdx.x; q < 4096; q += 256) {
+    const int a = R * 64 + (q >> 6), c = S * 64 + (q & 63);
+    if (a >= C.b || c > a) continue;
+    add_entry(m, padded(map[a], P.p, P.tp), padded(map[c], P.p, P.tp), u[q]);
   }
 }
 
-// backward gather: v = [y_P; -x_B]
-__global__ void k_nd_bgather(int n, const int2* __restrict__ item, const NdFrontDev* __restrict__ fr,
-                             const int64_t* __restrict__ bidx, const double* __restrict__ y,
-                             const double* __restrict__ x, double* __restrict__ w) {
-  const int g = blockIdx.x * blockDim.x + threadIdx.x;
-  if (g >= n) return;
-  const int2 it = item[g];
+constexpr int kChunk = 1024;  // vector entries staged at a time
+
+// Forward, one workgroup per (front, boundary tile row): the front's
+// right-hand side w_P (its rows of b plus the children's update entries, kept
+// for the backward pass by tile row 0) and u = w_B - G w_P for the tile's rows.
+__global__ void __launch_bounds__(256) k_nd_forward(const int2* __restrict__ item, const NdFrontDev* __restrict__ fr,
+                                                    const int64_t* __restrict__ gptr, const int64_t* __restrict__ gidx,
+                                                    const double* __restrict__ b, const double* __restrict__ tiles,
+                                                    double* __restrict__ w, double* ustore) {
+  __shared__ double xs[kChunk];
+  __shared__ double ys[64];
+  const int2 it = item[blockIdx.x];
   const NdFrontDev F = fr[it.x];
-  const int f = it.y;
-  w[F.w_off + f] = f < F.p ? y[F.dof0 + f] : -x[bidx[F.bidx_off + (f - F.p)]];
+  const int rt = it.y, t = threadIdx.x, wv = t >> 6, lane = t & 63, P = F.tp * 64;
+  auto gathered = [&](int f) {
+    double v = 0.0;
+    const int64_t k0 = gptr[F.g_off + f], k1 = gptr[F.g_off + f + 1];
+    for (int64_t k = k0; k < k1; ++k) v += ustore[gidx[k]];
+    return v;
+  };
+  const bool rows = rt < F.tb;
+  const int r = rt * 64 + t;
+  double wb = 0.0;
+  if (rows && t < 64 && r < F.b) wb = gathered(F.p + r);
+  double acc[16];
+#pragma unroll
+  for (int k = 0; k < 16; ++k) acc[k] = 0.0;
+  for (int c0 = 0; c0 < P; c0 += kChunk) {
+    const int c1 = min(P, c0 + kChunk);
+    __syncthreads();
+    for (int f = c0 + t; f < c1; f += 256) {
+      const double v = f < F.p ? b[F.dof0 + f] + gathered(f) : 0.0;
+      xs[f - c0] = v;
+      if (rt == 0) w[F.w_off + f] = v;
+    }
+    __syncthreads();
+    if (!rows) continue;
+    for (int J = c0 >> 6; J < (c1 >> 6); ++J) {
+      const double* T = tiles + (F.t_off + tile_at(F.tp + rt, J)) * 4096 + wv * 64 + lane;
+      const double xv = xs[J * 64 - c0 + lane];
+#pragma unroll
+      for (int k = 0; k < 16; ++k) acc[k] += T[k * 256] * xv;
+    }
+  }
+  if (!rows) return;
+#pragma unroll
+  for (int k = 0; k < 16; ++k) {
+    double v = acc[k];
+#pragma unroll
+    for (int o = 32; o >= 1; o >>= 1) v += __shfl_xor(v, o);
+    if (lane == 0) ys[wv + 4 * k] = v;
+  }
+  __syncthreads();
+  if (t < 64 && r < F.b) ustore[F.u_off + r] = wb - ys[t];
 }
 
-// backward GEMV, one wavefront per pivot row i: x_i = sum_{j >= i} MB[i][j] v_j
-__global__ void __launch_bounds__(256) k_nd_bgemv(int n, const int2* __restrict__ item,
-                                                  const NdFrontDev* __restrict__ fr, const double* __restrict__ MB,
-                                                  const double* __restrict__ w, double* __restrict__ x) {
-  const int row = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
-  if (row >= n) return;
-  const int2 it = item[row];
+// Backward, one workgroup per (front, pivot tile I): x_I = -((-A11^-1) w_P +
+// G^T x_B) over the tile rows of the front.
+__global__ void __launch_bounds__(256) k_nd_backward(const int2* __restrict__ item, const NdFrontDev* __restrict__ fr,
+                                                     const int64_t* __restrict__ bidx,
+                                                     const double* __restrict__ tiles, const double* __restrict__ w,
+                                                     double* x) {
+  __shared__ double xs[kChunk];
+  __shared__ double ys[64], yt[4][64];
+  const int2 it = item[blockIdx.x];
   const NdFrontDev F = fr[it.x];
-  const int i = it.y;
-  const int m = F.p + F.b;
-  const double* A = MB + F.mb_off + (int64_t)i * m;
-  const double* v = w + F.w_off;
-  double s = 0.0;
-  for (int j = i + lane; j < m; j += 64) s += A[j] * v[j];
-  s = wave_sum(s);
-  if (lane == 0) x[F.dof0 + i] = s;
+  const int I = it.y, t = threadIdx.x, wv = t >> 6, lane = t & 63, P = F.tp * 64, m = P + F.tb * 64;
+  double accN[16], accT = 0.0;
+#pragma unroll
+  for (int k = 0; k < 16; ++k) accN[k] = 0.0;
+  for (int c0 = 0; c0 < m; c0 += kChunk) {
+    const int c1 = min(m, c0 + kChunk);
+    __syncthreads();
+    for (int f = c0 + t; f < c1; f += 256)
+      xs[f - c0] = f < P ? w[F.w_off + f] : (f - P < F.b ? x[bidx[F.bidx_off + (f - P)]] : 0.0);
+    __syncthreads();
+    for (int J = c0 >> 6; J < (c1 >> 6); ++J) {
+      const double* xj = xs + (J * 64 - c0);
+      if (J <= I) {
+        const double* T = tiles + (F.t_off + tile_at(I, J)) * 4096 + wv * 64 + lane;
+        const double xv = xj[lane];
+#pragma unroll
+        for (int k = 0; k < 16; ++k) accN[k] += T[k * 256] * xv;
+      } else {
+        const double* T = tiles + (F.t_off + tile_at(J, I)) * 4096 + wv * 64 + lane;
+#pragma unroll
+        for (int k = 0; k < 16; ++k) accT += T[k * 256] * xj[wv + 4 * k];
+      }
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < 16; ++k) {
+    double v = accN[k];
+#pragma unroll
+    for (int o = 32; o >= 1; o >>= 1) v += __shfl_xor(v, o);
+    if (lane == 0) ys[wv + 4 * k] = v;
+  }
+  yt[wv][lane] = accT;
+  __syncthreads();
+  const int f = I * 64 + t;
+  if (t < 64 && f < F.p) x[F.dof0 + f] = -(ys[t] + ((yt[0][t] + yt[1][t]) + (yt[2][t] + yt[3][t])));
 }
 
 // level vector (T) -> pos-ordered FP64 right-hand side, and back
@@ -340,8 +377,8 @@ NdBottom::NdBottom(int64_t nb, const int32_t* base, const int32_t* nbr, const ui
   };
   // device-side front table, work lists per depth, gather lists, maps
   std::vector<NdFrontDev> fd(fr_.size());
-  int64_t mf = 0, wofs = 0, uofs = 0, bofs = 0, gofs = 0, ustore = 0;
-  size_t maxm2 = 0, maxbp = 0;
+  int64_t toff = 0, wofs = 0, uofs = 0, bofs = 0, gofs = 0;
+  std::vector<int32_t> ent_of;
   std::vector<int64_t> gptr, gidx, bidx;
   std::vector<int32_t> emap;
   for (size_t t = 0; t < fr_.size(); ++t) {
@@ -351,11 +388,13 @@ NdBottom::NdBottom(int64_t nb, const int32_t* base, const int32_t* nbr, const ui
     D.b = 3 * (int)F.bnd.size();
     const int m = D.p + D.b;
     D.dof0 = 3 * F.pos0;
-    D.mf_off = mf;
-    D.mb_off = mf;  // MB has the same size and offsets in its own store
-    mf += (int64_t)m * D.p;
+    D.tp = (D.p + 63) / 64;
+    D.tb = (D.b + 63) / 64;
+    D.parent = F.parent;
+    D.t_off = toff;
+    toff += tile_at(D.tp + D.tb, 0);
     D.w_off = wofs;
-    wofs += m;
+    wofs += D.tp * 64;
     D.u_off = uofs;
     uofs += D.b;
     D.bidx_off = bofs;
@@ -363,16 +402,12 @@ NdBottom::NdBottom(int64_t nb, const int32_t* base, const int32_t* nbr, const ui
       for (int c = 0; c < 3; ++c) bidx.push_back(3 * q + c);
     bofs += D.b;
     D.g_off = gofs;
-    F.ustore_off = ustore;
-    ustore += (int64_t)D.b * D.b;
-    maxm2 = std::max(maxm2, (size_t)m * m);
-    maxbp = std::max(maxbp, (size_t)D.b * D.p);
     // gather lists: children's update entries mapped into this front
     std::vector<std::vector<int64_t>> contrib(m);
     for (int c : F.kids) {
       const Front& C = fr_[c];
       const NdFrontDev& CD = fd[c];
-      fr_[c].emap_off = (int64_t)emap.size();
+      fd[c].emap_off = (int64_t)emap.size();
       for (size_t k = 0; k < C.bnd.size(); ++k) {
         const int lq = local(F, C.bnd[k]);
         if (lq < 0) throw std::runtime_error("nested dissection: a child's boundary node is missing from its parent");
@@ -389,7 +424,6 @@ NdBottom::NdBottom(int64_t nb, const int32_t* base, const int32_t* nbr, const ui
     }
     gofs += m + 1;
     // stencil entries: pivot i, spoke s, neighbour j later in the front
-    F.ent_off = (int64_t)ent_.size();
     for (int64_t k = F.pos0; k < F.pos0 + F.np; ++k) {
       const int32_t i = piv_nodes[k];
       const int li = (int)(k - F.pos0);
@@ -399,38 +433,65 @@ NdBottom::NdBottom(int64_t nb, const int32_t* base, const int32_t* nbr, const ui
         const int lj = local(F, pos[j]);
         if (lj < 0 || lj < li) continue;  // eliminated earlier, or an earlier pivot's entry
         ent_.push_back(make_int4(slot[i], s, 3 * li, 3 * lj));
+        ent_of.push_back((int32_t)t);
       }
     }
-    F.nent = (int64_t)ent_.size() - F.ent_off;
   }
-  mstore_ = mf;
+  ntile_ = toff;
   wlen_ = wofs;
   ulen_ = uofs;
-  ustore_len_ = ustore;
-  maxm2_ = maxm2;
-  maxbp_ = maxbp;
+  ent_of_ = std::move(ent_of);
   fdev_ = std::move(fd);
   gptr_ = std::move(gptr);
   gidx_ = std::move(gidx);
   bidx_ = std::move(bidx);
   emap_ = std::move(emap);
-  // work items per depth: fgather/fgemv/bgather over (front, 0..m), bgemv over (front, 0..p)
-  items_.clear();
-  piv_items_.clear();
-  lvl_off_.assign(maxdepth_ + 2, 0);
-  piv_off_.assign(maxdepth_ + 2, 0);
+  // per depth: the solve's work items (front, boundary tile row; front, pivot
+  // tile), the children to add (first and second ones) and the sweep batch
+  depth_.resize(maxdepth_ + 1);
+  int64_t maxpan = 0, maxid = 0;
   for (int d = 0; d <= maxdepth_; ++d) {
-    lvl_off_[d] = (int64_t)items_.size();
-    piv_off_[d] = (int64_t)piv_items_.size();
+    Depth& D = depth_[d];
+    D.fwd0 = (int64_t)items_.size();
+    for (size_t t = 0; t < fr_.size(); ++t)
+      if (fr_[t].depth == d)
+        for (int r = 0; r < std::max(1, fdev_[t].tb); ++r) items_.push_back(make_int2((int)t, r));
+    D.bwd0 = (int64_t)items_.size();
+    for (size_t t = 0; t < fr_.size(); ++t)
+      if (fr_[t].depth == d)
+        for (int r = 0; r < fdev_[t].tp; ++r) items_.push_back(make_int2((int)t, r));
+    D.end = (int64_t)items_.size();
+    std::vector<SweepMat> mats;
     for (size_t t = 0; t < fr_.size(); ++t) {
       if (fr_[t].depth != d) continue;
-      const int m = fdev_[t].p + fdev_[t].b;
-      for (int f = 0; f < m; ++f) items_.push_back(make_int2((int)t, f));
-      for (int f = 0; f < fdev_[t].p; ++f) piv_items_.push_back(make_int2((int)t, f));
+      mats.push_back(SweepMat{fdev_[t].t_off, fdev_[t].tp, fdev_[t].tp + fdev_[t].tb, 0, (int32_t)t});
+    }
+    std::stable_sort(mats.begin(), mats.end(), [](const SweepMat& a, const SweepMat& b) { return a.np > b.np; });
+    int64_t pan = 0;
+    for (SweepMat& m : mats) {
+      m.pan = (int32_t)pan;
+      pan += m.nt;
+    }
+    maxpan = std::max(maxpan, pan);
+    D.mat0 = (int64_t)mats_.size();
+    mats_.insert(mats_.end(), mats.begin(), mats.end());
+    D.batch.h = std::move(mats);
+    for (int o = 0; o < 2; ++o) {
+      D.kid0[o] = (int64_t)kids_.size();
+      D.kid_tiles[o] = 0;
+      for (size_t t = 0; t < fr_.size(); ++t) {
+        if (fr_[t].depth != d || (int)fr_[t].kids.size() <= o) continue;
+        const int c = fr_[t].kids[o];
+        if (fdev_[c].b == 0) continue;
+        kids_.push_back(c);
+        D.kid_tiles[o] = std::max(D.kid_tiles[o], tile_at(fdev_[c].tb, 0));
+      }
+      D.nkid[o] = (int64_t)kids_.size() - D.kid0[o];
     }
   }
-  lvl_off_[maxdepth_ + 1] = (int64_t)items_.size();
-  piv_off_[maxdepth_ + 1] = (int64_t)piv_items_.size();
+  maxid = (int64_t)fr_.size();
+  npan_ = maxpan;
+  nid_ = maxid;
 }
 
 void NdBottom::upload(hipStream_t st) {
@@ -441,104 +502,88 @@ void NdBottom::upload(hipStream_t st) {
   upload_vec(d_emap_, emap_, st);
   upload_vec(d_ent_, ent_, st);
   upload_vec(d_items_, items_, st);
-  upload_vec(d_piv_items_, piv_items_, st);
+  upload_vec(d_ent_of_, ent_of_, st);
+  upload_vec(d_mats_, mats_, st);
+  upload_vec(d_kids_, kids_, st);
   upload_vec(d_var_of_, var_of_, st);
-  mfs_.alloc((size_t)mstore_ * 8);
-  mbs_.alloc((size_t)mstore_ * 8);
+  const size_t tile = 4096 * 8;
+  tiles_.alloc((size_t)std::max<int64_t>(ntile_, 1) * tile);
+  panw_.alloc((size_t)std::max<int64_t>(npan_, 1) * tile);
+  panx_.alloc((size_t)std::max<int64_t>(npan_, 1) * tile);
+  dinv_.alloc((size_t)std::max<int64_t>(nid_, 1) * tile);
+  info_.alloc((size_t)std::max<int64_t>(nid_, 1) * sizeof(int));
+  for (Depth& D : depth_) {
+    D.batch.d = static_cast<SweepMat*>(d_mats_.p) + D.mat0;
+    D.batch.panw = static_cast<double*>(panw_.p);
+    D.batch.panx = static_cast<double*>(panx_.p);
+    D.batch.dinv = static_cast<double*>(dinv_.p);
+    D.batch.info = static_cast<int*>(info_.p);
+  }
   w_.alloc((size_t)std::max<int64_t>(wlen_, 1) * 8);
   u_.alloc((size_t)std::max<int64_t>(ulen_, 1) * 8);
   bx_.alloc((size_t)std::max<int64_t>(ndof_, 1) * 8);
-  y_.alloc((size_t)std::max<int64_t>(ndof_, 1) * 8);
   x_.alloc((size_t)std::max<int64_t>(ndof_, 1) * 8);
   NDCHK(hipStreamSynchronize(st));
 }
 
 size_t NdBottom::device_bytes() const {
   size_t s = 0;
-  for (const DevMem* d : {&d_fr_, &d_gptr_, &d_gidx_, &d_bidx_, &d_emap_, &d_ent_, &d_items_, &d_piv_items_,
-                          &d_var_of_, &mfs_, &mbs_, &w_, &u_, &bx_, &y_, &x_})
+  for (const DevMem* d : {&d_fr_, &d_gptr_, &d_gidx_, &d_bidx_, &d_emap_, &d_ent_, &d_ent_of_, &d_items_, &d_mats_,
+                          &d_kids_, &d_var_of_, &tiles_, &panw_, &panx_, &dinv_, &info_, &w_, &u_, &bx_, &x_})
     s += d->bytes;
   return s;
 }
 
 // ------------------------------------------------------------------ numeric
-void NdBottom::factor(const double* ST, hipStream_t st, rocblas_handle rb) {
-  DevMem F, T, U, info;
-  F.alloc(std::max<size_t>(maxm2_, 1) * 8);
-  T.alloc(std::max<size_t>(maxbp_, 1) * 8);
-  U.alloc((size_t)std::max<int64_t>(ustore_len_, 1) * 8);
-  info.alloc(2 * std::max<size_t>(fr_.size(), 1) * sizeof(rocblas_int));
-  NDCHK(hipMemsetAsync(info.p, 0, info.bytes, st));
-  double* Fp = static_cast<double*>(F.p);
-  double* Tp = static_cast<double*>(T.p);
-  double* Up = static_cast<double*>(U.p);
-  rocblas_int* ip = static_cast<rocblas_int*>(info.p);
-  const double one = 1.0, mone = -1.0;
-  for (size_t t = 0; t < fr_.size(); ++t) {
-    const Front& Fr = fr_[t];
-    const NdFrontDev& D = fdev_[t];
-    const int p = D.p, b = D.b, m = p + b;
-    NDCHK(hipMemsetAsync(Fp, 0, (size_t)m * m * 8, st));
-    if (Fr.nent > 0)
-      k_nd_assemble<<<grid(Fr.nent * 9), 256, 0, st>>>((int)Fr.nent, static_cast<const int4*>(d_ent_.p) + Fr.ent_off,
-                                                      ST, m, Fp);
-    for (int c : Fr.kids) {
-      const int bc = fdev_[c].b;
-      if (bc == 0) continue;
-      k_nd_extend_add<<<grid((int64_t)bc * bc), 256, 0, st>>>(bc, Up + fr_[c].ustore_off,
-                                                              static_cast<const int*>(d_emap_.p) + fr_[c].emap_off, m,
-                                                              Fp);
-    }
-    NDRB(rocsolver_dpotrf(rb, rocblas_fill_lower, p, Fp, m, ip + 2 * t));
-    if (b > 0) {
-      NDRB(rocblas_dtrsm(rb, rocblas_side_right, rocblas_fill_lower, rocblas_operation_transpose,
-                         rocblas_diagonal_non_unit, b, p, &one, Fp, m, Fp + p, m));
-      NDRB(rocblas_dsyrk(rb, rocblas_fill_lower, rocblas_operation_none, b, p, &mone, Fp + p, m, &one,
-                         Fp + p + (int64_t)p * m, m));
-      NDCHK(hipMemcpy2DAsync(Up + Fr.ustore_off, (size_t)b * 8, Fp + p + (int64_t)p * m, (size_t)m * 8,
-                             (size_t)b * 8, b, hipMemcpyDeviceToDevice, st));
-    }
-    NDRB(rocsolver_dtrtri(rb, rocblas_fill_lower, rocblas_diagonal_non_unit, p, Fp, m, ip + 2 * t + 1));
-    if (b > 0)
-      NDRB(rocblas_dtrmm(rb, rocblas_side_right, rocblas_fill_lower, rocblas_operation_none,
-                         rocblas_diagonal_non_unit, b, p, &one, Fp, m, Fp + p, m, Tp, b));
-    k_nd_pack<<<grid((int64_t)m * p), 256, 0, st>>>(p, b, m, Fp, Tp, static_cast<double*>(mfs_.p) + D.mf_off,
-                                                    static_cast<double*>(mbs_.p) + D.mb_off);
+void NdBottom::factor(const double* ST, hipStream_t st) {
+  if (fr_.empty()) return;
+  const NdFrontDev* fr = static_cast<const NdFrontDev*>(d_fr_.p);
+  double* tiles = static_cast<double*>(tiles_.p);
+  NDCHK(hipMemsetAsync(tiles_.p, 0, tiles_.bytes, st));
+  NDCHK(hipMemsetAsync(info_.p, 0, info_.bytes, st));
+  k_nd_pad<<<(unsigned)fr_.size(), 64, 0, st>>>(fr, tiles);
+  const int64_t n = (int64_t)ent_.size();
+  if (n > 0)
+    k_nd_assemble<<<grid(n * 9), 256, 0, st>>>(n, static_cast<const int4*>(d_ent_.p),
+                                               static_cast<const int*>(d_ent_of_.p), fr, ST, tiles);
+  for (int d = maxdepth_; d >= 0; --d) {
+    const Depth& D = depth_[d];
+    for (int o = 0; o < 2; ++o)
+      for (int64_t k = 0; k < D.nkid[o]; k += 32768)
+        k_nd_extend_add<<<dim3((unsigned)D.kid_tiles[o], (unsigned)std::min<int64_t>(32768, D.nkid[o] - k)), 256, 0,
+                          st>>>(static_cast<const int*>(d_kids_.p) + D.kid0[o] + k, fr,
+                                static_cast<const int*>(d_emap_.p), tiles);
+    sweep_run(st, D.batch, tiles);
   }
-  std::vector<rocblas_int> h(2 * fr_.size());
-  if (!h.empty())
-    NDCHK(hipMemcpyAsync(h.data(), info.p, h.size() * sizeof(rocblas_int), hipMemcpyDeviceToHost, st));
+  std::vector<int> h(fr_.size());
+  NDCHK(hipMemcpyAsync(h.data(), info_.p, h.size() * sizeof(int), hipMemcpyDeviceToHost, st));
   NDCHK(hipStreamSynchronize(st));
   for (size_t t = 0; t < fr_.size(); ++t)
-    if (h[2 * t] != 0 || h[2 * t + 1] != 0)
-      throw NdNotSpd("bottom Cholesky failed: front " + std::to_string(t) + " (" +
-                     std::to_string(fdev_[t].p) + " pivots) is not positive definite at its pivot " +
-                     std::to_string(h[2 * t] ? h[2 * t] : h[2 * t + 1]));
+    if (h[t] != 0)
+      throw NdNotSpd("bottom Cholesky failed: front " + std::to_string(t) + " (" + std::to_string(fdev_[t].p) +
+                     " pivots) is not positive definite at its pivot " + std::to_string(h[t]));
 }
 
 // ------------------------------------------------------------------ solve
 void NdBottom::solve_pos(hipStream_t st) {
   const NdFrontDev* fr = static_cast<const NdFrontDev*>(d_fr_.p);
   const int2* items = static_cast<const int2*>(d_items_.p);
-  const int2* pit = static_cast<const int2*>(d_piv_items_.p);
+  const double* tiles = static_cast<const double*>(tiles_.p);
   double* w = static_cast<double*>(w_.p);
   double* u = static_cast<double*>(u_.p);
-  double* y = static_cast<double*>(y_.p);
   double* x = static_cast<double*>(x_.p);
-  const double* b = static_cast<const double*>(bx_.p);
   for (int d = maxdepth_; d >= 0; --d) {
-    const int64_t o = lvl_off_[d], n = lvl_off_[d + 1] - o;
-    if (n == 0) continue;
-    k_nd_fgather<<<grid(n), 256, 0, st>>>((int)n, items + o, fr, static_cast<const int64_t*>(d_gptr_.p),
-                                          static_cast<const int64_t*>(d_gidx_.p), b, u, w);
-    k_nd_fgemv<<<grid(n, 4), 256, 0, st>>>((int)n, items + o, fr, static_cast<const double*>(mfs_.p), w, y, u);
+    const Depth& D = depth_[d];
+    if (D.bwd0 > D.fwd0)
+      k_nd_forward<<<(unsigned)(D.bwd0 - D.fwd0), 256, 0, st>>>(
+          items + D.fwd0, fr, static_cast<const int64_t*>(d_gptr_.p), static_cast<const int64_t*>(d_gidx_.p),
+          static_cast<const double*>(bx_.p), tiles, w, u);
   }
-  for (int d = 0; d <= maxdepth_; ++d) {
-    const int64_t o = lvl_off_[d], n = lvl_off_[d + 1] - o;
-    const int64_t po = piv_off_[d], pn = piv_off_[d + 1] - po;
-    if (n == 0) continue;
-    k_nd_bgather<<<grid(n), 256, 0, st>>>((int)n, items + o, fr, static_cast<const int64_t*>(d_bidx_.p), y, x, w);
-    k_nd_bgemv<<<grid(pn, 4), 256, 0, st>>>((int)pn, pit + po, fr, static_cast<const double*>(mbs_.p), w, x);
+  for (int d = 0; d <= maxdepth_ && !fr_.empty(); ++d) {
+    const Depth& D = depth_[d];
+    if (D.end > D.bwd0)
+      k_nd_backward<<<(unsigned)(D.end - D.bwd0), 256, 0, st>>>(items + D.bwd0, fr,
+                                                                static_cast<const int64_t*>(d_bidx_.p), tiles, w, x);
   }
 }
 
@@ -557,7 +602,7 @@ NdStats NdBottom::stats() const {
   NdStats s;
   s.fronts = (int64_t)fr_.size();
   s.depth = maxdepth_ + 1;
-  s.factor_entries = mstore_;
+  s.factor_entries = ntile_ * 4096;
   for (const NdFrontDev& D : fdev_) s.max_front = std::max<int64_t>(s.max_front, D.p + D.b);
   return s;
 }

@@ -2,13 +2,14 @@
 // multifrontal Cholesky factorization on the GPU (see bottom_nd.hip).
 #pragma once
 #include <hip/hip_runtime.h>
-#include <rocblas/rocblas.h>
 
 #include <cstdint>
 #include <functional>
 #include <stdexcept>
 #include <string>
 #include <vector>
+
+#include "sweep.hpp"
 
 namespace spg {
 
@@ -31,13 +32,15 @@ struct DevMem {
 // one front as the solve kernels see it; dofs are in elimination order
 struct NdFrontDev {
   int64_t dof0;      // first pivot dof (the pivots are dof0 .. dof0 + p - 1)
-  int64_t mf_off;    // [M; G], m x p row-major, in the forward store
-  int64_t mb_off;    // [M^T G^T], p x m row-major, in the backward store
-  int64_t w_off;     // m entries of solve workspace
+  int64_t t_off;     // first tile of its packed matrix (tp + tb tile rows)
+  int64_t w_off;     // 64 tp entries of solve workspace
   int64_t u_off;     // b entries: this front's forward update vector
   int64_t bidx_off;  // b entries: dof index of each boundary dof
   int64_t g_off;     // m + 1 entries of the gather list's row pointer
+  int64_t emap_off;  // b entries: local dof in the parent of each boundary dof
   int32_t p, b;      // pivot and boundary dofs
+  int32_t tp, tb;    // the same in tiles of 64
+  int32_t parent;    // -1 at the root
 };
 
 struct NdStats {
@@ -53,7 +56,7 @@ class NdBottom {
   void upload(hipStream_t st);
   // numeric factorization from the level's FP64 stencils (st_index layout);
   // throws NdNotSpd for a front that is not positive definite
-  void factor(const double* ST, hipStream_t st, rocblas_handle rb);
+  void factor(const double* ST, hipStream_t st);
   // u = A^-1 b on the level's vectors (inactive nodes: u = b), FP64 inside
   template <class T>
   void solve(int nb, const T* b, T* u, hipStream_t st);
@@ -68,7 +71,6 @@ class NdBottom {
     int depth = 0, parent = -1;
     std::vector<int> kids;
     std::vector<int64_t> bnd;  // positions of the boundary nodes, ascending
-    int64_t ustore_off = 0, emap_off = 0, ent_off = 0, nent = 0;
   };
   void solve_pos(hipStream_t st);
 
@@ -80,12 +82,20 @@ class NdBottom {
   std::vector<int64_t> gptr_, gidx_, bidx_;
   std::vector<int32_t> emap_;
   std::vector<int4> ent_;
-  std::vector<int2> items_, piv_items_;
-  std::vector<int64_t> lvl_off_, piv_off_;
-  int64_t mstore_ = 0, wlen_ = 0, ulen_ = 0, ustore_len_ = 0;
-  size_t maxm2_ = 0, maxbp_ = 0;
-  DevMem d_fr_, d_gptr_, d_gidx_, d_bidx_, d_emap_, d_ent_, d_items_, d_piv_items_, d_var_of_;
-  DevMem mfs_, mbs_, w_, u_, bx_, y_, x_;
+  std::vector<int2> items_;
+  std::vector<int32_t> ent_of_, kids_;
+  std::vector<SweepMat> mats_;
+  // one tree depth: ranges of items_ (forward, backward), of kids_ (first and
+  // second children) and of mats_, and its sweep batch
+  struct Depth {
+    int64_t fwd0 = 0, bwd0 = 0, end = 0, mat0 = 0;
+    int64_t kid0[2] = {0, 0}, nkid[2] = {0, 0}, kid_tiles[2] = {0, 0};
+    SweepBatch batch;
+  };
+  std::vector<Depth> depth_;
+  int64_t ntile_ = 0, npan_ = 0, nid_ = 0, wlen_ = 0, ulen_ = 0;
+  DevMem d_fr_, d_gptr_, d_gidx_, d_bidx_, d_emap_, d_ent_, d_ent_of_, d_items_, d_mats_, d_kids_, d_var_of_;
+  DevMem tiles_, panw_, panx_, dinv_, info_, w_, u_, bx_, x_;
 };
 
 }  // namespace spg

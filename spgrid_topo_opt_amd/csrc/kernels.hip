@@ -12,6 +12,7 @@
 #include <cstdlib>
 
 #include "kernels.hpp"
+#include "sweep.hpp"
 
 namespace spg {
 
@@ -2501,10 +2502,14 @@ __global__ void __launch_bounds__(TPB) k_galerkin_assemble(int nb, const int* __
 }
 
 // ------------------------------------------------------------------- bottom
-__global__ void k_dense_assemble(int nb, const int* __restrict__ nbr, const uint8_t* __restrict__ flags,
-                                 const double* __restrict__ ST, const int* __restrict__ var_of, int64_t n,
-                                 double* __restrict__ A) {
+__global__ void k_tile_assemble(int nb, const int* __restrict__ nbr, const uint8_t* __restrict__ flags,
+                                const double* __restrict__ ST, const int* __restrict__ var_of, int64_t n, int nT,
+                                double* __restrict__ tiles) {
   const int gid = blockIdx.x * blockDim.x + threadIdx.x;
+  if (gid < nT * 64 - n) {  // identity in the padding
+    const int64_t r = n + gid;
+    tiles[tile_at((int)(r >> 6), (int)(r >> 6)) * 4096 + (r & 63) * 65] = 1.0;
+  }
   if (gid >= nb * 64) return;
   const int blk = gid >> 6, l = gid & 63;
   const int vi = var_of[gid];
@@ -2518,18 +2523,19 @@ __global__ void k_dense_assemble(int nb, const int* __restrict__ nbr, const uint
     const int vj = var_of[bb * 64 + loc3(a, b, c)];
     if (vj < 0) continue;
     for (int v = 0; v < 3; ++v)
-      for (int w = 0; w < 3; ++w) A[(int64_t)(vi + v) + (int64_t)(vj + w) * n] = ST[st_index(blk, l, s * 9 + v * 3 + w)];
+      for (int w = 0; w < 3; ++w) {
+        const int r = vi + v, q = vj + w;
+        if ((r >> 6) >= (q >> 6))
+          tiles[tile_at(r >> 6, q >> 6) * 4096 + (r & 63) * 64 + (q & 63)] = ST[st_index(blk, l, s * 9 + v * 3 + w)];
+      }
   }
 }
-__global__ void k_symmetrize_lower(double* A, int64_t n) {
-  const int64_t gid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (gid >= n * n) return;
-  const int64_t i = gid % n, j = gid / n;  // A[i + j n]
-  if (i < j) A[i + j * n] = A[j + i * n];
-}
-__global__ void k_set_diagonal(double* A, int64_t n, double v) {
+__global__ void k_tile_negate(double* __restrict__ a, float* __restrict__ b, int64_t n) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) A[i + i * n] = v;
+  if (i >= n) return;
+  const double v = -a[i];
+  a[i] = v;
+  b[i] = (float)v;
 }
 template <class T>
 __global__ void k_bottom_gather(int nb, const int* __restrict__ var_of, const T* __restrict__ b, T* x) {
@@ -2547,23 +2553,6 @@ __global__ void k_bottom_scatter(int nb, const int* __restrict__ var_of, const T
   const int vi = var_of[gid];
   const int blk = gid >> 6, l = gid & 63;
   for (int c = 0; c < 3; ++c) u[vidx(blk, c, l)] = vi >= 0 ? y[vi + c] : b[vidx(blk, c, l)];
-}
-
-// The symmetric bottom inverse kept as its lower triangle in 64x64 tiles:
-// tile (I, J), I >= J, at index I(I+1)/2 + J, row-major, zero padded.
-template <class T>
-__global__ void k_pack_sym_tiles(const double* __restrict__ A, int64_t nv, int nT, T* __restrict__ tiles) {
-  const int64_t gid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const int64_t ntile = (int64_t)nT * (nT + 1) / 2;
-  if (gid >= ntile * 4096) return;
-  const int64_t tile = gid >> 12;
-  const int e = (int)(gid & 4095);
-  int I = (int)((sqrt(8.0 * (double)tile + 1.0) - 1.0) * 0.5);
-  while ((int64_t)(I + 1) * (I + 2) / 2 <= tile) ++I;
-  while ((int64_t)I * (I + 1) / 2 > tile) --I;
-  const int J = (int)(tile - (int64_t)I * (I + 1) / 2);
-  const int64_t row = (int64_t)I * 64 + (e >> 6), col = (int64_t)J * 64 + (e & 63);
-  tiles[gid] = (row < nv && col < nv) ? (T)A[row + col * nv] : T(0);
 }
 
 // y = A x with the packed tiles.  Workgroup (I, s) takes the tile columns
@@ -3285,9 +3274,14 @@ void launch_galerkin_assemble(hipStream_t st, const LevelDev& L, const int* cell
   k_galerkin_assemble<<<nblk((int64_t)L.nb * 64), TPB, 0, st>>>(L.nb, L.nbr, L.flags, cell_row, Cm, dx, ST);
 }
 void launch_stencil_to_float(hipStream_t st, const double* a, float* b, int64_t n) { launch_cast_d2f(st, a, b, n); }
-void launch_dense_assemble(hipStream_t st, const LevelDev& L, const double* ST, const int* var_of, int64_t n,
-                           double* A) {
-  k_dense_assemble<<<nblk((int64_t)L.nb * 64), TPB, 0, st>>>(L.nb, L.nbr, L.flags, ST, var_of, n, A);
+void launch_tile_assemble(hipStream_t st, const LevelDev& L, const double* ST, const int* var_of, int64_t n, int nT,
+                          double* tiles) {
+  // the first threads also write the padding: at least 64 of them
+  k_tile_assemble<<<nblk(std::max<int64_t>((int64_t)L.nb * 64, 64)), TPB, 0, st>>>(L.nb, L.nbr, L.flags, ST, var_of, n,
+                                                                                  nT, tiles);
+}
+void launch_tile_negate(hipStream_t st, double* a, float* b, int64_t n) {
+  if (n > 0) k_tile_negate<<<nblk(n), TPB, 0, st>>>(a, b, n);
 }
 void launch_list_nslot(hipStream_t st, const LevelDev& L, int n, const int* list, int* out) {
   if (n > 0) k_bnd_nslot<<<nblk((int64_t)n * 27), TPB, 0, st>>>(n, list, L.nbr, out);
@@ -3309,12 +3303,6 @@ void launch_density_update(hipStream_t st, int64_t n, const int* slot, const dou
                            double emin, double rmin, double* E64, float* E32, double* rho) {
   if (n > 0) k_density_update<<<nblk(n), TPB, 0, st>>>(n, slot, dens, penalty, emin, rmin, E64, E32, rho);
 }
-void launch_set_diagonal(hipStream_t st, double* A, int64_t n, double v) {
-  k_set_diagonal<<<nblk(n), TPB, 0, st>>>(A, n, v);
-}
-void launch_symmetrize_lower(hipStream_t st, double* A, int64_t n) {
-  k_symmetrize_lower<<<nblk(n * n), TPB, 0, st>>>(A, n);
-}
 template <class T>
 void launch_bottom_gather(hipStream_t st, const LevelDev& L, const int* var_of, const T* b, T* x) {
   k_bottom_gather<T><<<nblk((int64_t)L.nb * 64), TPB, 0, st>>>(L.nb, var_of, b, x);
@@ -3322,11 +3310,6 @@ void launch_bottom_gather(hipStream_t st, const LevelDev& L, const int* var_of, 
 template <class T>
 void launch_bottom_scatter(hipStream_t st, const LevelDev& L, const int* var_of, const T* y, const T* b, T* u) {
   k_bottom_scatter<T><<<nblk((int64_t)L.nb * 64), TPB, 0, st>>>(L.nb, var_of, y, b, u);
-}
-template <class T>
-void launch_pack_sym_tiles(hipStream_t st, const double* A, int64_t nv, int nT, T* tiles) {
-  const int64_t n = (int64_t)nT * (nT + 1) / 2 * 4096;
-  k_pack_sym_tiles<T><<<nblk(n), TPB, 0, st>>>(A, nv, nT, tiles);
 }
 int symv_splits(int nT) { return std::max(1, std::min(nT, 2048 / std::max(nT, 1))); }
 template <class T>
@@ -3388,7 +3371,6 @@ void launch_set_entries(hipStream_t st, double* v, const int* idx, const double*
                                       int);                                                                     \
   template void launch_bottom_gather<T>(hipStream_t, const LevelDev&, const int*, const T*, T*);                 \
   template void launch_bottom_scatter<T>(hipStream_t, const LevelDev&, const int*, const T*, const T*, T*);      \
-  template void launch_pack_sym_tiles<T>(hipStream_t, const double*, int64_t, int, T*);                          \
   template void launch_symv<T>(hipStream_t, int, const T*, const T*, T*, T*);
 SPG_INST(float)
 SPG_INST(double)

@@ -200,10 +200,12 @@ int bmap_max_nodes();
 void launch_bmap_build(hipStream_t st, const LevelDev& L, int sweeps, bool level0, double* const M[2],
                        float* const F[2]);
 // bottom
-void launch_dense_assemble(hipStream_t st, const LevelDev& L, const double* ST, const int* var_of, int64_t n,
-                           double* A);
-void launch_symmetrize_lower(hipStream_t st, double* A, int64_t n);
-void launch_set_diagonal(hipStream_t st, double* A, int64_t n, double v);  // A[i + i n] = v
+// the bottom matrix (n unknowns) in packed lower-triangle 64x64 tiles (nT tile
+// rows, cleared by the caller), identity in the padding; and afterwards
+// a = -a with a rounded FP32 copy
+void launch_tile_assemble(hipStream_t st, const LevelDev& L, const double* ST, const int* var_of, int64_t n, int nT,
+                          double* tiles);
+void launch_tile_negate(hipStream_t st, double* a, float* b, int64_t n);
 void launch_bnd_nslot(hipStream_t st, const LevelDev& L, int* out);  // fills LevelDev::bnslot
 // density update on the device: err |= 1 NaN, 2 deactivation, 4 activation
 void launch_density_check(hipStream_t st, int64_t n, const int* slot, const double* dens, const double* E64,
@@ -214,11 +216,8 @@ template <class T>
 void launch_bottom_gather(hipStream_t st, const LevelDev& L, const int* var_of, const T* b, T* x);
 template <class T>
 void launch_bottom_scatter(hipStream_t st, const LevelDev& L, const int* var_of, const T* y, const T* b, T* u);
-// symmetric matrix in packed lower-triangle 64x64 tiles: pack from a dense
-// column-major FP64 matrix, and y = A x (x, y padded to nT*64; part holds
-// symv_splits(nT) * nT * 64 partial sums)
-template <class T>
-void launch_pack_sym_tiles(hipStream_t st, const double* A, int64_t nv, int nT, T* tiles);
+// symmetric matrix in packed lower-triangle 64x64 tiles: y = A x (x, y padded
+// to nT*64; part holds symv_splits(nT) * nT * 64 partial sums)
 int symv_splits(int nT);
 template <class T>
 void launch_symv(hipStream_t st, int nT, const T* tiles, const T* x, T* part, T* y);

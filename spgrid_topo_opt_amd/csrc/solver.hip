@@ -1,7 +1,6 @@
 // solver.hip -- see solver.hpp.
 #include <hip/hip_runtime.h>
 #include <rocblas/rocblas.h>
-#include <rocsolver/rocsolver.h>
 
 #include <algorithm>
 #include <chrono>
@@ -50,11 +49,11 @@ static constexpr double kFp32PassReduction = 1e-6;
 // bandwidth-bound GEMV per V-cycle), the nested-dissection Cholesky
 // (bottom_nd.hip) above it, unless spg_config.bottom_dense_max sets another
 // limit; SPG_BOTTOM=dense|nd overrides both (dense stays limited to
-// kMaxDenseBottomDofs: its inverse is O(n^2)).  Per density update the
-// dense inverse costs 7, 22, 70 and 192 ms at 1.9 K, 4.6 K, 9 K and 15 K
-// unknowns, the nested dissection 8, 19, 37 and 62 ms, which then costs
-// about 0.08 ms more per V-cycle at 9 K: the dense inverse pays when many
-// solves share a factorization.
+// kMaxDenseBottomDofs: its inverse is O(n^2)).  A whole density update takes 5.5
+// / 112 / 552 ms with the dense inverse and 1.4 / 3.0 / 4.2 ms with the nested
+// dissection at 4.1 K / 12.7 K / 21.9 K unknowns; the bottom solve of an FP32
+// V-cycle 31 / 107 / 297 us against 89 / 164 / 216 us: the dense inverse pays
+// when many solves share a factorization.
 static constexpr int64_t kDenseBottomDofs = 16384;
 static constexpr int64_t kMaxDenseBottomDofs = 60000;
 
@@ -384,7 +383,7 @@ void Solver::build_operators() {
   mark("Galerkin levels");
   build_boundary_rows();
   mark("boundary rows");
-  // bottom: FP64 Cholesky of the Dirichlet-deleted stencil matrix, then its inverse
+  // bottom: FP64 inverse or factorization of the Dirichlet-deleted stencil matrix
   // (Multigrid_Hierarchy.h:332-341; Elasticity_Matrix.cpp:15-233 factorizes with PARDISO)
   const int B = L - 1;
   const LevelDesc& D = lay_.lv[B];
@@ -413,7 +412,7 @@ void Solver::build_operators() {
         nd_ = std::make_unique<NdBottom>(D.nb, D.base.data(), D.nbr.data(), D.flags.data(), D_ACTIVE);
         nd_->upload(st_);
       }
-      nd_->factor(lv_[B].st64.as<double>(), st_, rb_);
+      nd_->factor(lv_[B].st64.as<double>(), st_);
       mark("bottom (nested dissection)");
     } catch (const NdNotSpd& e) {
       throw SpgError(SPG_E_SINGULAR, e.what());
@@ -425,59 +424,45 @@ void Solver::build_operators() {
     return;
   }
   nd_.reset();
-  upload(var_of_, var);
-  DBuf Ainv;
-  Ainv.alloc((size_t)nv * nv * 8);
-  info_.alloc(16);
-  HIPCHK(hipMemsetAsync(Ainv.p, 0, (size_t)nv * nv * 8, st_));
-  launch_dense_assemble(st_, lv_[B].d, lv_[B].st64.as<double>(), var_of_.as<int>(), nv, Ainv.as<double>());
-  if (nv * nv <= (int64_t)std::numeric_limits<int32_t>::max()) {
-    RBCHK(rocsolver_dpotrf(rb_, rocblas_fill_lower, (rocblas_int)nv, Ainv.as<double>(), (rocblas_int)nv,
-                           info_.as<rocblas_int>()));
-    int hinfo = 0;
-    HIPCHK(hipMemcpyAsync(&hinfo, info_.p, sizeof(int), hipMemcpyDeviceToHost, st_));
-    sync();
-    if (hinfo != 0)
-      throw SpgError(SPG_E_SINGULAR, "bottom Cholesky failed: leading minor " + std::to_string(hinfo) +
-                                         " not positive definite");
-    RBCHK(rocsolver_dpotri(rb_, rocblas_fill_lower, (rocblas_int)nv, Ainv.as<double>(), (rocblas_int)nv,
-                           info_.as<rocblas_int>()));
-  } else {
-    // more than 2^31 entries: the 32-bit interfaces overflow their offsets, so
-    // factor with the 64-bit one and form A^-1 = L^-T L^-1 = X^T X, X = L^-1
-    RBCHK(rocsolver_dpotrf_64(rb_, rocblas_fill_lower, nv, Ainv.as<double>(), nv, info_.as<int64_t>()));
-    int64_t hinfo = 0;
-    HIPCHK(hipMemcpyAsync(&hinfo, info_.p, sizeof(int64_t), hipMemcpyDeviceToHost, st_));
-    sync();
-    if (hinfo != 0)
-      throw SpgError(SPG_E_SINGULAR, "bottom Cholesky failed: leading minor " + std::to_string(hinfo) +
-                                         " not positive definite");
-    DBuf X;
-    X.alloc((size_t)nv * nv * 8);
-    HIPCHK(hipMemsetAsync(X.p, 0, (size_t)nv * nv * 8, st_));
-    launch_set_diagonal(st_, X.as<double>(), nv, 1.0);
-    RBCHK(rocblas_dtrsm_64(rb_, rocblas_side_left, rocblas_fill_lower, rocblas_operation_none,
-                           rocblas_diagonal_non_unit, nv, nv, &one, Ainv.as<double>(), nv, X.as<double>(), nv));
-    RBCHK(rocblas_dsyrk_64(rb_, rocblas_fill_lower, rocblas_operation_transpose, nv, nv, &one, X.as<double>(), nv,
-                           &zero, Ainv.as<double>(), nv));
-    sync();
-  }
-  launch_symmetrize_lower(st_, Ainv.as<double>(), nv);
-  // packed lower-triangle tiles (FP64 for the FP64 cycle, rounded to FP32 for the FP32 cycle)
+  // the matrix in packed lower-triangle 64x64 tiles (padding rows are
+  // identity), its inverse by the block sweep in place, and the FP32 copy for
+  // the FP32 cycle
   nT_ = (int)((nv + 63) / 64);
   const size_t ntile = (size_t)nT_ * (nT_ + 1) / 2;
   const size_t npad = (size_t)nT_ * 64;
-  tiles64_.alloc(ntile * 4096 * 8);
-  tiles32_.alloc(ntile * 4096 * 4);
-  launch_pack_sym_tiles<double>(st_, Ainv.as<double>(), nv, nT_, tiles64_.as<double>());
-  launch_pack_sym_tiles<float>(st_, Ainv.as<double>(), nv, nT_, tiles32_.as<float>());
-  for (DBuf* d : {&xb64_, &yb64_}) d->alloc(npad * 8);
-  for (DBuf* d : {&xb32_, &yb32_}) d->alloc(npad * 4);
-  pb64_.alloc((size_t)symv_splits(nT_) * npad * 8);
-  pb32_.alloc((size_t)symv_splits(nT_) * npad * 4);
-  HIPCHK(hipMemsetAsync(xb64_.p, 0, npad * 8, st_));
-  HIPCHK(hipMemsetAsync(xb32_.p, 0, npad * 4, st_));
+  if (!tiles64_.p) {
+    upload(var_of_, var);
+    tiles64_.alloc(ntile * 4096 * 8);
+    tiles32_.alloc(ntile * 4096 * 4);
+    for (DBuf* d : {&panw_, &panx_}) d->alloc((size_t)nT_ * 4096 * 8);
+    dinv_.alloc(4096 * 8);
+    info_.alloc(sizeof(int));
+    const std::vector<SweepMat> one_mat{SweepMat{0, nT_, nT_, 0, 0}};
+    upload(smat_, one_mat);
+    sweep_.h = one_mat;
+    sweep_.d = smat_.as<SweepMat>();
+    sweep_.panw = panw_.as<double>();
+    sweep_.panx = panx_.as<double>();
+    sweep_.dinv = dinv_.as<double>();
+    sweep_.info = info_.as<int>();
+    for (DBuf* d : {&xb64_, &yb64_}) d->alloc(npad * 8);
+    for (DBuf* d : {&xb32_, &yb32_}) d->alloc(npad * 4);
+    pb64_.alloc((size_t)symv_splits(nT_) * npad * 8);
+    pb32_.alloc((size_t)symv_splits(nT_) * npad * 4);
+    HIPCHK(hipMemsetAsync(xb64_.p, 0, npad * 8, st_));
+    HIPCHK(hipMemsetAsync(xb32_.p, 0, npad * 4, st_));
+  }
+  HIPCHK(hipMemsetAsync(tiles64_.p, 0, tiles64_.bytes, st_));
+  HIPCHK(hipMemsetAsync(info_.p, 0, sizeof(int), st_));
+  launch_tile_assemble(st_, lv_[B].d, lv_[B].st64.as<double>(), var_of_.as<int>(), nv, nT_, tiles64_.as<double>());
+  sweep_run(st_, sweep_, tiles64_.as<double>());
+  launch_tile_negate(st_, tiles64_.as<double>(), tiles32_.as<float>(), (int64_t)ntile * 4096);
+  int hinfo = 0;
+  HIPCHK(hipMemcpyAsync(&hinfo, info_.p, sizeof(int), hipMemcpyDeviceToHost, st_));
   sync();
+  if (hinfo != 0)
+    throw SpgError(SPG_E_SINGULAR, "bottom Cholesky failed: leading minor " + std::to_string(hinfo) +
+                                       " not positive definite");
   mark("bottom (dense inverse)");
 }
 

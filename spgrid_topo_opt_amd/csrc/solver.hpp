@@ -18,6 +18,7 @@
 #include "bottom_nd.hpp"
 #include "kernels.hpp"
 #include "layout.hpp"
+#include "sweep.hpp"
 
 namespace spg {
 
@@ -155,6 +156,8 @@ class Solver {
   int nT_ = 0;  // 64-row tiles of the bottom inverse
   bool bottom64_ = false;  // FP32 cycles apply the FP64 bottom inverse
   bool coarse64_ = false;  // FP32 cycles run the explicit levels in FP64
+  SweepBatch sweep_;
+  DBuf smat_, panw_, panx_, dinv_;
   DBuf var_of_, info_, tiles64_, tiles32_, xb64_, yb64_, xb32_, yb32_, pb64_, pb32_;
   std::unique_ptr<NdBottom> nd_;  // nested-dissection Cholesky bottom (large bottoms)
   // PCG / outer vectors (level 0)

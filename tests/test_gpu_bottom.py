@@ -104,3 +104,23 @@ def test_bottom_dense_max_picks_the_bottom(monkeypatch):
         outs.append(out)
         s.close()
     assert rel(outs[0], outs[1]) < 1e-8
+
+
+@pytest.mark.parametrize("kind", ["dense", "nd"])
+@pytest.mark.parametrize("shape", [(2, 2, 2), (3, 3, 3), (4, 3, 2), (9, 6, 5), (15, 7, 7)])
+def test_bottom_sweep_at_tile_edges(shape, kind, monkeypatch):
+    """one-level problems whose bottom has 81, 192 (whole 64-tiles), 180, 1260
+    and 3072 unknowns: K x = b to 1e-11 of b (about 10^4 products a row at
+    condition numbers up to 10^5 of the residual form)"""
+    monkeypatch.setenv("SPG_BOTTOM", kind)
+    s = _lib.Solver(W.box(*shape, seed=2, mg_levels=1))
+    gx, gf = s.level_nodes(0)
+    rng = np.random.default_rng(7)
+    b = rng.standard_normal((len(gx), 3))
+    b[(gf & 1) == 0] = 0
+    b[((gf[:, None] >> (1 + np.arange(3))) & 1).astype(bool)] = 0
+    for prec, tol in ((1, 1e-11), (0, 1e-3)):
+        x = s.kernel(_lib.OP_BOTTOM, 0, None, b, precision=prec)
+        r = s.kernel(_lib.OP_OPERATOR, 0, x, None, precision=1) - b
+        assert np.abs(r).max() < tol * np.abs(b).max(), prec
+    s.close()
