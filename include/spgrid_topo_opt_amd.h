@@ -247,6 +247,16 @@ int spg_oc_trial(int64_t n, const uint8_t *mask, const double *rho, const double
                  double min_density, double fixed_density, int32_t exclude_fixed, double dc_shift, double *out,
                  double *volume, double *change);
 
+/* The whole OC update (optimality_criterion.cpp:19-146): the reference's
+ * bisection on the multiplier, from [1e-20, 1e20] down to a relative bracket of
+ * 1e-7, for the volume `target`, then the new densities (out, device [n]),
+ * *change = max |new - rho| and *multiplier = the last one tried (both host,
+ * may be NULL).  The same sequence and result as one spg_oc_trial per step,
+ * with several multipliers evaluated in each pass over the cells.            */
+int spg_oc_update(int64_t n, const uint8_t *mask, const double *rho, const double *dc, double target, double step,
+                  double min_density, double fixed_density, int32_t exclude_fixed, double dc_shift, double *out,
+                  double *change, double *multiplier);
+
 /* spg_oc_trial without any allocation.  No counterpart in the reference: it
  * is for callers that cannot allocate device or pinned memory (code under
  * HIP graph capture, tight optimizer loops, harnesses that forbid hipMalloc).

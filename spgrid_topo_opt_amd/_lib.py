@@ -33,7 +33,7 @@ EXPORTS = [
     "spg_solve_adjoint_device", "spg_sensitivity_device", "spg_num_levels", "spg_level_size", "spg_level_nodes",
     "spg_kernel", "spg_level_stencils", "spg_bench_apply", "spg_bench_kernel", "spg_get_info",
     "spg_update_density_device", "spg_filter_sensitivity", "spg_oc_trial", "spg_set_initial_guess_device",
-    "spg_oc_trial_noalloc",
+    "spg_oc_trial_noalloc", "spg_oc_update",
 ]
 
 
@@ -147,6 +147,8 @@ def lib():
                                    C.c_double, vp, dp, dp]
         L.spg_oc_trial_noalloc.argtypes = [C.c_int64, vp, vp, vp, C.c_double, C.c_double, C.c_double,
                                            C.c_double, C.c_int32, C.c_double, vp, vp, vp]
+        L.spg_oc_update.argtypes = [C.c_int64, vp, vp, vp, C.c_double, C.c_double, C.c_double, C.c_double, C.c_int32,
+                                    C.c_double, vp, dp, dp]
         L.fem_solve.argtypes = [vp, vp]
         L.fem_solve.restype = None
         L.fem_solve_test.argtypes = [vp, vp]
@@ -349,6 +351,16 @@ def oc_trial(n, mask_ptr, rho_ptr, dc_ptr, mid, step, min_density, out_ptr=None,
                               min_density, fixed_density, 1 if exclude_fixed else 0, dc_shift,
                               C.c_void_p(out_ptr) if out_ptr else None, C.byref(vol), C.byref(ch)))
     return vol.value, ch.value
+
+
+def oc_update(n, mask_ptr, rho_ptr, dc_ptr, target, step, min_density, out_ptr, fixed_density=1.0,
+              exclude_fixed=True, dc_shift=0.0):
+    """the OC bisection over device arrays (spg_oc_update); returns (max change, last multiplier)"""
+    ch, mid = C.c_double(0.0), C.c_double(0.0)
+    _check(lib().spg_oc_update(n, C.c_void_p(mask_ptr), C.c_void_p(rho_ptr), C.c_void_p(dc_ptr), target, step,
+                               min_density, fixed_density, 1 if exclude_fixed else 0, dc_shift, C.c_void_p(out_ptr),
+                               C.byref(ch), C.byref(mid)))
+    return ch.value, mid.value
 
 
 def oc_trial_noalloc(n, mask_ptr, rho_ptr, dc_ptr, mid, step, min_density, result_ptr, out_ptr=None,

@@ -13,7 +13,7 @@ iterate() at :1289-1331): differentiable GPU FEM solves for torch.
 * :func:`filter_sensitivity` / :func:`oc_update` -- the density-weighted cone
   filter (spgrid_topo_opt.cpp:527-574) and the bisection optimality-criterion
   update (optimizer/optimality_criterion.cpp:19-146), HIP kernels of the same
-  library (spg_filter_sensitivity, spg_oc_trial).
+  library (spg_filter_sensitivity, spg_oc_update).
 
 Densities are tensors of shape (nblocks*64,) in the input block order of the
 Problem (index block*64 + i*16 + j*4 + k), float64 on cuda.
@@ -223,8 +223,8 @@ def oc_update(rho, dc, inside, volume_fraction, step_limit=0.2, min_density=0.0,
     the volume nor in the container size.  shift = min(0, min over the inside
     cells of -dc) with smart_oc, else 0.  The volume must equal volume_fraction
     times (container cells - fixed inside cells); container cells default to
-    the updated cells.  Each trial is the HIP kernel spg_oc_trial; the
-    bisection sequence is the reference's."""
+    the updated cells.  The bisection (spg_oc_update) runs the reference's
+    sequence, several multipliers to a pass."""
     if not rho.is_cuda:
         raise RuntimeError("oc_update runs on the GPU (HIP kernel); got a CPU tensor")
     n = inside.sum().item() if container_cells is None else container_cells
@@ -241,20 +241,10 @@ def oc_update(rho, dc, inside, volume_fraction, step_limit=0.2, min_density=0.0,
     mask = mask.contiguous()
     shift = min(0.0, (-dc[inside]).min().item()) if smart_oc and bool(inside.any()) else 0.0
     torch.cuda.synchronize(rho.device)
-    kw = dict(fixed_density=fixed_cell_density, exclude_fixed=exclude_fixed_cells, dc_shift=shift)
-    lower, upper = 1e-20, 1e20
-    mid = 0.5 * (lower + upper)
-    while lower * (1 + 1e-7) < upper:
-        mid = 0.5 * (lower + upper)
-        vol, _ = _lib.oc_trial(rho.numel(), mask.data_ptr(), rho.data_ptr(), dc.data_ptr(), mid, step_limit,
-                               min_density, **kw)
-        if vol > target:
-            lower = mid
-        else:
-            upper = mid
     new = torch.empty_like(rho)
-    _, change = _lib.oc_trial(rho.numel(), mask.data_ptr(), rho.data_ptr(), dc.data_ptr(), mid, step_limit,
-                              min_density, new.data_ptr(), **kw)
+    change, _ = _lib.oc_update(rho.numel(), mask.data_ptr(), rho.data_ptr(), dc.data_ptr(), target, step_limit,
+                               min_density, new.data_ptr(), fixed_density=fixed_cell_density,
+                               exclude_fixed=exclude_fixed_cells, dc_shift=shift)
     return new, change
 
 

@@ -285,3 +285,43 @@ def test_filter_and_oc_kernels_match_torch_reference(filter_size):
         new_r, change_r, _ = TR.oc_update(rho, dc2, grid.inside, 0.3, 0.2, 0.0, **kw)
         assert (new - new_r).abs().max().item() < 1e-9, kw
         assert abs(change - change_r) < 1e-9, kw
+
+
+@pytest.mark.parametrize("n", [1, 255, 4097, 300_000])
+@pytest.mark.parametrize("kind", ["usual", "tiny gradients", "target out of reach", "negative density"])
+def test_oc_update_follows_the_bisection_of_single_trials(n, kind):
+    """spg_oc_update against the bisection with one spg_oc_trial per step: the
+    same multiplier and the same densities, bit for bit (both end with the
+    same trial kernel at the last multiplier)"""
+    from spgrid_topo_opt_amd import _lib
+    g = torch.Generator(device="cuda").manual_seed(n)
+    rho = torch.rand(n, generator=g, device="cuda", dtype=torch.float64) * 0.6 + 0.1
+    dc = -torch.rand(n, generator=g, device="cuda", dtype=torch.float64)
+    mask = (torch.rand(n, generator=g, device="cuda", dtype=torch.float64) < 0.9).to(torch.uint8)
+    mask |= (torch.rand(n, generator=g, device="cuda", dtype=torch.float64) < 0.05).to(torch.uint8) << 1
+    share = 0.35
+    if kind == "tiny gradients":
+        dc *= 1e-14
+    elif kind == "target out of reach":
+        share = 3.0
+    elif kind == "negative density":
+        rho[::7] *= -1.0
+    target = share * n
+    kw = dict(fixed_density=0.7, exclude_fixed=n % 2 == 0, dc_shift=-0.01 if n == 4097 else 0.0)
+    torch.cuda.synchronize()
+    lower, upper, mid = 1e-20, 1e20, 0.0
+    while lower * (1 + 1e-7) < upper:
+        mid = 0.5 * (lower + upper)
+        vol, _ = _lib.oc_trial(n, mask.data_ptr(), rho.data_ptr(), dc.data_ptr(), mid, 0.2, 0.01, **kw)
+        if vol > target:
+            lower = mid
+        else:
+            upper = mid
+    want = torch.empty_like(rho)
+    _, ch = _lib.oc_trial(n, mask.data_ptr(), rho.data_ptr(), dc.data_ptr(), mid, 0.2, 0.01, want.data_ptr(), **kw)
+    got = torch.full_like(rho, -1.0)
+    torch.cuda.synchronize()
+    change, last = _lib.oc_update(n, mask.data_ptr(), rho.data_ptr(), dc.data_ptr(), target, 0.2, 0.01,
+                                  got.data_ptr(), **kw)
+    assert last == mid and change == ch
+    assert torch.equal(got, want)
