@@ -2084,6 +2084,266 @@ __global__ void __launch_bounds__(64) k_bnd_flow(BndOff L, ColourOrder ord, Colo
   }
 }
 
+// Full Gauss-Seidel sweep of a small level by data flow: one launch instead of
+// one per colour, a one-wave workgroup per block (an octet of lanes per node,
+// lane g loading spokes g, g+8, g+16, g+24).  A neighbour of a colour later in the sweep still holds
+// its old value in u, since its update waits for this node's; one of an
+// earlier colour is taken from its tagged entry once that carries this
+// launch's `epoch`.  Every node of a block publishes, active or not.  As in
+// k_bnd_flow waits are on earlier steps only and bounded.  Bound by one
+// store-to-load hop per colour step; the next step's loads that need no wait go
+// out before the wait.
+// Sweep by flow / by launches back to back, FP32 and FP64: level 0 23 / 35 and
+// 28 / 48 us at 45 blocks, 30 / 36 us at 1377 (FP32); explicit levels 23 / 37
+// and 26 / 42 us at 225 blocks, 25 / 33 and 30 / 42 us at 441.
+// Most blocks, all resident together: half of what the registers let the 256
+// CUs hold (level 0: 4 and 2 waves per SIMD in FP32 and FP64, explicit levels 2
+// and 1).
+template <class T>
+struct FlowBlocks {
+  static constexpr int gs0 = sizeof(T) == 4 ? 2048 : 1024;
+  static constexpr int st = sizeof(T) == 4 ? 1024 : 512;
+};
+template <class T>
+struct SweepFetch {
+  T x[4][3];    // plain values (own and later colours)
+  int slot[4];  // -1 absent
+  T b[3], di[6];
+  int blk, l;   // the octet's node
+  int early;    // bit t: spoke t waits for the tagged entry
+  uint8_t fl;
+};
+// the part that waits for nothing; `shfl` needs the whole wave
+template <class T>
+__device__ __forceinline__ void sweep_fetch(SweepFetch<T>& F, int blk, int colour, unsigned early_colours, int nb_l,
+                                            const uint8_t* __restrict__ flags, const T* __restrict__ u,
+                                            const T* __restrict__ b) {
+  const int lane = threadIdx.x, k = lane >> 3, g = lane & 7;
+  const int l = colour_node(colour, k), li = l >> 4, lj = (l >> 2) & 3, lk = l & 3;
+  F.blk = blk;
+  F.l = l;
+  F.early = 0;
+#pragma unroll
+  for (int t = 0; t < 4; ++t) {
+    const int s = g + 8 * t;
+    const int ox = s / 9 - 1, oy = (s / 3) % 3 - 1, oz = s % 3 - 1;
+    const int x = li + ox, y = lj + oy, z = lk + oz;
+    const int sp = s < 27 ? ring_spoke(x, y, z) : 13;
+    const int bb = __shfl(nb_l, sp);
+    F.slot[t] = s < 27 && bb >= 0 ? bb * 64 + loc3(x, y, z) : -1;
+    const int c2 = colour ^ (((ox & 1) << 2) | ((oy & 1) << 1) | (oz & 1));
+    if (F.slot[t] >= 0 && ((early_colours >> c2) & 1)) F.early |= 1 << t;
+#pragma unroll
+    for (int c = 0; c < 3; ++c)
+      F.x[t][c] = F.slot[t] >= 0 && !((F.early >> t) & 1) ? u[vidx(F.slot[t] >> 6, c, F.slot[t] & 63)] : T(0);
+  }
+  F.fl = 0;
+  F.b[0] = F.b[1] = F.b[2] = T(0);
+  if (g == 5) {
+    F.fl = flags[blk * 64 + l];
+#pragma unroll
+    for (int c = 0; c < 3; ++c) F.b[c] = b[vidx(blk, c, l)];
+  }
+}
+// waits for the earlier colours' entries; false after a time-out
+template <class T>
+__device__ __forceinline__ bool sweep_wait(SweepFetch<T>& F, unsigned epoch, const TagWord* tu, int* err,
+                                           unsigned long long limit) {
+  constexpr int W = TagPack<T>::W, NW = 3 * W;
+  unsigned long long t0 = 0;
+  for (bool first = true;; first = false) {
+    bool ok = true;
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      if (!((F.early >> t) & 1)) continue;
+      TagWord w[NW];
+#pragma unroll
+      for (int k = 0; k < NW; ++k) w[k] = tag_load(tu + (size_t)F.slot[t] * NW + k);
+#pragma unroll
+      for (int k = 0; k < NW; ++k) ok = ok && (unsigned)(w[k] >> 32) == epoch;
+#pragma unroll
+      for (int v = 0; v < 3; ++v) TagPack<T>::get(w + v * W, F.x[t][v]);
+    }
+    if (__all(ok)) return true;
+    if (first) t0 = wall_clock64();
+    else if (wall_clock64() - t0 > limit) {
+      if (threadIdx.x == 0) __hip_atomic_fetch_or(err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      return false;
+    }
+  }
+}
+// the node's update by lane g = 5 (spoke 13 = (g 5, t 1) is the node itself),
+// published and stored
+template <class T>
+__device__ __forceinline__ void sweep_update(const SweepFetch<T>& F, T f0, T f1, T f2, unsigned epoch, TagWord* tu,
+                                             T* __restrict__ u) {
+  constexpr int W = TagPack<T>::W, NW = 3 * W;
+  if ((threadIdx.x & 7) != 5) return;
+  T n0 = F.x[1][0], n1 = F.x[1][1], n2 = F.x[1][2];
+  const T* d = F.di;
+  if (F.fl & 1) {
+    const T r0 = F.b[0] - f0, r1 = F.b[1] - f1, r2 = F.b[2] - f2;
+    n0 += d[0] * r0 + d[3] * r1 + d[4] * r2;
+    n1 += d[3] * r0 + d[1] * r1 + d[5] * r2;
+    n2 += d[4] * r0 + d[5] * r1 + d[2] * r2;
+  }
+  if (F.fl & 2) n0 = T(0);
+  if (F.fl & 4) n1 = T(0);
+  if (F.fl & 8) n2 = T(0);
+  TagWord* p = tu + (size_t)(F.blk * 64 + F.l) * NW;
+  TagPack<T>::put(p, n0, epoch);
+  TagPack<T>::put(p + W, n1, epoch);
+  TagPack<T>::put(p + 2 * W, n2, epoch);
+  if (F.fl & 0x0F) {
+    u[vidx(F.blk, 0, F.l)] = n0;
+    u[vidx(F.blk, 1, F.l)] = n1;
+    u[vidx(F.blk, 2, F.l)] = n2;
+  }
+}
+// colours that come before step st in the sweep, as a mask
+__device__ __forceinline__ unsigned colours_before(const ColourOrder& ord, int st) {
+  unsigned m = 0;
+  for (int i = 0; i < st; ++i) m |= 1u << ord.at(i);
+  return m;
+}
+
+// explicit level: rows from the stored stencils
+template <class T>
+struct StFlow {
+  SweepFetch<T> f;
+  T m[36];
+};
+template <class T>
+__global__ void __launch_bounds__(64) k_st_flow(ColourOrder ord, const int* __restrict__ nbr,
+                                                const uint8_t* __restrict__ flags, const T* __restrict__ ST, T* u,
+                                                const T* __restrict__ b, TagWord* tu, unsigned epoch, int* err,
+                                                unsigned long long limit) {
+  const int lane = threadIdx.x, k = lane >> 3, g = lane & 7, blk = blockIdx.x;
+  const int nb_l = lane == 13 ? blk : (lane < 27 ? nbr[blk * 27 + lane] : -1);
+  auto fetch = [&](StFlow<T>& F, int st) {
+    const int c = ord.at(st);
+    const T* S = ST + ((int64_t)blk * 8 + c) * 1944;
+#pragma unroll
+    for (int e = 0; e < 27; ++e) F.m[e] = S[e * 64 + lane];
+#pragma unroll
+    for (int e = 0; e < 9; ++e) F.m[27 + e] = g < 3 ? S[1728 + e * 24 + k * 3 + g] : T(0);
+    sweep_fetch<T>(F.f, blk, c, colours_before(ord, st), nb_l, flags, u, b);
+  };
+  auto update = [&](StFlow<T>& F) -> bool {
+    if (g == 5) {
+      const T* m = F.m + 9;
+      T* d = F.f.di;
+      d[0] = m[0]; d[1] = m[4]; d[2] = m[8]; d[3] = m[1]; d[4] = m[2]; d[5] = m[5];
+      if (F.f.fl & 1) dirichlet_inverse(d, F.f.fl);
+    }
+    if (!sweep_wait<T>(F.f, epoch, tu, err, limit)) return false;
+    T a0 = 0, a1 = 0, a2 = 0;
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      const T* m = F.m + t * 9;
+      const T* x = F.f.x[t];
+      a0 = fmaT(m[0], x[0], a0);
+      a0 = fmaT(m[1], x[1], a0);
+      a0 = fmaT(m[2], x[2], a0);
+      a1 = fmaT(m[3], x[0], a1);
+      a1 = fmaT(m[4], x[1], a1);
+      a1 = fmaT(m[5], x[2], a1);
+      a2 = fmaT(m[6], x[0], a2);
+      a2 = fmaT(m[7], x[1], a2);
+      a2 = fmaT(m[8], x[2], a2);
+    }
+    a0 = octet_sum(a0);
+    a1 = octet_sum(a1);
+    a2 = octet_sum(a2);
+    sweep_update<T>(F.f, a0, a1, a2, epoch, tu, u);
+    return true;
+  };
+  StFlow<T> X, Y;
+  fetch(X, 0);
+  for (int st = 0; st < 8; st += 2) {
+    fetch(Y, st + 1);
+    if (!update(X)) return;
+    if (st + 2 < 8) fetch(X, st + 2);
+    if (!update(Y)) return;
+  }
+}
+
+// level 0: matrix-free rows, lane I = g adding the cell of which the node is
+// corner I; the 27 neighbours pass through LDS
+template <class T>
+struct Gs0Flow {
+  SweepFetch<T> f;
+  T e;
+};
+template <class T>
+__global__ void __launch_bounds__(64) k_gs0_flow(ColourOrder ord, const int* __restrict__ nbr,
+                                                 const uint8_t* __restrict__ flags, const T* __restrict__ E, T dx, T* u,
+                                                 const T* __restrict__ b, TagWord* tu, unsigned epoch, int* err,
+                                                 unsigned long long limit) {
+  constexpr int HS = 85;  // row stride of an octet's 27 x 3 values
+  __shared__ T hs[8 * HS];
+  const int lane = threadIdx.x, k = lane >> 3, I = lane & 7, blk = blockIdx.x;
+  const int nb_l = lane == 13 ? blk : (lane < 27 ? nbr[blk * 27 + lane] : -1);
+  const int ix = (I >> 2) & 1, iy = (I >> 1) & 1, iz = I & 1;
+  T* H = hs + k * HS;
+  auto fetch = [&](Gs0Flow<T>& F, int st) {
+    const int c = ord.at(st);
+    sweep_fetch<T>(F.f, blk, c, colours_before(ord, st), nb_l, flags, u, b);
+    const int l = F.f.l, cx = (l >> 4) - ix, cy = ((l >> 2) & 3) - iy, cz = (l & 3) - iz;
+    const int eb = __shfl(nb_l, ring_spoke(cx, cy, cz));
+    F.e = eb >= 0 ? E[eb * 64 + loc3(cx, cy, cz)] : T(0);
+  };
+  auto update = [&](Gs0Flow<T>& F) -> bool {
+    const T e = F.e;
+    {
+      // the inverse self block, before the wait
+      const T sx = ix ? T(-1) : T(1), sy = iy ? T(-1) : T(1), sz = iz ? T(-1) : T(1);
+      const T S = dx * octet_sum(e), Sxy = dx * octet_sum(sx * sy * e), Sxz = dx * octet_sum(sx * sz * e),
+              Syz = dx * octet_sum(sy * sz * e);
+      T* d = F.f.di;
+      d[0] = KT<T>::k(0) * S;
+      d[1] = KT<T>::k(4) * S;
+      d[2] = KT<T>::k(8) * S;
+      d[3] = KT<T>::k(1) * Sxy;
+      d[4] = KT<T>::k(2) * Sxz;
+      d[5] = KT<T>::k(5) * Syz;
+      if (F.f.fl & 1) dirichlet_inverse(d, F.f.fl);
+    }
+    if (!sweep_wait<T>(F.f, epoch, tu, err, limit)) return false;
+    // a wavefront's LDS operations execute in order: its last reads of hs are
+    // done before these writes, and the writes before the reads below
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+      if (I + 8 * t < 27)
+#pragma unroll
+        for (int v = 0; v < 3; ++v) H[(I + 8 * t) * 3 + v] = F.f.x[t][v];
+    __builtin_amdgcn_wave_barrier();
+    asm volatile("" ::: "memory");
+    auto U = [&](int J, T& v0, T& v1, T& v2) {
+      const int sp = (((J >> 2) & 1) - ix + 1) * 9 + (((J >> 1) & 1) - iy + 1) * 3 + ((J & 1) - iz + 1);
+      v0 = H[sp * 3];
+      v1 = H[sp * 3 + 1];
+      v2 = H[sp * 3 + 2];
+    };
+    T f0, f1, f2;
+    corner_row<T>(I, e, U, f0, f1, f2);
+    f0 = dx * octet_sum(f0);
+    f1 = dx * octet_sum(f1);
+    f2 = dx * octet_sum(f2);
+    sweep_update<T>(F.f, f0, f1, f2, epoch, tu, u);
+    return true;
+  };
+  Gs0Flow<T> X, Y;
+  fetch(X, 0);
+  for (int st = 0; st < 8; st += 2) {
+    fetch(Y, st + 1);
+    if (!update(X)) return;
+    if (st + 2 < 8) fetch(X, st + 2);
+    if (!update(Y)) return;
+  }
+}
+
 // workgroup size of the boundary phase: two register sets of BndFetch per lane
 template <class T>
 struct BndThreads {
@@ -2937,6 +3197,19 @@ static bool launch_bnd0_phase(hipStream_t st, const LevelDev& L, T dx, T* u, con
                                                L.b0node, bD, bt, dx, u);
   return true;
 }
+// longest wait of a data-flow kernel in wall-clock ticks: 50 ms
+// (SPG_COOP_LIMIT_TICKS shortens it: tests force the time-out path)
+static unsigned long long flow_wait_limit() {
+  if (const char* e = std::getenv("SPG_COOP_LIMIT_TICKS"))
+    if (std::atoll(e) > 0) return (unsigned long long)std::atoll(e);
+  static const unsigned long long wait_50ms = [] {
+    int dev = 0, khz = 0;
+    (void)hipGetDevice(&dev);
+    if (hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, dev) != hipSuccess || khz <= 0) khz = 100000;
+    return (unsigned long long)khz * 50;
+  }();
+  return wait_50ms;
+}
 // boundary phase by data flow (k_bnd_flow); false if the level has no tables
 // for it or a cooperative launch is refused (the caller then runs another
 // path; `loud` reports a refused launch on stderr).  SPG_COOP_WG caps the
@@ -2954,16 +3227,7 @@ static bool launch_bnd_flow(hipStream_t st, const LevelDev& L, T* u, const T* b,
   int G = std::min(groups, BF_MAX_WG);
   if (const char* e = std::getenv("SPG_COOP_WG"))
     if (std::atoi(e) > 0) G = std::min(G, std::atoi(e));
-  static const unsigned long long wait_50ms = [] {
-    int dev = 0, khz = 0;
-    (void)hipGetDevice(&dev);
-    if (hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, dev) != hipSuccess || khz <= 0) khz = 100000;
-    return (unsigned long long)khz * 50;
-  }();
-  // SPG_COOP_LIMIT_TICKS shortens the wait (tests force the time-out path)
-  unsigned long long lim = wait_50ms;
-  if (const char* e = std::getenv("SPG_COOP_LIMIT_TICKS"))
-    if (std::atoll(e) > 0) lim = (unsigned long long)std::atoll(e);
+  unsigned long long lim = flow_wait_limit();
   TagWord* tu = static_cast<TagWord*>(L.btag);
   k_bnd_rhs<T><<<(n + 31) / 32, 256, 0, st>>>(n, L.bnd, L.bslot, A, u, b, bt, tu);
   BndOff o;
@@ -3132,6 +3396,21 @@ void launch_gs0(hipStream_t st, const LevelDev& L, const T* E, T dx, T* u, const
     k_gs0_colour<T><<<nwg, 64 * GS_WAVES, 0, st>>>(L.nb, colour, L.nbr, L.flags, E, dx, u, b);
   }
 }
+// one whole sweep by data flow where the level has the tagged entries for it
+static bool sweep_flows(const LevelDev& L, int most) {
+  return L.stag && L.epoch && L.coop && !L.coop_off && L.nb <= most;
+}
+template <class T>
+void launch_gs0_sweep(hipStream_t st, const LevelDev& L, const T* E, T dx, T* u, const T* b, bool forward,
+                      const T* bcm) {
+  if (sweep_flows(L, FlowBlocks<T>::gs0) && !std::getenv("SPG_GS_KERNEL")) {
+    k_gs0_flow<T><<<L.nb, 64, 0, st>>>(
+        colour_order(true, forward), L.nbr, L.flags, E, dx, u, b, static_cast<TagWord*>(L.stag), ++*L.epoch,
+        reinterpret_cast<int*>(L.coop + 1), flow_wait_limit());
+    return;
+  }
+  for (int c = 0; c < 8; ++c) launch_gs0<T>(st, L, E, dx, u, b, sweep_colour(true, forward, c), nullptr, 0, bcm);
+}
 template <class T>
 void launch_gs0_boundary(hipStream_t st, const LevelDev& L, const T* E, T dx, T* u, const T* b, int sweeps,
                          bool forward) {
@@ -3171,6 +3450,16 @@ template <class T>
 void launch_st_gs(hipStream_t st, const LevelDev& L, const T* ST, T* u, const T* b, int colour) {
   const int nwg = (L.nb + GS_WAVES - 1) / GS_WAVES;
   k_st_colour<T, 0><<<nwg, 64 * GS_WAVES, 0, st>>>(L.nb, colour, L.nbr, L.flags, ST, u, b, nullptr);
+}
+template <class T>
+void launch_st_sweep(hipStream_t st, const LevelDev& L, const T* ST, T* u, const T* b, bool forward) {
+  if (sweep_flows(L, FlowBlocks<T>::st)) {
+    k_st_flow<T><<<L.nb, 64, 0, st>>>(
+        colour_order(false, forward), L.nbr, L.flags, ST, u, b, static_cast<TagWord*>(L.stag), ++*L.epoch,
+        reinterpret_cast<int*>(L.coop + 1), flow_wait_limit());
+    return;
+  }
+  for (int c = 0; c < 8; ++c) launch_st_gs<T>(st, L, ST, u, b, sweep_colour(false, forward, c));
 }
 template <class T>
 void launch_st_boundary(hipStream_t st, const LevelDev& L, const T* ST, T* u, const T* b, int sweeps, bool forward) {
@@ -3356,6 +3645,8 @@ void launch_set_entries(hipStream_t st, double* v, const int* idx, const double*
   template void launch_gs0_boundary<T>(hipStream_t, const LevelDev&, const T*, T, T*, const T*, int, bool);      \
   template void launch_st_residual<T>(hipStream_t, const LevelDev&, const T*, const T*, const T*, T*);           \
   template void launch_st_gs<T>(hipStream_t, const LevelDev&, const T*, T*, const T*, int);                      \
+  template void launch_gs0_sweep<T>(hipStream_t, const LevelDev&, const T*, T, T*, const T*, bool, const T*);    \
+  template void launch_st_sweep<T>(hipStream_t, const LevelDev&, const T*, T*, const T*, bool);                  \
   template void launch_st_boundary<T>(hipStream_t, const LevelDev&, const T*, T*, const T*, int, bool);          \
   template void launch_restrict<T>(hipStream_t, const LevelDev&, const T*, T*, T*);                              \
   template void launch_prolongate<T>(hipStream_t, const LevelDev&, const T*, T*);                                \

@@ -48,6 +48,10 @@ struct LevelDev {
   const double* b0E64 = nullptr;
   const float* b0D32 = nullptr;
   const double* b0D64 = nullptr;
+  // data-flow sweep of a small level: tagged entries [nb*64*6] 64-bit words and
+  // the launch number that marks them (counted up by every launch)
+  void* stag = nullptr;
+  unsigned* epoch = nullptr;
   // data-flow boundary phase: tagged iterate [n*6] 64-bit words (either
   // precision) and {unused, error word}
   void* btag = nullptr;
@@ -118,6 +122,11 @@ void launch_apply_dot(hipStream_t st, const LevelDev& L, const T* E, T dx, const
 template <class T>
 void launch_gs0(hipStream_t st, const LevelDev& L, const T* E, T dx, T* u, const T* b, int colour,
                 const uint8_t* dist = nullptr, int dmin = 0, const T* bcm = nullptr);
+// one full sweep (8 colours): by data flow where the level has `stag`, else one
+// launch per colour
+template <class T>
+void launch_gs0_sweep(hipStream_t st, const LevelDev& L, const T* E, T dx, T* u, const T* b, bool forward,
+                      const T* bcm = nullptr);
 // v in colour-major order: vcm[((c * nb + blk) * 3 + comp) * 8 + k] = v at the
 // k-th node of colour c in block blk (level-0 vectors)
 template <class T>
@@ -139,6 +148,8 @@ template <class T>
 void launch_st_residual(hipStream_t st, const LevelDev& L, const T* ST, const T* u, const T* b, T* r);
 template <class T>
 void launch_st_gs(hipStream_t st, const LevelDev& L, const T* ST, T* u, const T* b, int colour);
+template <class T>
+void launch_st_sweep(hipStream_t st, const LevelDev& L, const T* ST, T* u, const T* b, bool forward);
 template <class T>
 void launch_st_boundary(hipStream_t st, const LevelDev& L, const T* ST, T* u, const T* b, int sweeps, bool forward);
 // transfers

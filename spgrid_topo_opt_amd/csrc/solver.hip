@@ -38,6 +38,9 @@ static double now_s() {
 // builds both maps: 0.2, 1.0, 1.9 and 5.9 ms, which a solve of 25 V-cycles (4
 // phases each) earns back up to about here.
 static constexpr int kMaxDenseBoundary = 2560;
+// levels of at most this many blocks get the entries of the data-flow sweep
+// (FlowBlocks in kernels.hip has each kernel's own limit)
+static constexpr int kMaxFlowSweep = 2048;
 // pcg() result: a level-0 boundary phase reported a barrier time-out; the
 // pass is repeated with the per-colour list launches
 static constexpr int kCoopRetry = -100;
@@ -278,6 +281,14 @@ void Solver::upload_layout() {
       upload(R.gsnear, all);
       R.gsnslot.alloc(std::max<size_t>(all.size(), 1) * 27 * 4);
       launch_list_nslot(st_, R.d, (int)all.size(), R.gsnear.as<int>(), R.gsnslot.as<int>());
+    }
+    // SPG_GS_CMB compares the per-colour launches' reads of b: it keeps them
+    if (D.nb <= kMaxFlowSweep && (l > 0 ? D.is_explicit : cmb_mode_ < 0) && lv_[0].coop.p) {
+      R.stag.alloc((size_t)D.nb * 64 * 6 * 8);
+      HIPCHK(hipMemset(R.stag.p, 0, R.stag.bytes));
+      R.d.stag = R.stag.p;
+      R.d.epoch = &R.epoch;
+      R.d.coop = lv_[0].coop.as<unsigned>();
     }
     R.d.flags = R.flags.as<uint8_t>();
     R.d.base = R.base.as<int>();
@@ -751,11 +762,10 @@ void Solver::smooth(int l, T* u, const T* b, bool forward, const T* bcm) {
   } else {
     boundary();
   }
-  for (int i = first; i < cfg_.smooth_iters; ++i)
-    for (int c = 0; c < 8; ++c) {
-      if (l == 0) launch_gs0<T>(st_, R.d, E<T>(), dxT<T>(), u, b, sweep_colour(true, forward, c), nullptr, 0, bcm);
-      else launch_st_gs<T>(st_, R.d, R.st<T>(), u, b, sweep_colour(false, forward, c));
-    }
+  for (int i = first; i < cfg_.smooth_iters; ++i) {
+    if (l == 0) launch_gs0_sweep<T>(st_, R.d, E<T>(), dxT<T>(), u, b, forward, bcm);
+    else launch_st_sweep<T>(st_, R.d, R.st<T>(), u, b, forward);
+  }
   boundary();
 }
 
@@ -1245,13 +1255,8 @@ void Solver::run_kernel(int op, int level, int precision, int forward, const dou
           else launch_st_boundary<T>(st_, Ld, lv_[level].st<T>(), A.as<T>(), Bv.as<T>(), sweeps, fwd);
         } else {
           const T* bcm = level == 0 ? colour_major_b<T>(Bv.as<T>()) : nullptr;
-          for (int c = 0; c < 8; ++c) {
-            if (level == 0)
-              launch_gs0<T>(st_, Ld, E<T>(), dxT<T>(), A.as<T>(), Bv.as<T>(), sweep_colour(true, fwd, c), nullptr, 0,
-                            bcm);
-            else
-              launch_st_gs<T>(st_, Ld, lv_[level].st<T>(), A.as<T>(), Bv.as<T>(), sweep_colour(false, fwd, c));
-          }
+          if (level == 0) launch_gs0_sweep<T>(st_, Ld, E<T>(), dxT<T>(), A.as<T>(), Bv.as<T>(), fwd, bcm);
+          else launch_st_sweep<T>(st_, Ld, lv_[level].st<T>(), A.as<T>(), Bv.as<T>(), fwd);
         }
         get(A.as<T>(), nb);
         break;
@@ -1373,10 +1378,8 @@ double Solver::bench_kernel(int op, int level, int precision, int arg, int reps)
         case SPG_OP_GS_SWEEP: {
           if (level != 0 && !lay_.lv[level].is_explicit) throw SpgError(SPG_E_INVALID, "level has no smoother");
           const T* bcm = level == 0 ? colour_major_b<T>(b) : nullptr;
-          for (int c = 0; c < 8; ++c) {
-            if (level == 0) launch_gs0<T>(st_, R.d, E<T>(), dxT<T>(), u, b, sweep_colour(true, true, c), nullptr, 0, bcm);
-            else launch_st_gs<T>(st_, R.d, R.st<T>(), u, b, sweep_colour(false, true, c));
-          }
+          if (level == 0) launch_gs0_sweep<T>(st_, R.d, E<T>(), dxT<T>(), u, b, true, bcm);
+          else launch_st_sweep<T>(st_, R.d, R.st<T>(), u, b, true);
           break;
         }
         case SPG_OP_GS_BOUNDARY:

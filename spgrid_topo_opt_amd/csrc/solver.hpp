@@ -54,6 +54,8 @@ struct LevelRT {
   DBuf b0cslot, b0node, b0E64, b0E32, b0D64, b0D32;  // level-0 matrix-free boundary system
   DBuf btag, coop;  // data-flow boundary phase: tagged iterate; level 0: {unused, error word}
   DBuf ball, bmap64[2], bmap32[2], bmx64, bmx32;     // dense boundary maps
+  DBuf stag;                                         // data-flow sweep: tagged entries
+  unsigned epoch = 0;                                // its launches so far
   DBuf bnslot;                                       // level 0: neighbour slots of boundary nodes
   DBuf gsdist, gsnear, gsnslot;                      // level 0: band distances, near-band step lists, their slots
   int64_t gsnear_off[17] = {};                       // list (dir * 8 + step) = gsnear[off[i] .. off[i+1])

@@ -357,6 +357,33 @@ def test_dense_map_and_data_flow_match_step_by_step(level, shape, monkeypatch):
     s.close()
 
 
+@pytest.mark.parametrize("shape,levels,blocks", [((3, 3, 3), 1, 1), ((45, 23, 19), 3, 360), ((64, 32, 32), 3, 1377),
+                                                 ((64, 43, 43), 3, 2057)])
+def test_data_flow_sweep_matches_colour_launches(shape, levels, blocks, monkeypatch):
+    """a level-0 sweep in one launch (small levels; 1377 blocks only in FP32,
+    2057 blocks not) against the octet colour kernel, whose arithmetic it
+    shares: FP64 to 1e-13, FP32 to 1e-6 relative"""
+    s = _lib.Solver(W.box(*shape, seed=6, mg_levels=levels))
+    assert s.level_blocks(0) == blocks
+    gx, gf = s.level_nodes(0)
+    rng = np.random.default_rng(17)
+    u = rng.standard_normal((len(gx), 3)) * 1e-3
+    b = rng.standard_normal((len(gx), 3))
+    for fwd in (True, False):
+        for prec, tol in ((1, 1e-13), (0, 1e-6)):
+            monkeypatch.setenv("SPG_GS_KERNEL", "1")
+            want = s.kernel(_lib.OP_GS_SWEEP, 0, u, b, precision=prec, forward=fwd)
+            monkeypatch.delenv("SPG_GS_KERNEL")
+            for _ in range(2):  # entries of the launch before are not this one's
+                got = s.kernel(_lib.OP_GS_SWEEP, 0, u, b, precision=prec, forward=fwd)
+                assert rel(got, want) < tol, (fwd, prec)
+    if blocks == 360:
+        monkeypatch.setenv("SPG_COOP_LIMIT_TICKS", "1")
+        with pytest.raises(_lib.SpgError, match="timed out"):
+            s.kernel(_lib.OP_GS_SWEEP, 0, u, b, precision=0, forward=True)
+    s.close()
+
+
 @pytest.mark.parametrize("prec,tol", [(1, 1e-13), (0, 1e-6)])
 def test_restriction_and_prolongation(blocky, prec, tol):
     P = blocky
