@@ -43,7 +43,11 @@ namespace spg {
 
 namespace {
 
-constexpr int kLeafNodes = 64;  // a box of at most this many nodes is one front
+// a box of at most this many nodes is one front: fewer tree depths and launches
+// per solve against larger pivot blocks.  Solve with 64 / 192 / 400: 56 / 49 /
+// 46 us at 4,131 unknowns, 100 / 80 / 75 us at 9,006; density update 1.5 / 1.6 /
+// 2.0 and 8.5 / 8.5 / 9.2 ms.
+constexpr int kLeafNodes = 192;
 
 #define NDCHK(x)                                                                              \
   do {                                                                                        \
@@ -108,130 +112,154 @@ __global__ void __launch_bounds__(256) k_nd_extend_add(const int* __restrict__ c
   }
 }
 
-constexpr int kChunk = 1024;  // vector entries staged at a time
+// The solve reads every tile with the output along the lanes: output c of a
+// tile row adds T[r][c] v[r].  The multipliers of the forward pass and the
+// tiles above the diagonal of A11^-1 are kept transposed for that.
+__global__ void __launch_bounds__(256) k_nd_transpose(const NdFrontDev* __restrict__ fr,
+                                                      const double* __restrict__ tiles, double* __restrict__ tr) {
+  __shared__ double s[64][65];
+  const NdFrontDev F = fr[blockIdx.y];
+  const int64_t e = blockIdx.x, nsq = (int64_t)F.tp * (F.tp - 1) / 2;
+  if (e >= nsq + (int64_t)F.tb * F.tp) return;
+  int I, J;
+  if (e < nsq) {  // strictly lower tiles of the pivot block
+    I = (int)((sqrt(8.0 * (double)e + 1.0) + 1.0) * 0.5);
+    while ((int64_t)I * (I - 1) / 2 > e) --I;
+    while ((int64_t)(I + 1) * I / 2 <= e) ++I;
+    J = (int)(e - (int64_t)I * (I - 1) / 2);
+  } else {
+    I = F.tp + (int)((e - nsq) / F.tp);
+    J = (int)((e - nsq) % F.tp);
+  }
+  const double* t = tiles + (F.t_off + tile_at(I, J)) * 4096;
+  double* o = tr + (F.tr_off + e) * 4096;
+  for (int q = threadIdx.x; q < 4096; q += 256) s[q & 63][q >> 6] = t[q];
+  __syncthreads();
+  for (int q = threadIdx.x; q < 4096; q += 256) o[q] = s[q >> 6][q & 63];
+}
+
+constexpr int kWaves = 8;       // waves of a solve workgroup, a tile each at a time
+constexpr int kChunk = 2048;    // vector entries staged at a time
+static_assert(kChunk % (64 * kWaves) == 0, "a wave's tiles of a chunk start at its own number");
+
+// acc + sum_r T[r][lane] v[r]
+__device__ __forceinline__ double tile_dot(const double* __restrict__ T, const double* v, int lane, double acc) {
+  double a0 = acc, a1 = 0.0, a2 = 0.0, a3 = 0.0;
+#pragma unroll 8
+  for (int r = 0; r < 64; r += 4) {
+    a0 = __builtin_fma(T[r * 64 + lane], v[r], a0);
+    a1 = __builtin_fma(T[(r + 1) * 64 + lane], v[r + 1], a1);
+    a2 = __builtin_fma(T[(r + 2) * 64 + lane], v[r + 2], a2);
+    a3 = __builtin_fma(T[(r + 3) * 64 + lane], v[r + 3], a3);
+  }
+  return (a0 + a1) + (a2 + a3);
+}
+// sum of the waves' partial results of one output tile row, in wave order
+__device__ __forceinline__ double tile_sum(double acc, double (*ys)[64]) {
+  const int t = threadIdx.x;
+  ys[t >> 6][t & 63] = acc;
+  __syncthreads();
+  double v = 0.0;
+  if (t < 64)
+#pragma unroll
+    for (int w = 0; w < kWaves; ++w) v += ys[w][t];
+  return v;
+}
+// a front's own right-hand side at local dof f: its row of b (pivots) plus the
+// children's update entries
+template <class T>
+__device__ __forceinline__ double front_rhs(const NdFrontDev& F, int f, const int2* __restrict__ kid,
+                                            const int* __restrict__ vmap, const T* __restrict__ b,
+                                            const double* ustore) {
+  const int2 k = kid[F.k_off + f];
+  double v = f < F.p ? (double)b[vmap[F.dof0 + f]] : 0.0;
+  if (k.x >= 0) v += ustore[k.x];
+  if (k.y >= 0) v += ustore[k.y];
+  return v;
+}
 
 // Forward, one workgroup per (front, boundary tile row): the front's
-// right-hand side w_P (its rows of b plus the children's update entries, kept
-// for the backward pass by tile row 0) and u = w_B - G w_P for the tile's rows.
-__global__ void __launch_bounds__(256) k_nd_forward(const int2* __restrict__ item, const NdFrontDev* __restrict__ fr,
-                                                    const int64_t* __restrict__ gptr, const int64_t* __restrict__ gidx,
-                                                    const double* __restrict__ b, const double* __restrict__ tiles,
-                                                    double* __restrict__ w, double* ustore) {
-  __shared__ double xs[kChunk];
-  __shared__ double ys[64];
+// right-hand side w_P (kept for the backward pass by tile row 0) and u = w_B -
+// G w_P for the tile's rows.  Bound by the chain item, front, child map, update
+// entry, then the tiles; a wave per tile with one accumulator per lane keeps
+// its 64 rows in flight.  A solve of 9,006 unknowns takes 80 us in 15 launches
+// (150 us with a workgroup's waves splitting the rows of each tile).
+template <class T>
+__global__ void __launch_bounds__(64 * kWaves) k_nd_forward(const int2* __restrict__ item,
+                                                            const NdFrontDev* __restrict__ fr,
+                                                            const int2* __restrict__ kid, const int* __restrict__ vmap,
+                                                            const T* __restrict__ b, const double* __restrict__ tr,
+                                                            double* __restrict__ w, double* ustore) {
+  __shared__ __align__(16) double xs[kChunk];
+  __shared__ double ys[kWaves][64];
   const int2 it = item[blockIdx.x];
   const NdFrontDev F = fr[it.x];
   const int rt = it.y, t = threadIdx.x, wv = t >> 6, lane = t & 63, P = F.tp * 64;
-  auto gathered = [&](int f) {
-    double v = 0.0;
-    const int64_t k0 = gptr[F.g_off + f], k1 = gptr[F.g_off + f + 1];
-    for (int64_t k = k0; k < k1; ++k) v += ustore[gidx[k]];
-    return v;
-  };
   const bool rows = rt < F.tb;
   const int r = rt * 64 + t;
   double wb = 0.0;
-  if (rows && t < 64 && r < F.b) wb = gathered(F.p + r);
-  double acc[16];
-#pragma unroll
-  for (int k = 0; k < 16; ++k) acc[k] = 0.0;
+  if (rows && t < 64 && r < F.b) wb = front_rhs<T>(F, F.p + r, kid, vmap, b, ustore);
+  const double* G = tr + (F.tr_off + (int64_t)F.tp * (F.tp - 1) / 2 + (int64_t)rt * F.tp) * 4096;
+  double acc = 0.0;
   for (int c0 = 0; c0 < P; c0 += kChunk) {
     const int c1 = min(P, c0 + kChunk);
     __syncthreads();
-    for (int f = c0 + t; f < c1; f += 256) {
-      const double v = f < F.p ? b[F.dof0 + f] + gathered(f) : 0.0;
+    for (int f = c0 + t; f < c1; f += 64 * kWaves) {
+      const double v = f < F.p ? front_rhs<T>(F, f, kid, vmap, b, ustore) : 0.0;
       xs[f - c0] = v;
       if (rt == 0) w[F.w_off + f] = v;
     }
     __syncthreads();
     if (!rows) continue;
-    for (int J = c0 >> 6; J < (c1 >> 6); ++J) {
-      const double* T = tiles + (F.t_off + tile_at(F.tp + rt, J)) * 4096 + wv * 64 + lane;
-      const double xv = xs[J * 64 - c0 + lane];
-#pragma unroll
-      for (int k = 0; k < 16; ++k) acc[k] += T[k * 256] * xv;
-    }
+    for (int J = (c0 >> 6) + wv; J < (c1 >> 6); J += kWaves)
+      acc = tile_dot(G + (int64_t)J * 4096, xs + (J * 64 - c0), lane, acc);
   }
   if (!rows) return;
-#pragma unroll
-  for (int k = 0; k < 16; ++k) {
-    double v = acc[k];
-#pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) v += __shfl_xor(v, o);
-    if (lane == 0) ys[wv + 4 * k] = v;
-  }
-  __syncthreads();
-  if (t < 64 && r < F.b) ustore[F.u_off + r] = wb - ys[t];
+  const double s = tile_sum(acc, ys);
+  if (t < 64 && r < F.b) ustore[F.u_off + r] = wb - s;
 }
 
 // Backward, one workgroup per (front, pivot tile I): x_I = -((-A11^-1) w_P +
-// G^T x_B) over the tile rows of the front.
-__global__ void __launch_bounds__(256) k_nd_backward(const int2* __restrict__ item, const NdFrontDev* __restrict__ fr,
-                                                     const int64_t* __restrict__ bidx,
-                                                     const double* __restrict__ tiles, const double* __restrict__ w,
-                                                     double* x) {
-  __shared__ double xs[kChunk];
-  __shared__ double ys[64], yt[4][64];
+// G^T x_B) over the tile rows of the front, to x and to the level vector.
+template <class T>
+__global__ void __launch_bounds__(64 * kWaves) k_nd_backward(const int2* __restrict__ item,
+                                                             const NdFrontDev* __restrict__ fr,
+                                                             const int* __restrict__ bidx, const int* __restrict__ vmap,
+                                                             const double* __restrict__ tiles,
+                                                             const double* __restrict__ tr,
+                                                             const double* __restrict__ w, double* x,
+                                                             T* __restrict__ u) {
+  __shared__ __align__(16) double xs[kChunk];
+  __shared__ double ys[kWaves][64];
   const int2 it = item[blockIdx.x];
   const NdFrontDev F = fr[it.x];
   const int I = it.y, t = threadIdx.x, wv = t >> 6, lane = t & 63, P = F.tp * 64, m = P + F.tb * 64;
-  double accN[16], accT = 0.0;
-#pragma unroll
-  for (int k = 0; k < 16; ++k) accN[k] = 0.0;
+  double acc = 0.0;
   for (int c0 = 0; c0 < m; c0 += kChunk) {
     const int c1 = min(m, c0 + kChunk);
     __syncthreads();
-    for (int f = c0 + t; f < c1; f += 256)
+    for (int f = c0 + t; f < c1; f += 64 * kWaves)
       xs[f - c0] = f < P ? w[F.w_off + f] : (f - P < F.b ? x[bidx[F.bidx_off + (f - P)]] : 0.0);
     __syncthreads();
-    for (int J = c0 >> 6; J < (c1 >> 6); ++J) {
-      const double* xj = xs + (J * 64 - c0);
-      if (J <= I) {
-        const double* T = tiles + (F.t_off + tile_at(I, J)) * 4096 + wv * 64 + lane;
-        const double xv = xj[lane];
-#pragma unroll
-        for (int k = 0; k < 16; ++k) accN[k] += T[k * 256] * xv;
-      } else {
-        const double* T = tiles + (F.t_off + tile_at(J, I)) * 4096 + wv * 64 + lane;
-#pragma unroll
-        for (int k = 0; k < 16; ++k) accT += T[k * 256] * xj[wv + 4 * k];
-      }
+    for (int J = (c0 >> 6) + wv; J < (c1 >> 6); J += kWaves) {
+      const double* A = J >= I ? tiles + (F.t_off + tile_at(J, I)) * 4096
+                               : tr + (F.tr_off + (int64_t)I * (I - 1) / 2 + J) * 4096;
+      acc = tile_dot(A, xs + (J * 64 - c0), lane, acc);
     }
   }
-#pragma unroll
-  for (int k = 0; k < 16; ++k) {
-    double v = accN[k];
-#pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) v += __shfl_xor(v, o);
-    if (lane == 0) ys[wv + 4 * k] = v;
-  }
-  yt[wv][lane] = accT;
-  __syncthreads();
+  const double s = tile_sum(acc, ys);
   const int f = I * 64 + t;
-  if (t < 64 && f < F.p) x[F.dof0 + f] = -(ys[t] + ((yt[0][t] + yt[1][t]) + (yt[2][t] + yt[3][t])));
+  if (t < 64 && f < F.p) {
+    x[F.dof0 + f] = -s;
+    u[vmap[F.dof0 + f]] = (T)-s;
+  }
 }
 
-// level vector (T) -> pos-ordered FP64 right-hand side, and back
+// u = b at the inactive nodes
 template <class T>
-__global__ void k_nd_in(int nb, const int* __restrict__ var_of, const T* __restrict__ b, double* __restrict__ x) {
-  const int gid = blockIdx.x * blockDim.x + threadIdx.x;
-  if (gid >= nb * 64) return;
-  const int vi = var_of[gid];
-  if (vi < 0) return;
-  const int blk = gid >> 6, l = gid & 63;
-  for (int c = 0; c < 3; ++c) x[vi + c] = (double)b[(blk * 3 + c) * 64 + l];
-}
-template <class T>
-__global__ void k_nd_out(int nb, const int* __restrict__ var_of, const double* __restrict__ x,
-                         const T* __restrict__ b, T* __restrict__ u) {
-  const int gid = blockIdx.x * blockDim.x + threadIdx.x;
-  if (gid >= nb * 64) return;
-  const int vi = var_of[gid];
-  const int blk = gid >> 6, l = gid & 63;
-  for (int c = 0; c < 3; ++c) {
-    const int k = (blk * 3 + c) * 64 + l;
-    u[k] = vi >= 0 ? (T)x[vi + c] : b[k];
-  }
+__global__ void k_nd_rest(int n, const int* __restrict__ rest, const T* __restrict__ b, T* __restrict__ u) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) u[rest[i]] = b[rest[i]];
 }
 
 unsigned grid(int64_t n, int t = 256) { return (unsigned)((n + t - 1) / t); }
@@ -379,7 +407,9 @@ NdBottom::NdBottom(int64_t nb, const int32_t* base, const int32_t* nbr, const ui
   std::vector<NdFrontDev> fd(fr_.size());
   int64_t toff = 0, wofs = 0, uofs = 0, bofs = 0, gofs = 0;
   std::vector<int32_t> ent_of;
-  std::vector<int64_t> gptr, gidx, bidx;
+  std::vector<int2> kid;
+  std::vector<int32_t> bidx;
+  int64_t trofs = 0;
   std::vector<int32_t> emap;
   for (size_t t = 0; t < fr_.size(); ++t) {
     Front& F = fr_[t];
@@ -399,30 +429,28 @@ NdBottom::NdBottom(int64_t nb, const int32_t* base, const int32_t* nbr, const ui
     uofs += D.b;
     D.bidx_off = bofs;
     for (int64_t q : F.bnd)
-      for (int c = 0; c < 3; ++c) bidx.push_back(3 * q + c);
+      for (int c = 0; c < 3; ++c) bidx.push_back((int32_t)(3 * q + c));
     bofs += D.b;
-    D.g_off = gofs;
-    // gather lists: children's update entries mapped into this front
-    std::vector<std::vector<int64_t>> contrib(m);
-    for (int c : F.kids) {
+    D.k_off = gofs;
+    D.tr_off = trofs;
+    trofs += (int64_t)D.tp * (D.tp - 1) / 2 + (int64_t)D.tb * D.tp;
+    // children's update entries mapped into this front, at most two per dof
+    kid.resize(kid.size() + m, make_int2(-1, -1));
+    int2* km = kid.data() + gofs;
+    for (size_t o = 0; o < F.kids.size(); ++o) {
+      const int c = F.kids[o];
       const Front& C = fr_[c];
-      const NdFrontDev& CD = fd[c];
       fd[c].emap_off = (int64_t)emap.size();
       for (size_t k = 0; k < C.bnd.size(); ++k) {
         const int lq = local(F, C.bnd[k]);
         if (lq < 0) throw std::runtime_error("nested dissection: a child's boundary node is missing from its parent");
         for (int cc = 0; cc < 3; ++cc) {
           emap.push_back(3 * lq + cc);
-          contrib[3 * lq + cc].push_back(CD.u_off + 3 * (int64_t)k + cc);
+          (o == 0 ? km[3 * lq + cc].x : km[3 * lq + cc].y) = (int)(fd[c].u_off + 3 * (int64_t)k + cc);
         }
       }
     }
-    gptr.push_back((int64_t)gidx.size());
-    for (int f = 0; f < m; ++f) {
-      for (int64_t q : contrib[f]) gidx.push_back(q);
-      gptr.push_back((int64_t)gidx.size());
-    }
-    gofs += m + 1;
+    gofs += m;
     // stencil entries: pivot i, spoke s, neighbour j later in the front
     for (int64_t k = F.pos0; k < F.pos0 + F.np; ++k) {
       const int32_t i = piv_nodes[k];
@@ -442,8 +470,17 @@ NdBottom::NdBottom(int64_t nb, const int32_t* base, const int32_t* nbr, const ui
   ulen_ = uofs;
   ent_of_ = std::move(ent_of);
   fdev_ = std::move(fd);
-  gptr_ = std::move(gptr);
-  gidx_ = std::move(gidx);
+  kid_ = std::move(kid);
+  ntr_ = trofs;
+  if (uofs > INT32_MAX || ndof_ > INT32_MAX)
+    throw std::runtime_error("nested dissection: more than 2^31 - 1 solve entries");
+  vmap_.resize(ndof_);
+  for (int64_t s = 0; s < nb * 64; ++s)
+    for (int c = 0; c < 3; ++c) {
+      const int32_t k = (int32_t)((s >> 6) * 192 + c * 64 + (s & 63));
+      if (var_of_[s] >= 0) vmap_[var_of_[s] + c] = k;
+      else rest_.push_back(k);
+    }
   bidx_ = std::move(bidx);
   emap_ = std::move(emap);
   // per depth: the solve's work items (front, boundary tile row; front, pivot
@@ -496,8 +533,9 @@ NdBottom::NdBottom(int64_t nb, const int32_t* base, const int32_t* nbr, const ui
 
 void NdBottom::upload(hipStream_t st) {
   upload_vec(d_fr_, fdev_, st);
-  upload_vec(d_gptr_, gptr_, st);
-  upload_vec(d_gidx_, gidx_, st);
+  upload_vec(d_kid_, kid_, st);
+  upload_vec(d_vmap_, vmap_, st);
+  upload_vec(d_rest_, rest_, st);
   upload_vec(d_bidx_, bidx_, st);
   upload_vec(d_emap_, emap_, st);
   upload_vec(d_ent_, ent_, st);
@@ -505,9 +543,9 @@ void NdBottom::upload(hipStream_t st) {
   upload_vec(d_ent_of_, ent_of_, st);
   upload_vec(d_mats_, mats_, st);
   upload_vec(d_kids_, kids_, st);
-  upload_vec(d_var_of_, var_of_, st);
   const size_t tile = 4096 * 8;
   tiles_.alloc((size_t)std::max<int64_t>(ntile_, 1) * tile);
+  tr_.alloc((size_t)std::max<int64_t>(ntr_, 1) * tile);
   panw_.alloc((size_t)std::max<int64_t>(npan_, 1) * tile);
   panx_.alloc((size_t)std::max<int64_t>(npan_, 1) * tile);
   dinv_.alloc((size_t)std::max<int64_t>(nid_, 1) * tile);
@@ -521,15 +559,14 @@ void NdBottom::upload(hipStream_t st) {
   }
   w_.alloc((size_t)std::max<int64_t>(wlen_, 1) * 8);
   u_.alloc((size_t)std::max<int64_t>(ulen_, 1) * 8);
-  bx_.alloc((size_t)std::max<int64_t>(ndof_, 1) * 8);
   x_.alloc((size_t)std::max<int64_t>(ndof_, 1) * 8);
   NDCHK(hipStreamSynchronize(st));
 }
 
 size_t NdBottom::device_bytes() const {
   size_t s = 0;
-  for (const DevMem* d : {&d_fr_, &d_gptr_, &d_gidx_, &d_bidx_, &d_emap_, &d_ent_, &d_ent_of_, &d_items_, &d_mats_,
-                          &d_kids_, &d_var_of_, &tiles_, &panw_, &panx_, &dinv_, &info_, &w_, &u_, &bx_, &x_})
+  for (const DevMem* d : {&d_fr_, &d_kid_, &d_vmap_, &d_rest_, &d_bidx_, &d_emap_, &d_ent_, &d_ent_of_, &d_items_,
+                          &d_mats_, &d_kids_, &tiles_, &tr_, &panw_, &panx_, &dinv_, &info_, &w_, &u_, &x_})
     s += d->bytes;
   return s;
 }
@@ -555,6 +592,13 @@ void NdBottom::factor(const double* ST, hipStream_t st) {
                                 static_cast<const int*>(d_emap_.p), tiles);
     sweep_run(st, D.batch, tiles);
   }
+  int64_t most = 0;
+  for (const NdFrontDev& D : fdev_)
+    most = std::max(most, (int64_t)D.tp * (D.tp - 1) / 2 + (int64_t)D.tb * D.tp);
+  if (most > 0)
+    for (size_t f = 0; f < fr_.size(); f += 32768)
+      k_nd_transpose<<<dim3((unsigned)most, (unsigned)std::min<size_t>(32768, fr_.size() - f)), 256, 0, st>>>(
+          fr + f, tiles, static_cast<double*>(tr_.p));
   std::vector<int> h(fr_.size());
   NDCHK(hipMemcpyAsync(h.data(), info_.p, h.size() * sizeof(int), hipMemcpyDeviceToHost, st));
   NDCHK(hipStreamSynchronize(st));
@@ -565,44 +609,38 @@ void NdBottom::factor(const double* ST, hipStream_t st) {
 }
 
 // ------------------------------------------------------------------ solve
-void NdBottom::solve_pos(hipStream_t st) {
+template <class T>
+void NdBottom::solve(const T* b, T* u, hipStream_t st) {
   const NdFrontDev* fr = static_cast<const NdFrontDev*>(d_fr_.p);
   const int2* items = static_cast<const int2*>(d_items_.p);
+  const int* vmap = static_cast<const int*>(d_vmap_.p);
   const double* tiles = static_cast<const double*>(tiles_.p);
+  const double* tr = static_cast<const double*>(tr_.p);
   double* w = static_cast<double*>(w_.p);
-  double* u = static_cast<double*>(u_.p);
+  double* us = static_cast<double*>(u_.p);
   double* x = static_cast<double*>(x_.p);
-  for (int d = maxdepth_; d >= 0; --d) {
+  for (int d = (int)depth_.size() - 1; d >= 0; --d) {
     const Depth& D = depth_[d];
     if (D.bwd0 > D.fwd0)
-      k_nd_forward<<<(unsigned)(D.bwd0 - D.fwd0), 256, 0, st>>>(
-          items + D.fwd0, fr, static_cast<const int64_t*>(d_gptr_.p), static_cast<const int64_t*>(d_gidx_.p),
-          static_cast<const double*>(bx_.p), tiles, w, u);
+      k_nd_forward<T><<<(unsigned)(D.bwd0 - D.fwd0), 64 * kWaves, 0, st>>>(
+          items + D.fwd0, fr, static_cast<const int2*>(d_kid_.p), vmap, b, tr, w, us);
   }
-  for (int d = 0; d <= maxdepth_ && !fr_.empty(); ++d) {
-    const Depth& D = depth_[d];
+  for (const Depth& D : depth_)
     if (D.end > D.bwd0)
-      k_nd_backward<<<(unsigned)(D.end - D.bwd0), 256, 0, st>>>(items + D.bwd0, fr,
-                                                                static_cast<const int64_t*>(d_bidx_.p), tiles, w, x);
-  }
+      k_nd_backward<T><<<(unsigned)(D.end - D.bwd0), 64 * kWaves, 0, st>>>(
+          items + D.bwd0, fr, static_cast<const int*>(d_bidx_.p), vmap, tiles, tr, w, x, u);
+  const int n = (int)rest_.size();
+  if (n > 0) k_nd_rest<T><<<grid(n), 256, 0, st>>>(n, static_cast<const int*>(d_rest_.p), b, u);
 }
 
-template <class T>
-void NdBottom::solve(int nb, const T* b, T* u, hipStream_t st) {
-  const int* vo = static_cast<const int*>(d_var_of_.p);
-  k_nd_in<T><<<grid((int64_t)nb * 64), 256, 0, st>>>(nb, vo, b, static_cast<double*>(bx_.p));
-  solve_pos(st);
-  k_nd_out<T><<<grid((int64_t)nb * 64), 256, 0, st>>>(nb, vo, static_cast<const double*>(x_.p), b, u);
-}
-
-template void NdBottom::solve<float>(int, const float*, float*, hipStream_t);
-template void NdBottom::solve<double>(int, const double*, double*, hipStream_t);
+template void NdBottom::solve<float>(const float*, float*, hipStream_t);
+template void NdBottom::solve<double>(const double*, double*, hipStream_t);
 
 NdStats NdBottom::stats() const {
   NdStats s;
   s.fronts = (int64_t)fr_.size();
   s.depth = maxdepth_ + 1;
-  s.factor_entries = ntile_ * 4096;
+  s.factor_entries = (ntile_ + ntr_) * 4096;
   for (const NdFrontDev& D : fdev_) s.max_front = std::max<int64_t>(s.max_front, D.p + D.b);
   return s;
 }

@@ -36,7 +36,8 @@ struct NdFrontDev {
   int64_t w_off;     // 64 tp entries of solve workspace
   int64_t u_off;     // b entries: this front's forward update vector
   int64_t bidx_off;  // b entries: dof index of each boundary dof
-  int64_t g_off;     // m + 1 entries of the gather list's row pointer
+  int64_t tr_off;    // first tile of its transposed tiles (k_nd_transpose)
+  int64_t k_off;     // m entries of the child map: update entries of both children
   int64_t emap_off;  // b entries: local dof in the parent of each boundary dof
   int32_t p, b;      // pivot and boundary dofs
   int32_t tp, tb;    // the same in tiles of 64
@@ -59,7 +60,7 @@ class NdBottom {
   void factor(const double* ST, hipStream_t st);
   // u = A^-1 b on the level's vectors (inactive nodes: u = b), FP64 inside
   template <class T>
-  void solve(int nb, const T* b, T* u, hipStream_t st);
+  void solve(const T* b, T* u, hipStream_t st);
   int64_t dofs() const { return ndof_; }
   size_t device_bytes() const;
   NdStats stats() const;
@@ -72,14 +73,15 @@ class NdBottom {
     std::vector<int> kids;
     std::vector<int64_t> bnd;  // positions of the boundary nodes, ascending
   };
-  void solve_pos(hipStream_t st);
 
   int64_t nnode_ = 0, ndof_ = 0;
   int maxdepth_ = 0;
   std::vector<Front> fr_;
   std::vector<NdFrontDev> fdev_;
   std::vector<int32_t> var_of_;  // slot -> first dof, -1 if inactive
-  std::vector<int64_t> gptr_, gidx_, bidx_;
+  std::vector<int2> kid_;
+  // index of each dof in the level's vectors, and the entries of inactive nodes
+  std::vector<int32_t> vmap_, rest_, bidx_;
   std::vector<int32_t> emap_;
   std::vector<int4> ent_;
   std::vector<int2> items_;
@@ -93,9 +95,9 @@ class NdBottom {
     SweepBatch batch;
   };
   std::vector<Depth> depth_;
-  int64_t ntile_ = 0, npan_ = 0, nid_ = 0, wlen_ = 0, ulen_ = 0;
-  DevMem d_fr_, d_gptr_, d_gidx_, d_bidx_, d_emap_, d_ent_, d_ent_of_, d_items_, d_mats_, d_kids_, d_var_of_;
-  DevMem tiles_, panw_, panx_, dinv_, info_, w_, u_, bx_, x_;
+  int64_t ntile_ = 0, ntr_ = 0, npan_ = 0, nid_ = 0, wlen_ = 0, ulen_ = 0;
+  DevMem d_fr_, d_kid_, d_vmap_, d_rest_, d_bidx_, d_emap_, d_ent_, d_ent_of_, d_items_, d_mats_, d_kids_;
+  DevMem tiles_, tr_, panw_, panx_, dinv_, info_, w_, u_, x_;
 };
 
 }  // namespace spg

@@ -782,7 +782,7 @@ void Solver::bottom(const T* b, T* u) {
     // FP64 factors in both cycles: the FP32 cycle's right-hand side is
     // widened and the solution rounded, as the reference casts the PARDISO
     // result to float (Multigrid_Hierarchy.h:346-372, 439-451)
-    nd_->solve<T>(R.d.nb, b, u, st_);
+    nd_->solve<T>(b, u, st_);
     return;
   }
   const bool f = sizeof(T) == 4;
