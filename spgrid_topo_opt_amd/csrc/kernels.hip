@@ -106,6 +106,11 @@ __device__ __forceinline__ int xcd_chunk(int h, int n) {
   const int q = n >> 3, r = n & 7, x = h & 7, i = h >> 3;
   return (x < r ? x * (q + 1) : r * (q + 1) + (x - r) * q) + i;
 }
+// the same chunks, each from its end if rev
+__device__ __forceinline__ int xcd_chunk(int h, int n, bool rev) {
+  const int q = n >> 3, r = n & 7, x = h & 7, i = h >> 3, len = q + (x < r ? 1 : 0);
+  return (x < r ? x * (q + 1) : r * (q + 1) + (x - r) * q) + (rev ? len - 1 - i : i);
+}
 __device__ __forceinline__ int ring_side(int x) { return x < 0 ? 0 : (x > 3 ? 2 : 1); }
 __device__ __forceinline__ int ring_spoke(int x, int y, int z) {
   return ring_side(x) * 9 + ring_side(y) * 3 + ring_side(z);
@@ -843,12 +848,39 @@ __device__ __forceinline__ T quad_sum(T x) {
   return x;
 }
 
-// One colour of the level-0 sweep with 4 lanes per node: a wavefront owns
-// the colour-c nodes of 2 blocks; lane (k, q) adds the rows of colour node k
-// in its cells with corners I = q and q|4 (the reflection form of
-// corner_row), the quad sums, and lane q = 0 updates the node.  A 256-thread
-// workgroup stages the 5^3 halos of its 8 blocks.  Same race argument as
+// four consecutive values of a vector, 16-byte aligned
+__device__ __forceinline__ void load4(const float* __restrict__ p, float (&v)[4]) {
+  const float4 q = *reinterpret_cast<const float4*>(p);
+  v[0] = q.x;
+  v[1] = q.y;
+  v[2] = q.z;
+  v[3] = q.w;
+}
+__device__ __forceinline__ void load4(const double* __restrict__ p, double (&v)[4]) {
+  const double2 q = reinterpret_cast<const double2*>(p)[0], r = reinterpret_cast<const double2*>(p)[1];
+  v[0] = q.x;
+  v[1] = q.y;
+  v[2] = r.x;
+  v[3] = r.y;
+}
+
+// One colour of the level-0 sweep with 4 lanes per node: 32 threads own the 8
+// colour-c nodes of a block; lane (k, q) adds the rows of colour node k in its
+// cells with corners I = q and q|4 (the reflection form of corner_row), the
+// quad sums, and lane q = 0 updates the node.  Same race argument as
 // k_gs0_colour.
+// The 5^3 node halo comes in as 25 columns along z: four of a column's five
+// nodes are consecutive in one block (a vector load), the fifth is the next
+// block's nearest; the 4^3 cells likewise as 16 columns.  With that, fixed
+// offsets from four staged corner nodes and opposite directions of
+// neighbouring colours (a launch starts where the last one ended, on what the
+// caches still hold: 4 of 117 and 7 of 186 us a launch on the band), a sweep takes,
+// FP32 / FP64, where single-node staging took the first figures:
+//   128x64x64 box, 9.5 K blocks      62 / 82 -> 54 / 73 us
+//   256^3 shell, 82.8 K blocks       286 / 465 -> 258 / 427 us
+//   512x256x256 band, 246 K blocks   1067 -> 905 us FP32, 1429 us FP64
+// FP32 keeps the VALUs 94% busy (479 instructions a wave); the FP64 band moves
+// 805 MB a launch at 4.5 TB/s, what a copy reaches.
 // With `dist` given, only nodes at distance >= dmin from the boundary band
 // are updated (the far part of a sweep that runs beside the band phase).
 template <class T, int QB>
@@ -858,47 +890,52 @@ __global__ void __launch_bounds__(32 * QB) k_gs0_colour4(int nb, int colour, con
                                                          const uint8_t* __restrict__ dist, int dmin,
                                                          const T* __restrict__ bcm = nullptr,
                                                          const uint8_t* __restrict__ fcm = nullptr) {
-  static_assert(QB >= 4, "the 125-entry halo table is filled by one pass of the workgroup");
-  __shared__ T hu[QB][3][128];
+  constexpr int XS = 25, YS = 5, CS = 128;  // strides of the staged nodes: x, y (z 1), component
+  __shared__ T hu[QB][3 * CS];
+  __shared__ T he[QB][64];
   __shared__ int ht[QB][27];
-  __shared__ int htab[128];
   const int tid = threadIdx.x;
-  const int blk0 = xcd_chunk(blockIdx.x, gridDim.x) * QB;
+  const int blk0 = xcd_chunk(blockIdx.x, gridDim.x, (colour & 1) != 0) * QB;
   const int px = (colour >> 2) & 1, py = (colour >> 1) & 1, pz = colour & 1;
   if (tid < QB * 27) {
     const int bl = tid / 27, sp = tid - bl * 27, blk = blk0 + bl;
     ht[bl][sp] = blk < nb ? (sp == 13 ? blk : nbr[blk * 27 + sp]) : -1;
   }
-  if (tid < 125) htab[tid] = cHaloC[colour * 125 + tid];
-  __syncthreads();
   // lane roles after staging: block bl, node k of the colour, corner pair q
   const int bl = tid >> 5, k = (tid >> 2) & 7, q = tid & 3;
   const int blk = blk0 + bl;
-  const int nx = 2 * ((k >> 2) & 1) + 1, ny = 2 * ((k >> 1) & 1) + 1, nz = 2 * (k & 1) + 1;  // halo coords
-  const int l = loc3(px - 1 + nx, py - 1 + ny, pz - 1 + nz);
-  T ee[2], bv[3] = {T(0), T(0), T(0)};
+  const int kx = (k >> 2) & 1, ky = (k >> 1) & 1, kz = k & 1;
+  const int l = colour_node(colour, k);
+  __syncthreads();
+  T bv[3] = {T(0), T(0), T(0)};
   uint8_t fl = 0;
   bool skip = false;
   {
-    // 32 threads per block stage its 5^3 halo (4 passes, table in LDS).  The
-    // halo loads, this lane's two cell moduli and (lane q = 0) the node's
-    // flags and b are all issued before one wait.
-    const int rs = tid & 31;
-    T v[4][3];
+    const int z0 = pz ? 0 : 1, zx = pz ? 4 : 0;  // places of the four and of the fifth
+    const int ez = pz ? 2 : 0, el = pz ? 0 : 3;  // the fifth's block and local z
+    // threads 0 .. 25 of the 32 take a node column each, 16 a cell column;
+    // every load is issued before one wait
+    const int cid = tid & 31;
+    T v[3][4], w[3], ev[4], ew = T(0);
+    const int cx = px - 1 + cid / 5, cy = py - 1 + cid % 5;
+    const bool col = cid < 25;
+    {
+      const int sp = ring_side(cx) * 9 + ring_side(cy) * 3, o = ((cx & 3) << 4) | ((cy & 3) << 2);
+      const int bm = col ? ht[bl][sp + 1] : -1, bx = col ? ht[bl][sp + ez] : -1;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int hh = rs + 32 * i;
-      const int t = hh < 125 ? htab[hh] : 0;
-      const int bb = hh < 125 ? ht[bl][t >> 8] : -1;
-#pragma unroll
-      for (int c = 0; c < 3; ++c) v[i][c] = bb >= 0 ? u[vidx(bb, c, t & 255)] : T(0);
+      for (int c = 0; c < 3; ++c) {
+        v[c][0] = v[c][1] = v[c][2] = v[c][3] = w[c] = T(0);
+        if (bm >= 0) load4(u + vidx(bm, c, o), v[c]);
+        if (bx >= 0) w[c] = u[vidx(bx, c, o + el)];
+      }
     }
-#pragma unroll
-    for (int r = 0; r < 2; ++r) {
-      const int I = q | (r << 2);
-      const int ex = px - 1 + nx - ((I >> 2) & 1), ey = py - 1 + ny - ((I >> 1) & 1), ez = pz - 1 + nz - (I & 1);
-      const int eb = ht[bl][ring_spoke(ex, ey, ez)];
-      ee[r] = eb >= 0 ? E[eb * 64 + loc3(ex, ey, ez)] : T(0);
+    {
+      const int e = cid & 15, ex = px - 1 + (e >> 2), ey = py - 1 + (e & 3);
+      const int sp = ring_side(ex) * 9 + ring_side(ey) * 3, o = ((ex & 3) << 4) | ((ey & 3) << 2);
+      const int bm = cid < 16 ? ht[bl][sp + 1] : -1, bx = cid < 16 && !pz ? ht[bl][sp] : -1;
+      ev[0] = ev[1] = ev[2] = ev[3] = T(0);
+      if (bm >= 0) load4(E + bm * 64 + o, ev);
+      if (bx >= 0) ew = E[bx * 64 + o + 3];
     }
     if (q == 0 && blk < nb) {
       if (bcm) {
@@ -914,33 +951,60 @@ __global__ void __launch_bounds__(32 * QB) k_gs0_colour4(int nb, int colour, con
       }
       if (dist) skip = dist[blk * 64 + l] < dmin;
     }
+    if (col) {
+      T* h = hu[bl] + cid * YS;
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
-      if (rs + 32 * i < 125)
+      for (int c = 0; c < 3; ++c) {
 #pragma unroll
-        for (int c = 0; c < 3; ++c) hu[bl][c][rs + 32 * i] = v[i][c];
+        for (int z = 0; z < 4; ++z) h[c * CS + z0 + z] = v[c][z];
+        h[c * CS + zx] = w[c];
+      }
+    }
+    if (cid < 16) {
+      // the cells' z runs from pz - 1: one less than the columns hold
+      T* h = he[bl] + cid * 4;
+      if (pz) {
+#pragma unroll
+        for (int z = 0; z < 4; ++z) h[z] = ev[z];
+      } else {
+        h[0] = ew;
+#pragma unroll
+        for (int z = 0; z < 3; ++z) h[z + 1] = ev[z];
+      }
+    }
   }
   __syncthreads();
-  const T* H = &hu[bl][0][0];
+  const int iy = q >> 1, iz = q & 1;
+  // the node, and one step towards the lane's cells along y and z
+  const int hn = (2 * kx + 1) * XS + (2 * ky + 1) * YS + 2 * kz + 1;
+  const int dy = iy ? -YS : YS, dz = iz ? -1 : 1;
+  const T* H[4] = {hu[bl] + hn, hu[bl] + hn + dz, hu[bl] + hn + dy, hu[bl] + hn + dy + dz};
+  const T* Ec = he[bl] + (2 * kx + 1) * 16 + (2 * ky + 1 - iy) * 4 + 2 * kz + 1 - iz;
+  const T ee[2] = {Ec[0], Ec[-16]};
   T f0 = 0, f1 = 0, f2 = 0;
 #pragma unroll
   for (int r = 0; r < 2; ++r) {
-    const int I = q | (r << 2);
-    const int cx = nx - ((I >> 2) & 1), cy = ny - ((I >> 1) & 1), cz = nz - (I & 1);  // cell corner (halo)
-    auto U = [&](int J, T& v0, T& v1, T& v2) {
-      const int h = ((cx + ((J >> 2) & 1)) * 5 + (cy + ((J >> 1) & 1))) * 5 + (cz + (J & 1));
-      v0 = H[h];
-      v1 = H[128 + h];
-      v2 = H[256 + h];
-    };
-    T g0, g1, g2;
-    corner_row<T>(I, ee[r], U, g0, g1, g2);
-    f0 += g0;
-    f1 += g1;
-    f2 += g2;
+    // corner_row for I = q | 4r: node J of the cell seen from corner I is
+    // I ^ Jp, one step along each axis of which Jp has the bit
+    const T sx = r ? T(-1) : T(1), sy = iy ? T(-1) : T(1), sz = iz ? T(-1) : T(1);
+    T a[3][3] = {{0, 0, 0}, {0, 0, 0}, {0, 0, 0}};
+#pragma unroll
+    for (int Jp = 0; Jp < 8; ++Jp) {
+      const T* p = H[Jp & 3] + ((Jp & 4) ? (r ? -XS : XS) : 0);
+      const T x[3] = {p[0], p[CS], p[2 * CS]};
+      const int kb = Jp * 9;
+#pragma unroll
+      for (int v = 0; v < 3; ++v)
+#pragma unroll
+        for (int c = 0; c < 3; ++c) a[v][c] = fmaT(KT<T>::k(kb + 3 * v + c), x[c], a[v][c]);
+    }
+    const T ex = sx * ee[r], ey = sy * ee[r], ez = sz * ee[r];
+    f0 += sx * fmaT(ex, a[0][0], fmaT(ey, a[0][1], ez * a[0][2]));
+    f1 += sy * fmaT(ex, a[1][0], fmaT(ey, a[1][1], ez * a[1][2]));
+    f2 += sz * fmaT(ex, a[2][0], fmaT(ey, a[2][1], ez * a[2][2]));
   }
   // self block: corners q and q|4 differ in the x mirror only
-  const T sy = (q & 2) ? T(-1) : T(1), sz = (q & 1) ? T(-1) : T(1);
+  const T sy = iy ? T(-1) : T(1), sz = iz ? T(-1) : T(1);
   const T es = ee[0] + ee[1], ed = ee[0] - ee[1];
   f0 = dx * quad_sum(f0);
   f1 = dx * quad_sum(f1);
@@ -949,8 +1013,8 @@ __global__ void __launch_bounds__(32 * QB) k_gs0_colour4(int nb, int colour, con
           Syz = dx * quad_sum(sy * sz * es);
   if (q != 0 || blk >= nb || skip) return;
   T d[6] = {KT<T>::k(0) * S, KT<T>::k(4) * S, KT<T>::k(8) * S, KT<T>::k(1) * Sxy, KT<T>::k(2) * Sxz, KT<T>::k(5) * Syz};
-  const int hn = (nx * 5 + ny) * 5 + nz;
-  gs_node_update_b<T>(fl, d, f0, f1, f2, blk, l, H[hn], H[128 + hn], H[256 + hn], bv[0], bv[1], bv[2], u);
+  const T* n = H[0];
+  gs_node_update_b<T>(fl, d, f0, f1, f2, blk, l, n[0], n[CS], n[2 * CS], bv[0], bv[1], bv[2], u);
 }
 
 // Level-0 update of list node `s` (blk*64+l) by the 8 lanes of an octet,
