@@ -644,7 +644,7 @@ __device__ __forceinline__ T octet_sum(T x) {
 // needed and they are wave-uniform (scalar registers).  `U(J)` returns the 3
 // components of the cell's node J.  Result: the 3 rows times e (no dx).
 template <class T, class LoadU>
-__device__ __forceinline__ void corner_row(int I, T e, const LoadU& U, T& f0, T& f1, T& f2) {
+__device__ __forceinline__ void corner_row(int I, T e, const LoadU& U, T& f0, T& f1, T& f2, int k0 = 0) {
   const T sx = (I & 4) ? T(-1) : T(1), sy = (I & 2) ? T(-1) : T(1), sz = (I & 1) ? T(-1) : T(1);
   // partial sums per (row v, component w); the signs s_v s_w apply once at the end
   T a[3][3] = {{0, 0, 0}, {0, 0, 0}, {0, 0, 0}};
@@ -652,7 +652,7 @@ __device__ __forceinline__ void corner_row(int I, T e, const LoadU& U, T& f0, T&
   for (int Jp = 0; Jp < 8; ++Jp) {
     T v[3];
     U(I ^ Jp, v[0], v[1], v[2]);
-    const int kb = Jp * 9;
+    const int kb = k0 + Jp * 9;
 #pragma unroll
     for (int r = 0; r < 3; ++r)
 #pragma unroll
@@ -2149,163 +2149,193 @@ __global__ void __launch_bounds__(64) k_bnd_flow(BndOff L, ColourOrder ord, Colo
 }
 
 // Full Gauss-Seidel sweep of a small level by data flow: one launch instead of
-// one per colour, a one-wave workgroup per block (an octet of lanes per node,
-// lane g loading spokes g, g+8, g+16, g+24).  A neighbour of a colour later in the sweep still holds
-// its old value in u, since its update waits for this node's; one of an
-// earlier colour is taken from its tagged entry once that carries this
-// launch's `epoch`.  Every node of a block publishes, active or not.  As in
-// k_bnd_flow waits are on earlier steps only and bounded.  Bound by one
-// store-to-load hop per colour step; the next step's loads that need no wait go
-// out before the wait.
-// Sweep by flow / by launches back to back, FP32 and FP64: level 0 23 / 35 and
-// 28 / 48 us at 45 blocks, 30 / 36 us at 1377 (FP32); explicit levels 23 / 37
-// and 26 / 42 us at 225 blocks, 25 / 33 and 30 / 42 us at 441.
-// Most blocks, all resident together: half of what the registers let the 256
-// CUs hold (level 0: 4 and 2 waves per SIMD in FP32 and FP64, explicit levels 2
-// and 1).
+// one per colour, a one-wave workgroup per block.  The wave stages the block's
+// 6^3 node halo (and what else the rows need without waiting) once; after
+// each colour step it publishes the 8 nodes it has updated as tagged entries
+// and takes the up to 19 nodes of that colour around the block from theirs, a
+// word per lane, as soon as they carry this launch's `epoch`.  Every node of a
+// block publishes, active or not, so neighbouring blocks stay within one step.
+// The halo's first values come from u, which a block writes when it is done:
+// a value that is still needed belongs to a node whose update waits for this
+// block's first entries, and those go out after the halo is staged.  As in
+// k_bnd_flow waits are on earlier steps only and bounded.  Bound by a
+// store-to-load hop and one row evaluation per colour step (1.3 us); an octet
+// of lanes gathering each node's neighbours from u and the entries in every
+// step, 12 loads a lane for FP32, took 2.4 us.
+// Sweep in us, FP32 / FP64: this, by octet gather, by colour launches
+//   level 0, 45 blocks       15 / 17    24 / 29    33 / 41
+//            1377 blocks     21 / 39    30 / -     35 / 43
+//            3024 blocks     29 / 46    -          41 / 48
+//            2057 blocks     24 / 49    -          36 / 45
+//   explicit, 84 blocks      16 / 17    24 / 29
+//            251 blocks      17 / 18    23 / 26    37 / 42
+//            1229 blocks     25 / -     -          46 / 57
+// The lines: where the launches win (FP64 level 0), or half of the blocks that
+// the registers let the 256 CUs hold at once, so that two solvers' launches
+// fit beside each other.
 template <class T>
 struct FlowBlocks {
-  static constexpr int gs0 = sizeof(T) == 4 ? 2048 : 1024;
-  static constexpr int st = sizeof(T) == 4 ? 1024 : 512;
+  static constexpr int gs0 = sizeof(T) == 4 ? 4096 : 1536;
+  static constexpr int st = sizeof(T) == 4 ? 1536 : 1024;
 };
-template <class T>
-struct SweepFetch {
-  T x[4][3];    // plain values (own and later colours)
-  int slot[4];  // -1 absent
-  T b[3], di[6];
-  int blk, l;   // the octet's node
-  int early;    // bit t: spoke t waits for the tagged entry
-  uint8_t fl;
-};
-// the part that waits for nothing; `shfl` needs the whole wave
-template <class T>
-__device__ __forceinline__ void sweep_fetch(SweepFetch<T>& F, int blk, int colour, unsigned early_colours, int nb_l,
-                                            const uint8_t* __restrict__ flags, const T* __restrict__ u,
-                                            const T* __restrict__ b) {
-  const int lane = threadIdx.x, k = lane >> 3, g = lane & 7;
-  const int l = colour_node(colour, k), li = l >> 4, lj = (l >> 2) & 3, lk = l & 3;
-  F.blk = blk;
-  F.l = l;
-  F.early = 0;
-#pragma unroll
-  for (int t = 0; t < 4; ++t) {
-    const int s = g + 8 * t;
-    const int ox = s / 9 - 1, oy = (s / 3) % 3 - 1, oz = s % 3 - 1;
-    const int x = li + ox, y = lj + oy, z = lk + oz;
-    const int sp = s < 27 ? ring_spoke(x, y, z) : 13;
-    const int bb = __shfl(nb_l, sp);
-    F.slot[t] = s < 27 && bb >= 0 ? bb * 64 + loc3(x, y, z) : -1;
-    const int c2 = colour ^ (((ox & 1) << 2) | ((oy & 1) << 1) | (oz & 1));
-    if (F.slot[t] >= 0 && ((early_colours >> c2) & 1)) F.early |= 1 << t;
-#pragma unroll
-    for (int c = 0; c < 3; ++c)
-      F.x[t][c] = F.slot[t] >= 0 && !((F.early >> t) & 1) ? u[vidx(F.slot[t] >> 6, c, F.slot[t] & 63)] : T(0);
-  }
-  F.fl = 0;
-  F.b[0] = F.b[1] = F.b[2] = T(0);
-  if (g == 5) {
-    F.fl = flags[blk * 64 + l];
-#pragma unroll
-    for (int c = 0; c < 3; ++c) F.b[c] = b[vidx(blk, c, l)];
-  }
+// order of a wave's own LDS accesses: they execute in order, only the
+// compiler has to keep them so
+__device__ __forceinline__ void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
 }
-// waits for the earlier colours' entries; false after a time-out
+// place of the block's node l in its 6^3 halo
+__device__ __forceinline__ int halo_pos(int l) { return ((l >> 4) + 1) * 36 + (((l >> 2) & 3) + 1) * 6 + (l & 3) + 1; }
+// the 6^3 node halo of block blk in hu (component stride 216) and its
+// neighbour row in ht
 template <class T>
-__device__ __forceinline__ bool sweep_wait(SweepFetch<T>& F, unsigned epoch, const TagWord* tu, int* err,
-                                           unsigned long long limit) {
-  constexpr int W = TagPack<T>::W, NW = 3 * W;
+__device__ __forceinline__ void sweep_stage(int blk, const int* __restrict__ nbr, const T* u, T* hu, int* ht) {
+  const int lane = threadIdx.x;
+  int tab[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) tab[i] = lane + 64 * i < 216 ? cHalo6[lane + 64 * i] : -1;
+  if (lane < 27) ht[lane] = lane == 13 ? blk : nbr[blk * 27 + lane];
+  wave_lds_fence();
+  T v[4][3];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int bb = tab[i] >= 0 ? ht[tab[i] >> 8] : -1;
+#pragma unroll
+    for (int c = 0; c < 3; ++c) v[i][c] = bb >= 0 ? u[vidx(bb, c, tab[i] & 255)] : T(0);
+  }
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    if (lane + 64 * i < 216)
+#pragma unroll
+      for (int c = 0; c < 3; ++c) hu[c * 216 + lane + 64 * i] = v[i][c];
+}
+// the nodes of a colour around the block, from their tagged entries into the
+// halo; false after a time-out
+template <class T>
+__device__ __forceinline__ bool sweep_take(int colour, const int* ht, T* hu, const TagWord* tu, unsigned epoch,
+                                           int* err, unsigned long long limit) {
+  constexpr int W = TagPack<T>::W, NW = 3 * W, H = (NW + 1) / 2;
+  // lanes j and j + 32 share the words of node j of the 3^3 of that colour
+  const int j = threadIdx.x & 31, half = threadIdx.x >> 5;
+  const int px = (colour >> 2) & 1, py = (colour >> 1) & 1, pz = colour & 1;
+  const int x = 2 * (j / 9) - px, y = 2 * ((j / 3) % 3) - py, z = 2 * (j % 3) - pz;
+  const bool own = (unsigned)x < 4u && (unsigned)y < 4u && (unsigned)z < 4u;
+  const int bb = j < 27 && !own ? ht[ring_spoke(x, y, z)] : -1;
+  const TagWord* p = tu + ((size_t)bb * 64 + loc3(x, y, z)) * NW + half * H;
+  TagWord w[H];
   unsigned long long t0 = 0;
   for (bool first = true;; first = false) {
     bool ok = true;
 #pragma unroll
-    for (int t = 0; t < 4; ++t) {
-      if (!((F.early >> t) & 1)) continue;
-      TagWord w[NW];
-#pragma unroll
-      for (int k = 0; k < NW; ++k) w[k] = tag_load(tu + (size_t)F.slot[t] * NW + k);
-#pragma unroll
-      for (int k = 0; k < NW; ++k) ok = ok && (unsigned)(w[k] >> 32) == epoch;
-#pragma unroll
-      for (int v = 0; v < 3; ++v) TagPack<T>::get(w + v * W, F.x[t][v]);
+    for (int k = 0; k < H; ++k) {
+      w[k] = tag_word(0u, epoch);
+      if (bb >= 0 && half * H + k < NW) w[k] = tag_load(p + k);
     }
-    if (__all(ok)) return true;
+#pragma unroll
+    for (int k = 0; k < H; ++k) ok = ok && (unsigned)(w[k] >> 32) == epoch;
+    if (__all(ok)) break;
     if (first) t0 = wall_clock64();
     else if (wall_clock64() - t0 > limit) {
       if (threadIdx.x == 0) __hip_atomic_fetch_or(err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       return false;
     }
   }
+  typedef unsigned __attribute__((may_alias)) Half;
+  Half* h = reinterpret_cast<Half*>(hu);
+  const int pos = (x + 1) * 36 + (y + 1) * 6 + z + 1;
+#pragma unroll
+  for (int k = 0; k < H; ++k) {
+    const int i = half * H + k;
+    if (bb >= 0 && i < NW) h[((i / W) * 216 + pos) * W + i % W] = (unsigned)w[k];
+  }
+  return true;
 }
-// the node's update by lane g = 5 (spoke 13 = (g 5, t 1) is the node itself),
-// published and stored
+// u += D^-1 (b - f) of one node at halo position pos, published
 template <class T>
-__device__ __forceinline__ void sweep_update(const SweepFetch<T>& F, T f0, T f1, T f2, unsigned epoch, TagWord* tu,
-                                             T* __restrict__ u) {
-  constexpr int W = TagPack<T>::W, NW = 3 * W;
-  if ((threadIdx.x & 7) != 5) return;
-  T n0 = F.x[1][0], n1 = F.x[1][1], n2 = F.x[1][2];
-  const T* d = F.di;
-  if (F.fl & 1) {
-    const T r0 = F.b[0] - f0, r1 = F.b[1] - f1, r2 = F.b[2] - f2;
+__device__ __forceinline__ void sweep_node(uint8_t fl, const T (&d)[6], const T (&b)[3], T f0, T f1, T f2, T* hu,
+                                           int pos, unsigned epoch, TagWord* p) {
+  constexpr int W = TagPack<T>::W;
+  T n0 = hu[pos], n1 = hu[216 + pos], n2 = hu[432 + pos];
+  if (fl & 1) {
+    const T r0 = b[0] - f0, r1 = b[1] - f1, r2 = b[2] - f2;
     n0 += d[0] * r0 + d[3] * r1 + d[4] * r2;
     n1 += d[3] * r0 + d[1] * r1 + d[5] * r2;
     n2 += d[4] * r0 + d[5] * r1 + d[2] * r2;
   }
-  if (F.fl & 2) n0 = T(0);
-  if (F.fl & 4) n1 = T(0);
-  if (F.fl & 8) n2 = T(0);
-  TagWord* p = tu + (size_t)(F.blk * 64 + F.l) * NW;
+  if (fl & 2) n0 = T(0);
+  if (fl & 4) n1 = T(0);
+  if (fl & 8) n2 = T(0);
   TagPack<T>::put(p, n0, epoch);
   TagPack<T>::put(p + W, n1, epoch);
   TagPack<T>::put(p + 2 * W, n2, epoch);
-  if (F.fl & 0x0F) {
-    u[vidx(F.blk, 0, F.l)] = n0;
-    u[vidx(F.blk, 1, F.l)] = n1;
-    u[vidx(F.blk, 2, F.l)] = n2;
-  }
+  hu[pos] = n0;
+  hu[216 + pos] = n1;
+  hu[432 + pos] = n2;
 }
-// colours that come before step st in the sweep, as a mask
-__device__ __forceinline__ unsigned colours_before(const ColourOrder& ord, int st) {
-  unsigned m = 0;
-  for (int i = 0; i < st; ++i) m |= 1u << ord.at(i);
-  return m;
+// the finished block
+template <class T>
+__device__ __forceinline__ void sweep_store(int blk, const T* hu, T* u) {
+  const int l = threadIdx.x, pos = halo_pos(l);
+  wave_lds_fence();
+#pragma unroll
+  for (int c = 0; c < 3; ++c) u[vidx(blk, c, l)] = hu[c * 216 + pos];
 }
 
-// explicit level: rows from the stored stencils
+// explicit level: rows from the stored stencils, an octet of lanes per node,
+// lane g adding spokes g, g+8, g+16, g+24; the next step's stencils are loaded
+// before the wait
 template <class T>
 struct StFlow {
-  SweepFetch<T> f;
-  T m[36];
+  T m[36], b[3], di[6];
+  uint8_t fl;
 };
 template <class T>
 __global__ void __launch_bounds__(64) k_st_flow(ColourOrder ord, const int* __restrict__ nbr,
                                                 const uint8_t* __restrict__ flags, const T* __restrict__ ST, T* u,
                                                 const T* __restrict__ b, TagWord* tu, unsigned epoch, int* err,
                                                 unsigned long long limit) {
+  __shared__ T hu[3 * 216];
+  __shared__ int ht[28];
   const int lane = threadIdx.x, k = lane >> 3, g = lane & 7, blk = blockIdx.x;
-  const int nb_l = lane == 13 ? blk : (lane < 27 ? nbr[blk * 27 + lane] : -1);
   auto fetch = [&](StFlow<T>& F, int st) {
-    const int c = ord.at(st);
+    const int c = ord.at(st), l = colour_node(c, k);
     const T* S = ST + ((int64_t)blk * 8 + c) * 1944;
 #pragma unroll
     for (int e = 0; e < 27; ++e) F.m[e] = S[e * 64 + lane];
 #pragma unroll
     for (int e = 0; e < 9; ++e) F.m[27 + e] = g < 3 ? S[1728 + e * 24 + k * 3 + g] : T(0);
-    sweep_fetch<T>(F.f, blk, c, colours_before(ord, st), nb_l, flags, u, b);
+    F.fl = 0;
+    F.b[0] = F.b[1] = F.b[2] = T(0);
+    if (g == 5) {
+      F.fl = flags[blk * 64 + l];
+#pragma unroll
+      for (int v = 0; v < 3; ++v) F.b[v] = b[vidx(blk, v, l)];
+    }
   };
-  auto update = [&](StFlow<T>& F) -> bool {
+  // LDS step from the node to each of the lane's spokes
+  int off[4];
+#pragma unroll
+  for (int t = 0; t < 4; ++t) {
+    const int s = g + 8 * t;
+    off[t] = s < 27 ? (s / 9 - 1) * 36 + ((s / 3) % 3 - 1) * 6 + s % 3 - 1 : 0;
+  }
+  auto update = [&](StFlow<T>& F, int st) -> bool {
     if (g == 5) {
       const T* m = F.m + 9;
-      T* d = F.f.di;
+      T* d = F.di;
       d[0] = m[0]; d[1] = m[4]; d[2] = m[8]; d[3] = m[1]; d[4] = m[2]; d[5] = m[5];
-      if (F.f.fl & 1) dirichlet_inverse(d, F.f.fl);
+      if (F.fl & 1) dirichlet_inverse(d, F.fl);
     }
-    if (!sweep_wait<T>(F.f, epoch, tu, err, limit)) return false;
+    if (st && !sweep_take<T>(ord.at(st - 1), ht, hu, tu, epoch, err, limit)) return false;
+    wave_lds_fence();
+    const int l = colour_node(ord.at(st), k), pos = halo_pos(l);
     T a0 = 0, a1 = 0, a2 = 0;
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
       const T* m = F.m + t * 9;
-      const T* x = F.f.x[t];
+      T x[3];
+#pragma unroll
+      for (int v = 0; v < 3; ++v) x[v] = g + 8 * t < 27 ? hu[v * 216 + pos + off[t]] : T(0);
       a0 = fmaT(m[0], x[0], a0);
       a0 = fmaT(m[1], x[1], a0);
       a0 = fmaT(m[2], x[2], a0);
@@ -2319,93 +2349,90 @@ __global__ void __launch_bounds__(64) k_st_flow(ColourOrder ord, const int* __re
     a0 = octet_sum(a0);
     a1 = octet_sum(a1);
     a2 = octet_sum(a2);
-    sweep_update<T>(F.f, a0, a1, a2, epoch, tu, u);
+    // lane g = 5 holds spoke 13, the node itself
+    if (g == 5)
+      sweep_node<T>(F.fl, F.di, F.b, a0, a1, a2, hu, pos, epoch, tu + (size_t)(blk * 64 + l) * (3 * TagPack<T>::W));
     return true;
   };
   StFlow<T> X, Y;
   fetch(X, 0);
+  sweep_stage<T>(blk, nbr, u, hu, ht);
   for (int st = 0; st < 8; st += 2) {
     fetch(Y, st + 1);
-    if (!update(X)) return;
+    if (!update(X, st)) return;
     if (st + 2 < 8) fetch(X, st + 2);
-    if (!update(Y)) return;
+    if (!update(Y, st + 1)) return;
   }
+  sweep_store<T>(blk, hu, u);
 }
 
-// level 0: matrix-free rows, lane I = g adding the cell of which the node is
-// corner I; the 27 neighbours pass through LDS
-template <class T>
-struct Gs0Flow {
-  SweepFetch<T> f;
-  T e;
-};
+// level 0: matrix-free rows, an octet of lanes per node, lane I adding the
+// cell of which the node is corner I.  Lane (k, g) keeps b, flags and the
+// inverse self block of node k of colour g and updates it in that colour's
+// step.
 template <class T>
 __global__ void __launch_bounds__(64) k_gs0_flow(ColourOrder ord, const int* __restrict__ nbr,
                                                  const uint8_t* __restrict__ flags, const T* __restrict__ E, T dx, T* u,
                                                  const T* __restrict__ b, TagWord* tu, unsigned epoch, int* err,
                                                  unsigned long long limit) {
-  constexpr int HS = 85;  // row stride of an octet's 27 x 3 values
-  __shared__ T hs[8 * HS];
+  __shared__ T hu[3 * 216];
+  __shared__ T he[128];
+  __shared__ int ht[28];
   const int lane = threadIdx.x, k = lane >> 3, I = lane & 7, blk = blockIdx.x;
-  const int nb_l = lane == 13 ? blk : (lane < 27 ? nbr[blk * 27 + lane] : -1);
-  const int ix = (I >> 2) & 1, iy = (I >> 1) & 1, iz = I & 1;
-  T* H = hs + k * HS;
-  auto fetch = [&](Gs0Flow<T>& F, int st) {
-    const int c = ord.at(st);
-    sweep_fetch<T>(F.f, blk, c, colours_before(ord, st), nb_l, flags, u, b);
-    const int l = F.f.l, cx = (l >> 4) - ix, cy = ((l >> 2) & 3) - iy, cz = (l & 3) - iz;
-    const int eb = __shfl(nb_l, ring_spoke(cx, cy, cz));
-    F.e = eb >= 0 ? E[eb * 64 + loc3(cx, cy, cz)] : T(0);
-  };
-  auto update = [&](Gs0Flow<T>& F) -> bool {
-    const T e = F.e;
-    {
-      // the inverse self block, before the wait
-      const T sx = ix ? T(-1) : T(1), sy = iy ? T(-1) : T(1), sz = iz ? T(-1) : T(1);
-      const T S = dx * octet_sum(e), Sxy = dx * octet_sum(sx * sy * e), Sxz = dx * octet_sum(sx * sz * e),
-              Syz = dx * octet_sum(sy * sz * e);
-      T* d = F.f.di;
-      d[0] = KT<T>::k(0) * S;
-      d[1] = KT<T>::k(4) * S;
-      d[2] = KT<T>::k(8) * S;
-      d[3] = KT<T>::k(1) * Sxy;
-      d[4] = KT<T>::k(2) * Sxz;
-      d[5] = KT<T>::k(5) * Syz;
-      if (F.f.fl & 1) dirichlet_inverse(d, F.f.fl);
+  const int l0 = colour_node(I, k);
+  const uint8_t fl = flags[blk * 64 + l0];
+  T bv[3], di[6];
+#pragma unroll
+  for (int c = 0; c < 3; ++c) bv[c] = b[vidx(blk, c, l0)];
+  sweep_stage<T>(blk, nbr, u, hu, ht);
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+    if (lane + 64 * i < 125) {
+      const int t = cHalo5[lane + 64 * i], bb = ht[t >> 8];
+      he[lane + 64 * i] = bb >= 0 ? E[bb * 64 + (t & 255)] : T(0);
     }
-    if (!sweep_wait<T>(F.f, epoch, tu, err, limit)) return false;
-    // a wavefront's LDS operations execute in order: its last reads of hs are
-    // done before these writes, and the writes before the reads below
-    __builtin_amdgcn_wave_barrier();
+  wave_lds_fence();
+  {
+    const T* ec = he + (l0 >> 4) * 25 + ((l0 >> 2) & 3) * 5 + (l0 & 3);  // cell of corner 7
+    T e[8];
 #pragma unroll
-    for (int t = 0; t < 4; ++t)
-      if (I + 8 * t < 27)
-#pragma unroll
-        for (int v = 0; v < 3; ++v) H[(I + 8 * t) * 3 + v] = F.f.x[t][v];
-    __builtin_amdgcn_wave_barrier();
-    asm volatile("" ::: "memory");
+    for (int J = 0; J < 8; ++J) e[J] = ec[(J & 4 ? 0 : 25) + (J & 2 ? 0 : 5) + (J & 1 ? 0 : 1)];
+    const T p0 = e[0] + e[7], p1 = e[1] + e[6], p2 = e[2] + e[5], p3 = e[3] + e[4];
+    const T S = dx * ((p0 + p1) + (p2 + p3)), Sxy = dx * ((p0 + p1) - (p2 + p3)),
+            Sxz = dx * ((p0 + p2) - (p1 + p3)), Syz = dx * ((p0 + p3) - (p1 + p2));
+    di[0] = KT<T>::k(0) * S;
+    di[1] = KT<T>::k(4) * S;
+    di[2] = KT<T>::k(8) * S;
+    di[3] = KT<T>::k(1) * Sxy;
+    di[4] = KT<T>::k(2) * Sxz;
+    di[5] = KT<T>::k(5) * Syz;
+    if (fl & 1) dirichlet_inverse(di, fl);
+  }
+  const int ix = (I >> 2) & 1, iy = (I >> 1) & 1, iz = I & 1;
+  for (int st = 0; st < 8; ++st) {
+    // FP64: the constants are read again in each step, kept over the steps
+    // they would spill
+    int k0 = 0;
+    if constexpr (sizeof(T) == 8) asm volatile("" : "+s"(k0));
+    const int c = ord.at(st), l = colour_node(c, k), pos = halo_pos(l);
+    const T e = he[((l >> 4) + 1 - ix) * 25 + (((l >> 2) & 3) + 1 - iy) * 5 + (l & 3) + 1 - iz];
+    if (st && !sweep_take<T>(ord.at(st - 1), ht, hu, tu, epoch, err, limit)) return;
+    wave_lds_fence();
     auto U = [&](int J, T& v0, T& v1, T& v2) {
-      const int sp = (((J >> 2) & 1) - ix + 1) * 9 + (((J >> 1) & 1) - iy + 1) * 3 + ((J & 1) - iz + 1);
-      v0 = H[sp * 3];
-      v1 = H[sp * 3 + 1];
-      v2 = H[sp * 3 + 2];
+      const int h = pos + (((J >> 2) & 1) - ix) * 36 + (((J >> 1) & 1) - iy) * 6 + (J & 1) - iz;
+      v0 = hu[h];
+      v1 = hu[216 + h];
+      v2 = hu[432 + h];
     };
     T f0, f1, f2;
-    corner_row<T>(I, e, U, f0, f1, f2);
+    corner_row<T>(I, e, U, f0, f1, f2, k0);
     f0 = dx * octet_sum(f0);
     f1 = dx * octet_sum(f1);
     f2 = dx * octet_sum(f2);
-    sweep_update<T>(F.f, f0, f1, f2, epoch, tu, u);
-    return true;
-  };
-  Gs0Flow<T> X, Y;
-  fetch(X, 0);
-  for (int st = 0; st < 8; st += 2) {
-    fetch(Y, st + 1);
-    if (!update(X)) return;
-    if (st + 2 < 8) fetch(X, st + 2);
-    if (!update(Y)) return;
+    if (I == c)
+      sweep_node<T>(fl, di, bv, f0, f1, f2, hu, pos, epoch, tu + (size_t)(blk * 64 + l) * (3 * TagPack<T>::W));
   }
+  sweep_store<T>(blk, hu, u);
 }
 
 // workgroup size of the boundary phase: two register sets of BndFetch per lane

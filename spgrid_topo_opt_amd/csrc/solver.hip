@@ -40,7 +40,7 @@ static double now_s() {
 static constexpr int kMaxDenseBoundary = 2560;
 // levels of at most this many blocks get the entries of the data-flow sweep
 // (FlowBlocks in kernels.hip has each kernel's own limit)
-static constexpr int kMaxFlowSweep = 2048;
+static constexpr int kMaxFlowSweep = 4096;
 // pcg() result: a level-0 boundary phase reported a barrier time-out; the
 // pass is repeated with the per-colour list launches
 static constexpr int kCoopRetry = -100;

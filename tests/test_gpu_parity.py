@@ -358,10 +358,10 @@ def test_dense_map_and_data_flow_match_step_by_step(level, shape, monkeypatch):
 
 
 @pytest.mark.parametrize("shape,levels,blocks", [((3, 3, 3), 1, 1), ((45, 23, 19), 3, 360), ((64, 32, 32), 3, 1377),
-                                                 ((64, 43, 43), 3, 2057)])
+                                                 ((64, 43, 43), 3, 2057), ((64, 64, 64), 3, 4913)])
 def test_data_flow_sweep_matches_colour_launches(shape, levels, blocks, monkeypatch):
-    """a level-0 sweep in one launch (small levels; 1377 blocks only in FP32,
-    2057 blocks not) against the octet colour kernel, whose arithmetic it
+    """a level-0 sweep in one launch (small levels; 2057 blocks only in FP32,
+    4913 blocks not) against the octet colour kernel, whose arithmetic it
     shares: FP64 to 1e-13, FP32 to 1e-6 relative"""
     s = _lib.Solver(W.box(*shape, seed=6, mg_levels=levels))
     assert s.level_blocks(0) == blocks
