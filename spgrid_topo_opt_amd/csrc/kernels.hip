@@ -2186,15 +2186,15 @@ __device__ __forceinline__ void wave_lds_fence() {
 }
 // place of the block's node l in its 6^3 halo
 __device__ __forceinline__ int halo_pos(int l) { return ((l >> 4) + 1) * 36 + (((l >> 2) & 3) + 1) * 6 + (l & 3) + 1; }
-// the 6^3 node halo of block blk in hu (component stride 216) and its
-// neighbour row in ht
+// the 6^3 node halo of a block in hu (component stride 216) and its neighbour
+// row, of which lane i < 27 brings slot i, in ht
 template <class T>
-__device__ __forceinline__ void sweep_stage(int blk, const int* __restrict__ nbr, const T* u, T* hu, int* ht) {
+__device__ __forceinline__ void sweep_stage(int nb_l, const T* u, T* hu, int* ht) {
   const int lane = threadIdx.x;
   int tab[4];
 #pragma unroll
   for (int i = 0; i < 4; ++i) tab[i] = lane + 64 * i < 216 ? cHalo6[lane + 64 * i] : -1;
-  if (lane < 27) ht[lane] = lane == 13 ? blk : nbr[blk * 27 + lane];
+  if (lane < 27) ht[lane] = nb_l;
   wave_lds_fence();
   T v[4][3];
 #pragma unroll
@@ -2209,18 +2209,21 @@ __device__ __forceinline__ void sweep_stage(int blk, const int* __restrict__ nbr
 #pragma unroll
       for (int c = 0; c < 3; ++c) hu[c * 216 + lane + 64 * i] = v[i][c];
 }
-// the nodes of a colour around the block, from their tagged entries into the
-// halo; false after a time-out
-template <class T>
-__device__ __forceinline__ bool sweep_take(int colour, const int* ht, T* hu, const TagWord* tu, unsigned epoch,
-                                           int* err, unsigned long long limit) {
+// the nodes of a colour around the block, from their tagged entries (of blocks
+// `id`; with MASK only the nodes in the blocks' bit masks `hm`) into the halo
+// once they carry `tag` or a later one; false after a time-out
+template <class T, bool MASK>
+__device__ __forceinline__ bool sweep_take(int colour, const int* id, const unsigned long long* hm, T* hu,
+                                           const TagWord* tu, unsigned tag, int* err, unsigned long long limit) {
   constexpr int W = TagPack<T>::W, NW = 3 * W, H = (NW + 1) / 2;
   // lanes j and j + 32 share the words of node j of the 3^3 of that colour
   const int j = threadIdx.x & 31, half = threadIdx.x >> 5;
   const int px = (colour >> 2) & 1, py = (colour >> 1) & 1, pz = colour & 1;
   const int x = 2 * (j / 9) - px, y = 2 * ((j / 3) % 3) - py, z = 2 * (j % 3) - pz;
   const bool own = (unsigned)x < 4u && (unsigned)y < 4u && (unsigned)z < 4u;
-  const int bb = j < 27 && !own ? ht[ring_spoke(x, y, z)] : -1;
+  const int sp = ring_spoke(x, y, z);
+  int bb = j < 27 && !own ? id[sp] : -1;
+  if (MASK && bb >= 0 && !((hm[sp] >> loc3(x, y, z)) & 1)) bb = -1;
   const TagWord* p = tu + ((size_t)bb * 64 + loc3(x, y, z)) * NW + half * H;
   TagWord w[H];
   unsigned long long t0 = 0;
@@ -2228,11 +2231,11 @@ __device__ __forceinline__ bool sweep_take(int colour, const int* ht, T* hu, con
     bool ok = true;
 #pragma unroll
     for (int k = 0; k < H; ++k) {
-      w[k] = tag_word(0u, epoch);
+      w[k] = tag_word(0u, tag);
       if (bb >= 0 && half * H + k < NW) w[k] = tag_load(p + k);
     }
 #pragma unroll
-    for (int k = 0; k < H; ++k) ok = ok && (unsigned)(w[k] >> 32) == epoch;
+    for (int k = 0; k < H; ++k) ok = ok && (int)((unsigned)(w[k] >> 32) - tag) >= 0;
     if (__all(ok)) break;
     if (first) t0 = wall_clock64();
     else if (wall_clock64() - t0 > limit) {
@@ -2326,7 +2329,7 @@ __global__ void __launch_bounds__(64) k_st_flow(ColourOrder ord, const int* __re
       d[0] = m[0]; d[1] = m[4]; d[2] = m[8]; d[3] = m[1]; d[4] = m[2]; d[5] = m[5];
       if (F.fl & 1) dirichlet_inverse(d, F.fl);
     }
-    if (st && !sweep_take<T>(ord.at(st - 1), ht, hu, tu, epoch, err, limit)) return false;
+    if (st && !sweep_take<T, false>(ord.at(st - 1), ht, nullptr, hu, tu, epoch, err, limit)) return false;
     wave_lds_fence();
     const int l = colour_node(ord.at(st), k), pos = halo_pos(l);
     T a0 = 0, a1 = 0, a2 = 0;
@@ -2356,7 +2359,7 @@ __global__ void __launch_bounds__(64) k_st_flow(ColourOrder ord, const int* __re
   };
   StFlow<T> X, Y;
   fetch(X, 0);
-  sweep_stage<T>(blk, nbr, u, hu, ht);
+  sweep_stage<T>(lane == 13 ? blk : lane < 27 ? nbr[blk * 27 + lane] : -1, u, hu, ht);
   for (int st = 0; st < 8; st += 2) {
     fetch(Y, st + 1);
     if (!update(X, st)) return;
@@ -2371,6 +2374,59 @@ __global__ void __launch_bounds__(64) k_st_flow(ColourOrder ord, const int* __re
 // inverse self block of node k of colour g and updates it in that colour's
 // step.
 template <class T>
+struct Gs0Own {
+  T b[3], di[6];
+  uint8_t fl;
+};
+// the block's 5^3 cells in he; before it the node's b and flags, after it the
+// inverse self blocks
+template <class T>
+__device__ __forceinline__ void gs0_stage(Gs0Own<T>& O, int blk, const int* ht, const T* __restrict__ E, T dx, T* he) {
+  const int lane = threadIdx.x, l0 = colour_node(lane & 7, lane >> 3);
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+    if (lane + 64 * i < 125) {
+      const int t = cHalo5[lane + 64 * i], bb = ht[t >> 8];
+      he[lane + 64 * i] = bb >= 0 ? E[bb * 64 + (t & 255)] : T(0);
+    }
+  wave_lds_fence();
+  const T* ec = he + (l0 >> 4) * 25 + ((l0 >> 2) & 3) * 5 + (l0 & 3);  // cell of corner 7
+  T e[8];
+#pragma unroll
+  for (int J = 0; J < 8; ++J) e[J] = ec[(J & 4 ? 0 : 25) + (J & 2 ? 0 : 5) + (J & 1 ? 0 : 1)];
+  const T p0 = e[0] + e[7], p1 = e[1] + e[6], p2 = e[2] + e[5], p3 = e[3] + e[4];
+  const T S = dx * ((p0 + p1) + (p2 + p3)), Sxy = dx * ((p0 + p1) - (p2 + p3)), Sxz = dx * ((p0 + p2) - (p1 + p3)),
+          Syz = dx * ((p0 + p3) - (p1 + p2));
+  O.di[0] = KT<T>::k(0) * S;
+  O.di[1] = KT<T>::k(4) * S;
+  O.di[2] = KT<T>::k(8) * S;
+  O.di[3] = KT<T>::k(1) * Sxy;
+  O.di[4] = KT<T>::k(2) * Sxz;
+  O.di[5] = KT<T>::k(5) * Syz;
+  if (O.fl & 1) dirichlet_inverse(O.di, O.fl);
+}
+// the rows of the octets' nodes l at halo positions pos; every lane of an
+// octet has the result
+template <class T>
+__device__ __forceinline__ void gs0_rows(int l, int pos, const T* he, const T* hu, T dx, T& f0, T& f1, T& f2) {
+  const int I = threadIdx.x & 7, ix = (I >> 2) & 1, iy = (I >> 1) & 1, iz = I & 1;
+  // FP64: the constants are read again in each step, kept over the steps
+  // they would spill
+  int k0 = 0;
+  if constexpr (sizeof(T) == 8) asm volatile("" : "+s"(k0));
+  const T e = he[((l >> 4) + 1 - ix) * 25 + (((l >> 2) & 3) + 1 - iy) * 5 + (l & 3) + 1 - iz];
+  auto U = [&](int J, T& v0, T& v1, T& v2) {
+    const int h = pos + (((J >> 2) & 1) - ix) * 36 + (((J >> 1) & 1) - iy) * 6 + (J & 1) - iz;
+    v0 = hu[h];
+    v1 = hu[216 + h];
+    v2 = hu[432 + h];
+  };
+  corner_row<T>(I, e, U, f0, f1, f2, k0);
+  f0 = dx * octet_sum(f0);
+  f1 = dx * octet_sum(f1);
+  f2 = dx * octet_sum(f2);
+}
+template <class T>
 __global__ void __launch_bounds__(64) k_gs0_flow(ColourOrder ord, const int* __restrict__ nbr,
                                                  const uint8_t* __restrict__ flags, const T* __restrict__ E, T dx, T* u,
                                                  const T* __restrict__ b, TagWord* tu, unsigned epoch, int* err,
@@ -2380,59 +2436,79 @@ __global__ void __launch_bounds__(64) k_gs0_flow(ColourOrder ord, const int* __r
   __shared__ int ht[28];
   const int lane = threadIdx.x, k = lane >> 3, I = lane & 7, blk = blockIdx.x;
   const int l0 = colour_node(I, k);
-  const uint8_t fl = flags[blk * 64 + l0];
-  T bv[3], di[6];
+  Gs0Own<T> O;
+  O.fl = flags[blk * 64 + l0];
 #pragma unroll
-  for (int c = 0; c < 3; ++c) bv[c] = b[vidx(blk, c, l0)];
-  sweep_stage<T>(blk, nbr, u, hu, ht);
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-    if (lane + 64 * i < 125) {
-      const int t = cHalo5[lane + 64 * i], bb = ht[t >> 8];
-      he[lane + 64 * i] = bb >= 0 ? E[bb * 64 + (t & 255)] : T(0);
-    }
-  wave_lds_fence();
-  {
-    const T* ec = he + (l0 >> 4) * 25 + ((l0 >> 2) & 3) * 5 + (l0 & 3);  // cell of corner 7
-    T e[8];
-#pragma unroll
-    for (int J = 0; J < 8; ++J) e[J] = ec[(J & 4 ? 0 : 25) + (J & 2 ? 0 : 5) + (J & 1 ? 0 : 1)];
-    const T p0 = e[0] + e[7], p1 = e[1] + e[6], p2 = e[2] + e[5], p3 = e[3] + e[4];
-    const T S = dx * ((p0 + p1) + (p2 + p3)), Sxy = dx * ((p0 + p1) - (p2 + p3)),
-            Sxz = dx * ((p0 + p2) - (p1 + p3)), Syz = dx * ((p0 + p3) - (p1 + p2));
-    di[0] = KT<T>::k(0) * S;
-    di[1] = KT<T>::k(4) * S;
-    di[2] = KT<T>::k(8) * S;
-    di[3] = KT<T>::k(1) * Sxy;
-    di[4] = KT<T>::k(2) * Sxz;
-    di[5] = KT<T>::k(5) * Syz;
-    if (fl & 1) dirichlet_inverse(di, fl);
-  }
-  const int ix = (I >> 2) & 1, iy = (I >> 1) & 1, iz = I & 1;
+  for (int c = 0; c < 3; ++c) O.b[c] = b[vidx(blk, c, l0)];
+  sweep_stage<T>(lane == 13 ? blk : lane < 27 ? nbr[blk * 27 + lane] : -1, u, hu, ht);
+  gs0_stage<T>(O, blk, ht, E, dx, he);
   for (int st = 0; st < 8; ++st) {
-    // FP64: the constants are read again in each step, kept over the steps
-    // they would spill
-    int k0 = 0;
-    if constexpr (sizeof(T) == 8) asm volatile("" : "+s"(k0));
     const int c = ord.at(st), l = colour_node(c, k), pos = halo_pos(l);
-    const T e = he[((l >> 4) + 1 - ix) * 25 + (((l >> 2) & 3) + 1 - iy) * 5 + (l & 3) + 1 - iz];
-    if (st && !sweep_take<T>(ord.at(st - 1), ht, hu, tu, epoch, err, limit)) return;
+    if (st && !sweep_take<T, false>(ord.at(st - 1), ht, nullptr, hu, tu, epoch, err, limit)) return;
     wave_lds_fence();
-    auto U = [&](int J, T& v0, T& v1, T& v2) {
-      const int h = pos + (((J >> 2) & 1) - ix) * 36 + (((J >> 1) & 1) - iy) * 6 + (J & 1) - iz;
-      v0 = hu[h];
-      v1 = hu[216 + h];
-      v2 = hu[432 + h];
-    };
     T f0, f1, f2;
-    corner_row<T>(I, e, U, f0, f1, f2, k0);
-    f0 = dx * octet_sum(f0);
-    f1 = dx * octet_sum(f1);
-    f2 = dx * octet_sum(f2);
+    gs0_rows<T>(l, pos, he, hu, dx, f0, f1, f2);
     if (I == c)
-      sweep_node<T>(fl, di, bv, f0, f1, f2, hu, pos, epoch, tu + (size_t)(blk * 64 + l) * (3 * TagPack<T>::W));
+      sweep_node<T>(O.fl, O.di, O.b, f0, f1, f2, hu, pos, epoch, tu + (size_t)(blk * 64 + l) * (3 * TagPack<T>::W));
   }
   sweep_store<T>(blk, hu, u);
+}
+
+// Level-0 boundary phase by data flow: the sweep kernel's scheme over the
+// blocks that hold boundary nodes (fb_* in LevelDev), for several sweeps of
+// which only the boundary nodes are updated, published (tag `last` + sweep + 1)
+// and stored; the others keep what the halo holds.  A wave may run ahead of a
+// neighbouring block only in nodes that no boundary node of that block
+// touches, so a later tag than the one waited for is as good.
+// Bound by 1.4 us a colour step: a load of the entries (0.6 us, at times two
+// or three until the neighbours' are there) and the row.  A phase of 3 sweeps,
+// FP32 / FP64 us, against k_bnd_rhs and k_bnd_flow: 38.6 / 43.0 and 46.7 / 62.9
+// at 855 nodes, 41.8 / 48.8 and 53.1 / 82.3 at 12,675.  Two loads half a round
+// trip apart gave 37 / 44 and twice the time of a sweep of 3000 blocks; all
+// but the last colour's part of the row before the wait 44 / 45; a pause
+// between the loads 40 / 43.
+template <class T>
+__global__ void __launch_bounds__(64) k_gs0_bnd_flow(ColourOrder ord, int sweeps, const int* __restrict__ fblk,
+                                                     const int* __restrict__ fnbr, const int* __restrict__ fid,
+                                                     const unsigned long long* __restrict__ fmask,
+                                                     const uint8_t* __restrict__ flags, const T* __restrict__ E, T dx,
+                                                     T* u, const T* __restrict__ b, TagWord* tu, unsigned last,
+                                                     int* err, unsigned long long limit) {
+  __shared__ T hu[3 * 216];
+  __shared__ T he[128];
+  __shared__ unsigned long long hm[28];
+  __shared__ int ht[28], id[28];
+  const int lane = threadIdx.x, k = lane >> 3, I = lane & 7, i = blockIdx.x, blk = fblk[i];
+  const int l0 = colour_node(I, k);
+  Gs0Own<T> O;
+  O.fl = flags[blk * 64 + l0];
+#pragma unroll
+  for (int c = 0; c < 3; ++c) O.b[c] = b[vidx(blk, c, l0)];
+  int nb_l = -1;
+  if (lane < 27) {
+    nb_l = fnbr[i * 27 + lane];
+    id[lane] = fid[i * 27 + lane];
+    hm[lane] = fmask[i * 27 + lane];
+  }
+  sweep_stage<T>(nb_l, u, hu, ht);
+  gs0_stage<T>(O, blk, ht, E, dx, he);
+  const unsigned long long own = hm[13];
+  for (int st = 0; st < 8 * sweeps; ++st) {
+    const int c = ord.at(st & 7), l = colour_node(c, k), pos = halo_pos(l);
+    if (st && !sweep_take<T, true>(ord.at((st - 1) & 7), id, hm, hu, tu, last + ((st - 1) >> 3) + 1, err, limit)) return;
+    wave_lds_fence();
+    const bool set = (own >> l) & 1;
+    if (!__any(set)) continue;
+    T f0, f1, f2;
+    gs0_rows<T>(l, pos, he, hu, dx, f0, f1, f2);
+    if (I == c && set)
+      sweep_node<T>(O.fl, O.di, O.b, f0, f1, f2, hu, pos, last + (st >> 3) + 1,
+                    tu + (size_t)(i * 64 + l) * (3 * TagPack<T>::W));
+  }
+  wave_lds_fence();
+  if ((own >> lane) & 1)
+#pragma unroll
+    for (int c = 0; c < 3; ++c) u[vidx(blk, c, lane)] = hu[c * 216 + halo_pos(lane)];
 }
 
 // workgroup size of the boundary phase: two register sets of BndFetch per lane
@@ -3350,6 +3426,38 @@ static bool launch_bnd_flow(hipStream_t st, const LevelDev& L, T* u, const T* b,
                hipGetErrorString(e));
   return false;
 }
+// level-0 boundary phase over blocks (k_gs0_bnd_flow); false as above.  A cap
+// on the workgroups needs the node-list kernel.
+template <class T>
+static bool launch_gs0_bnd_flow(hipStream_t st, const LevelDev& L, const T* E, T dx, T* u, const T* b, int sweeps,
+                                bool forward, bool loud) {
+  if (!L.fb_last || !L.coop || L.coop_off || L.fb_n > FlowBlocks<T>::gs0) return false;
+  if (const char* e = std::getenv("SPG_COOP_WG"))
+    if (std::atoi(e) > 0) return false;
+  ColourOrder ord = colour_order(true, forward);
+  TagWord* tu = static_cast<TagWord*>(L.fb_tag);
+  int* err = reinterpret_cast<int*>(L.coop + 1);
+  unsigned last = *L.fb_last;
+  unsigned long long lim = flow_wait_limit();
+  *L.fb_last += (unsigned)sweeps;
+  const char* cl = std::getenv("SPG_COOP_LAUNCH");
+  if (!(cl && std::atoi(cl) == 1)) {
+    k_gs0_bnd_flow<T><<<L.fb_n, 64, 0, st>>>(ord, sweeps, L.fb_blk, L.fb_nbr, L.fb_id, L.fb_mask, L.flags, E, dx, u, b,
+                                            tu, last, err, lim);
+    return true;
+  }
+  const int *fblk = L.fb_blk, *fnbr = L.fb_nbr, *fid = L.fb_id;
+  const unsigned long long* fmask = L.fb_mask;
+  const uint8_t* flags = L.flags;
+  void* args[] = {&ord, &sweeps, &fblk, &fnbr, &fid, &fmask, &flags, &E, &dx, &u, &b, &tu, &last, &err, &lim};
+  const hipError_t e = hipLaunchCooperativeKernel((const void*)k_gs0_bnd_flow<T>, dim3(L.fb_n), dim3(64), args, 0, st);
+  if (e == hipSuccess) return true;
+  (void)hipGetLastError();
+  if (loud)
+    std::fprintf(stderr, "spgrid_topo_opt_amd: cooperative boundary phase not launched (%s); using the list path\n",
+                 hipGetErrorString(e));
+  return false;
+}
 template <class T>
 struct BmapPtr;
 template <>
@@ -3508,12 +3616,14 @@ void launch_gs0_boundary(hipStream_t st, const LevelDev& L, const T* E, T dx, T*
   if (sweeps <= 0 || L.bnd_off[8] == 0) return;
   int path = boundary_path();
   // Automatic choice beyond the dense map (solver.hip has that line), FP32 per phase of 3 sweeps on the 256^3 shell (3655
-  // boundary nodes): data flow 45 us, grid barriers between the steps 87 us,
-  // per-colour list launches 145 us, single workgroup 154 us (one CU's VALU
-  // work).  The lists remain for a refused cooperative launch and after a
+  // boundary nodes): data flow over blocks 40 us, over node groups 47 us (the
+  // way for more blocks than FlowBlocks has), grid barriers between the steps
+  // 87 us, per-colour list launches 145 us, single workgroup 154 us (one CU's
+  // VALU work).  The lists remain for a refused cooperative launch and after a
   // time-out.
   if (path == 0 && launch_bnd_map<T>(st, L, u, b, sweeps, forward)) return;
   if (path == 0 || path == 5) {
+    if (launch_gs0_bnd_flow<T>(st, L, E, dx, u, b, sweeps, forward, path == 5)) return;
     if (launch_bnd_flow<T>(st, L, u, b, sweeps, true, forward, path == 5)) return;
     path = 2;
   }

@@ -56,6 +56,17 @@ struct LevelDev {
   // precision) and {unused, error word}
   void* btag = nullptr;
   unsigned* coop = nullptr;
+  // level-0 boundary phase by data flow over the blocks that hold boundary
+  // nodes: their number and slots, per block the slots of its 27 neighbours,
+  // those blocks' places in this list (-1 if not in it) and the bit masks of
+  // their boundary nodes, the tagged entries [fb_n*64*6] and the last tag given
+  int fb_n = 0;
+  const int* fb_blk = nullptr;
+  const int* fb_nbr = nullptr;
+  const int* fb_id = nullptr;
+  const unsigned long long* fb_mask = nullptr;
+  void* fb_tag = nullptr;
+  unsigned* fb_last = nullptr;
   int coop_off = 0;  // 1 after a wait timed out: the list launches take over
   // slots of all neighbours of the boundary nodes ([n*32], in or outside the
   // set), and dense maps of one boundary phase (forward, backward colour

@@ -236,6 +236,42 @@ void Solver::upload_layout() {
         R.d.coop = lv_[0].coop.as<unsigned>();  // one error word for every level
       }
     }
+    if (l == 0 && !bnd.empty()) {
+      // the blocks that hold boundary nodes
+      std::vector<int32_t> id((size_t)D.nb, -1), blk;
+      for (const int32_t s : bnd) id[(size_t)(s >> 6)] = 0;
+      for (int64_t i = 0; i < D.nb; ++i)
+        if (id[(size_t)i] == 0) {
+          id[(size_t)i] = (int32_t)blk.size();
+          blk.push_back((int32_t)i);
+        }
+      if (blk.size() <= (size_t)kMaxFlowSweep) {
+        std::vector<unsigned long long> own(blk.size(), 0), mask(blk.size() * 27, 0);
+        for (const int32_t s : bnd) own[(size_t)id[(size_t)(s >> 6)]] |= 1ull << (s & 63);
+        std::vector<int32_t> nb27(blk.size() * 27), id27(blk.size() * 27, -1);
+        for (size_t i = 0; i < blk.size(); ++i)
+          for (int k = 0; k < 27; ++k) {
+            const int32_t q = k == 13 ? blk[i] : D.nbr[(size_t)blk[i] * 27 + k];
+            nb27[i * 27 + k] = q;
+            if (q < 0 || id[(size_t)q] < 0) continue;
+            id27[i * 27 + k] = id[(size_t)q];
+            mask[i * 27 + k] = own[(size_t)id[(size_t)q]];
+          }
+        upload(R.fb_blk, blk);
+        upload(R.fb_nbr, nb27);
+        upload(R.fb_id, id27);
+        upload(R.fb_mask, mask);
+        R.fb_tag.alloc(blk.size() * 64 * 6 * 8);
+        HIPCHK(hipMemset(R.fb_tag.p, 0, R.fb_tag.bytes));
+        R.d.fb_n = (int)blk.size();
+        R.d.fb_blk = R.fb_blk.as<int>();
+        R.d.fb_nbr = R.fb_nbr.as<int>();
+        R.d.fb_id = R.fb_id.as<int>();
+        R.d.fb_mask = R.fb_mask.as<unsigned long long>();
+        R.d.fb_tag = R.fb_tag.p;
+        R.d.fb_last = &R.fb_last;
+      }
+    }
     if (!D.bnd_cslot.empty()) {
       upload(R.b0cslot, D.bnd_cslot);
       upload(R.b0node, D.bnd_cnode);

@@ -56,6 +56,8 @@ struct LevelRT {
   DBuf ball, bmap64[2], bmap32[2], bmx64, bmx32;     // dense boundary maps
   DBuf stag;                                         // data-flow sweep: tagged entries
   unsigned epoch = 0;                                // its launches so far
+  DBuf fb_blk, fb_nbr, fb_id, fb_mask, fb_tag;       // data-flow boundary phase: blocks, tagged entries
+  unsigned fb_last = 0;                              // last tag given
   DBuf bnslot;                                       // level 0: neighbour slots of boundary nodes
   DBuf gsdist, gsnear, gsnslot;                      // level 0: band distances, near-band step lists, their slots
   int64_t gsnear_off[17] = {};                       // list (dir * 8 + step) = gsnear[off[i] .. off[i+1])

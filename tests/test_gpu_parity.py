@@ -333,10 +333,12 @@ def test_boundary_phase_multi_sweep(blocky, path, monkeypatch):
                 assert rel(got, want) < tol, (lv, fwd, prec)
 
 
-@pytest.mark.parametrize("level,shape", [(0, (12, 8, 8)), (0, (12, 22, 21)), (0, (12, 22, 22)), (2, (24, 92, 92))])
+@pytest.mark.parametrize("level,shape", [(0, (12, 8, 8)), (0, (12, 22, 21)), (0, (12, 22, 22)), (0, (12, 160, 160)),
+                                         (2, (24, 92, 92))])
 def test_dense_map_and_data_flow_match_step_by_step(level, shape, monkeypatch):
     """the automatic boundary phase (level-0 sets of 405 and 2530 nodes: dense
-    map, 2645 nodes and an explicit-level set of 2880: data flow) against the
+    map, 2645 nodes and an explicit-level set of 2880: data flow, 129,605 on
+    level 0: by node groups in FP64) against the
     colour steps one after the other, from an iterate that is not zero at the
     Dirichlet components; FP64 to 1e-11, FP32 to 1e-4 relative (sums of up to
     7590 products in another order)"""
