@@ -2748,15 +2748,26 @@ __device__ inline void cg_stage(CgScalars* sc, int stage) {
     sc->singular = 0;
   }
 }
+__device__ inline void cg_report(const CgReport& rep, double nrm, int singular) {
+  const unsigned long long b = (unsigned long long)__double_as_longlong(nrm);
+  const unsigned part[kReportWords] = {(unsigned)b, (unsigned)(b >> 32),
+                                       (singular ? 1u : 0u) | (rep.err && *rep.err ? 2u : 0u)};
+#pragma unroll
+  for (int i = 0; i < kReportWords; ++i)
+    __hip_atomic_store(rep.host + i, ((unsigned long long)rep.seq << 32) | part[i], __ATOMIC_RELAXED,
+                       __HIP_MEMORY_SCOPE_SYSTEM);
+}
 template <int OP>
 __global__ void __launch_bounds__(RED_T) k_final(const double* part, int np, double* out, CgScalars* sc = nullptr,
-                                                 int stage = -1) {
+                                                 int stage = -1, CgReport rep = CgReport(),
+                                                 const CgScalars* rsc = nullptr) {
   double s = 0.0;
   for (int i = threadIdx.x; i < np; i += blockDim.x) s = OP == 0 ? s + part[i] : fmax(s, part[i]);
   s = block_reduce<OP>(s);
   if (threadIdx.x == 0) {
     *out = s;
     if (sc) cg_stage(sc, stage);
+    if (rep.host) cg_report(rep, s, rsc->singular);
   }
 }
 
@@ -3719,10 +3730,11 @@ void launch_dot(hipStream_t st, const T* a, const T* b, int64_t n, double* parti
   k_final<0><<<1, RED_T, 0, st>>>(partial, (int)g, out);
 }
 template <class T>
-void launch_linf(hipStream_t st, const T* a, int64_t n, double* partial, double* out) {
+void launch_linf(hipStream_t st, const T* a, int64_t n, double* partial, double* out, const CgReport& rep,
+                 const CgScalars* sc) {
   const unsigned g = red_grid(n);
   k_linf_part<T><<<g, RED_T, 0, st>>>(a, n, partial);
-  k_final<1><<<1, RED_T, 0, st>>>(partial, (int)g, out);
+  k_final<1><<<1, RED_T, 0, st>>>(partial, (int)g, out, nullptr, -1, rep, sc);
 }
 void launch_sumsq(hipStream_t st, const double* a, int64_t n, double* partial, double* out) {
   const unsigned g = red_grid(n);
@@ -3735,12 +3747,12 @@ void launch_cg_direction(hipStream_t st, T* s, const T* z, const CgScalars* sc, 
 }
 template <class T>
 void launch_cg_update(hipStream_t st, T* x, T* r, const T* s, const T* q, CgScalars* sc, int64_t n, int stage,
-                      T* zclear) {
+                      T* zclear, const CgReport& rep) {
   // caller passes the partial buffer right after the scalars block
   double* part = reinterpret_cast<double*>(sc + 1);
   const unsigned g = red_grid(n);
   k_cg_update<T><<<g, RED_T, 0, st>>>(x, r, s, q, sc, n, part, zclear);
-  k_final<1><<<1, RED_T, 0, st>>>(part, (int)g, &sc->nrm, stage >= 0 ? sc : nullptr, stage);
+  k_final<1><<<1, RED_T, 0, st>>>(part, (int)g, &sc->nrm, stage >= 0 ? sc : nullptr, stage, rep, sc);
 }
 void launch_cg_scalars(hipStream_t st, CgScalars* sc, int stage) { k_cg_scalars<<<1, 64, 0, st>>>(sc, stage); }
 template <class T>
@@ -3855,9 +3867,11 @@ void launch_set_entries(hipStream_t st, double* v, const int* idx, const double*
   template void launch_copy<T>(hipStream_t, const T*, T*, int64_t);                                              \
   template void launch_axpy_d<T>(hipStream_t, double*, const T*, int64_t);                                       \
   template void launch_dot<T>(hipStream_t, const T*, const T*, int64_t, double*, double*);                       \
-  template void launch_linf<T>(hipStream_t, const T*, int64_t, double*, double*);                                \
+  template void launch_linf<T>(hipStream_t, const T*, int64_t, double*, double*, const CgReport&,                \
+                               const CgScalars*);                                \
   template void launch_cg_direction<T>(hipStream_t, T*, const T*, const CgScalars*, int64_t);                    \
-  template void launch_cg_update<T>(hipStream_t, T*, T*, const T*, const T*, CgScalars*, int64_t, int, T*);    \
+  template void launch_cg_update<T>(hipStream_t, T*, T*, const T*, const T*, CgScalars*, int64_t, int, T*,     \
+                                    const CgReport&);                                                           \
   template void launch_project<T>(hipStream_t, const LevelDev&, T*, bool);                                       \
   template void launch_project_dot<T>(hipStream_t, const LevelDev&, T*, const T*, double*, double*, CgScalars*,  \
                                       int);                                                                     \

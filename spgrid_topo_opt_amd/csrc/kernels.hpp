@@ -113,6 +113,18 @@ struct CgScalars {
   int pad;
 };
 
+// What a PCG iteration's last kernel tells the host: words of pinned host
+// memory that carry a 32-bit part of the report and the report's number
+// (halves of ||r||_inf; bit 0 singular, bit 1 a data-flow wait timed out, from
+// `err`).  The host reads them as they arrive, without a copy or a
+// synchronisation.
+struct CgReport {
+  unsigned long long* host = nullptr;
+  unsigned seq = 0;
+  const int* err = nullptr;
+};
+static constexpr int kReportWords = 3;
+
 // The element matrix K0 = mu K_mu + lambda K_la and the halo tables, in the
 // device's constant memory (one set per device: Solver::activate uploads
 // its material's before its kernels run).  Synchronous.
@@ -183,14 +195,15 @@ int64_t reduce_partials(int64_t n);
 template <class T>
 void launch_dot(hipStream_t st, const T* a, const T* b, int64_t n, double* partial, double* out);
 template <class T>
-void launch_linf(hipStream_t st, const T* a, int64_t n, double* partial, double* out);
+void launch_linf(hipStream_t st, const T* a, int64_t n, double* partial, double* out,
+                 const CgReport& rep = CgReport(), const CgScalars* sc = nullptr);
 void launch_sumsq(hipStream_t st, const double* a, int64_t n, double* partial, double* out);
 // PCG steps (scalars on device)
 template <class T>
 void launch_cg_direction(hipStream_t st, T* s, const T* z, const CgScalars* sc, int64_t n);  // s = beta s + z
 template <class T>
 void launch_cg_update(hipStream_t st, T* x, T* r, const T* s, const T* q, CgScalars* sc, int64_t n, int stage = -1,
-                      T* zclear = nullptr);
+                      T* zclear = nullptr, const CgReport& rep = CgReport());
 void launch_cg_scalars(hipStream_t st, CgScalars* sc, int stage);  // 0: after rho, 1: after sq, 2: end
 // (the reductions above take `sc, stage` to run a stage in their last kernel)
 // projections

@@ -44,8 +44,8 @@ static constexpr int kMaxFlowSweep = 4096;
 // pcg() result: a level-0 boundary phase reported a barrier time-out; the
 // pass is repeated with the per-colour list launches
 static constexpr int kCoopRetry = -100;
-// byte offset of the barrier error word in the pinned scalar buffer
-static constexpr int kCoopWordOffset = 192;
+// byte offset of the PCG report in the pinned scalar buffer
+static constexpr int kReportOffset = 128;
 // relative residual reduction one FP32 MG-PCG pass is asked for at most
 static constexpr double kFp32PassReduction = 1e-6;
 // bottom solve: the dense FP64 inverse up to this many unknowns (one
@@ -357,7 +357,8 @@ void Solver::upload_layout() {
   scal_.alloc(sizeof(CgScalars) + reduce_partials(0) * sizeof(double));
   part_.alloc((reduce_partials(0) + 16) * sizeof(double));
   apart_.alloc(apply_dot_partials(lv_[0].d.nb) * sizeof(double));
-  HIPCHK(hipHostMalloc((void**)&hscal_, 256));
+  HIPCHK(hipHostMalloc((void**)&hscal_, 256, hipHostMallocCoherent));
+  std::memset(hscal_, 0, 256);
 }
 
 // Galerkin position matrices of one depth for this solver's K0, on its
@@ -764,7 +765,7 @@ const T* Solver::colour_major_b(const T* b0) {
 }
 
 template <class T>
-void Solver::smooth(int l, T* u, const T* b, bool forward, const T* bcm) {
+void Solver::smooth(int l, T* u, const T* b, bool forward, const T* bcm, Part part) {
   const LevelRT& R = lv_[l];
   // Multigrid_Hierarchy.h:577-586 / 605-617: boundary sweeps, full sweeps, boundary sweeps
   auto boundary = [&] {
@@ -772,6 +773,10 @@ void Solver::smooth(int l, T* u, const T* b, bool forward, const T* bcm) {
     else launch_st_boundary<T>(st_, R.d, R.st<T>(), u, b, cfg_.boundary_iters, forward);
   };
   int first = 0;
+  if (part == Part::kFirst) {
+    boundary();
+    return;
+  }
   if (l == 0 && overlap_ && R.gsdist.p && cfg_.smooth_iters > 0 && cfg_.boundary_iters > 0) {
     // The boundary phase writes only band nodes.  The first sweep's step-c
     // update of a node farther than c + 1 from the band reads nothing that
@@ -795,7 +800,7 @@ void Solver::smooth(int l, T* u, const T* b, bool forward, const T* bcm) {
                          b);
     }
     first = 1;
-  } else {
+  } else if (part == Part::kAll) {
     boundary();
   }
   for (int i = first; i < cfg_.smooth_iters; ++i) {
@@ -840,7 +845,7 @@ void Solver::bottom(const T* b, T* u) {
 // FP32 cycle whose explicit levels (and bottom) run in FP64: the level
 // handed over is restricted in FP32 and widened, and widened corrections are
 // rounded back before the FP32 prolongation
-void Solver::vcycle_coarse64(const float* b0, float* z, bool z_is_zero) {
+void Solver::vcycle_coarse64(const float* b0, float* z, bool z_is_zero, Part part) {
   const int L = lay_.nlev;
   const int ex = lay_.explicit_level;
   if (!z_is_zero) launch_zero<float>(st_, z, lv_[0].n3);
@@ -858,7 +863,7 @@ void Solver::vcycle_coarse64(const float* b0, float* z, bool z_is_zero) {
     } else {
       float* u = l == 0 ? z : lv_[l].u<float>();
       const float* b = l == 0 ? b0 : lv_[l].b<float>();
-      if (sm) smooth<float>(l, u, b, true, l == 0 ? bcm : nullptr);
+      if (sm) smooth<float>(l, u, b, true, l == 0 ? bcm : nullptr, l == 0 ? part : Part::kAll);
       if (dn) launch_zero<double>(st_, lv_[l + 1].u<double>(), lv_[l + 1].n3);
       else launch_zero<float>(st_, lv_[l + 1].u<float>(), lv_[l + 1].n3);
       if (sm) {
@@ -887,12 +892,20 @@ void Solver::vcycle_coarse64(const float* b0, float* z, bool z_is_zero) {
   }
 }
 
+bool Solver::has_first_part() const {
+  return lay_.use_mg && lay_.nlev > 1 && lay_.explicit_level > 0 && !overlap_ && cfg_.boundary_iters > 0;
+}
+
 template <class T>
-void Solver::vcycle(const T* b0, T* z, bool z_is_zero) {
+void Solver::vcycle(const T* b0, T* z, bool z_is_zero, Part part) {
+  if (part == Part::kFirst) {
+    smooth<T>(0, z, b0, true, nullptr, part);
+    return;
+  }
   const int L = lay_.nlev;
   const int ex = lay_.explicit_level;
   if (sizeof(T) == 4 && coarse64_ && lay_.use_mg && L > ex) {
-    vcycle_coarse64(reinterpret_cast<const float*>(b0), reinterpret_cast<float*>(z), z_is_zero);
+    vcycle_coarse64(reinterpret_cast<const float*>(b0), reinterpret_cast<float*>(z), z_is_zero, part);
     return;
   }
   if (!lay_.use_mg) {
@@ -909,7 +922,7 @@ void Solver::vcycle(const T* b0, T* z, bool z_is_zero) {
     T* u = l == 0 ? z : lv_[l].u<T>();
     const T* b = l == 0 ? b0 : lv_[l].b<T>();
     const bool sm = (l == 0 || l >= ex);
-    if (sm) smooth<T>(l, u, b, true, l == 0 ? bcm : nullptr);
+    if (sm) smooth<T>(l, u, b, true, l == 0 ? bcm : nullptr, l == 0 ? part : Part::kAll);
     // the restriction also clears the coarse iterate
     if (sm) {
       level_residual<T>(l, u, b, lv_[l].r<T>());
@@ -931,6 +944,44 @@ void Solver::vcycle(const T* b0, T* z, bool z_is_zero) {
 // CONJUGATE_GRADIENT_4Ch::Solve (CG/CONJUGATE_GRADIENT.cpp:21-61): projected
 // PCG on x (starting at 0) with the L_inf stop test; scalars stay FP64 on the
 // device, the host reads ||r||_inf once per iteration.
+CgReport Solver::report() {
+  CgReport r;
+  r.host = reinterpret_cast<unsigned long long*>(reinterpret_cast<char*>(hscal_) + kReportOffset);
+  r.seq = ++report_seq_;
+  if (lv_[0].coop.p && !lv_[0].d.coop_off) r.err = lv_[0].coop.as<int>() + 1;
+  return r;
+}
+
+// Each word carries the report's number, so the values are complete once all
+// words do; the stream's state is looked at now and then so that a failed
+// kernel ends the wait.
+void Solver::wait_report(double* nrm, unsigned* bits) {
+  const unsigned long long* w =
+      reinterpret_cast<const unsigned long long*>(reinterpret_cast<const char*>(hscal_) + kReportOffset);
+  unsigned long long v[kReportWords];
+  auto arrived = [&] {
+    bool ok = true;
+    for (int i = 0; i < kReportWords; ++i) {
+      v[i] = __atomic_load_n(w + i, __ATOMIC_ACQUIRE);
+      ok = ok && (unsigned)(v[i] >> 32) == report_seq_;
+    }
+    return ok;
+  };
+  for (unsigned spin = 1; !arrived(); ++spin) {
+    if (spin % 65536 == 0) {
+      const hipError_t e = hipStreamQuery(st_);
+      if (e == hipErrorNotReady) continue;
+      HIPCHK(e);
+      if (!arrived()) throw SpgError(SPG_E_HIP, "PCG: the stream is idle and the residual has not arrived");
+      break;
+    }
+    __builtin_ia32_pause();
+  }
+  const unsigned long long b = (v[0] & 0xffffffffull) | (v[1] << 32);
+  std::memcpy(nrm, &b, sizeof(b));
+  *bits = (unsigned)v[2];
+}
+
 template <class T>
 int Solver::pcg(T* x, T* r, double tol, int maxit, int* iters, double* last_nrm) {
   const LevelRT& R0 = lv_[0];
@@ -945,17 +996,24 @@ int Solver::pcg(T* x, T* r, double tol, int maxit, int* iters, double* last_nrm)
   launch_zero<T>(st_, z, n);
   launch_project<T>(st_, R0.d, r, true);
   launch_cg_scalars(st_, sc, 3);
-  launch_linf<T>(st_, r, n, part, &sc->nrm);
+  launch_linf<T>(st_, r, n, part, &sc->nrm, report(), sc);
   int it = 0;
   int rc = SPG_E_NOT_CONVERGED;
-  unsigned* coop_word = reinterpret_cast<unsigned*>(reinterpret_cast<char*>(hscal_) + kCoopWordOffset);
   const bool coop = lv_[0].coop.p && !lv_[0].d.coop_off;
+  // The next V-cycle's first boundary phase, which changes nothing but z, is
+  // launched before the host reads the residual: the device has work while the
+  // host decides and launches the rest.  With that, and the report written by
+  // the iteration's last kernel instead of two copies and a synchronisation,
+  // the device no longer idles between iterations.
+  const bool split = has_first_part();
+  bool ahead = false;
   for (;; ++it) {
-    HIPCHK(hipMemcpyAsync(hscal_, sc, sizeof(CgScalars), hipMemcpyDeviceToHost, st_));
-    if (coop) HIPCHK(hipMemcpyAsync(coop_word, lv_[0].coop.as<unsigned>() + 1, sizeof(unsigned),
-                                    hipMemcpyDeviceToHost, st_));
-    sync();
-    if (coop && *coop_word) {
+    ahead = split && it < maxit;
+    if (ahead) vcycle<T>(r, z, true, Part::kFirst);
+    double nrm;
+    unsigned bits;
+    wait_report(&nrm, &bits);
+    if (bits & 2) {
       // the last V-cycle's boundary phase ended early: its result is not a
       // Gauss-Seidel sweep.  Switch to the list launches for good and let
       // the caller repeat the pass.
@@ -968,34 +1026,35 @@ int Solver::pcg(T* x, T* r, double tol, int maxit, int* iters, double* last_nrm)
       *iters = it;
       return kCoopRetry;
     }
-    const CgScalars* h = reinterpret_cast<const CgScalars*>(hscal_);
-    *last_nrm = h->nrm;
+    *last_nrm = nrm;
     if (print_residuals_) {
       FILE* o = print_residuals_ == 2 ? stderr : stdout;
-      std::fprintf(o, "%.9g\n", h->nrm);
+      std::fprintf(o, "%.9g\n", nrm);
       std::fflush(o);
     }
-    if (h->singular) {
+    if (bits & 1) {
       rc = SPG_E_SINGULAR;
       break;
     }
-    if (std::isnan(h->nrm)) {
+    if (std::isnan(nrm)) {
       rc = SPG_E_NAN;
       break;
     }
-    if (h->nrm <= tol) {
+    if (nrm <= tol) {
       rc = SPG_OK;
       break;
     }
     if (it == maxit) break;
-    vcycle<T>(r, z, true);  // z was cleared before the loop / by the last update
+    vcycle<T>(r, z, true, ahead ? Part::kRest : Part::kAll);  // z was cleared before the loop / by the last update
     // the scalar stages (beta, alpha, rho_old) run in the last kernel of
     // the reduction they follow
     launch_project_dot<T>(st_, R0.d, z, r, part, &sc->rho, sc, 0);
     launch_cg_direction<T>(st_, s, z, sc, n);
     launch_apply_dot<T>(st_, R0.d, E<T>(), dxT<T>(), s, q, apart_.as<double>(), part, &sc->sq, sc, 1);
-    launch_cg_update<T>(st_, x, r, s, q, sc, n, 2, z);
+    launch_cg_update<T>(st_, x, r, s, q, sc, n, 2, z, report());
   }
+  // a time-out in a phase whose result nobody uses is nobody's error
+  if (ahead && coop) HIPCHK(hipMemsetAsync(lv_[0].coop.as<unsigned>() + 1, 0, sizeof(unsigned), st_));
   *iters = it;
   return rc;
 }
@@ -1461,7 +1520,7 @@ double Solver::bench_kernel(int op, int level, int precision, int arg, int reps)
   return (double)ms * 1e-3 / reps;
 }
 
-template void Solver::vcycle<float>(const float*, float*, bool);
-template void Solver::vcycle<double>(const double*, double*, bool);
+template void Solver::vcycle<float>(const float*, float*, bool, Part);
+template void Solver::vcycle<double>(const double*, double*, bool, Part);
 
 }  // namespace spg

@@ -107,10 +107,16 @@ class Solver {
 
  private:
   // z = M b0; `z_is_zero` says the caller has already cleared z
-  template <class T> void vcycle(const T* b0, T* z, bool z_is_zero = false);
-  void vcycle_coarse64(const float* b0, float* z, bool z_is_zero);
+  // Part: all of it, or its first boundary phase and everything after that
+  // (which the PCG loop launches before and after it has read the residual)
+  enum class Part { kAll, kFirst, kRest };
+  bool has_first_part() const;
+  template <class T> void vcycle(const T* b0, T* z, bool z_is_zero = false, Part part = Part::kAll);
+  CgReport report();                             // for the next report() / wait_report() pair
+  void wait_report(double* nrm, unsigned* bits);  // the last one handed out
+  void vcycle_coarse64(const float* b0, float* z, bool z_is_zero, Part part);
   void pack_records(const int32_t* base, int hdr, uint8_t* dst) const;
-  template <class T> void smooth(int l, T* u, const T* b, bool forward, const T* bcm = nullptr);
+  template <class T> void smooth(int l, T* u, const T* b, bool forward, const T* bcm = nullptr, Part part = Part::kAll);
   // the level-0 colour sweeps read b and the flags from colour-major copies
   // when the level's working set exceeds the memory-side cache (or
   // SPG_GS_CMB=1); returns the copy of b0 to pass, or null
@@ -172,6 +178,7 @@ class Solver {
   DBuf apart_;  // per-workgroup partials of the fused operator apply + dot
   DBuf fcm_, bcm_;  // level-0 flags and b in colour-major order (either precision)
   double* hscal_ = nullptr;
+  unsigned report_seq_ = 0;
   mutable void* stage_ = nullptr;  // pinned staging of the output records
   mutable size_t stage_bytes_ = 0;
   double setup_s_ = 0.0;
