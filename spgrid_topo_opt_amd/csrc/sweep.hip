@@ -15,9 +15,10 @@
 // tiles on the matrix cores (v_mfma_f64_16x16x4), both operands staged in LDS,
 // the result tile in registers.  Small batches are bound by the serial
 // inversion of the diagonal tiles (64 dependent pivots each).  Per density update,
-// against partial Cholesky front by front through rocSOLVER and rocBLAS: 37 ->
-// 2.0 ms (9,006 unknowns, nested dissection), 16 -> 1.1 ms (4,131, nested
-// dissection), 9 -> 1.9 ms (2,016, dense).
+// against partial Cholesky front by front through rocSOLVER and rocBLAS, at the
+// scalar inversion: 37 -> 2.0 ms (9,006 unknowns, nested dissection), 16 -> 1.1
+// ms (4,131, nested dissection), 9 -> 1.9 ms (2,016, dense); the 16x16 blocks
+// take another 0.3 ms from the last two.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -65,38 +66,94 @@ __device__ __forceinline__ void acc_pos(int i, int j, int q, int& row, int& col)
   col = (w & 1) * 32 + j * 16 + (l & 15);
 }
 
-// In place: the 64x64 SPD tile in LDS -> minus its inverse in the tile store,
-// the inverse in dinv; one scalar sweep per pivot, a thread holding 16 rows of
-// one column, the pivot row passed through LDS (one barrier a pivot).
-__device__ void invert_tile(const double (*s)[LD], double (*rowbuf)[64], double* __restrict__ tile,
-                            double* __restrict__ dinv, int* __restrict__ info, int pivot0) {
-  const int w = threadIdx.x >> 6, c = threadIdx.x & 63;
-  double a[16];
+template <int CTRL>
+__device__ __forceinline__ double dpp_d(double x) {
+  const long long v = __double_as_longlong(x);
+  const int lo = __builtin_amdgcn_update_dpp(0, (int)(v & 0xffffffffll), CTRL, 0xF, 0xF, true);
+  const int hi = __builtin_amdgcn_update_dpp(0, (int)(v >> 32), CTRL, 0xF, 0xF, true);
+  return __longlong_as_double(((long long)hi << 32) | (long long)(unsigned)lo);
+}
+// value of one lane, the same for all, in scalar registers
+__device__ __forceinline__ double lane_d(double x, int lane) {
+  const long long v = __double_as_longlong(x);
+  const unsigned lo = __builtin_amdgcn_readlane((int)(v & 0xffffffffll), lane);
+  const unsigned hi = __builtin_amdgcn_readlane((int)(v >> 32), lane);
+  return __longlong_as_double(((long long)hi << 32) | (long long)lo);
+}
+// one scalar sweep of a 16x16 SPD block held by a wave (lane l: rows
+// 4 (l>>4) + i, column l & 15), pivot KK and the following ones; the block
+// becomes minus its inverse
+template <int KK>
+__device__ __forceinline__ void sweep16(double (&a)[4], int& bad, int pivot0) {
+  if constexpr (KK < 16) {
+    const int l = threadIdx.x & 63, g = l >> 4, c = l & 15;
+    constexpr int gk = KK >> 2, ik = KK & 3;
+    const double d = lane_d(a[ik], 16 * gk + KK);
+    const double row = __shfl(a[ik], 16 * gk + c, 64);
+    double ci[4];  // the pivot column: lane KK of each 16 (row_newbcast)
 #pragma unroll
-  for (int i = 0; i < 16; ++i) a[i] = s[16 * w + i][c];
+    for (int i = 0; i < 4; ++i) ci[i] = dpp_d<0x150 + KK>(a[i]);
+    if (!(d > 0.0) && bad == 0) bad = pivot0 + KK + 1;
+    const double inv = 1.0 / d, pr = row * inv;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) a[i] = c == KK ? ci[i] * inv : __builtin_fma(-ci[i], pr, a[i]);
+    if (g == gk) a[ik] = c == KK ? -inv : pr;
+    sweep16<KK + 1>(a, bad, pivot0);
+  }
+}
+
+// The 64x64 SPD tile in LDS -> minus its inverse in the tile store, the
+// inverse in dinv, by the block sweep above with 16x16 blocks.  Every wave
+// inverts the pivot block D (no barrier between its 16 dependent pivots), then
+// wave r takes row block r: W_r^T = D^-1 X_r^T, whose result registers are the
+// left operand of A_rj -= W_r X_j^T when the sum over k runs in the order that
+// they hold.  Two barriers per block.  Against a scalar sweep with a barrier
+// for each of the 64 pivots, a thread holding 16 rows of a column: first tile
+// 33.5 -> 19.1 us, a trailing step with its next diagonal tile 38.0 -> 25.7 us.
+__device__ void invert_tile(double (*s)[LD], double* __restrict__ tile, double* __restrict__ dinv,
+                            int* __restrict__ info, int pivot0) {
+  const int r = threadIdx.x >> 6, l = threadIdx.x & 63, g = l >> 4, c = l & 15;
   int bad = 0;
-  for (int o = 0; o < 4; ++o)
+  for (int K = 0; K < 4; ++K) {
+    const int o = 16 * K;
+    double a[4];
 #pragma unroll
-    for (int kk = 0; kk < 16; ++kk) {
-      const int k = 16 * o + kk;
-      double* rb = rowbuf[k & 1];
-      if (w == o) rb[c] = a[kk];
-      __syncthreads();
-      const double d = rb[k];
-      if (!(d > 0.0) && bad == 0) bad = pivot0 + k + 1;
-      const double inv = 1.0 / d, pr = rb[c] * inv;
+    for (int i = 0; i < 4; ++i) a[i] = s[o + 4 * g + i][o + c];
+    sweep16<0>(a, bad, pivot0 + o);
+    d4 wt = {};
+    if (r != K) {
 #pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        // the pivot column by symmetry
-        const double ci = rb[16 * w + i];
-        a[i] = c == k ? ci * inv : __builtin_fma(-ci, pr, a[i]);
+      for (int i = 0; i < 4; ++i)
+        wt = __builtin_amdgcn_mfma_f64_16x16x4f64(-a[i], s[16 * r + c][o + 4 * g + i], wt, 0, 0, 0);
+      for (int j = 0; j < 4; ++j) {
+        if (j == K) continue;
+        d4 acc;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) acc[q] = s[16 * r + 4 * q + g][16 * j + c];
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+          acc = __builtin_amdgcn_mfma_f64_16x16x4f64(-wt[q], s[16 * j + c][o + 4 * q + g], acc, 0, 0, 0);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) s[16 * r + 4 * q + g][16 * j + c] = acc[q];
       }
-      if (w == o) a[kk] = c == k ? -inv : pr;
     }
+    __syncthreads();  // the panel has been read
+    if (r != K) {
 #pragma unroll
-  for (int i = 0; i < 16; ++i) {
-    tile[(16 * w + i) * 64 + c] = a[i];
-    dinv[(16 * w + i) * 64 + c] = -a[i];
+      for (int q = 0; q < 4; ++q) {
+        s[16 * r + c][o + 4 * q + g] = wt[q];
+        s[o + 4 * q + g][16 * r + c] = wt[q];
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) s[o + 4 * g + i][o + c] = a[i];
+    }
+    __syncthreads();
+  }
+  for (int e = threadIdx.x; e < 4096; e += 256) {
+    const double v = s[e >> 6][e & 63];
+    tile[e] = v;
+    dinv[e] = -v;
   }
   if (threadIdx.x == 0 && bad && *info == 0) *info = bad;
 }
@@ -105,12 +162,11 @@ __device__ void invert_tile(const double (*s)[LD], double (*rowbuf)[64], double*
 __global__ void __launch_bounds__(256) k_sw_first(const SweepMat* __restrict__ mats, double* tiles, double* dinv,
                                                   int* info) {
   __shared__ __align__(16) double s[64][LD];
-  __shared__ double rowbuf[2][64];
   const SweepMat M = mats[blockIdx.x];
   double* t = tiles + M.off * 4096;
   stage(t, s, 1.0);
   __syncthreads();
-  invert_tile(s, rowbuf, t, dinv + (int64_t)M.id * 4096, info + M.id, 0);
+  invert_tile(s, t, dinv + (int64_t)M.id * 4096, info + M.id, 0);
 }
 
 // panels of step k: X_i = A_iK (kept for the trailing tiles), W_i = X_i D^-1,
@@ -155,7 +211,6 @@ __global__ void __launch_bounds__(256) k_sw_trail(const SweepMat* __restrict__ m
                                                   const double* __restrict__ panw, const double* __restrict__ panx,
                                                   double* dinv, int* info) {
   __shared__ __align__(16) double sw[64][LD], sx[64][LD];
-  __shared__ double rowbuf[2][64];
   const SweepMat M = mats[blockIdx.y];
   const bool more = k + 1 < M.np;
   int i, j;
@@ -202,7 +257,7 @@ __global__ void __launch_bounds__(256) k_sw_trail(const SweepMat* __restrict__ m
       }
   if (next) {
     __syncthreads();
-    invert_tile(sw, rowbuf, t, dinv + (int64_t)M.id * 4096, info + M.id, 64 * (k + 1));
+    invert_tile(sw, t, dinv + (int64_t)M.id * 4096, info + M.id, 64 * (k + 1));
   }
 }
 
