@@ -247,15 +247,14 @@ void launch_density_check(hipStream_t st, int64_t n, const int* slot, const doub
                           int* err);
 void launch_density_update(hipStream_t st, int64_t n, const int* slot, const double* dens, double penalty,
                            double emin, double rmin, double* E64, float* E32, double* rho);
-template <class T>
-void launch_bottom_gather(hipStream_t st, const LevelDev& L, const int* var_of, const T* b, T* x);
-template <class T>
-void launch_bottom_scatter(hipStream_t st, const LevelDev& L, const int* var_of, const T* y, const T* b, T* u);
-// symmetric matrix in packed lower-triangle 64x64 tiles: y = A x (x, y padded
-// to nT*64; part holds symv_splits(nT) * nT * 64 partial sums)
-int symv_splits(int nT);
-template <class T>
-void launch_symv(hipStream_t st, int nT, const T* tiles, const T* x, T* part, T* y);
+// Bottom solve with the dense inverse in packed lower-triangle 64x64 tiles of
+// type A: u = inverse of b on the active nodes, b on the others.  `vslot`: place
+// in b of every variable (-1 in the padding to nT*64), `var_of`: first variable
+// of a node (-1 if inactive); part holds bottom_splits(nT) * nT * 64 sums.
+int bottom_splits(int nT);
+template <class T, class A>
+void launch_bottom_dense(hipStream_t st, const LevelDev& L, int nT, const A* tiles, const int* vslot,
+                         const int* var_of, const T* b, A* part, T* u);
 // sensitivity: per level-0 slot (cell): dc = -p rho^(p-1)(1-Emin) a_e^T K0 u_e,
 // and with `obj` given *obj = the objective (deterministic sum; `bpart` holds
 // apply_dot_partials(nb) doubles, `part` reduce_partials)

@@ -52,11 +52,11 @@ static constexpr double kFp32PassReduction = 1e-6;
 // bandwidth-bound GEMV per V-cycle), the nested-dissection Cholesky
 // (bottom_nd.hip) above it, unless spg_config.bottom_dense_max sets another
 // limit; SPG_BOTTOM=dense|nd overrides both (dense stays limited to
-// kMaxDenseBottomDofs: its inverse is O(n^2)).  A whole density update takes 5.5
-// / 112 / 552 ms with the dense inverse and 1.4 / 3.0 / 4.2 ms with the nested
-// dissection at 4.1 K / 12.7 K / 21.9 K unknowns; the bottom solve of an FP32
-// V-cycle 31 / 107 / 297 us against 89 / 164 / 216 us: the dense inverse pays
-// when many solves share a factorization.
+// kMaxDenseBottomDofs: its inverse is O(n^2)).  A whole density update takes 2.9
+// / 5.1 / 41 ms with the dense inverse and 2.1 / 1.2 / 8.0 ms with the nested
+// dissection at 2.0 K / 4.1 K / 9.0 K unknowns (other levels' work included);
+// the bottom solve of an FP32 V-cycle 6.6 / 15 / 48 us against 33 / 50 / 80 us:
+// the dense inverse pays when many solves share a factorization.
 static constexpr int64_t kDenseBottomDofs = 16384;
 static constexpr int64_t kMaxDenseBottomDofs = 60000;
 
@@ -493,12 +493,13 @@ void Solver::build_operators() {
     sweep_.panx = panx_.as<double>();
     sweep_.dinv = dinv_.as<double>();
     sweep_.info = info_.as<int>();
-    for (DBuf* d : {&xb64_, &yb64_}) d->alloc(npad * 8);
-    for (DBuf* d : {&xb32_, &yb32_}) d->alloc(npad * 4);
-    pb64_.alloc((size_t)symv_splits(nT_) * npad * 8);
-    pb32_.alloc((size_t)symv_splits(nT_) * npad * 4);
-    HIPCHK(hipMemsetAsync(xb64_.p, 0, npad * 8, st_));
-    HIPCHK(hipMemsetAsync(xb32_.p, 0, npad * 4, st_));
+    std::vector<int32_t> vslot(npad, -1);
+    for (size_t i = 0; i < var.size(); ++i)
+      if (var[i] >= 0)
+        for (int c = 0; c < 3; ++c) vslot[(size_t)var[i] + c] = (int32_t)((i >> 6) * 192 + c * 64 + (i & 63));
+    upload(vslot_, vslot);
+    pb64_.alloc((size_t)bottom_splits(nT_) * npad * 8);
+    pb32_.alloc((size_t)bottom_splits(nT_) * npad * 4);
   }
   HIPCHK(hipMemsetAsync(tiles64_.p, 0, tiles64_.bytes, st_));
   HIPCHK(hipMemsetAsync(info_.p, 0, sizeof(int), st_));
@@ -826,20 +827,12 @@ void Solver::bottom(const T* b, T* u) {
     nd_->solve<T>(b, u, st_);
     return;
   }
-  const bool f = sizeof(T) == 4;
-  T* x = f ? (T*)xb32_.p : (T*)xb64_.p;
-  T* y = f ? (T*)yb32_.p : (T*)yb64_.p;
-  launch_bottom_gather<T>(st_, R.d, var_of_.as<int>(), b, x);
-  if (f && bottom64_) {
-    // FP32 cycle with the FP64 inverse: widen, apply, round back
-    const int64_t npad = (int64_t)nT_ * 64;
-    launch_cast_f2d(st_, (const float*)x, xb64_.as<double>(), npad);
-    launch_symv<double>(st_, nT_, tiles64_.as<double>(), xb64_.as<double>(), pb64_.as<double>(), yb64_.as<double>());
-    launch_cast_d2f(st_, yb64_.as<double>(), (float*)y, npad);
-  } else {
-    launch_symv<T>(st_, nT_, f ? (const T*)tiles32_.p : (const T*)tiles64_.p, x, f ? (T*)pb32_.p : (T*)pb64_.p, y);
-  }
-  launch_bottom_scatter<T>(st_, R.d, var_of_.as<int>(), y, b, u);
+  const int *vs = vslot_.as<int>(), *vo = var_of_.as<int>();
+  // FP32 cycle with the FP64 inverse: widened, applied and rounded back
+  if (sizeof(T) == 8 || bottom64_)
+    launch_bottom_dense<T, double>(st_, R.d, nT_, tiles64_.as<double>(), vs, vo, b, pb64_.as<double>(), u);
+  else
+    launch_bottom_dense<T, float>(st_, R.d, nT_, tiles32_.as<float>(), vs, vo, b, pb32_.as<float>(), u);
 }
 
 // FP32 cycle whose explicit levels (and bottom) run in FP64: the level

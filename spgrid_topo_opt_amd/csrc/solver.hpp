@@ -168,7 +168,7 @@ class Solver {
   bool coarse64_ = false;  // FP32 cycles run the explicit levels in FP64
   SweepBatch sweep_;
   DBuf smat_, panw_, panx_, dinv_;
-  DBuf var_of_, info_, tiles64_, tiles32_, xb64_, yb64_, xb32_, yb32_, pb64_, pb32_;
+  DBuf var_of_, vslot_, info_, tiles64_, tiles32_, pb64_, pb32_;
   std::unique_ptr<NdBottom> nd_;  // nested-dissection Cholesky bottom (large bottoms)
   // PCG / outer vectors (level 0)
   DBuf x32_, rr32_, s32_, q32_, z32_, x64_, rr64_, s64_, q64_, z64_;
