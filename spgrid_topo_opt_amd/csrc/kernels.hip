@@ -2805,6 +2805,29 @@ __global__ void __launch_bounds__(1024) k_sum_wide(const double* __restrict__ pa
 }
 
 // ----------------------------------------------------------------------- PCG
+// Small levels: the kernel that needs a reduction's result adds the partials
+// itself, every workgroup the same sum in the same order, instead of a launch
+// of one workgroup before it (2-5 us with its gap, against about 1 us here).
+// The first workgroup writes the scalars; none of those it writes is read here.
+// Line: at most 4096 blocks, i.e. 1024 partials of z . r and 4096 of s . q.
+static bool sum_in_consumer(int nb) { return nb <= 4096 && !std::getenv("SPG_SUM_WIDE_MAX"); }
+__device__ __forceinline__ double sum_partials(const double* __restrict__ part, int np) {
+  double s = 0.0;
+  for (int i = threadIdx.x; i < np; i += RED_T) s += part[i];
+  return block_reduce<0>(s);
+}
+template <class T>
+__global__ void __launch_bounds__(RED_T) k_cg_direction_sum(T* s, const T* __restrict__ z, CgScalars* sc, int64_t n,
+                                                            const double* __restrict__ part, int np) {
+  const double rho_old = sc->rho_old, rho = sum_partials(part, np), b = rho / rho_old;
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    sc->rho = rho;
+    sc->beta = b;
+  }
+  const T beta = (T)b;
+  for (int64_t i = (int64_t)blockIdx.x * RED_T + threadIdx.x; i < n; i += (int64_t)gridDim.x * RED_T)
+    s[i] = beta * s[i] + z[i];
+}
 template <class T>
 __global__ void k_cg_direction(T* s, const T* z, const CgScalars* sc, int64_t n) {
   int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -2812,12 +2835,10 @@ __global__ void k_cg_direction(T* s, const T* z, const CgScalars* sc, int64_t n)
   const T beta = (T)sc->beta;  // CG_VECTOR::Copy(c,x,y) rounds c to T (CG_VECTOR.cpp:96-114)
   s[i] = beta * s[i] + z[i];
 }
-template <class T>
 // x += alpha s, r -= alpha q, partial max |r|; with `zc` also clears zc
 // (the next V-cycle's iterate)
-__global__ void __launch_bounds__(RED_T) k_cg_update(T* x, T* r, const T* s, const T* q, const CgScalars* sc, int64_t n,
-                                                      double* part, T* zc) {
-  const T alpha = (T)sc->alpha;
+template <class T>
+__device__ __forceinline__ void cg_update(T alpha, T* x, T* r, const T* s, const T* q, int64_t n, double* part, T* zc) {
   double m = 0.0;
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
     x[i] = alpha * s[i] + x[i];
@@ -2828,6 +2849,24 @@ __global__ void __launch_bounds__(RED_T) k_cg_update(T* x, T* r, const T* s, con
   }
   m = block_reduce<1>(m);
   if (threadIdx.x == 0) part[blockIdx.x] = m;
+}
+template <class T>
+__global__ void __launch_bounds__(RED_T) k_cg_update(T* x, T* r, const T* s, const T* q, const CgScalars* sc, int64_t n,
+                                                      double* part, T* zc) {
+  cg_update<T>((T)sc->alpha, x, r, s, q, n, part, zc);
+}
+template <class T>
+__global__ void __launch_bounds__(RED_T) k_cg_update_sum(T* x, T* r, const T* s, const T* q, CgScalars* sc, int64_t n,
+                                                          double* part, T* zc, const double* __restrict__ bpart,
+                                                          int np) {
+  const double rho = sc->rho, sq = sum_partials(bpart, np);
+  const double alpha = sq != 0.0 ? rho / sq : (double)FLT_MAX;
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    sc->sq = sq;
+    sc->alpha = alpha;
+    sc->singular = !(sq > 0.0);
+  }
+  cg_update<T>((T)alpha, x, r, s, q, n, part, zc);
 }
 __global__ void k_cg_scalars(CgScalars* sc, int stage) {
   if (threadIdx.x == 0) cg_stage(sc, stage);
@@ -3283,8 +3322,8 @@ void launch_apply(hipStream_t st, const LevelDev& L, const T* E, T dx, const T* 
 }
 int64_t apply_dot_partials(int64_t nb) { return nb > RED_MAX_WG ? nb : RED_MAX_WG; }
 template <class T>
-void launch_apply_dot(hipStream_t st, const LevelDev& L, const T* E, T dx, const T* in, T* out, double* bpart,
-                      double* part, double* dot, CgScalars* sc, int stage) {
+int launch_apply_dot(hipStream_t st, const LevelDev& L, const T* E, T dx, const T* in, T* out, double* bpart,
+                     double* part, double* dot, CgScalars* sc, int stage) {
   // 256^3 shell, 18 iterations: mixed 42.8 vs 43.1 ms, FP64 60.0 vs 60.5 ms
   // against the apply followed by a separate dot
   const int nwg = (L.nb + AP_WAVES - 1) / AP_WAVES;
@@ -3296,6 +3335,7 @@ void launch_apply_dot(hipStream_t st, const LevelDev& L, const T* E, T dx, const
     k_apply_lds<T, double, 3><<<nwg, 64 * AP_WAVES, 0, st>>>(L.nb, L.nbr, L.flags, E, dx, in, nullptr, out, bpart);
   else
     k_apply_lds<T, T, 3><<<nwg, 64 * AP_WAVES, 0, st>>>(L.nb, L.nbr, L.flags, E, dx, in, nullptr, out, bpart);
+  if (sum_in_consumer(L.nb)) return L.nb;
   // one workgroup sums up to 65536 partials; beyond that two stages
   // (SPG_SUM_WIDE_MAX lowers the limit so that tests reach both forms)
   int wide_max = 65536;
@@ -3307,6 +3347,7 @@ void launch_apply_dot(hipStream_t st, const LevelDev& L, const T* E, T dx, const
     k_sum_part<<<g, RED_T, 0, st>>>(bpart, L.nb, part);
     k_final<0><<<1, RED_T, 0, st>>>(part, (int)g, dot, sc, stage);
   }
+  return 0;
 }
 static ColourOrder colour_order(bool level0, bool forward) {
   ColourOrder o{0};
@@ -3763,25 +3804,29 @@ void launch_sumsq(hipStream_t st, const double* a, int64_t n, double* partial, d
   k_final<0><<<1, RED_T, 0, st>>>(partial, (int)g, out);
 }
 template <class T>
-void launch_cg_direction(hipStream_t st, T* s, const T* z, const CgScalars* sc, int64_t n) {
-  k_cg_direction<T><<<nblk(n), TPB, 0, st>>>(s, z, sc, n);
+void launch_cg_direction(hipStream_t st, T* s, const T* z, CgScalars* sc, int64_t n, const double* part, int np) {
+  if (np > 0) k_cg_direction_sum<T><<<red_grid(n), RED_T, 0, st>>>(s, z, sc, n, part, np);
+  else k_cg_direction<T><<<nblk(n), TPB, 0, st>>>(s, z, sc, n);
 }
 template <class T>
 void launch_cg_update(hipStream_t st, T* x, T* r, const T* s, const T* q, CgScalars* sc, int64_t n, int stage,
-                      T* zclear, const CgReport& rep) {
+                      T* zclear, const CgReport& rep, const double* bpart, int np) {
   // caller passes the partial buffer right after the scalars block
   double* part = reinterpret_cast<double*>(sc + 1);
   const unsigned g = red_grid(n);
-  k_cg_update<T><<<g, RED_T, 0, st>>>(x, r, s, q, sc, n, part, zclear);
+  if (np > 0) k_cg_update_sum<T><<<g, RED_T, 0, st>>>(x, r, s, q, sc, n, part, zclear, bpart, np);
+  else k_cg_update<T><<<g, RED_T, 0, st>>>(x, r, s, q, sc, n, part, zclear);
   k_final<1><<<1, RED_T, 0, st>>>(part, (int)g, &sc->nrm, stage >= 0 ? sc : nullptr, stage, rep, sc);
 }
 void launch_cg_scalars(hipStream_t st, CgScalars* sc, int stage) { k_cg_scalars<<<1, 64, 0, st>>>(sc, stage); }
 template <class T>
-void launch_project_dot(hipStream_t st, const LevelDev& L, T* v, const T* w, double* partial, double* out,
-                        CgScalars* sc, int stage) {
+int launch_project_dot(hipStream_t st, const LevelDev& L, T* v, const T* w, double* partial, double* out,
+                       CgScalars* sc, int stage) {
   const unsigned g = red_grid((int64_t)L.nb * 64);
   k_project_dot_part<T><<<g, RED_T, 0, st>>>(L.nb, L.flags, v, w, partial);
+  if (sum_in_consumer(L.nb)) return (int)g;
   k_final<0><<<1, RED_T, 0, st>>>(partial, (int)g, out, sc, stage);
+  return 0;
 }
 template <class T>
 void launch_project(hipStream_t st, const LevelDev& L, T* v, bool nullspace) {
@@ -3868,7 +3913,7 @@ void launch_set_entries(hipStream_t st, double* v, const int* idx, const double*
 
 #define SPG_INST(T)                                                                                              \
   template void launch_apply<T>(hipStream_t, const LevelDev&, const T*, T, const T*, const T*, T*, int);         \
-  template void launch_apply_dot<T>(hipStream_t, const LevelDev&, const T*, T, const T*, T*, double*, double*,   \
+  template int launch_apply_dot<T>(hipStream_t, const LevelDev&, const T*, T, const T*, T*, double*, double*,   \
                                     double*, CgScalars*, int);                                                  \
   template void launch_gs0<T>(hipStream_t, const LevelDev&, const T*, T, T*, const T*, int, const uint8_t*, int,  \
                               const T*);                                                                        \
@@ -3889,11 +3934,11 @@ void launch_set_entries(hipStream_t st, double* v, const int* idx, const double*
   template void launch_dot<T>(hipStream_t, const T*, const T*, int64_t, double*, double*);                       \
   template void launch_linf<T>(hipStream_t, const T*, int64_t, double*, double*, const CgReport&,                \
                                const CgScalars*);                                \
-  template void launch_cg_direction<T>(hipStream_t, T*, const T*, const CgScalars*, int64_t);                    \
+  template void launch_cg_direction<T>(hipStream_t, T*, const T*, CgScalars*, int64_t, const double*, int);       \
   template void launch_cg_update<T>(hipStream_t, T*, T*, const T*, const T*, CgScalars*, int64_t, int, T*,     \
-                                    const CgReport&);                                                           \
+                                    const CgReport&, const double*, int);                                       \
   template void launch_project<T>(hipStream_t, const LevelDev&, T*, bool);                                       \
-  template void launch_project_dot<T>(hipStream_t, const LevelDev&, T*, const T*, double*, double*, CgScalars*,  \
+  template int launch_project_dot<T>(hipStream_t, const LevelDev&, T*, const T*, double*, double*, CgScalars*,  \
                                       int);
 
 SPG_INST(float)

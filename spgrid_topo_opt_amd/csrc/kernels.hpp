@@ -136,9 +136,11 @@ void launch_apply(hipStream_t st, const LevelDev& L, const T* E, T dx, const T* 
 // out = P K in (mode 2) and *dot = in . out (deterministic); `bpart` holds
 // apply_dot_partials(nb) doubles, `part` reduce_partials(n) doubles
 int64_t apply_dot_partials(int64_t nb);
+// this and launch_project_dot return how many partials (of `bpart`, of
+// `partial`) the next CG kernel has to add up; 0: the sum and its stage are done
 template <class T>
-void launch_apply_dot(hipStream_t st, const LevelDev& L, const T* E, T dx, const T* in, T* out, double* bpart,
-                      double* part, double* dot, CgScalars* sc = nullptr, int stage = -1);
+int launch_apply_dot(hipStream_t st, const LevelDev& L, const T* E, T dx, const T* in, T* out, double* bpart,
+                     double* part, double* dot, CgScalars* sc = nullptr, int stage = -1);
 // level-0 GS: one colour over all blocks; all boundary sweeps of one phase.
 // With `bcm` (b in colour-major order, launch_colour_major) and the level's
 // flags_cm, the colour kernel reads b and the flags of its colour only.
@@ -200,10 +202,11 @@ void launch_linf(hipStream_t st, const T* a, int64_t n, double* partial, double*
 void launch_sumsq(hipStream_t st, const double* a, int64_t n, double* partial, double* out);
 // PCG steps (scalars on device)
 template <class T>
-void launch_cg_direction(hipStream_t st, T* s, const T* z, const CgScalars* sc, int64_t n);  // s = beta s + z
+void launch_cg_direction(hipStream_t st, T* s, const T* z, CgScalars* sc, int64_t n, const double* part = nullptr,
+                         int np = 0);  // s = beta s + z
 template <class T>
 void launch_cg_update(hipStream_t st, T* x, T* r, const T* s, const T* q, CgScalars* sc, int64_t n, int stage = -1,
-                      T* zclear = nullptr, const CgReport& rep = CgReport());
+                      T* zclear = nullptr, const CgReport& rep = CgReport(), const double* bpart = nullptr, int np = 0);
 void launch_cg_scalars(hipStream_t st, CgScalars* sc, int stage);  // 0: after rho, 1: after sq, 2: end
 // (the reductions above take `sc, stage` to run a stage in their last kernel)
 // projections
@@ -211,7 +214,7 @@ template <class T>
 void launch_project(hipStream_t st, const LevelDev& L, T* v, bool nullspace);
 // v = P P_null v, then *out = v . w (deterministic two-stage sum)
 template <class T>
-void launch_project_dot(hipStream_t st, const LevelDev& L, T* v, const T* w, double* partial, double* out,
+int launch_project_dot(hipStream_t st, const LevelDev& L, T* v, const T* w, double* partial, double* out,
                         CgScalars* sc = nullptr, int stage = -1);
 // Galerkin assembly (FP64)
 void launch_galerkin_gather(hipStream_t st, int64_t ncell, int depth, const int* cell_fine_blocks,

@@ -1041,10 +1041,10 @@ int Solver::pcg(T* x, T* r, double tol, int maxit, int* iters, double* last_nrm)
     vcycle<T>(r, z, true, ahead ? Part::kRest : Part::kAll);  // z was cleared before the loop / by the last update
     // the scalar stages (beta, alpha, rho_old) run in the last kernel of
     // the reduction they follow
-    launch_project_dot<T>(st_, R0.d, z, r, part, &sc->rho, sc, 0);
-    launch_cg_direction<T>(st_, s, z, sc, n);
-    launch_apply_dot<T>(st_, R0.d, E<T>(), dxT<T>(), s, q, apart_.as<double>(), part, &sc->sq, sc, 1);
-    launch_cg_update<T>(st_, x, r, s, q, sc, n, 2, z, report());
+    const int nr = launch_project_dot<T>(st_, R0.d, z, r, part, &sc->rho, sc, 0);
+    launch_cg_direction<T>(st_, s, z, sc, n, part, nr);
+    const int nq = launch_apply_dot<T>(st_, R0.d, E<T>(), dxT<T>(), s, q, apart_.as<double>(), part, &sc->sq, sc, 1);
+    launch_cg_update<T>(st_, x, r, s, q, sc, n, 2, z, report(), apart_.as<double>(), nq);
   }
   // a time-out in a phase whose result nobody uses is nobody's error
   if (ahead && coop) HIPCHK(hipMemsetAsync(lv_[0].coop.as<unsigned>() + 1, 0, sizeof(unsigned), st_));
