@@ -2681,6 +2681,11 @@ int64_t reduce_partials(int64_t n) {
   (void)n;
   return RED_MAX_WG;
 }
+// a thread per element as far as the partials reach: small levels are bound by
+// latency, where four elements a thread (red_grid) cost three more rounds
+static inline unsigned fine_grid(int64_t n) {
+  return (unsigned)std::max<int64_t>(1, std::min<int64_t>((n + RED_T - 1) / RED_T, RED_MAX_WG));
+}
 static inline unsigned red_grid(int64_t n) {
   int64_t g = (n + RED_T * 4 - 1) / (RED_T * 4);
   if (g < 1) g = 1;
@@ -3805,7 +3810,7 @@ void launch_sumsq(hipStream_t st, const double* a, int64_t n, double* partial, d
 }
 template <class T>
 void launch_cg_direction(hipStream_t st, T* s, const T* z, CgScalars* sc, int64_t n, const double* part, int np) {
-  if (np > 0) k_cg_direction_sum<T><<<red_grid(n), RED_T, 0, st>>>(s, z, sc, n, part, np);
+  if (np > 0) k_cg_direction_sum<T><<<fine_grid(n), RED_T, 0, st>>>(s, z, sc, n, part, np);
   else k_cg_direction<T><<<nblk(n), TPB, 0, st>>>(s, z, sc, n);
 }
 template <class T>
@@ -3813,7 +3818,7 @@ void launch_cg_update(hipStream_t st, T* x, T* r, const T* s, const T* q, CgScal
                       T* zclear, const CgReport& rep, const double* bpart, int np) {
   // caller passes the partial buffer right after the scalars block
   double* part = reinterpret_cast<double*>(sc + 1);
-  const unsigned g = red_grid(n);
+  const unsigned g = np > 0 ? fine_grid(n) : red_grid(n);
   if (np > 0) k_cg_update_sum<T><<<g, RED_T, 0, st>>>(x, r, s, q, sc, n, part, zclear, bpart, np);
   else k_cg_update<T><<<g, RED_T, 0, st>>>(x, r, s, q, sc, n, part, zclear);
   k_final<1><<<1, RED_T, 0, st>>>(part, (int)g, &sc->nrm, stage >= 0 ? sc : nullptr, stage, rep, sc);
@@ -3822,7 +3827,8 @@ void launch_cg_scalars(hipStream_t st, CgScalars* sc, int stage) { k_cg_scalars<
 template <class T>
 int launch_project_dot(hipStream_t st, const LevelDev& L, T* v, const T* w, double* partial, double* out,
                        CgScalars* sc, int stage) {
-  const unsigned g = red_grid((int64_t)L.nb * 64);
+  const int64_t n = (int64_t)L.nb * 64;
+  const unsigned g = sum_in_consumer(L.nb) ? fine_grid(n) : red_grid(n);
   k_project_dot_part<T><<<g, RED_T, 0, st>>>(L.nb, L.flags, v, w, partial);
   if (sum_in_consumer(L.nb)) return (int)g;
   k_final<0><<<1, RED_T, 0, st>>>(partial, (int)g, out, sc, stage);
