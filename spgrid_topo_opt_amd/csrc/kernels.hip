@@ -2511,6 +2511,60 @@ __global__ void __launch_bounds__(64) k_gs0_bnd_flow(ColourOrder ord, int sweeps
     for (int c = 0; c < 3; ++c) u[vidx(blk, c, lane)] = hu[c * 216 + halo_pos(lane)];
 }
 
+// Stiffness apply of small levels: a workgroup of 8 waves per block instead of
+// a wave, an octet of lanes per node adding a cell each (corner_row), so that
+// few blocks still fill the device and a wave evaluates 72 products a lane
+// instead of 576 with their constants streamed in.  Modes as k_apply_lds, 0 to 3.
+template <class T, int MODE>
+__global__ void __launch_bounds__(512) k_apply_oct(const int* __restrict__ nbr, const uint8_t* __restrict__ flags,
+                                                   const T* __restrict__ E, T dx, const T* __restrict__ in,
+                                                   const T* __restrict__ b, T* __restrict__ out,
+                                                   double* __restrict__ dpart = nullptr) {
+  __shared__ T hu[3 * 216];
+  __shared__ T he[128];
+  __shared__ int ht[28];
+  __shared__ double dp[8];
+  const int tid = threadIdx.x, lane = tid & 63, I = lane & 7, blk = blockIdx.x;
+  const int l = tid >> 3, pos = halo_pos(l);
+  // threads 0 .. 215 stage a node each, 256 .. 380 a cell
+  const int t = tid < 216 ? cHalo6[tid] : (tid >= 256 && tid < 381 ? cHalo5[tid - 256] : -1);
+  if (tid < 27) ht[tid] = tid == 13 ? blk : nbr[blk * 27 + tid];
+  // lane I < 3 of a node's octet writes component I
+  const bool wr = I < 3;
+  uint8_t fl = 0;
+  T bv = T(0);
+  if (MODE > 0 && wr) fl = flags[blk * 64 + l];
+  if (MODE == 1 && wr) bv = b[vidx(blk, I, l)];
+  __syncthreads();
+  const int bb = t >= 0 ? ht[t >> 8] : -1;
+  if (tid < 216) {
+    T v[3];
+#pragma unroll
+    for (int c = 0; c < 3; ++c) v[c] = bb >= 0 ? in[vidx(bb, c, t & 255)] : T(0);
+#pragma unroll
+    for (int c = 0; c < 3; ++c) hu[c * 216 + tid] = v[c];
+  } else if (t >= 0) {
+    he[tid - 256] = bb >= 0 ? E[bb * 64 + (t & 255)] : T(0);
+  }
+  __syncthreads();
+  T f0, f1, f2;
+  gs0_rows<T>(l, pos, he, hu, dx, f0, f1, f2);
+  const T f = I == 0 ? f0 : (I == 1 ? f1 : f2);
+  double d = 0.0;
+  if (wr) {
+    const T o = (fl & (2 << I)) ? T(0) : (MODE == 1 ? bv - f : f);
+    out[vidx(blk, I, l)] = o;
+    if (MODE == 3) d = (double)hu[I * 216 + pos] * (double)o;
+  }
+  if (MODE == 3) {
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) d += __shfl_down(d, o, 64);
+    if (lane == 0) dp[tid >> 6] = d;
+    __syncthreads();
+    if (tid == 0) dpart[blk] = ((dp[0] + dp[1]) + (dp[2] + dp[3])) + ((dp[4] + dp[5]) + (dp[6] + dp[7]));
+  }
+}
+
 // workgroup size of the boundary phase: two register sets of BndFetch per lane
 template <class T>
 struct BndThreads {
@@ -3312,6 +3366,21 @@ static void launch_apply_cell(hipStream_t st, const LevelDev& L, const T* E, T d
   else
     k_apply_cell<T, 3><<<nwg, 64 * AP_WAVES, 0, st>>>(L.nb, L.nbr, L.flags, E, k, dx, in, b, out, dpart);
 }
+// most blocks of k_apply_oct: residual, an octet of lanes against a lane per
+// node, FP32 / FP64 us: 3.3 / 4.0 and 6.5 / 8.2 at 360 blocks, 5.8 / 7.3 and
+// 6.8 / 8.8 at 1377, 10.2 / 14.9 and 8.5 / 10.7 at 3024 (a device full of waves
+// pays the halo eight lanes a node)
+static constexpr int kMaxOctApply = 1536;
+template <class T>
+static bool launch_apply_oct(hipStream_t st, const LevelDev& L, const T* E, T dx, const T* in, const T* b, T* out,
+                             int mode, double* dpart = nullptr) {
+  if (L.nb > kMaxOctApply) return false;
+  if (mode == 0) k_apply_oct<T, 0><<<L.nb, 512, 0, st>>>(L.nbr, L.flags, E, dx, in, b, out);
+  else if (mode == 1) k_apply_oct<T, 1><<<L.nb, 512, 0, st>>>(L.nbr, L.flags, E, dx, in, b, out);
+  else if (mode == 2) k_apply_oct<T, 2><<<L.nb, 512, 0, st>>>(L.nbr, L.flags, E, dx, in, b, out);
+  else k_apply_oct<T, 3><<<L.nb, 512, 0, st>>>(L.nbr, L.flags, E, dx, in, b, out, dpart);
+  return true;
+}
 template <class T>
 void launch_apply(hipStream_t st, const LevelDev& L, const T* E, T dx, const T* in, const T* b, T* out, int mode) {
   if (apply_cell(sizeof(T) == 4, mode)) {
@@ -3321,7 +3390,7 @@ void launch_apply(hipStream_t st, const LevelDev& L, const T* E, T dx, const T* 
     k_apply_lds<T, T, 4><<<nwg, 64 * AP_WAVES, 0, st>>>(L.nb, L.nbr, L.flags, E, dx, in, b, out);
   } else if (sizeof(T) == 4 && ((acc64_modes() >> mode) & 1)) {
     launch_apply_t<T, double>(st, L, E, dx, in, b, out, mode);
-  } else {
+  } else if (!launch_apply_oct<T>(st, L, E, dx, in, b, out, mode)) {
     launch_apply_t<T, T>(st, L, E, dx, in, b, out, mode);
   }
 }
@@ -3338,7 +3407,7 @@ int launch_apply_dot(hipStream_t st, const LevelDev& L, const T* E, T dx, const 
     k_apply_lds<T, T, 5><<<nwg, 64 * AP_WAVES, 0, st>>>(L.nb, L.nbr, L.flags, E, dx, in, nullptr, out, bpart);
   else if (sizeof(T) == 4 && ((acc64_modes() >> 2) & 1))
     k_apply_lds<T, double, 3><<<nwg, 64 * AP_WAVES, 0, st>>>(L.nb, L.nbr, L.flags, E, dx, in, nullptr, out, bpart);
-  else
+  else if (!launch_apply_oct<T>(st, L, E, dx, in, nullptr, out, 3, bpart))
     k_apply_lds<T, T, 3><<<nwg, 64 * AP_WAVES, 0, st>>>(L.nb, L.nbr, L.flags, E, dx, in, nullptr, out, bpart);
   if (sum_in_consumer(L.nb)) return L.nb;
   // one workgroup sums up to 65536 partials; beyond that two stages

@@ -386,6 +386,28 @@ def test_data_flow_sweep_matches_colour_launches(shape, levels, blocks, monkeypa
     s.close()
 
 
+@pytest.mark.parametrize("shape,blocks", [((3, 3, 3), 1), ((45, 23, 19), 360), ((61, 43, 35), 1584)])
+def test_apply_forms_agree(shape, blocks, monkeypatch):
+    """apply, residual and operator row by row (eight lanes a node up to 1536
+    blocks, one beyond) against the cell-by-cell form in FP64, which shares none
+    of their arithmetic; sums of up to 192 products of nodal noise: FP64 to
+    1e-13, FP32 to 1e-6 relative"""
+    s = _lib.Solver(W.box(*shape, seed=9, mg_levels=1 if blocks == 1 else 3))
+    assert s.level_blocks(0) == blocks
+    n = len(s.level_nodes(0)[0])
+    rng = np.random.default_rng(23)
+    u = rng.standard_normal((n, 3)).astype(np.float32).astype(np.float64)
+    b = rng.standard_normal((n, 3)).astype(np.float32).astype(np.float64)
+    for op in (_lib.OP_APPLY, _lib.OP_RESIDUAL, _lib.OP_OPERATOR):
+        monkeypatch.setenv("SPG_APPLY_CELL", "1")
+        want = s.kernel(op, 0, u, b, precision=1)
+        monkeypatch.setenv("SPG_APPLY_CELL", "0")
+        for prec, tol in ((1, 1e-13), (0, 1e-6)):
+            assert rel(s.kernel(op, 0, u, b, precision=prec), want) < tol, (op, prec)
+        monkeypatch.delenv("SPG_APPLY_CELL")
+    s.close()
+
+
 @pytest.mark.parametrize("prec,tol", [(1, 1e-13), (0, 1e-6)])
 def test_restriction_and_prolongation(blocky, prec, tol):
     P = blocky
