@@ -1771,10 +1771,14 @@ __global__ void __launch_bounds__(BM_THREADS) k_bmap_build(int n, BndOff L, Colo
 
 // Dense boundary map apply: u_B += M x, x the residual of the boundary
 // equations (node-major).  Rows are padded to a multiple of 64 entries
-// (zeros), one wavefront per row streams it with 16-byte loads, four in flight
-// per lane, and reduces in a fixed order.  A Dirichlet row holds a single 1,
-// so its component ends at u - u = 0.  Bound by streaming M from HBM or the
-// memory-side cache.
+// (zeros); a workgroup takes a row, each of its four waves a quarter with
+// 16-byte loads, four in flight per lane, and the sum has a fixed order.  A
+// Dirichlet row holds a single 1, so its component ends at u - u = 0.  Bound
+// by streaming M, mostly from the memory-side cache (FP64 at 2400 nodes: 415 MB
+// in about 23 us).  A whole phase against a wave per row, FP32 / FP64: 17.5 /
+// 29.0 and 18.5 / 30.5 us at 2400 nodes, 6.8 / 8.2 and 7.4 / 8.4 at 405; 8 or 16
+// loads in flight gave 20 / 31 and 23 / 36, not reading Dirichlet rows 20 / 31
+// (their kind is two dependent loads away).
 template <class T>
 __device__ __forceinline__ T dot4(const typename Vec4<T>::type& a, const typename Vec4<T>::type& b, T acc);
 template <>
@@ -1787,31 +1791,34 @@ __device__ __forceinline__ double dot4<double>(const double2& a, const double2& 
 }
 // row 3i+c belongs to boundary node list[i], component c
 template <class T>
-__global__ void __launch_bounds__(256) k_bmap_gemv(int rows, int Kp, const T* __restrict__ M, const T* __restrict__ x,
+__global__ void __launch_bounds__(256) k_bmap_gemv(int Kp, const T* __restrict__ M, const T* __restrict__ x,
                                                    const int* __restrict__ list, T* __restrict__ u) {
   using V = typename Vec4<T>::type;
   constexpr int PER = 16 / sizeof(T);
-  const int r = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
-  if (r >= rows) return;
+  __shared__ T sh[4];
+  const int r = blockIdx.x, w = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const V* row = reinterpret_cast<const V*>(M + (int64_t)r * Kp);
   const V* xv = reinterpret_cast<const V*>(x);
-  const int nv = Kp / PER;
+  // wave w's quarter of the row, in whole 64-entry pieces
+  const int nv = Kp / PER, per = (nv + 255) / 256 * 64, end = min(nv, (w + 1) * per);
   T a0 = 0, a1 = 0, a2 = 0, a3 = 0;
-  int k = lane;
-  for (; k + 192 < nv; k += 256) {
+  int k = w * per + lane;
+  for (; k + 192 < end; k += 256) {
     const V m0 = row[k], m1 = row[k + 64], m2 = row[k + 128], m3 = row[k + 192];
     a0 = dot4<T>(m0, xv[k], a0);
     a1 = dot4<T>(m1, xv[k + 64], a1);
     a2 = dot4<T>(m2, xv[k + 128], a2);
     a3 = dot4<T>(m3, xv[k + 192], a3);
   }
-  for (; k < nv; k += 64) a0 = dot4<T>(row[k], xv[k], a0);
+  for (; k < end; k += 64) a0 = dot4<T>(row[k], xv[k], a0);
   T acc = (a0 + a1) + (a2 + a3);
 #pragma unroll
   for (int o = 32; o >= 1; o >>= 1) acc += __shfl_xor(acc, o);
-  if (lane == 0) {
+  if (lane == 0) sh[w] = acc;
+  __syncthreads();
+  if (threadIdx.x == 0) {
     const int i = r / 3, c = r - 3 * i, node = list[i];
-    u[vidx(node >> 6, c, node & 63)] += acc;
+    u[vidx(node >> 6, c, node & 63)] += (sh[0] + sh[1]) + (sh[2] + sh[3]);
   }
 }
 // ------------------------------------- level-0 matrix-free boundary phase
@@ -2463,7 +2470,7 @@ __global__ void __launch_bounds__(64) k_gs0_flow(ColourOrder ord, const int* __r
 // Bound by 1.4 us a colour step: a load of the entries (0.6 us, at times two
 // or three until the neighbours' are there) and the row.  A phase of 3 sweeps,
 // FP32 / FP64 us, against k_bnd_rhs and k_bnd_flow: 38.6 / 43.0 and 46.7 / 62.9
-// at 855 nodes, 41.8 / 48.8 and 53.1 / 82.3 at 12,675.  Two loads half a round
+// at 1425 nodes, 41.8 / 48.8 and 53.1 / 82.3 at 21,125.  Two loads half a round
 // trip apart gave 37 / 44 and twice the time of a sweep of 3000 blocks; all
 // but the last colour's part of the row before the wait 44 / 45; a pause
 // between the loads 40 / 43.
@@ -3627,7 +3634,7 @@ static bool launch_bnd_map(hipStream_t st, const LevelDev& L, T* u, const T* b, 
   const int n = L.bnd_off[8];
   T* x = BmapPtr<T>::x(L);  // zero past 3n
   k_bnd_res<T><<<(n + 31) / 32, 256, 0, st>>>(n, L.bnd, L.ball, BndPtr<T>::A(L), L.flags, u, b, x);
-  k_bmap_gemv<T><<<(3 * n + 3) / 4, 256, 0, st>>>(3 * n, (int)bmap_stride(n), M, x, L.bnd, u);
+  k_bmap_gemv<T><<<3 * n, 256, 0, st>>>((int)bmap_stride(n), M, x, L.bnd, u);
   return true;
 }
 void launch_bnd0_setup(hipStream_t st, const LevelDev& L, const int* cslot, const double* E, double dx, double* bE,

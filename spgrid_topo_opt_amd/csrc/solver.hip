@@ -33,9 +33,9 @@ static double now_s() {
 
 // Boundary phases over at most this many nodes run as one dense map (2 maps x
 // 3n x 3n entries in FP64 and FP32).  Level-0 phase by map / by data flow, FP32
-// and FP64: 7.6 / 45 and 8.5 / 62 us at 405 nodes, 9.8 / 47 and 17 / 62 at 1425,
-// 18 / 46 and 30 / 61 at 2400, 25 / 46 and 42 / 62 at 3000.  A density update
-// builds both maps: 0.2, 1.0, 1.9 and 5.9 ms, which a solve of 25 V-cycles (4
+// and FP64: 9.8 / 39 and 16 / 43 us at 1425 nodes, 17.5 / 40 and 29 / 44 at
+// 2400, 25 / 40 and 42 / 45 at 3000.  A density update builds both maps: 0.2 ms
+// at 405 nodes, 1.0, 1.9 and 5.9 at these, which a solve of 25 V-cycles (4
 // phases each) earns back up to about here.
 static constexpr int kMaxDenseBoundary = 2560;
 // levels of at most this many blocks get the entries of the data-flow sweep
