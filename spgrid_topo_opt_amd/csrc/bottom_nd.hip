@@ -546,15 +546,13 @@ void NdBottom::upload(hipStream_t st) {
   const size_t tile = 4096 * 8;
   tiles_.alloc((size_t)std::max<int64_t>(ntile_, 1) * tile);
   tr_.alloc((size_t)std::max<int64_t>(ntr_, 1) * tile);
-  panw_.alloc((size_t)std::max<int64_t>(npan_, 1) * tile);
-  panx_.alloc((size_t)std::max<int64_t>(npan_, 1) * tile);
-  dinv_.alloc((size_t)std::max<int64_t>(nid_, 1) * tile);
+  pan_.alloc((size_t)std::max<int64_t>(npan_, 1) * tile);
+  minv_.alloc((size_t)std::max<int64_t>(nid_, 1) * tile);
   info_.alloc((size_t)std::max<int64_t>(nid_, 1) * sizeof(int));
   for (Depth& D : depth_) {
     D.batch.d = static_cast<SweepMat*>(d_mats_.p) + D.mat0;
-    D.batch.panw = static_cast<double*>(panw_.p);
-    D.batch.panx = static_cast<double*>(panx_.p);
-    D.batch.dinv = static_cast<double*>(dinv_.p);
+    D.batch.pan = static_cast<double*>(pan_.p);
+    D.batch.minv = static_cast<double*>(minv_.p);
     D.batch.info = static_cast<int*>(info_.p);
   }
   w_.alloc((size_t)std::max<int64_t>(wlen_, 1) * 8);
@@ -566,7 +564,7 @@ void NdBottom::upload(hipStream_t st) {
 size_t NdBottom::device_bytes() const {
   size_t s = 0;
   for (const DevMem* d : {&d_fr_, &d_kid_, &d_vmap_, &d_rest_, &d_bidx_, &d_emap_, &d_ent_, &d_ent_of_, &d_items_,
-                          &d_mats_, &d_kids_, &tiles_, &tr_, &panw_, &panx_, &dinv_, &info_, &w_, &u_, &x_})
+                          &d_mats_, &d_kids_, &tiles_, &tr_, &pan_, &minv_, &info_, &w_, &u_, &x_})
     s += d->bytes;
   return s;
 }

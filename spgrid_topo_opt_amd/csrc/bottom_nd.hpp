@@ -97,7 +97,7 @@ class NdBottom {
   std::vector<Depth> depth_;
   int64_t ntile_ = 0, ntr_ = 0, npan_ = 0, nid_ = 0, wlen_ = 0, ulen_ = 0;
   DevMem d_fr_, d_kid_, d_vmap_, d_rest_, d_bidx_, d_emap_, d_ent_, d_ent_of_, d_items_, d_mats_, d_kids_;
-  DevMem tiles_, tr_, panw_, panx_, dinv_, info_, w_, u_, x_;
+  DevMem tiles_, tr_, pan_, minv_, info_, w_, u_, x_;
 };
 
 }  // namespace spg

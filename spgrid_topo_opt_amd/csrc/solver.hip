@@ -482,16 +482,15 @@ void Solver::build_operators() {
     upload(var_of_, var);
     tiles64_.alloc(ntile * 4096 * 8);
     tiles32_.alloc(ntile * 4096 * 4);
-    for (DBuf* d : {&panw_, &panx_}) d->alloc((size_t)nT_ * 4096 * 8);
-    dinv_.alloc(4096 * 8);
+    pan_.alloc((size_t)nT_ * 4096 * 8);
+    minv_.alloc(4096 * 8);
     info_.alloc(sizeof(int));
     const std::vector<SweepMat> one_mat{SweepMat{0, nT_, nT_, 0, 0}};
     upload(smat_, one_mat);
     sweep_.h = one_mat;
     sweep_.d = smat_.as<SweepMat>();
-    sweep_.panw = panw_.as<double>();
-    sweep_.panx = panx_.as<double>();
-    sweep_.dinv = dinv_.as<double>();
+    sweep_.pan = pan_.as<double>();
+    sweep_.minv = minv_.as<double>();
     sweep_.info = info_.as<int>();
     std::vector<int32_t> vslot(npad, -1);
     for (size_t i = 0; i < var.size(); ++i)

@@ -167,7 +167,7 @@ class Solver {
   bool bottom64_ = false;  // FP32 cycles apply the FP64 bottom inverse
   bool coarse64_ = false;  // FP32 cycles run the explicit levels in FP64
   SweepBatch sweep_;
-  DBuf smat_, panw_, panx_, dinv_;
+  DBuf smat_, pan_, minv_;
   DBuf var_of_, vslot_, info_, tiles64_, tiles32_, pb64_, pb32_;
   std::unique_ptr<NdBottom> nd_;  // nested-dissection Cholesky bottom (large bottoms)
   // PCG / outer vectors (level 0)

@@ -6,19 +6,25 @@
 // the front's inverse, its multipliers A21 A11^-1 and its update matrix, which
 // is all that the bottom solve needs.  The pivots met on the way are those of
 // the Cholesky factorization, so the matrix is positive definite exactly when
-// all are positive, and the inverse is as accurate as the one from the
-// Cholesky factors.
+// all are positive.
+//
+// D^-1 is never applied as one matrix: with D = L L^T and M = L^-1, the panel is
+// Y_i = A_iK M^T, the update A_ij -= Y_i Y_j^T and W_i = Y_i M.  An update
+// through W_i = A_iK D^-1 loses the soft parts of a design behind a solid pivot
+// (moduli 1 and 9e-9, 3 K to 7 K unknowns, residual of a solve: 6e6 to 6e7 of
+// the right-hand side, this form and LAPACK's Cholesky 2e-7 to 1.5e-6).
 //
 // Every step is two launches over the whole batch: the panels, then the
-// trailing tiles; the workgroup of the next diagonal tile also inverts it, so
+// trailing tiles; the workgroup of the next diagonal tile also factors it, so
 // that serial part runs beside the others.  The products are 64x64x64 FP64
 // tiles on the matrix cores (v_mfma_f64_16x16x4), both operands staged in LDS,
 // the result tile in registers.  Small batches are bound by the serial
-// inversion of the diagonal tiles (64 dependent pivots each).  Per density update,
-// against partial Cholesky front by front through rocSOLVER and rocBLAS, at the
-// scalar inversion: 37 -> 2.0 ms (9,006 unknowns, nested dissection), 16 -> 1.1
-// ms (4,131, nested dissection), 9 -> 1.9 ms (2,016, dense); the 16x16 blocks
-// take another 0.3 ms from the last two.
+// factorization of the diagonal tiles (64 dependent pivots each).  A density
+// update, against one tile inverse applied as a matrix: dense 3,072 unknowns
+// 2.8 -> 3.2 ms, nested dissection 1.3 -> 1.6 ms and, at 15,120, 2.9 -> 3.2 ms
+// (partial Cholesky front by front through rocSOLVER: 12.6, 12.6 and 62 ms).
+// The residual of a solve is 0.4 to 1.3 times rocSOLVER's over 3 K to 15 K
+// unknowns, ordinary and high-contrast designs.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -59,6 +65,33 @@ __device__ __forceinline__ void mm64(const double (*A)[LD], const double (*B)[LD
     acc[1][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(a1, b1, acc[1][1], 0, 0, 0);
   }
 }
+// acc += A B over K = 64, and acc += A^T A, results placed as above
+__device__ __forceinline__ void mm64n(const double (*A)[LD], const double (*B)[LD], d4 (&acc)[2][2]) {
+  const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
+  const int ra = (w >> 1) * 32 + (l & 15), rb = (w & 1) * 32 + (l & 15), k0 = l >> 4;
+#pragma unroll
+  for (int k = 0; k < 64; k += 4) {
+    const double a0 = A[ra][k + k0], a1 = A[ra + 16][k + k0];
+    const double b0 = B[k + k0][rb], b1 = B[k + k0][rb + 16];
+    acc[0][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(a0, b0, acc[0][0], 0, 0, 0);
+    acc[0][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(a0, b1, acc[0][1], 0, 0, 0);
+    acc[1][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(a1, b0, acc[1][0], 0, 0, 0);
+    acc[1][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(a1, b1, acc[1][1], 0, 0, 0);
+  }
+}
+__device__ __forceinline__ void mm64sq(const double (*A)[LD], d4 (&acc)[2][2]) {
+  const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
+  const int ra = (w >> 1) * 32 + (l & 15), rb = (w & 1) * 32 + (l & 15), k0 = l >> 4;
+#pragma unroll
+  for (int k = 0; k < 64; k += 4) {
+    const double a0 = A[k + k0][ra], a1 = A[k + k0][ra + 16];
+    const double b0 = A[k + k0][rb], b1 = A[k + k0][rb + 16];
+    acc[0][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(a0, b0, acc[0][0], 0, 0, 0);
+    acc[0][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(a0, b1, acc[0][1], 0, 0, 0);
+    acc[1][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(a1, b0, acc[1][0], 0, 0, 0);
+    acc[1][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(a1, b1, acc[1][1], 0, 0, 0);
+  }
+}
 // position of element q of sub-tile (i, j) of the caller's accumulators
 __device__ __forceinline__ void acc_pos(int i, int j, int q, int& row, int& col) {
   const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
@@ -80,11 +113,13 @@ __device__ __forceinline__ double lane_d(double x, int lane) {
   const unsigned hi = __builtin_amdgcn_readlane((int)(v >> 32), lane);
   return __longlong_as_double(((long long)hi << 32) | (long long)lo);
 }
-// one scalar sweep of a 16x16 SPD block held by a wave (lane l: rows
-// 4 (l>>4) + i, column l & 15), pivot KK and the following ones; the block
-// becomes minus its inverse
+// P = L L^T of a 16x16 SPD block held by a wave (lane l: rows 4 (l>>4) + i,
+// column l & 15), pivot KK and the following ones.  Elimination by columns: at
+// the end column c holds, above the diagonal, row c of the inverse of the unit
+// triangular factor, and `dc` the pivot L_cc^2 (its root is taken once, not in
+// the chain of pivots).
 template <int KK>
-__device__ __forceinline__ void sweep16(double (&a)[4], int& bad, int pivot0) {
+__device__ __forceinline__ void chol16(double (&a)[4], double& dc, int& bad, int pivot0) {
   if constexpr (KK < 16) {
     const int l = threadIdx.x & 63, g = l >> 4, c = l & 15;
     constexpr int gk = KK >> 2, ik = KK & 3;
@@ -94,104 +129,145 @@ __device__ __forceinline__ void sweep16(double (&a)[4], int& bad, int pivot0) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) ci[i] = dpp_d<0x150 + KK>(a[i]);
     if (!(d > 0.0) && bad == 0) bad = pivot0 + KK + 1;
-    const double inv = 1.0 / d, pr = row * inv;
+    const double pr = row * (1.0 / d);
+    dc = c == KK ? d : dc;
+    if (c > KK) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) a[i] = c == KK ? ci[i] * inv : __builtin_fma(-ci[i], pr, a[i]);
-    if (g == gk) a[ik] = c == KK ? -inv : pr;
-    sweep16<KK + 1>(a, bad, pivot0);
+      for (int i = 0; i < 4; ++i) a[i] = (g == gk && i == ik) ? -pr : __builtin_fma(-ci[i], pr, a[i]);
+    }
+    chol16<KK + 1>(a, dc, bad, pivot0);
   }
 }
 
-// The 64x64 SPD tile in LDS -> minus its inverse in the tile store, the
-// inverse in dinv, by the block sweep above with 16x16 blocks.  Every wave
-// inverts the pivot block D (no barrier between its 16 dependent pivots), then
-// wave r takes row block r: W_r^T = D^-1 X_r^T, whose result registers are the
-// left operand of A_rj -= W_r X_j^T when the sum over k runs in the order that
-// they hold.  Two barriers per block.  Against a scalar sweep with a barrier
-// for each of the 64 pivots, a thread holding 16 rows of a column: first tile
-// 33.5 -> 19.1 us, a trailing step with its next diagonal tile 38.0 -> 25.7 us.
-__device__ void invert_tile(double (*s)[LD], double* __restrict__ tile, double* __restrict__ dinv,
+// The 64x64 SPD tile in LDS (lower blocks and whole diagonal blocks are read)
+// -> M = L^-1 in minv, -M^T M = minus the inverse in the tile store, by blocks
+// of 16.  Every wave factors the pivot block (no barrier between its 16
+// dependent pivots); wave r below it takes row block r: Y_r^T = M_KK A_rK^T,
+// whose result registers are the left operand of A_rj -= Y_r Y_j^T and of the
+// rows of M, T_rc -= Y_r M_Kc, when the sum over k runs in the order that they
+// hold; the pivot's own wave finishes M_Kc = M_KK T_Kc.  Y_j^T waits in the block
+// above the diagonal, which holds nothing else.  Two barriers per block.
+__device__ void factor_tile(double (*s)[LD], double (*mk)[17], double* __restrict__ tile, double* __restrict__ minv,
                             int* __restrict__ info, int pivot0) {
   const int r = threadIdx.x >> 6, l = threadIdx.x & 63, g = l >> 4, c = l & 15;
   int bad = 0;
   for (int K = 0; K < 4; ++K) {
     const int o = 16 * K;
-    double a[4];
+    double a[4], dc = 1.0;
 #pragma unroll
     for (int i = 0; i < 4; ++i) a[i] = s[o + 4 * g + i][o + c];
-    sweep16<0>(a, bad, pivot0 + o);
-    d4 wt = {};
-    if (r != K) {
+    chol16<0>(a, dc, bad, pivot0 + o);
+    const double rs = 1.0 / sqrt(dc);
+    double m[4];  // M_KK[c][4 g + i]
+#pragma unroll
+    for (int i = 0; i < 4; ++i) m[i] = 4 * g + i < c ? a[i] * rs : (4 * g + i == c ? rs : 0.0);
+    d4 y = {};
+    if (r > K) {
 #pragma unroll
       for (int i = 0; i < 4; ++i)
-        wt = __builtin_amdgcn_mfma_f64_16x16x4f64(-a[i], s[16 * r + c][o + 4 * g + i], wt, 0, 0, 0);
-      for (int j = 0; j < 4; ++j) {
-        if (j == K) continue;
-        d4 acc;
+        y = __builtin_amdgcn_mfma_f64_16x16x4f64(m[i], s[16 * r + c][o + 4 * g + i], y, 0, 0, 0);
 #pragma unroll
-        for (int q = 0; q < 4; ++q) acc[q] = s[16 * r + 4 * q + g][16 * j + c];
+      for (int q = 0; q < 4; ++q) s[o + 4 * q + g][16 * r + c] = y[q];
+    } else if (r == K) {
+      for (int j = 0; j < K; ++j) {
+        d4 acc = {};
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          acc = __builtin_amdgcn_mfma_f64_16x16x4f64(m[i], s[o + 4 * g + i][16 * j + c], acc, 0, 0, 0);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) s[o + 4 * q + g][16 * j + c] = acc[q];
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i) mk[c][4 * g + i] = m[i];
+    }
+    __syncthreads();  // the pivot block has been read, Y and row K of M are there
+    if (r > K) {
+      for (int j = 0; j <= r; ++j) {
+        d4 acc = {};
 #pragma unroll
         for (int q = 0; q < 4; ++q)
-          acc = __builtin_amdgcn_mfma_f64_16x16x4f64(-wt[q], s[16 * j + c][o + 4 * q + g], acc, 0, 0, 0);
+          acc = __builtin_amdgcn_mfma_f64_16x16x4f64(-y[q], j == K ? mk[4 * q + g][c] : s[o + 4 * q + g][16 * j + c],
+                                                     acc, 0, 0, 0);
 #pragma unroll
-        for (int q = 0; q < 4; ++q) s[16 * r + 4 * q + g][16 * j + c] = acc[q];
+        for (int q = 0; q < 4; ++q) {
+          double* p = &s[16 * r + 4 * q + g][16 * j + c];
+          *p = j == K ? acc[q] : *p + acc[q];
+        }
       }
-    }
-    __syncthreads();  // the panel has been read
-    if (r != K) {
+    } else if (r == K) {
 #pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        s[16 * r + c][o + 4 * q + g] = wt[q];
-        s[o + 4 * q + g][16 * r + c] = wt[q];
-      }
-    } else {
-#pragma unroll
-      for (int i = 0; i < 4; ++i) s[o + 4 * g + i][o + c] = a[i];
+      for (int i = 0; i < 4; ++i) s[o + c][o + 4 * g + i] = m[i];
     }
     __syncthreads();
   }
   for (int e = threadIdx.x; e < 4096; e += 256) {
-    const double v = s[e >> 6][e & 63];
-    tile[e] = v;
-    dinv[e] = -v;
+    const int i = e >> 6, j = e & 63;
+    if ((j >> 4) > (i >> 4)) s[i][j] = 0.0;
+    minv[e] = s[i][j];
   }
+  __syncthreads();
+  d4 acc[2][2] = {};
+  mm64sq(s, acc);
+#pragma unroll
+  for (int p = 0; p < 2; ++p)
+#pragma unroll
+    for (int b = 0; b < 2; ++b)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        int i, j;
+        acc_pos(p, b, q, i, j);
+        tile[i * 64 + j] = -acc[p][b][q];
+      }
   if (threadIdx.x == 0 && bad && *info == 0) *info = bad;
 }
 
 // the first diagonal tile of every matrix
-__global__ void __launch_bounds__(256) k_sw_first(const SweepMat* __restrict__ mats, double* tiles, double* dinv,
+__global__ void __launch_bounds__(256) k_sw_first(const SweepMat* __restrict__ mats, double* tiles, double* minv,
                                                   int* info) {
   __shared__ __align__(16) double s[64][LD];
+  __shared__ double mk[16][17];
   const SweepMat M = mats[blockIdx.x];
   double* t = tiles + M.off * 4096;
   stage(t, s, 1.0);
   __syncthreads();
-  invert_tile(s, t, dinv + (int64_t)M.id * 4096, info + M.id, 0);
+  factor_tile(s, mk, t, minv + (int64_t)M.id * 4096, info + M.id, 0);
 }
 
-// panels of step k: X_i = A_iK (kept for the trailing tiles), W_i = X_i D^-1,
-// A_iK = W_i
+// panels of step k: Y_i = A_iK M^T (kept for the trailing tiles), A_iK = Y_i M
 __global__ void __launch_bounds__(256) k_sw_panel(const SweepMat* __restrict__ mats, int k, double* tiles,
-                                                  double* __restrict__ panw, double* __restrict__ panx,
-                                                  const double* __restrict__ dinv) {
-  __shared__ __align__(16) double sx[64][LD], sd[64][LD];
+                                                  double* __restrict__ pan, const double* __restrict__ minv) {
+  __shared__ __align__(16) double sx[64][LD], sm[64][LD];
   const SweepMat M = mats[blockIdx.y];
   const int i = blockIdx.x;
   if (i >= M.nt || i == k) return;
   const bool below = i > k;
   double* t = tiles + (M.off + (below ? tile_at(i, k) : tile_at(k, i))) * 4096;
-  double* X = panx + (int64_t)(M.pan + i) * 4096;
-  double* W = panw + (int64_t)(M.pan + i) * 4096;
-  stage(dinv + (int64_t)M.id * 4096, sd, 1.0);
+  double* Y = pan + (int64_t)(M.pan + i) * 4096;
+  stage(minv + (int64_t)M.id * 4096, sm, 1.0);
   if (below) {
     stage(t, sx, 1.0);
   } else {
     for (int e = threadIdx.x; e < 4096; e += 256) sx[e & 63][e >> 6] = t[e];
   }
   __syncthreads();
-  for (int e = threadIdx.x; e < 4096; e += 256) X[e] = sx[e >> 6][e & 63];
   d4 acc[2][2] = {};
-  mm64(sx, sd, acc);
+  mm64(sx, sm, acc);
+  __syncthreads();  // sx is reused
+#pragma unroll
+  for (int a = 0; a < 2; ++a)
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        int r, c;
+        acc_pos(a, b, q, r, c);
+        Y[r * 64 + c] = acc[a][b][q];
+        sx[r][c] = acc[a][b][q];
+      }
+      acc[a][b] = d4{};
+    }
+  __syncthreads();
+  mm64n(sx, sm, acc);
 #pragma unroll
   for (int a = 0; a < 2; ++a)
 #pragma unroll
@@ -200,17 +276,16 @@ __global__ void __launch_bounds__(256) k_sw_panel(const SweepMat* __restrict__ m
       for (int q = 0; q < 4; ++q) {
         int r, c;
         acc_pos(a, b, q, r, c);
-        W[r * 64 + c] = acc[a][b][q];
         t[below ? r * 64 + c : c * 64 + r] = acc[a][b][q];
       }
 }
 
-// trailing tiles of step k: A_ij -= W_i X_j^T, i >= j, both != k.  Workgroup 0
-// takes the next diagonal tile and inverts it.
+// trailing tiles of step k: A_ij -= Y_i Y_j^T, i >= j, both != k.  Workgroup 0
+// takes the next diagonal tile and factors it.
 __global__ void __launch_bounds__(256) k_sw_trail(const SweepMat* __restrict__ mats, int k, double* tiles,
-                                                  const double* __restrict__ panw, const double* __restrict__ panx,
-                                                  double* dinv, int* info) {
+                                                  const double* __restrict__ pan, double* minv, int* info) {
   __shared__ __align__(16) double sw[64][LD], sx[64][LD];
+  __shared__ double mk[16][17];
   const SweepMat M = mats[blockIdx.y];
   const bool more = k + 1 < M.np;
   int i, j;
@@ -227,7 +302,9 @@ __global__ void __launch_bounds__(256) k_sw_trail(const SweepMat* __restrict__ m
     if (i == k || j == k || (more && i == k + 1 && j == k + 1)) return;
   }
   double* t = tiles + (M.off + tile_at(i, j)) * 4096;
-  d4 acc[2][2];
+  // the product is summed by itself and added once: 64 terms added to a tile
+  // that holds the sums of the steps before would each round at its size
+  d4 acc[2][2] = {}, old[2][2];
 #pragma unroll
   for (int a = 0; a < 2; ++a)
 #pragma unroll
@@ -236,10 +313,10 @@ __global__ void __launch_bounds__(256) k_sw_trail(const SweepMat* __restrict__ m
       for (int q = 0; q < 4; ++q) {
         int r, c;
         acc_pos(a, b, q, r, c);
-        acc[a][b][q] = t[r * 64 + c];
+        old[a][b][q] = t[r * 64 + c];
       }
-  stage(panw + (int64_t)(M.pan + i) * 4096, sw, -1.0);
-  stage(panx + (int64_t)(M.pan + j) * 4096, sx, 1.0);
+  stage(pan + (int64_t)(M.pan + i) * 4096, sw, -1.0);
+  stage(pan + (int64_t)(M.pan + j) * 4096, sx, 1.0);
   __syncthreads();
   mm64(sw, sx, acc);
   const bool next = blockIdx.x == 0;
@@ -252,12 +329,13 @@ __global__ void __launch_bounds__(256) k_sw_trail(const SweepMat* __restrict__ m
       for (int q = 0; q < 4; ++q) {
         int r, c;
         acc_pos(a, b, q, r, c);
-        if (next) sw[r][c] = acc[a][b][q];
-        else t[r * 64 + c] = acc[a][b][q];
+        const double v = old[a][b][q] + acc[a][b][q];
+        if (next) sw[r][c] = v;
+        else t[r * 64 + c] = v;
       }
   if (next) {
     __syncthreads();
-    invert_tile(sw, t, dinv + (int64_t)M.id * 4096, info + M.id, 64 * (k + 1));
+    factor_tile(sw, mk, t, minv + (int64_t)M.id * 4096, info + M.id, 64 * (k + 1));
   }
 }
 
@@ -272,15 +350,14 @@ void sweep_run(hipStream_t st, const SweepBatch& b, double* tiles) {
     if (h[0].np == 0) break;  // sorted by decreasing np
     int live = n;
     while (live > 0 && h[live - 1].np == 0) --live;
-    k_sw_first<<<live, 256, 0, st>>>(d, tiles, b.dinv, b.info);
+    k_sw_first<<<live, 256, 0, st>>>(d, tiles, b.minv, b.info);
     for (int k = 0; k < h[0].np; ++k) {
       while (live > 0 && h[live - 1].np <= k) --live;
       int nt = 0;
       for (int i = 0; i < live; ++i) nt = std::max(nt, h[i].nt);
       if (nt == 1) break;  // a single tile is done
-      k_sw_panel<<<dim3(nt, live), 256, 0, st>>>(d, k, tiles, b.panw, b.panx, b.dinv);
-      k_sw_trail<<<dim3((unsigned)(tile_at(nt, 0) + 1), live), 256, 0, st>>>(d, k, tiles, b.panw, b.panx, b.dinv,
-                                                                             b.info);
+      k_sw_panel<<<dim3(nt, live), 256, 0, st>>>(d, k, tiles, b.pan, b.minv);
+      k_sw_trail<<<dim3((unsigned)(tile_at(nt, 0) + 1), live), 256, 0, st>>>(d, k, tiles, b.pan, b.minv, b.info);
     }
   }
 }

@@ -16,7 +16,7 @@ struct SweepMat {
   int64_t off;
   int32_t np, nt;
   int32_t pan;  // first tile of its panels
-  int32_t id;   // slot of its diagonal inverse and of its error word
+  int32_t id;   // slot of its diagonal factor and of its error word
 };
 
 __host__ __device__ inline int64_t tile_at(int I, int J) { return (int64_t)I * (I + 1) / 2 + J; }
@@ -25,7 +25,7 @@ __host__ __device__ inline int64_t tile_at(int I, int J) { return (int64_t)I * (
 struct SweepBatch {
   std::vector<SweepMat> h;  // by decreasing np
   SweepMat* d = nullptr;    // device copy of h
-  double *panw = nullptr, *panx = nullptr, *dinv = nullptr;
+  double *pan = nullptr, *minv = nullptr;  // panels, inverse factors of the diagonal tiles
   int* info = nullptr;      // per id: 0, or 1 + the first pivot that is not positive
 };
 

@@ -124,3 +124,27 @@ def test_bottom_sweep_at_tile_edges(shape, kind, monkeypatch):
         r = s.kernel(_lib.OP_OPERATOR, 0, x, None, precision=1) - b
         assert np.abs(r).max() < tol * np.abs(b).max(), prec
     s.close()
+
+
+@pytest.mark.parametrize("kind", ["dense", "nd"])
+@pytest.mark.parametrize("shape", [(15, 7, 7), (11, 9, 9), (23, 14, 13)])
+def test_bottom_of_a_high_contrast_design(shape, kind, monkeypatch):
+    """a tenth of the cells solid, the others at density 0.002 (SIMP moduli 1
+    and 9e-9): condition numbers of 5e10 to 1.5e11, at which an inverse from
+    Cholesky factors leaves a residual of about eps cond |b| (2e-16 x 1.5e11 =
+    3.3e-5 is the bound; LAPACK's own leaves 3e-7 to 1.4e-6 on the first two),
+    and one from explicit inverses of pivot blocks does not converge"""
+    monkeypatch.setenv("SPG_BOTTOM", kind)
+    p = W.box(*shape, seed=2, mg_levels=1)
+    cells = p.density > 0
+    p.density[cells] = np.where(np.random.default_rng(3).random(int(cells.sum())) < 0.1, 1.0, 2e-3)
+    s = _lib.Solver(p)
+    gx, gf = s.level_nodes(0)
+    rng = np.random.default_rng(7)
+    b = rng.standard_normal((len(gx), 3))
+    b[(gf & 1) == 0] = 0
+    b[((gf[:, None] >> (1 + np.arange(3))) & 1).astype(bool)] = 0
+    x = s.kernel(_lib.OP_BOTTOM, 0, None, b, precision=1)
+    r = s.kernel(_lib.OP_OPERATOR, 0, x, None, precision=1) - b
+    assert np.abs(r).max() < 3.3e-5 * np.abs(b).max()
+    s.close()
