@@ -2030,7 +2030,7 @@ __global__ void __launch_bounds__(64) k_bnd_flow(BndOff L, ColourOrder ord, Colo
                                                  const int* __restrict__ list, const int* __restrict__ bci,
                                                  const T* __restrict__ A, const uint8_t* __restrict__ flags,
                                                  const T* __restrict__ bt, TagWord* tu, T* __restrict__ u, int* err,
-                                                 unsigned long long limit) {
+                                                 unsigned long long limit, int who) {
   constexpr int W = TagPack<T>::W, NW = 3 * W;
   const int lane = threadIdx.x, oct = lane >> 3, g = lane & 7;
   const int G = gridDim.x, steps = sweeps * 8;
@@ -2090,7 +2090,7 @@ __global__ void __launch_bounds__(64) k_bnd_flow(BndOff L, ColourOrder ord, Colo
       if (__all(ok)) break;
       if (first) t0 = wall_clock64();
       else if (wall_clock64() - t0 > limit) {
-        if (lane == 0) __hip_atomic_fetch_or(err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (lane == 0) __hip_atomic_fetch_or(err, who, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         return false;
       }
     }
@@ -2178,8 +2178,8 @@ __global__ void __launch_bounds__(64) k_bnd_flow(BndOff L, ColourOrder ord, Colo
 //            251 blocks      17 / 18    23 / 26    37 / 42
 //            1229 blocks     25 / -     -          46 / 57
 // The lines: where the launches win (FP64 level 0), or half of the blocks that
-// the registers let the 256 CUs hold at once, so that two solvers' launches
-// fit beside each other.
+// the registers let the 256 CUs hold at once, which leaves the other solvers of
+// a device something of its budget (flow_budget.hpp).
 template <class T>
 struct FlowBlocks {
   static constexpr int gs0 = sizeof(T) == 4 ? 4096 : 1536;
@@ -2219,7 +2219,7 @@ __device__ __forceinline__ void sweep_stage(int nb_l, const T* u, T* hu, int* ht
 // the nodes of a colour around the block, from their tagged entries (of blocks
 // `id`; with MASK only the nodes in the blocks' bit masks `hm`) into the halo
 // once they carry `tag` or a later one; false after a time-out
-template <class T, bool MASK>
+template <class T, bool MASK, int who>
 __device__ __forceinline__ bool sweep_take(int colour, const int* id, const unsigned long long* hm, T* hu,
                                            const TagWord* tu, unsigned tag, int* err, unsigned long long limit) {
   constexpr int W = TagPack<T>::W, NW = 3 * W, H = (NW + 1) / 2;
@@ -2246,7 +2246,7 @@ __device__ __forceinline__ bool sweep_take(int colour, const int* id, const unsi
     if (__all(ok)) break;
     if (first) t0 = wall_clock64();
     else if (wall_clock64() - t0 > limit) {
-      if (threadIdx.x == 0) __hip_atomic_fetch_or(err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (threadIdx.x == 0) __hip_atomic_fetch_or(err, who, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       return false;
     }
   }
@@ -2336,7 +2336,7 @@ __global__ void __launch_bounds__(64) k_st_flow(ColourOrder ord, const int* __re
       d[0] = m[0]; d[1] = m[4]; d[2] = m[8]; d[3] = m[1]; d[4] = m[2]; d[5] = m[5];
       if (F.fl & 1) dirichlet_inverse(d, F.fl);
     }
-    if (st && !sweep_take<T, false>(ord.at(st - 1), ht, nullptr, hu, tu, epoch, err, limit)) return false;
+    if (st && !sweep_take<T, false, kFlowSt>(ord.at(st - 1), ht, nullptr, hu, tu, epoch, err, limit)) return false;
     wave_lds_fence();
     const int l = colour_node(ord.at(st), k), pos = halo_pos(l);
     T a0 = 0, a1 = 0, a2 = 0;
@@ -2451,7 +2451,7 @@ __global__ void __launch_bounds__(64) k_gs0_flow(ColourOrder ord, const int* __r
   gs0_stage<T>(O, blk, ht, E, dx, he);
   for (int st = 0; st < 8; ++st) {
     const int c = ord.at(st), l = colour_node(c, k), pos = halo_pos(l);
-    if (st && !sweep_take<T, false>(ord.at(st - 1), ht, nullptr, hu, tu, epoch, err, limit)) return;
+    if (st && !sweep_take<T, false, kFlowGs0>(ord.at(st - 1), ht, nullptr, hu, tu, epoch, err, limit)) return;
     wave_lds_fence();
     T f0, f1, f2;
     gs0_rows<T>(l, pos, he, hu, dx, f0, f1, f2);
@@ -2502,7 +2502,9 @@ __global__ void __launch_bounds__(64) k_gs0_bnd_flow(ColourOrder ord, int sweeps
   const unsigned long long own = hm[13];
   for (int st = 0; st < 8 * sweeps; ++st) {
     const int c = ord.at(st & 7), l = colour_node(c, k), pos = halo_pos(l);
-    if (st && !sweep_take<T, true>(ord.at((st - 1) & 7), id, hm, hu, tu, last + ((st - 1) >> 3) + 1, err, limit)) return;
+    if (st && !sweep_take<T, true, kFlowBnd0>(ord.at((st - 1) & 7), id, hm, hu, tu, last + ((st - 1) >> 3) + 1, err,
+                                              limit))
+      return;
     wave_lds_fence();
     const bool set = (own >> l) & 1;
     if (!__any(set)) continue;
@@ -2817,7 +2819,7 @@ __device__ inline void cg_stage(CgScalars* sc, int stage) {
 __device__ inline void cg_report(const CgReport& rep, double nrm, int singular) {
   const unsigned long long b = (unsigned long long)__double_as_longlong(nrm);
   const unsigned part[kReportWords] = {(unsigned)b, (unsigned)(b >> 32),
-                                       (singular ? 1u : 0u) | (rep.err && *rep.err ? 2u : 0u)};
+                                       (singular ? 1u : 0u) | (rep.err ? (unsigned)*rep.err << 1 : 0u)};
 #pragma unroll
   for (int i = 0; i < kReportWords; ++i)
     __hip_atomic_store(rep.host + i, ((unsigned long long)rep.seq << 32) | part[i], __ATOMIC_RELAXED,
@@ -3531,86 +3533,116 @@ static unsigned long long flow_wait_limit() {
   }();
   return wait_50ms;
 }
-// boundary phase by data flow (k_bnd_flow); false if the level has no tables
-// for it or a cooperative launch is refused (the caller then runs another
-// path; `loud` reports a refused launch on stderr).  SPG_COOP_WG caps the
-// workgroup count (tests use it to make a wave take several node groups per
-// colour step).
-template <class T>
-static bool launch_bnd_flow(hipStream_t st, const LevelDev& L, T* u, const T* b, int sweeps, bool level0, bool forward,
-                            bool loud) {
-  const int n = L.bnd_off[8];
-  const T* A = BndPtr<T>::A(L);
-  T* bt = BndPtr<T>::bt(L);
-  if (!A || !bt || !L.bci || !L.bslot || !L.btag || !L.coop || L.coop_off) return false;
-  int groups = 1;
-  for (int c = 0; c < 8; ++c) groups = std::max(groups, (L.bnd_off[c + 1] - L.bnd_off[c] + 7) / 8);
-  int G = std::min(groups, BF_MAX_WG);
-  if (const char* e = std::getenv("SPG_COOP_WG"))
-    if (std::atoi(e) > 0) G = std::min(G, std::atoi(e));
-  unsigned long long lim = flow_wait_limit();
-  TagWord* tu = static_cast<TagWord*>(L.btag);
-  k_bnd_rhs<T><<<(n + 31) / 32, 256, 0, st>>>(n, L.bnd, L.bslot, A, u, b, bt, tu);
-  BndOff o;
-  for (int c = 0; c < 9; ++c) o.off[c] = L.bnd_off[c];
-  ColourOrder ord = colour_order(level0, forward), pos{0};
-  for (int i = 0; i < 8; ++i) pos.v |= (unsigned)i << (4 * ord.at(i));
-  const int* list = L.bnd;
-  const int* bci = L.bci;
-  const uint8_t* flags = L.flags;
-  int* err = reinterpret_cast<int*>(L.coop + 1);
-  int sw = sweeps;
-  // An ordinary launch by default: the solver's stream runs one kernel at a
-  // time, so the one-wave workgroups (at most 512: 2 per CU) all start at
-  // once on the empty device.  The cooperative launch API guarantees that
-  // even while other streams fill the device, but costs about 40 us per
-  // phase; SPG_COOP_LAUNCH=1 selects it.  Either way a wait ends after the
-  // limit and is reported.
-  const char* cl = std::getenv("SPG_COOP_LAUNCH");
-  if (!(cl && std::atoi(cl) == 1)) {
-    k_bnd_flow<T><<<G, 64, 0, st>>>(o, ord, pos, sw, list, bci, A, flags, bt, tu, u, err, lim);
-    return true;
-  }
-  void* args[] = {&o, &ord, &pos, &sw, &list, &bci, &A, &flags, &bt, &tu, &u, &err, &lim};
-  const hipError_t e = hipLaunchCooperativeKernel((const void*)k_bnd_flow<T>, dim3(G), dim3(64), args, 0, st);
-  if (e == hipSuccess) return true;
-  (void)hipGetLastError();
-  if (loud)
-    std::fprintf(stderr, "spgrid_topo_opt_amd: cooperative boundary phase not launched (%s); using the list path\n",
-               hipGetErrorString(e));
-  return false;
+// A data-flow launch: an ordinary one, for which the caller holds the device's
+// budget, or with SPG_COOP_LAUNCH=1 one through the cooperative launch API,
+// which starts all workgroups together whatever else runs (about 40 us more a
+// launch) or refuses.  False if refused: the caller takes another path; `loud`
+// reports that on stderr.
+static bool coop_launch() {
+  const char* e = std::getenv("SPG_COOP_LAUNCH");
+  return e && std::atoi(e) == 1;
 }
-// level-0 boundary phase over blocks (k_gs0_bnd_flow); false as above.  A cap
-// on the workgroups needs the node-list kernel.
 template <class T>
-static bool launch_gs0_bnd_flow(hipStream_t st, const LevelDev& L, const T* E, T dx, T* u, const T* b, int sweeps,
-                                bool forward, bool loud) {
-  if (!L.fb_last || !L.coop || L.coop_off || L.fb_n > FlowBlocks<T>::gs0) return false;
-  if (const char* e = std::getenv("SPG_COOP_WG"))
-    if (std::atoi(e) > 0) return false;
-  ColourOrder ord = colour_order(true, forward);
-  TagWord* tu = static_cast<TagWord*>(L.fb_tag);
-  int* err = reinterpret_cast<int*>(L.coop + 1);
-  unsigned last = *L.fb_last;
-  unsigned long long lim = flow_wait_limit();
-  *L.fb_last += (unsigned)sweeps;
-  const char* cl = std::getenv("SPG_COOP_LAUNCH");
-  if (!(cl && std::atoi(cl) == 1)) {
-    k_gs0_bnd_flow<T><<<L.fb_n, 64, 0, st>>>(ord, sweeps, L.fb_blk, L.fb_nbr, L.fb_id, L.fb_mask, L.flags, E, dx, u, b,
-                                            tu, last, err, lim);
+struct SameType {
+  using type = T;
+};
+template <class... P>
+static bool launch_flow(void (*kernel)(P...), int waves, hipStream_t st, bool loud, typename SameType<P>::type... p) {
+  if (!coop_launch()) {
+    kernel<<<waves, 64, 0, st>>>(p...);
     return true;
   }
-  const int *fblk = L.fb_blk, *fnbr = L.fb_nbr, *fid = L.fb_id;
-  const unsigned long long* fmask = L.fb_mask;
-  const uint8_t* flags = L.flags;
-  void* args[] = {&ord, &sweeps, &fblk, &fnbr, &fid, &fmask, &flags, &E, &dx, &u, &b, &tu, &last, &err, &lim};
-  const hipError_t e = hipLaunchCooperativeKernel((const void*)k_gs0_bnd_flow<T>, dim3(L.fb_n), dim3(64), args, 0, st);
+  void* args[] = {const_cast<void*>(static_cast<const volatile void*>(&p))...};
+  const hipError_t e = hipLaunchCooperativeKernel((const void*)kernel, dim3(waves), dim3(64), args, 0, st);
   if (e == hipSuccess) return true;
   (void)hipGetLastError();
   if (loud)
     std::fprintf(stderr, "spgrid_topo_opt_amd: cooperative boundary phase not launched (%s); using the list path\n",
                  hipGetErrorString(e));
   return false;
+}
+// waves of the level's boundary phase by node groups; 0 if it has no tables for it
+static int bnd_flow_waves(const LevelDev& L) {
+  if (!L.bci || !L.bslot || !L.btag || !L.coop || L.flow == kFlowNone) return 0;
+  int groups = 1;
+  for (int c = 0; c < 8; ++c) groups = std::max(groups, (L.bnd_off[c + 1] - L.bnd_off[c] + 7) / 8);
+  return std::min(groups, L.flow == kFlowFew ? kFlowFewWaves : BF_MAX_WG);
+}
+// waves of the level-0 boundary phase over blocks; 0 as above
+template <class T>
+static int gs0_bnd_flow_waves(const LevelDev& L) {
+  return L.fb_last && L.coop && L.flow == kFlowAll && L.fb_n <= FlowBlocks<T>::gs0 ? L.fb_n : 0;
+}
+// waves of a whole sweep by data flow; 0 where the level has no tagged entries
+// for it or more blocks than `most`
+static int sweep_flow_waves(const LevelDev& L, int most) {
+  return L.stag && L.epoch && L.coop && L.flow == kFlowAll && L.nb <= most ? L.nb : 0;
+}
+// one-wave workgroups of a kernel that fit a CU
+template <class F>
+static int flow_fit(F kernel) {
+  int n = 0;
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, reinterpret_cast<const void*>(kernel), 64, 0) != hipSuccess) {
+    (void)hipGetLastError();
+    n = 1;
+  }
+  return n;
+}
+template <class T>
+static void add_flow_need_t(FlowNeed& need, const LevelDev& L, bool level0) {
+  static const int fit_bnd = flow_fit(k_bnd_flow<T>), fit_bnd0 = flow_fit(k_gs0_bnd_flow<T>),
+                   fit_gs0 = flow_fit(k_gs0_flow<T>), fit_st = flow_fit(k_st_flow<T>);
+  need.add(bnd_flow_waves(L), fit_bnd);
+  if (level0) {
+    need.add(gs0_bnd_flow_waves<T>(L), fit_bnd0);
+    need.add(sweep_flow_waves(L, FlowBlocks<T>::gs0), fit_gs0);
+  } else {
+    need.add(sweep_flow_waves(L, FlowBlocks<T>::st), fit_st);
+  }
+}
+void add_flow_need(FlowNeed& need, const LevelDev& L, bool level0, bool fp64, FlowUse use) {
+  LevelDev l = L;
+  l.flow = use;
+  if (fp64) add_flow_need_t<double>(need, l, level0);
+  else add_flow_need_t<float>(need, l, level0);
+}
+// boundary phase by data flow (k_bnd_flow); false if the level has no tables
+// for it or the launch is refused (the caller then runs another path).
+// SPG_COOP_WG caps the workgroup count (tests use it to make a wave take
+// several node groups per colour step).
+template <class T>
+static bool launch_bnd_flow(hipStream_t st, const LevelDev& L, T* u, const T* b, int sweeps, bool level0, bool forward,
+                            bool loud) {
+  const int n = L.bnd_off[8];
+  const T* A = BndPtr<T>::A(L);
+  T* bt = BndPtr<T>::bt(L);
+  int G = bnd_flow_waves(L);
+  if (!A || !bt || G == 0) return false;
+  if (const char* e = std::getenv("SPG_COOP_WG"))
+    if (std::atoi(e) > 0) G = std::min(G, std::atoi(e));
+  TagWord* tu = static_cast<TagWord*>(L.btag);
+  k_bnd_rhs<T><<<(n + 31) / 32, 256, 0, st>>>(n, L.bnd, L.bslot, A, u, b, bt, tu);
+  BndOff o;
+  for (int c = 0; c < 9; ++c) o.off[c] = L.bnd_off[c];
+  ColourOrder ord = colour_order(level0, forward), pos{0};
+  for (int i = 0; i < 8; ++i) pos.v |= (unsigned)i << (4 * ord.at(i));
+  return launch_flow(k_bnd_flow<T>, G, st, loud, o, ord, pos, sweeps, L.bnd, L.bci, A, L.flags, (const T*)bt, tu, u,
+                     reinterpret_cast<int*>(L.coop + 1), flow_wait_limit(), (int)(level0 ? kFlowBnd0 : kFlowBndSt));
+}
+// level-0 boundary phase over blocks (k_gs0_bnd_flow); false as above.  A cap
+// on the workgroups needs the node-list kernel.
+template <class T>
+static bool launch_gs0_bnd_flow(hipStream_t st, const LevelDev& L, const T* E, T dx, T* u, const T* b, int sweeps,
+                                bool forward, bool loud) {
+  const int waves = gs0_bnd_flow_waves<T>(L);
+  if (waves == 0) return false;
+  if (const char* e = std::getenv("SPG_COOP_WG"))
+    if (std::atoi(e) > 0) return false;
+  const unsigned last = *L.fb_last;
+  *L.fb_last += (unsigned)sweeps;
+  return launch_flow(k_gs0_bnd_flow<T>, waves, st, loud, colour_order(true, forward), sweeps, L.fb_blk, L.fb_nbr,
+                     L.fb_id, L.fb_mask, L.flags, E, dx, u, b, static_cast<TagWord*>(L.fb_tag), last,
+                     reinterpret_cast<int*>(L.coop + 1), flow_wait_limit());
 }
 template <class T>
 struct BmapPtr;
@@ -3749,19 +3781,14 @@ void launch_gs0(hipStream_t st, const LevelDev& L, const T* E, T dx, T* u, const
     k_gs0_colour<T><<<nwg, 64 * GS_WAVES, 0, st>>>(L.nb, colour, L.nbr, L.flags, E, dx, u, b);
   }
 }
-// one whole sweep by data flow where the level has the tagged entries for it
-static bool sweep_flows(const LevelDev& L, int most) {
-  return L.stag && L.epoch && L.coop && !L.coop_off && L.nb <= most;
-}
 template <class T>
 void launch_gs0_sweep(hipStream_t st, const LevelDev& L, const T* E, T dx, T* u, const T* b, bool forward,
                       const T* bcm) {
-  if (sweep_flows(L, FlowBlocks<T>::gs0) && !std::getenv("SPG_GS_KERNEL")) {
-    k_gs0_flow<T><<<L.nb, 64, 0, st>>>(
-        colour_order(true, forward), L.nbr, L.flags, E, dx, u, b, static_cast<TagWord*>(L.stag), ++*L.epoch,
-        reinterpret_cast<int*>(L.coop + 1), flow_wait_limit());
+  const int waves = std::getenv("SPG_GS_KERNEL") ? 0 : sweep_flow_waves(L, FlowBlocks<T>::gs0);
+  if (waves > 0 && launch_flow(k_gs0_flow<T>, waves, st, false, colour_order(true, forward), L.nbr, L.flags, E, dx, u,
+                               b, static_cast<TagWord*>(L.stag), ++*L.epoch, reinterpret_cast<int*>(L.coop + 1),
+                               flow_wait_limit()))
     return;
-  }
   for (int c = 0; c < 8; ++c) launch_gs0<T>(st, L, E, dx, u, b, sweep_colour(true, forward, c), nullptr, 0, bcm);
 }
 template <class T>
@@ -3808,12 +3835,11 @@ void launch_st_gs(hipStream_t st, const LevelDev& L, const T* ST, T* u, const T*
 }
 template <class T>
 void launch_st_sweep(hipStream_t st, const LevelDev& L, const T* ST, T* u, const T* b, bool forward) {
-  if (sweep_flows(L, FlowBlocks<T>::st)) {
-    k_st_flow<T><<<L.nb, 64, 0, st>>>(
-        colour_order(false, forward), L.nbr, L.flags, ST, u, b, static_cast<TagWord*>(L.stag), ++*L.epoch,
-        reinterpret_cast<int*>(L.coop + 1), flow_wait_limit());
+  const int waves = sweep_flow_waves(L, FlowBlocks<T>::st);
+  if (waves > 0 && launch_flow(k_st_flow<T>, waves, st, false, colour_order(false, forward), L.nbr, L.flags, ST, u, b,
+                               static_cast<TagWord*>(L.stag), ++*L.epoch, reinterpret_cast<int*>(L.coop + 1),
+                               flow_wait_limit()))
     return;
-  }
   for (int c = 0; c < 8; ++c) launch_st_gs<T>(st, L, ST, u, b, sweep_colour(false, forward, c));
 }
 template <class T>

@@ -10,6 +10,8 @@
 
 #include <cstdint>
 
+#include "flow_budget.hpp"
+
 namespace spg {
 
 // constants of the strain-form cell operator per unit modulus: 9mu, 4.5la,
@@ -18,6 +20,14 @@ struct CellConsts {
   double d = 0, t = 0, s = 0, w = 0, q = 0, c3 = 0;
 };
 CellConsts cell_consts(double mu, double lambda);
+
+// Data-flow kernels wait between workgroups, so their waves must run together:
+// which of them a call may use follows from what the device's budget
+// (flow_budget.hpp) has left.
+enum FlowUse { kFlowNone = 0, kFlowFew = 1, kFlowAll = 2 };  // few: boundary phases by at most kFlowFewWaves
+static constexpr int kFlowFewWaves = 64;
+// the error word's bits: whose wait timed out
+enum FlowWho { kFlowBnd0 = 1, kFlowBndSt = 2, kFlowGs0 = 4, kFlowSt = 8 };
 
 struct LevelDev {
   int nb = 0;
@@ -67,7 +77,7 @@ struct LevelDev {
   const unsigned long long* fb_mask = nullptr;
   void* fb_tag = nullptr;
   unsigned* fb_last = nullptr;
-  int coop_off = 0;  // 1 after a wait timed out: the list launches take over
+  int flow = 0;  // which data-flow kernels this call may use (FlowUse)
   // slots of all neighbours of the boundary nodes ([n*32], in or outside the
   // set), and dense maps of one boundary phase (forward, backward colour
   // order) for `bmap_sweeps` sweeps with their input ([bmap_stride(n)])
@@ -115,8 +125,8 @@ struct CgScalars {
 
 // What a PCG iteration's last kernel tells the host: words of pinned host
 // memory that carry a 32-bit part of the report and the report's number
-// (halves of ||r||_inf; bit 0 singular, bit 1 a data-flow wait timed out, from
-// `err`).  The host reads them as they arrive, without a copy or a
+// (halves of ||r||_inf; bit 0 singular, from bit 1 on the error word `err`:
+// FlowWho of data-flow waits that timed out).  The host reads them as they arrive, without a copy or a
 // synchronisation.
 struct CgReport {
   unsigned long long* host = nullptr;
@@ -141,6 +151,9 @@ int64_t apply_dot_partials(int64_t nb);
 template <class T>
 int launch_apply_dot(hipStream_t st, const LevelDev& L, const T* E, T dx, const T* in, T* out, double* bpart,
                      double* part, double* dot, CgScalars* sc = nullptr, int stage = -1);
+// what the level's data-flow kernels take of the device at most, of one
+// precision, under `use`
+void add_flow_need(FlowNeed& need, const LevelDev& L, bool level0, bool fp64, FlowUse use);
 // level-0 GS: one colour over all blocks; all boundary sweeps of one phase.
 // With `bcm` (b in colour-major order, launch_colour_major) and the level's
 // flags_cm, the colour kernel reads b and the flags of its colour only.

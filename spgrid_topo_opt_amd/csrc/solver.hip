@@ -41,9 +41,9 @@ static constexpr int kMaxDenseBoundary = 2560;
 // levels of at most this many blocks get the entries of the data-flow sweep
 // (FlowBlocks in kernels.hip has each kernel's own limit)
 static constexpr int kMaxFlowSweep = 4096;
-// pcg() result: a level-0 boundary phase reported a barrier time-out; the
-// pass is repeated with the per-colour list launches
-static constexpr int kCoopRetry = -100;
+// pcg() result: a data-flow kernel reported a wait that timed out; the pass is
+// repeated with per-colour launches
+static constexpr int kFlowRetry = -100;
 // byte offset of the PCG report in the pinned scalar buffer
 static constexpr int kReportOffset = 128;
 // relative residual reduction one FP32 MG-PCG pass is asked for at most
@@ -179,19 +179,75 @@ void Solver::activate() {
   k.lambda = cfg_.lambda;
 }
 
-void Solver::check_coop() {
+// names of the FlowWho bits
+static std::string flow_names(unsigned who) {
+  static const std::pair<unsigned, const char*> kNames[] = {{kFlowBnd0, "level-0 boundary phase"},
+                                                            {kFlowBndSt, "boundary phase of an explicit level"},
+                                                            {kFlowGs0, "level-0 sweep"},
+                                                            {kFlowSt, "sweep of an explicit level"}};
+  std::string s;
+  for (const auto& [bit, name] : kNames)
+    if (who & bit) s += (s.empty() ? "" : ", ") + std::string(name);
+  return s;
+}
+
+void Solver::check_flow() {
   if (lv_.empty() || !lv_[0].coop.p) return;
   unsigned w[2] = {0, 0};
   HIPCHK(hipMemcpyAsync(w, lv_[0].coop.p, sizeof(w), hipMemcpyDeviceToHost, st_));
   HIPCHK(hipStreamSynchronize(st_));
   if (w[1]) {
-    // reported once: the next phase starts from a clear word
+    // reported once: the next kernel starts from a clear word
     HIPCHK(hipMemsetAsync(static_cast<unsigned*>(lv_[0].coop.p) + 1, 0, sizeof(unsigned), st_));
     HIPCHK(hipStreamSynchronize(st_));
-    throw SpgError(SPG_E_HIP,
-                   "level-0 boundary phase: a wait timed out (workgroups not resident together; "
-                   "SPG_COOP_LAUNCH=1 uses the cooperative launch API, SPG_BOUNDARY_PATH=2 per-colour launches)");
+    throw SpgError(SPG_E_HIP, flow_names(w[1]) +
+                                  ": a wait timed out (workgroups not resident together; SPG_COOP_LAUNCH=1 uses the "
+                                  "cooperative launch API, SPG_DATA_FLOW=0 per-colour launches on every level)");
   }
+}
+
+// waves of data-flow kernels that the solvers of this process have on each device
+static FlowBudget& flow_budget() {
+  static FlowBudget* b = new FlowBudget();  // outlives every solver
+  return *b;
+}
+
+void Solver::set_flow(FlowUse use) {
+  for (LevelRT& R : lv_) R.d.flow = use;
+}
+
+// All data-flow kernels if their waves fit beside those that other solvers have
+// on the device; else boundary phases by few waves; else none.  A cooperative
+// launch makes its own room.  SPG_DATA_FLOW=0: none.
+Solver::FlowLease::FlowLease(Solver& s, int precision) : s_(s) {
+  const char* sw = std::getenv("SPG_DATA_FLOW");
+  const char* coop = std::getenv("SPG_COOP_LAUNCH");
+  FlowUse use = kFlowNone;
+  if (s.flow_dead_ || (sw && std::atoi(sw) == 0)) {
+  } else if (coop && std::atoi(coop) == 1) {
+    use = kFlowAll;
+  } else {
+    int cus = 0;
+    HIPCHK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, s.cfg_.device));
+    for (const FlowUse u : {kFlowAll, kFlowFew}) {
+      need_ = FlowNeed();
+      for (size_t l = 0; l < s.lv_.size(); ++l) {
+        if (precision != 1) add_flow_need(need_, s.lv_[l].d, l == 0, false, u);
+        if (precision == 1 || s.coarse64_) add_flow_need(need_, s.lv_[l].d, l == 0, true, u);
+      }
+      held_ = need_.cus == 0.0 || flow_budget().take(s.cfg_.device, cus, need_);
+      if (!held_) continue;
+      held_ = need_.cus > 0.0;
+      use = u;
+      break;
+    }
+  }
+  s_.set_flow(use);
+}
+
+Solver::FlowLease::~FlowLease() {
+  s_.set_flow(kFlowNone);
+  if (held_) flow_budget().give(s_.cfg_.device, need_);
 }
 
 void Solver::upload_layout() {
@@ -940,7 +996,7 @@ CgReport Solver::report() {
   CgReport r;
   r.host = reinterpret_cast<unsigned long long*>(reinterpret_cast<char*>(hscal_) + kReportOffset);
   r.seq = ++report_seq_;
-  if (lv_[0].coop.p && !lv_[0].d.coop_off) r.err = lv_[0].coop.as<int>() + 1;
+  if (lv_[0].coop.p && lv_[0].d.flow) r.err = lv_[0].coop.as<int>() + 1;
   return r;
 }
 
@@ -991,7 +1047,7 @@ int Solver::pcg(T* x, T* r, double tol, int maxit, int* iters, double* last_nrm)
   launch_linf<T>(st_, r, n, part, &sc->nrm, report(), sc);
   int it = 0;
   int rc = SPG_E_NOT_CONVERGED;
-  const bool coop = lv_[0].coop.p && !lv_[0].d.coop_off;
+  const bool flows = lv_[0].coop.p && lv_[0].d.flow;
   // The next V-cycle's first boundary phase, which changes nothing but z, is
   // launched before the host reads the residual: the device has work while the
   // host decides and launches the rest.  With that, and the report written by
@@ -1005,18 +1061,20 @@ int Solver::pcg(T* x, T* r, double tol, int maxit, int* iters, double* last_nrm)
     double nrm;
     unsigned bits;
     wait_report(&nrm, &bits);
-    if (bits & 2) {
-      // the last V-cycle's boundary phase ended early: its result is not a
-      // Gauss-Seidel sweep.  Switch to the list launches for good and let
-      // the caller repeat the pass.
+    if (bits >> 1) {
+      // a kernel of the last V-cycle ended early: its result is not a
+      // Gauss-Seidel sweep.  Use none of them any more and let the caller
+      // repeat the pass.
       HIPCHK(hipMemsetAsync(lv_[0].coop.as<unsigned>() + 1, 0, sizeof(unsigned), st_));
       sync();
-      for (LevelRT& R : lv_) R.d.coop_off = 1;
+      flow_dead_ = true;
+      set_flow(kFlowNone);
       std::fprintf(stderr,
-                   "spgrid_topo_opt_amd: level-0 boundary phase barrier timed out (workgroups not resident "
-                   "together); continuing with per-colour launches\n");
+                   "spgrid_topo_opt_amd: %s: a wait timed out (workgroups not resident together); continuing with "
+                   "per-colour launches\n",
+                   flow_names(bits >> 1).c_str());
       *iters = it;
-      return kCoopRetry;
+      return kFlowRetry;
     }
     *last_nrm = nrm;
     if (print_residuals_) {
@@ -1046,7 +1104,7 @@ int Solver::pcg(T* x, T* r, double tol, int maxit, int* iters, double* last_nrm)
     launch_cg_update<T>(st_, x, r, s, q, sc, n, 2, z, report(), apart_.as<double>(), nq);
   }
   // a time-out in a phase whose result nobody uses is nobody's error
-  if (ahead && coop) HIPCHK(hipMemsetAsync(lv_[0].coop.as<unsigned>() + 1, 0, sizeof(unsigned), st_));
+  if (ahead && flows) HIPCHK(hipMemsetAsync(lv_[0].coop.as<unsigned>() + 1, 0, sizeof(unsigned), st_));
   *iters = it;
   return rc;
 }
@@ -1057,6 +1115,7 @@ void Solver::reset_to_ud(double* u) {
 }
 
 int Solver::solve_rhs(const spg_solve_params& prm, double* u, const double* f, spg_info* info, bool warm) {
+  const FlowLease lease(*this, prm.precision);
   const LevelRT& R0 = lv_[0];
   const int64_t n = R0.n3;
   const double t0 = now_s();
@@ -1113,9 +1172,9 @@ int Solver::solve_rhs(const spg_solve_params& prm, double* u, const double* f, s
         launch_cast_d2f(st_, res_.as<double>(), rr32_.as<float>(), n);
         prc = pcg<float>(x32_.as<float>(), rr32_.as<float>(), tolp, prm.max_iterations, &it, &last);
       }
-      if (prc != kCoopRetry) break;
+      if (prc != kFlowRetry) break;
       total += it;
-      if (attempt > 0) throw SpgError(SPG_E_HIP, "boundary phase failed after the switch to list launches");
+      if (attempt > 0) throw SpgError(SPG_E_HIP, "a data-flow wait timed out after the switch to per-colour launches");
     }
     if (prm.precision == 1) launch_axpy_d<double>(st_, u, x64_.as<double>(), n);
     else launch_axpy_d<float>(st_, u, x32_.as<float>(), n);
@@ -1142,7 +1201,7 @@ int Solver::solve_rhs(const spg_solve_params& prm, double* u, const double* f, s
     info->r_start_linf = rstart;
     info->warm_reused = reused ? 1 : 0;
   }
-  check_coop();
+  check_flow();
   if (rc == SPG_OK && !conv) rc = SPG_E_NOT_CONVERGED;
   return rc;
 }
@@ -1301,6 +1360,7 @@ void Solver::run_kernel(int op, int level, int precision, int forward, const dou
                         double* out) {
   activate();
   if (level < 0 || level >= lay_.nlev) throw SpgError(SPG_E_INVALID, "level out of range");
+  const FlowLease lease(*this, precision);
   auto body = [&](auto tag) {
     using T = decltype(tag);
     auto put = [&](DBuf& d, const double* h, int64_t nb) {
@@ -1395,7 +1455,7 @@ void Solver::run_kernel(int op, int level, int precision, int forward, const dou
   };
   if (precision == 1) body(double());
   else body(float());
-  check_coop();
+  check_flow();
 }
 
 void Solver::level_stencils(int level, double* out) {
@@ -1443,6 +1503,7 @@ double Solver::bench_kernel(int op, int level, int precision, int arg, int reps)
   activate();
   if (level < 0 || level >= lay_.nlev) throw SpgError(SPG_E_INVALID, "level out of range");
   const int B = lay_.nlev - 1;
+  const FlowLease lease(*this, precision);
   hipEvent_t e0, e1;
   HIPCHK(hipEventCreate(&e0));
   HIPCHK(hipEventCreate(&e1));
@@ -1508,7 +1569,7 @@ double Solver::bench_kernel(int op, int level, int precision, int arg, int reps)
   HIPCHK(hipEventElapsedTime(&ms, e0, e1));
   (void)hipEventDestroy(e0);
   (void)hipEventDestroy(e1);
-  check_coop();
+  check_flow();
   return (double)ms * 1e-3 / reps;
 }
 

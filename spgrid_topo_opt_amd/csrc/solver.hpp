@@ -143,9 +143,25 @@ class Solver {
   void upload_layout();
   double read_scalar(const double* dev);
   void sync();
-  // throws (once per event) if a cooperative boundary phase reported a
-  // barrier time-out
-  void check_coop();
+  // throws (once per event) if a data-flow kernel reported a wait that timed out
+  void check_flow();
+  // A call's share of its device's budget of waves that wait for each other
+  // (flow_budget.hpp), given back when the call ends; sets what the levels may
+  // use meanwhile.
+  class FlowLease {
+   public:
+    FlowLease(Solver& s, int precision);
+    ~FlowLease();
+    FlowLease(const FlowLease&) = delete;
+    FlowLease& operator=(const FlowLease&) = delete;
+
+   private:
+    Solver& s_;
+    FlowNeed need_;
+    bool held_ = false;
+  };
+  void set_flow(FlowUse use);
+  bool flow_dead_ = false;  // a wait has timed out in a solve: no data-flow kernels any more
 
   spg_config cfg_;
   Layout lay_;
