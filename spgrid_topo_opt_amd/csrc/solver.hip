@@ -525,6 +525,8 @@ void Solver::build_operators() {
     } catch (const std::exception& e) {
       throw SpgError(SPG_E_HIP, std::string("nested-dissection bottom: ") + e.what());
     }
+    build_boundary_maps();
+    mark("boundary maps");
     return;
   }
   nd_.reset();
@@ -568,6 +570,8 @@ void Solver::build_operators() {
     throw SpgError(SPG_E_SINGULAR, "bottom Cholesky failed: leading minor " + std::to_string(hinfo) +
                                        " not positive definite");
   mark("bottom (dense inverse)");
+  build_boundary_maps();
+  mark("boundary maps");
 }
 
 // coefficient rows of the boundary system of every smoothed level
@@ -586,41 +590,78 @@ void Solver::build_boundary_rows() {
     else if (lay_.lv[l].is_explicit) launch_bnd_coef_st(st_, R.d, R.st64.as<double>(), R.bA64.as<double>());
     else continue;
     launch_cast_d2f(st_, R.bA64.as<double>(), R.bA32.as<float>(), (int64_t)n * 288);
-    // small boundary sets: each phase becomes one dense map
-    if (n <= kMaxDenseBoundary && cfg_.boundary_iters > 0) {
-      const size_t entries = (size_t)3 * n * bmap_stride(n);
-      for (int d = 0; d < 2; ++d)
-        if (!R.bmap64[d].p) {
-          // padding columns stay zero: the build writes columns < 3n only
-          R.bmap64[d].alloc(entries * 8);
-          R.bmap32[d].alloc(entries * 4);
-          HIPCHK(hipMemsetAsync(R.bmap64[d].p, 0, entries * 8, st_));
-          HIPCHK(hipMemsetAsync(R.bmap32[d].p, 0, entries * 4, st_));
-          R.d.bmap64[d] = R.bmap64[d].as<double>();
-          R.d.bmap32[d] = R.bmap32[d].as<float>();
-        }
-      double* const M[2] = {R.bmap64[0].as<double>(), R.bmap64[1].as<double>()};
-      float* const F[2] = {R.bmap32[0].as<float>(), R.bmap32[1].as<float>()};
-      launch_bmap_build(st_, R.d, cfg_.boundary_iters, l == 0, M, F);
-      if (!R.bmx64.p) {
-        const size_t nx = (size_t)bmap_stride(n);
-        const LevelDesc& D = lay_.lv[l];
-        std::vector<int32_t> list, all(D.bnd_ci.size());
-        for (int c = 0; c < 8; ++c) list.insert(list.end(), D.bnd_list[c].begin(), D.bnd_list[c].end());
-        for (size_t e = 0; e < all.size(); ++e) all[e] = D.bnd_ci[e] >= 0 ? list[D.bnd_ci[e]] : D.bnd_slot[e];
-        upload(R.ball, all);
-        R.d.ball = R.ball.as<int>();
-        R.bmx64.alloc(nx * 8);
-        R.bmx32.alloc(nx * 4);
-        HIPCHK(hipMemsetAsync(R.bmx64.p, 0, nx * 8, st_));
-        HIPCHK(hipMemsetAsync(R.bmx32.p, 0, nx * 4, st_));
-      }
-      R.d.bmx64 = R.bmx64.as<double>();
-      R.d.bmx32 = R.bmx32.as<float>();
-      R.d.bmap_sweeps = cfg_.boundary_iters;
-    }
   }
   sync();
+}
+
+// Small boundary sets: each phase becomes one dense map.  The maps are optional
+// (up to 1.4 GB a level), so they come after everything the solve needs, and a
+// level for which there is no memory runs its phases by data flow instead.
+void Solver::build_boundary_maps() {
+  if (cfg_.boundary_iters <= 0) return;
+  for (int l = 0; l < lay_.nlev; ++l) {
+    LevelRT& R = lv_[l];
+    const int n = R.d.bnd_off[8];
+    if (n == 0 || !R.bA64.p || n > kMaxDenseBoundary || R.no_maps) continue;
+    if (l > 0 && !lay_.lv[l].is_explicit) continue;
+    if (!R.d.bmap_sweeps && !alloc_boundary_maps(l)) {
+      R.no_maps = true;
+      continue;
+    }
+    double* const M[2] = {R.bmap64[0].as<double>(), R.bmap64[1].as<double>()};
+    float* const F[2] = {R.bmap32[0].as<float>(), R.bmap32[1].as<float>()};
+    launch_bmap_build(st_, R.d, cfg_.boundary_iters, l == 0, M, F);
+  }
+  sync();
+}
+
+bool Solver::alloc_boundary_maps(int l) {
+  LevelRT& R = lv_[l];
+  const int n = R.d.bnd_off[8];
+  const size_t entries = (size_t)3 * n * bmap_stride(n), nx = (size_t)bmap_stride(n);
+  try {
+    // SPG_MAP_MAX_MB: what the maps of a level may take
+    const char* e = std::getenv("SPG_MAP_MAX_MB");
+    if (e && (double)entries * 24.0 > std::atof(e) * 1048576.0) throw SpgError(SPG_E_HIP, "SPG_MAP_MAX_MB");
+    for (int d = 0; d < 2; ++d) {
+      R.bmap64[d].alloc(entries * 8);
+      R.bmap32[d].alloc(entries * 4);
+    }
+    const LevelDesc& D = lay_.lv[l];
+    std::vector<int32_t> list, all(D.bnd_ci.size());
+    for (int c = 0; c < 8; ++c) list.insert(list.end(), D.bnd_list[c].begin(), D.bnd_list[c].end());
+    for (size_t k = 0; k < all.size(); ++k) all[k] = D.bnd_ci[k] >= 0 ? list[D.bnd_ci[k]] : D.bnd_slot[k];
+    upload(R.ball, all);
+    R.bmx64.alloc(nx * 8);
+    R.bmx32.alloc(nx * 4);
+  } catch (const SpgError&) {
+    (void)hipGetLastError();
+    for (DBuf* b : {&R.bmap64[0], &R.bmap64[1], &R.bmap32[0], &R.bmap32[1], &R.ball, &R.bmx64, &R.bmx32}) b->alloc(0);
+    if (!R.btag.p && lv_[0].coop.p) {  // an explicit level of this size has none yet
+      try {
+        R.btag.alloc((size_t)n * 6 * 8);
+        R.d.btag = R.btag.p;
+        R.d.coop = lv_[0].coop.as<unsigned>();
+      } catch (const SpgError&) {
+        (void)hipGetLastError();  // its phases run in one workgroup
+      }
+    }
+    return false;
+  }
+  for (int d = 0; d < 2; ++d) {
+    // padding columns stay zero: the build writes columns < 3n only
+    HIPCHK(hipMemsetAsync(R.bmap64[d].p, 0, entries * 8, st_));
+    HIPCHK(hipMemsetAsync(R.bmap32[d].p, 0, entries * 4, st_));
+    R.d.bmap64[d] = R.bmap64[d].as<double>();
+    R.d.bmap32[d] = R.bmap32[d].as<float>();
+  }
+  HIPCHK(hipMemsetAsync(R.bmx64.p, 0, nx * 8, st_));
+  HIPCHK(hipMemsetAsync(R.bmx32.p, 0, nx * 4, st_));
+  R.d.ball = R.ball.as<int>();
+  R.d.bmx64 = R.bmx64.as<double>();
+  R.d.bmx32 = R.bmx32.as<float>();
+  R.d.bmap_sweeps = cfg_.boundary_iters;
+  return true;
 }
 
 // The lowest i in [0, n) with ev(i) != 0, and ev there (n and 0 if none):

@@ -54,6 +54,7 @@ struct LevelRT {
   DBuf b0cslot, b0node, b0E64, b0E32, b0D64, b0D32;  // level-0 matrix-free boundary system
   DBuf btag, coop;  // data-flow boundary phase: tagged iterate; level 0: {unused, error word}
   DBuf ball, bmap64[2], bmap32[2], bmx64, bmx32;     // dense boundary maps
+  bool no_maps = false;                              // there was no memory for them
   DBuf stag;                                         // data-flow sweep: tagged entries
   unsigned epoch = 0;                                // its launches so far
   DBuf fb_blk, fb_nbr, fb_id, fb_mask, fb_tag;       // data-flow boundary phase: blocks, tagged entries
@@ -140,6 +141,8 @@ class Solver {
   // only when another material was the last one used on the device)
   void activate();
   void build_boundary_rows();
+  void build_boundary_maps();
+  bool alloc_boundary_maps(int l);
   void upload_layout();
   double read_scalar(const double* dev);
   void sync();

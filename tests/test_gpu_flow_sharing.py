@@ -115,3 +115,31 @@ def test_solvers_on_several_threads(coop, monkeypatch, capfd):
     assert "timed out" not in capfd.readouterr().err
     for s in solvers:
         s.close()
+
+
+@pytest.mark.parametrize("shape,levels,level", [((45, 23, 19), 3, 0), ((24, 40, 40), 4, 2)])
+def test_dense_maps_that_get_no_memory(shape, levels, level, monkeypatch):
+    """the maps refused at creation: the solver is created without them, its
+    boundary phases (of the level's own sweep count) run by data flow, solves
+    reach the same solution, also after a density update"""
+    p = W.box(*shape, seed=5, mg_levels=levels)
+    with_maps = _lib.Solver(p)
+    monkeypatch.setenv("SPG_MAP_MAX_MB", "0")
+    s = _lib.Solver(p)
+    monkeypatch.delenv("SPG_MAP_MAX_MB")
+    # two maps in FP64 and FP32 of at least this level's set
+    gx, gf = s.level_nodes(level)
+    assert with_maps.info()["hbm_bytes"] - s.info()["hbm_bytes"] > 10e6
+    rng = np.random.default_rng(11)
+    u, b = rng.standard_normal((len(gx), 3)) * 1e-3, rng.standard_normal((len(gx), 3))
+    u[(gf & 1) == 0] = 0
+    for prec, tol in ((1, 1e-11), (0, 1e-4)):
+        want = with_maps.kernel(_lib.OP_GS_BOUNDARY, level, u, b, precision=prec, sweeps=3)
+        assert rel(s.kernel(_lib.OP_GS_BOUNDARY, level, u, b, precision=prec, sweeps=3), want) < tol
+    for density in (p.density, p.density * 0.9):
+        for x in (s, with_maps):
+            x.update_density(density)
+        want, got = (x.solve(tolerance=1e-10, precision=1)[0] for x in (with_maps, s))
+        assert rel(got[..., :3], want[..., :3]) < 1e-8
+    s.close()
+    with_maps.close()
