@@ -11,6 +11,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstdint>
+#include <exception>
 #include <limits>
 #include <mutex>
 #include <string>
@@ -250,7 +251,6 @@ __global__ void __launch_bounds__(64 * (OC_MIDS + 1)) k_oc_many_final(int np, co
 // per-device scratch of the OC reduction, allocated on first use
 struct OcScratch {
   double* part = nullptr;
-  double* res = nullptr;
   double* host = nullptr;  // pinned, written by the final kernels of a pass
   int np = 0;
 };
@@ -358,9 +358,9 @@ extern "C" int spg_oc_trial(int64_t n, const uint8_t* mask, const double* rho, c
 // it starts with; then the next four levels of its tree.  An answer within
 // rounding of the target is taken from a trial of that multiplier alone, so
 // the sequence is that of one trial per step: 8 passes instead of about 90.
-extern "C" int spg_oc_update(int64_t n, const uint8_t* mask, const double* rho, const double* dc, double target,
-                             double step, double min_density, double fixed_density, int32_t exclude_fixed,
-                             double dc_shift, double* out, double* change, double* multiplier) {
+static int oc_update(int64_t n, const uint8_t* mask, const double* rho, const double* dc, double target, double step,
+                     double min_density, double fixed_density, int32_t exclude_fixed, double dc_shift, double* out,
+                     double* change, double* multiplier) {
   if (!mask || !rho || !dc || !out) return fail(SPG_E_INVALID, "null argument");
   if (n < 0) return fail(SPG_E_INVALID, "negative cell count");
   std::lock_guard<std::mutex> lock(g_oc_mu);
@@ -450,6 +450,17 @@ extern "C" int spg_oc_update(int64_t n, const uint8_t* mask, const double* rho, 
   if (change) *change = vc[1];
   if (multiplier) *multiplier = mid;
   return SPG_OK;
+}
+
+extern "C" int spg_oc_update(int64_t n, const uint8_t* mask, const double* rho, const double* dc, double target,
+                             double step, double min_density, double fixed_density, int32_t exclude_fixed,
+                             double dc_shift, double* out, double* change, double* multiplier) {
+  try {  // the lists of multipliers are allocated
+    return oc_update(n, mask, rho, dc, target, step, min_density, fixed_density, exclude_fixed, dc_shift, out, change,
+                     multiplier);
+  } catch (const std::exception& e) {
+    return fail(SPG_E_HIP, e.what());
+  }
 }
 
 // ------------------------------------------------ OC trial without allocation
