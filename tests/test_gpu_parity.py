@@ -408,6 +408,30 @@ def test_apply_forms_agree(shape, blocks, monkeypatch):
     s.close()
 
 
+@pytest.mark.parametrize("shape,blocks", [((3, 3, 3), 1), ((45, 23, 19), 360), ((61, 43, 35), 1584)])
+def test_krylov_operator_by_rows_in_fp32(shape, blocks, monkeypatch):
+    """the FP32 Krylov operator by rows with FP32 sums (eight lanes a node up to
+    1536 blocks, which the default leaves to the cell form or to FP64 sums)
+    against the cell form in FP64, to 1e-6 relative, and its fused dot product
+    in whole solves: FP32 PCG with it, and FP64 PCG, whose operator is by rows
+    by default, to the oracle's solution"""
+    p = W.box(*shape, seed=9, mg_levels=1 if blocks == 1 else 3)
+    s = _lib.Solver(p)
+    assert s.level_blocks(0) == blocks
+    u = np.random.default_rng(23).standard_normal((len(s.level_nodes(0)[0]), 3)).astype(np.float32).astype(np.float64)
+    monkeypatch.setenv("SPG_APPLY_CELL", "1")
+    want = s.kernel(_lib.OP_OPERATOR, 0, u, None, precision=1)
+    monkeypatch.setenv("SPG_APPLY_CELL", "0")
+    monkeypatch.setenv("SPG_ACC64_MODES", "0")
+    assert rel(s.kernel(_lib.OP_OPERATOR, 0, u, None, precision=0), want) < 1e-6
+    o = O.Oracle(p)
+    u_o = o.pack(o.solve(tolerance=1e-12, max_iterations=500)[0])[..., :3]
+    for out, info in (s.solve_mixed(tolerance=1e-8), s.solve(tolerance=1e-10, precision=1)):
+        assert info["converged"] == 1
+        assert np.linalg.norm(out[..., :3] - u_o) / np.linalg.norm(u_o) < 1e-6
+    s.close()
+
+
 @pytest.mark.parametrize("prec,tol", [(1, 1e-13), (0, 1e-6)])
 def test_restriction_and_prolongation(blocky, prec, tol):
     P = blocky
