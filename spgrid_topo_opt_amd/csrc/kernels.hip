@@ -2170,16 +2170,17 @@ __global__ void __launch_bounds__(64) k_bnd_flow(BndOff L, ColourOrder ord, Colo
 // of lanes gathering each node's neighbours from u and the entries in every
 // step, 12 loads a lane for FP32, took 2.4 us.
 // Sweep in us, FP32 / FP64: this, by octet gather, by colour launches
-//   level 0, 45 blocks       15 / 17    24 / 29    33 / 41
-//            1377 blocks     21 / 39    30 / -     35 / 43
-//            3024 blocks     29 / 46    -          41 / 48
-//            2057 blocks     24 / 49    -          36 / 45
+//   level 0, 180 blocks      16 / 18    25 / 29    35 / 40
+//            1377 blocks     21 / 40    30 / -     34 / 40
+//            2057 blocks     25 / 49    -          35 / 43
+//            2750 blocks     28 / 58    -          37 / 46
+//            3575 blocks     35 / 77    -          38 / 46
 //   explicit, 84 blocks      16 / 17    24 / 29
 //            251 blocks      17 / 18    23 / 26    37 / 42
 //            1229 blocks     25 / -     -          46 / 57
-// The lines: where the launches win (FP64 level 0), or half of the blocks that
-// the registers let the 256 CUs hold at once, which leaves the other solvers of
-// a device something of its budget (flow_budget.hpp).
+// The lines: where the launches win (level 0), or half of the blocks that the
+// registers let the 256 CUs hold at once, which leaves the other solvers of a
+// device something of its budget (flow_budget.hpp).
 template <class T>
 struct FlowBlocks {
   static constexpr int gs0 = sizeof(T) == 4 ? 4096 : 1536;
@@ -3689,7 +3690,6 @@ static void launch_bmap_build_nc(hipStream_t st, const LevelDev& L, int sweeps, 
       n, o, colour_order(level0, true), colour_order(level0, false), sweeps, L.bnd, L.bci, L.bA64, L.flags, M[0], M[1],
       F[0], F[1]);
 }
-int bmap_max_nodes() { return (int)(kMaxLds / 24); }
 void launch_bmap_build(hipStream_t st, const LevelDev& L, int sweeps, bool level0, double* const M[2],
                        float* const F[2]) {
   const int n = L.bnd_off[8];
@@ -3755,7 +3755,7 @@ void launch_gs0(hipStream_t st, const LevelDev& L, const T* E, T dx, T* u, const
   // 359 / 571 us; a persistent, software-pipelined quad kernel with buffer
   // loads 389 / 600 us (118 VGPRs: 4 waves per SIMD); a cell corner per
   // wavefront with table-driven staging 436 / 726 us.  The quad kernel keeps
-  // the VALUs about 94% busy, and with fewer VALU instructions the latency of
+  // the VALUs 81% busy here, and with fewer VALU instructions the latency of
   // its two dependent load phases (neighbour rows, then the halo) sets the
   // same time.
   const int kind = e && std::atoi(e) > 0 ? std::atoi(e) : 3;

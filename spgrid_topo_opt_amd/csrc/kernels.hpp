@@ -245,9 +245,8 @@ void launch_bnd_coef_st(hipStream_t st, const LevelDev& L, const double* ST, dou
 // row stride of the dense boundary map of an n-node boundary set: 3n padded to 64
 __host__ __device__ inline int64_t bmap_stride(int n) { return ((int64_t)3 * n + 63) / 64 * 64; }
 // dense maps (3n x 3n, row-major, stride bmap_stride(n)) of a boundary phase,
-// [0] forward and [1] backward, in FP64 and rounded to FP32, for at most
-// bmap_max_nodes() nodes; the padding columns must hold zeros
-int bmap_max_nodes();
+// [0] forward and [1] backward, in FP64 and rounded to FP32, for at most 6826
+// nodes (a column of 3n doubles in the LDS); the padding columns must hold zeros
 void launch_bmap_build(hipStream_t st, const LevelDev& L, int sweeps, bool level0, double* const M[2],
                        float* const F[2]);
 // bottom

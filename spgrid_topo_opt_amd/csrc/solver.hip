@@ -33,10 +33,16 @@ static double now_s() {
 
 // Boundary phases over at most this many nodes run as one dense map (2 maps x
 // 3n x 3n entries in FP64 and FP32).  Level-0 phase by map / by data flow, FP32
-// and FP64: 9.8 / 39 and 16 / 43 us at 1425 nodes, 17.5 / 40 and 29 / 44 at
-// 2400, 25 / 40 and 42 / 45 at 3000.  A density update builds both maps: 0.2 ms
-// at 405 nodes, 1.0, 1.9 and 5.9 at these, which a solve of 25 V-cycles (4
-// phases each) earns back up to about here.
+// and FP64, and what both maps add to a density update:
+//   405 nodes    7.1 / 36 us    8.2 / 41 us   0.36 ms
+//   1425         9.8 / 38       16 / 43       1.2
+//   2400         17 / 39        29 / 44       2.6
+//   3000         23 / 38        41 / 43       6.0
+// At four phases a V-cycle the maps are earned back after 3, 11, 30 and 99
+// FP32 V-cycles, and 3, 11, 43 and over 500 FP64 ones.  The line is drawn for
+// solves on kept operators and for FP32.  One FP64 solve of 25 V-cycles after
+// each update earns them back up to about 1,900 nodes and loses about 1 ms of
+// 10 at 2,400: there the data flow would be the faster way.
 static constexpr int kMaxDenseBoundary = 2560;
 // levels of at most this many blocks get the entries of the data-flow sweep
 // (FlowBlocks in kernels.hip has each kernel's own limit)
@@ -52,10 +58,10 @@ static constexpr double kFp32PassReduction = 1e-6;
 // bandwidth-bound GEMV per V-cycle), the nested-dissection Cholesky
 // (bottom_nd.hip) above it, unless spg_config.bottom_dense_max sets another
 // limit; SPG_BOTTOM=dense|nd overrides both (dense stays limited to
-// kMaxDenseBottomDofs: its inverse is O(n^2)).  A whole density update takes 2.9
-// / 5.1 / 41 ms with the dense inverse and 2.1 / 1.2 / 8.0 ms with the nested
-// dissection at 2.0 K / 4.1 K / 9.0 K unknowns (other levels' work included);
-// the bottom solve of an FP32 V-cycle 6.6 / 15 / 48 us against 33 / 50 / 80 us:
+// kMaxDenseBottomDofs: its inverse is O(n^2)).A whole density update takes 4.1
+// / 5.0 / 49 ms with the dense inverse and 3.0 / 1.9 / 3.7 ms with the nested
+// dissection at 2.0 K / 4.1 K / 11.6 K unknowns (other levels' work included);
+// the bottom solve of an FP32 V-cycle 6.5 / 15 / 80 us against 33 / 49 / 101 us:
 // the dense inverse pays when many solves share a factorization.
 static constexpr int64_t kDenseBottomDofs = 16384;
 static constexpr int64_t kMaxDenseBottomDofs = 60000;
