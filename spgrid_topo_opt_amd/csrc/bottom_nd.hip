@@ -547,7 +547,7 @@ void NdBottom::upload(hipStream_t st) {
   tiles_.alloc((size_t)std::max<int64_t>(ntile_, 1) * tile);
   tr_.alloc((size_t)std::max<int64_t>(ntr_, 1) * tile);
   pan_.alloc((size_t)std::max<int64_t>(npan_, 1) * tile);
-  minv_.alloc((size_t)std::max<int64_t>(nid_, 1) * tile);
+  minv_.alloc((size_t)std::max<int64_t>(nid_, 1) * 2 * tile);
   info_.alloc((size_t)std::max<int64_t>(nid_, 1) * sizeof(int));
   for (Depth& D : depth_) {
     D.batch.d = static_cast<SweepMat*>(d_mats_.p) + D.mat0;

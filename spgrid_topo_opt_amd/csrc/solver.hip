@@ -58,10 +58,10 @@ static constexpr double kFp32PassReduction = 1e-6;
 // bandwidth-bound GEMV per V-cycle), the nested-dissection Cholesky
 // (bottom_nd.hip) above it, unless spg_config.bottom_dense_max sets another
 // limit; SPG_BOTTOM=dense|nd overrides both (dense stays limited to
-// kMaxDenseBottomDofs: its inverse is O(n^2)).A whole density update takes 4.1
-// / 5.0 / 49 ms with the dense inverse and 3.0 / 1.9 / 3.7 ms with the nested
+// kMaxDenseBottomDofs: its inverse is O(n^2)).A whole density update takes 3.8
+// / 4.4 / 46 ms with the dense inverse and 3.0 / 1.8 / 3.3 ms with the nested
 // dissection at 2.0 K / 4.1 K / 11.6 K unknowns (other levels' work included);
-// the bottom solve of an FP32 V-cycle 6.5 / 15 / 80 us against 33 / 49 / 101 us:
+// the bottom solve of an FP32 V-cycle 6.5 / 15 / 76 us against 33 / 49 / 101 us:
 // the dense inverse pays when many solves share a factorization.
 static constexpr int64_t kDenseBottomDofs = 16384;
 static constexpr int64_t kMaxDenseBottomDofs = 60000;
@@ -547,7 +547,7 @@ void Solver::build_operators() {
     tiles64_.alloc(ntile * 4096 * 8);
     tiles32_.alloc(ntile * 4096 * 4);
     pan_.alloc((size_t)nT_ * 4096 * 8);
-    minv_.alloc(4096 * 8);
+    minv_.alloc(2 * 4096 * 8);
     info_.alloc(sizeof(int));
     const std::vector<SweepMat> one_mat{SweepMat{0, nT_, nT_, 0, 0}};
     upload(smat_, one_mat);

@@ -14,15 +14,18 @@
 // (moduli 1 and 9e-9, 3 K to 7 K unknowns, residual of a solve: 6e6 to 6e7 of
 // the right-hand side, this form and LAPACK's Cholesky 2e-7 to 1.5e-6).
 //
-// Every step is two launches over the whole batch: the panels, then the
+// Every step is two launches over the whole batch: the panels Y, then the
 // trailing tiles; the workgroup of the next diagonal tile also factors it, so
-// that serial part runs beside the others.  The products are 64x64x64 FP64
+// that serial part runs beside the others, and so do W and -D^-1, which nothing
+// in the step waits for.  The products are 64x64x64 FP64
 // tiles on the matrix cores (v_mfma_f64_16x16x4), both operands staged in LDS,
 // the result tile in registers.  Small batches are bound by the serial
 // factorization of the diagonal tiles (64 dependent pivots each).  A density
-// update, against one tile inverse applied as a matrix: dense 3,072 unknowns
-// 2.8 -> 3.2 ms, nested dissection 1.3 -> 1.6 ms and, at 15,120, 2.9 -> 3.2 ms
-// (partial Cholesky front by front through rocSOLVER: 12.6, 12.6 and 62 ms).
+// update, against one tile inverse applied as a matrix: dense 2.8 -> 2.6 ms at
+// 3,072 unknowns, nested dissection 1.3 -> 1.3 ms there and 2.9 -> 2.7 ms at
+// 15,120 (partial Cholesky front by front through rocSOLVER: 12.6, 12.6 and 62
+// ms); with W and -D^-1 in the chain of the panel and of the factorization 3.2,
+// 1.6 and 3.2 ms.
 // The residual of a solve is 0.4 to 1.3 times rocSOLVER's over 3 K to 15 K
 // unknowns, ordinary and high-contrast designs.
 #include <hip/hip_runtime.h>
@@ -58,6 +61,16 @@ __device__ __forceinline__ void put_half(const double2 (&v)[4], double (*s)[HLD]
     s[r][c + 1] = sgn * v[i].y;
   }
 }
+// stage rows 32h .. 32h + 31
+__device__ __forceinline__ void stage_rows(const double* __restrict__ t, int h, double (*s)[LD]) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int e = threadIdx.x + 256 * i, r = e >> 5, c = (e & 31) * 2;
+    const double2 v = *reinterpret_cast<const double2*>(t + (32 * h + r) * 64 + c);
+    s[r][c] = v.x;
+    s[r][c + 1] = v.y;
+  }
+}
 // stage a row-major 64x64 tile, times sgn
 __device__ __forceinline__ void stage(const double* __restrict__ t, double (*s)[LD], double sgn) {
   for (int e = threadIdx.x; e < 2048; e += 256) {
@@ -84,12 +97,13 @@ __device__ __forceinline__ void mm64(const double (*A)[S], const double (*B)[S],
     acc[1][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(a1, b1, acc[1][1], 0, 0, 0);
   }
 }
-// acc += A B over K = 64, and acc += A^T A, results placed as above
-__device__ __forceinline__ void mm64n(const double (*A)[LD], const double (*B)[LD], d4 (&acc)[2][2]) {
+// acc += A B and acc += B^T B over 32 rows of B (A: the matching columns),
+// results placed as above
+__device__ __forceinline__ void mm32n(const double (*A)[HLD], const double (*B)[LD], d4 (&acc)[2][2]) {
   const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
   const int ra = (w >> 1) * 32 + (l & 15), rb = (w & 1) * 32 + (l & 15), k0 = l >> 4;
 #pragma unroll
-  for (int k = 0; k < 64; k += 4) {
+  for (int k = 0; k < 32; k += 4) {
     const double a0 = A[ra][k + k0], a1 = A[ra + 16][k + k0];
     const double b0 = B[k + k0][rb], b1 = B[k + k0][rb + 16];
     acc[0][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(a0, b0, acc[0][0], 0, 0, 0);
@@ -98,13 +112,13 @@ __device__ __forceinline__ void mm64n(const double (*A)[LD], const double (*B)[L
     acc[1][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(a1, b1, acc[1][1], 0, 0, 0);
   }
 }
-__device__ __forceinline__ void mm64sq(const double (*A)[LD], d4 (&acc)[2][2]) {
+__device__ __forceinline__ void mm32sq(const double (*B)[LD], d4 (&acc)[2][2]) {
   const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
   const int ra = (w >> 1) * 32 + (l & 15), rb = (w & 1) * 32 + (l & 15), k0 = l >> 4;
 #pragma unroll
-  for (int k = 0; k < 64; k += 4) {
-    const double a0 = A[k + k0][ra], a1 = A[k + k0][ra + 16];
-    const double b0 = A[k + k0][rb], b1 = A[k + k0][rb + 16];
+  for (int k = 0; k < 32; k += 4) {
+    const double a0 = B[k + k0][ra], a1 = B[k + k0][ra + 16];
+    const double b0 = B[k + k0][rb], b1 = B[k + k0][rb + 16];
     acc[0][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(a0, b0, acc[0][0], 0, 0, 0);
     acc[0][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(a0, b1, acc[0][1], 0, 0, 0);
     acc[1][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(a1, b0, acc[1][0], 0, 0, 0);
@@ -159,15 +173,16 @@ __device__ __forceinline__ void chol16(double (&a)[4], double& dc, int& bad, int
 }
 
 // The 64x64 SPD tile in LDS (lower blocks and whole diagonal blocks are read)
-// -> M = L^-1 in minv, -M^T M = minus the inverse in the tile store, by blocks
-// of 16.  Every wave factors the pivot block (no barrier between its 16
-// dependent pivots); wave r below it takes row block r: Y_r^T = M_KK A_rK^T,
-// whose result registers are the left operand of A_rj -= Y_r Y_j^T and of the
-// rows of M, T_rc -= Y_r M_Kc, when the sum over k runs in the order that they
-// hold; the pivot's own wave finishes M_Kc = M_KK T_Kc.  Y_j^T waits in the block
-// above the diagonal, which holds nothing else.  Two barriers per block.
-__device__ void factor_tile(double (*s)[LD], double (*mk)[17], double* __restrict__ tile, double* __restrict__ minv,
-                            int* __restrict__ info, int pivot0) {
+// -> M = L^-1 in minv, by blocks of 16.  Every wave factors the pivot block (no
+// barrier between its 16 dependent pivots); wave r below it takes row block r:
+// Y_r^T = M_KK A_rK^T, whose result registers are the left operand of A_rj -= Y_r
+// Y_j^T and of the rows of M, T_rc -= Y_r M_Kc, when the sum over k runs in the
+// order that they hold; the pivot's own wave finishes M_Kc = M_KK T_Kc.  Y_j^T
+// waits in the block above the diagonal, which holds nothing else.  Two barriers
+// per block.  Inlined: as a call it takes the caller 4 registers too many for
+// four workgroups a CU.
+__device__ __forceinline__ void factor_tile(double (*s)[LD], double (*mk)[17], double* __restrict__ minv,
+                                            int* __restrict__ info, int pivot0) {
   const int r = threadIdx.x >> 6, l = threadIdx.x & 63, g = l >> 4, c = l & 15;
   int bad = 0;
   for (int K = 0; K < 4; ++K) {
@@ -221,48 +236,35 @@ __device__ void factor_tile(double (*s)[LD], double (*mk)[17], double* __restric
   }
   for (int e = threadIdx.x; e < 4096; e += 256) {
     const int i = e >> 6, j = e & 63;
-    if ((j >> 4) > (i >> 4)) s[i][j] = 0.0;
-    minv[e] = s[i][j];
+    minv[e] = (j >> 4) > (i >> 4) ? 0.0 : s[i][j];
   }
-  __syncthreads();
-  d4 acc[2][2] = {};
-  mm64sq(s, acc);
-#pragma unroll
-  for (int p = 0; p < 2; ++p)
-#pragma unroll
-    for (int b = 0; b < 2; ++b)
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        int i, j;
-        acc_pos(p, b, q, i, j);
-        tile[i * 64 + j] = -acc[p][b][q];
-      }
   if (threadIdx.x == 0 && bad && *info == 0) *info = bad;
 }
 
 // the first diagonal tile of every matrix
-__global__ void __launch_bounds__(256) k_sw_first(const SweepMat* __restrict__ mats, double* tiles, double* minv,
+__global__ void __launch_bounds__(256) k_sw_first(const SweepMat* __restrict__ mats, const double* tiles,
+                                                  double* minv,
                                                   int* info) {
   __shared__ __align__(16) double s[64][LD];
   __shared__ double mk[16][17];
   const SweepMat M = mats[blockIdx.x];
-  double* t = tiles + M.off * 4096;
-  stage(t, s, 1.0);
+  stage(tiles + M.off * 4096, s, 1.0);
   __syncthreads();
-  factor_tile(s, mk, t, minv + (int64_t)M.id * 4096, info + M.id, 0);
+  factor_tile(s, mk, minv + (int64_t)M.id * 8192, info + M.id, 0);
 }
 
-// panels of step k: Y_i = A_iK M^T (kept for the trailing tiles), A_iK = Y_i M
-__global__ void __launch_bounds__(256) k_sw_panel(const SweepMat* __restrict__ mats, int k, double* tiles,
-                                                  double* __restrict__ pan, const double* __restrict__ minv) {
+// panels of step k: Y_i = A_iK M^T
+__global__ void __launch_bounds__(256) k_sw_panel(const SweepMat* __restrict__ mats, int k,
+                                                  const double* __restrict__ tiles, double* __restrict__ pan,
+                                                  const double* __restrict__ minv) {
   __shared__ __align__(16) double sx[64][LD], sm[64][LD];
   const SweepMat M = mats[blockIdx.y];
   const int i = blockIdx.x;
   if (i >= M.nt || i == k) return;
   const bool below = i > k;
-  double* t = tiles + (M.off + (below ? tile_at(i, k) : tile_at(k, i))) * 4096;
+  const double* t = tiles + (M.off + (below ? tile_at(i, k) : tile_at(k, i))) * 4096;
   double* Y = pan + (int64_t)(M.pan + i) * 4096;
-  stage(minv + (int64_t)M.id * 4096, sm, 1.0);
+  stage(minv + ((int64_t)M.id * 2 + (k & 1)) * 4096, sm, 1.0);
   if (below) {
     stage(t, sx, 1.0);
   } else {
@@ -271,22 +273,6 @@ __global__ void __launch_bounds__(256) k_sw_panel(const SweepMat* __restrict__ m
   __syncthreads();
   d4 acc[2][2] = {};
   mm64(sx, sm, acc);
-  __syncthreads();  // sx is reused
-#pragma unroll
-  for (int a = 0; a < 2; ++a)
-#pragma unroll
-    for (int b = 0; b < 2; ++b) {
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        int r, c;
-        acc_pos(a, b, q, r, c);
-        Y[r * 64 + c] = acc[a][b][q];
-        sx[r][c] = acc[a][b][q];
-      }
-      acc[a][b] = d4{};
-    }
-  __syncthreads();
-  mm64n(sx, sm, acc);
 #pragma unroll
   for (int a = 0; a < 2; ++a)
 #pragma unroll
@@ -295,18 +281,19 @@ __global__ void __launch_bounds__(256) k_sw_panel(const SweepMat* __restrict__ m
       for (int q = 0; q < 4; ++q) {
         int r, c;
         acc_pos(a, b, q, r, c);
-        t[below ? r * 64 + c : c * 64 + r] = acc[a][b][q];
+        Y[r * 64 + c] = acc[a][b][q];
       }
 }
 
-// trailing tiles of step k: A_ij -= Y_i Y_j^T, i >= j, both != k.  Workgroup 0
-// takes the next diagonal tile and factors it.
+// trailing tiles of step k: A_ij -= Y_i Y_j^T, i >= j, both != k; A_iK = Y_i M and
+// A_KK = -M^T M.  Workgroup 0 takes the next diagonal tile and factors it into
+// the other of its two places in minv, as the others still read this one.
 // Large matrices are bound by the loads and stores of the tiles: operands staged
-// in halves (37 KB of LDS, the second half's loads under the first product)
-// leave room for four workgroups a CU instead of two.  Density update of a dense
-// bottom 150 -> 102 ms at 15,120 unknowns, 1180 -> 815 ms at 30,720 (rocSOLVER
-// 187 and 1094 ms), 3.2 ms either way at 3,072.
-__global__ void __launch_bounds__(256) k_sw_trail(const SweepMat* __restrict__ mats, int k, double* tiles,
+// in halves (37 KB of LDS, the second half's loads under the first product) and
+// 125 registers leave room for four workgroups a CU (whole tiles: two).  Density
+// update of a dense bottom 150 -> 96 ms at 15,120 unknowns, 1180 -> 767 ms at
+// 30,720 (rocSOLVER 187 and 1094 ms), no difference at 3,072.
+__global__ void __launch_bounds__(256, 4) k_sw_trail(const SweepMat* __restrict__ mats, int k, double* tiles,
                                                   const double* __restrict__ pan, double* minv, int* info) {
   __shared__ __align__(16) double sm[2 * 64 * HLD];
   __shared__ double mk[16][17];
@@ -314,6 +301,8 @@ __global__ void __launch_bounds__(256) k_sw_trail(const SweepMat* __restrict__ m
   double(*sy)[HLD] = reinterpret_cast<double(*)[HLD]>(sm);
   double(*sx)[HLD] = reinterpret_cast<double(*)[HLD]>(sm + 64 * HLD);
   double(*sw)[LD] = reinterpret_cast<double(*)[LD]>(sm);
+  double(*sr)[LD] = reinterpret_cast<double(*)[LD]>(sm + 64 * HLD);
+  static_assert(64 * HLD >= 32 * LD, "32 rows take the place of an operand");
   const SweepMat M = mats[blockIdx.y];
   const bool more = k + 1 < M.np;
   int i, j;
@@ -327,9 +316,39 @@ __global__ void __launch_bounds__(256) k_sw_trail(const SweepMat* __restrict__ m
     while (tile_at(i + 1, 0) <= e) ++i;
     while (tile_at(i, 0) > e) --i;
     j = (int)(e - tile_at(i, 0));
-    if (i == k || j == k || (more && i == k + 1 && j == k + 1)) return;
+    if (more && i == k + 1 && j == k + 1) return;
   }
   double* t = tiles + (M.off + tile_at(i, j)) * 4096;
+  if (i == k || j == k) {
+    const double* Mk = minv + ((int64_t)M.id * 2 + (k & 1)) * 4096;
+    const double* Yp = pan + (int64_t)(M.pan + (i == k ? j : i)) * 4096;
+    const bool diag = i == j;
+    d4 acc[2][2] = {};
+    for (int h = 0; h < 2; ++h) {
+      if (h) __syncthreads();
+      stage_rows(Mk, h, sr);
+      if (!diag) {
+        double2 v[4];
+        load_half(Yp, h, v);
+        put_half(v, sy, 1.0);
+      }
+      __syncthreads();
+      if (diag) mm32sq(sr, acc);
+      else mm32n(sy, sr, acc);
+    }
+#pragma unroll
+    for (int a = 0; a < 2; ++a)
+#pragma unroll
+      for (int b = 0; b < 2; ++b)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          int r, c;
+          acc_pos(a, b, q, r, c);
+          if (diag) t[r * 64 + c] = -acc[a][b][q];
+          else t[i > k ? r * 64 + c : c * 64 + r] = acc[a][b][q];
+        }
+    return;
+  }
   // the product is summed by itself and added once: 64 terms added to a tile
   // that holds the sums of the steps before would each round at its size
   d4 acc[2][2] = {}, old[2][2];
@@ -374,7 +393,7 @@ __global__ void __launch_bounds__(256) k_sw_trail(const SweepMat* __restrict__ m
       }
   if (next) {
     __syncthreads();
-    factor_tile(sw, mk, t, minv + (int64_t)M.id * 4096, info + M.id, 64 * (k + 1));
+    factor_tile(sw, mk, minv + ((int64_t)M.id * 2 + ((k + 1) & 1)) * 4096, info + M.id, 64 * (k + 1));
   }
 }
 
@@ -394,8 +413,7 @@ void sweep_run(hipStream_t st, const SweepBatch& b, double* tiles) {
       while (live > 0 && h[live - 1].np <= k) --live;
       int nt = 0;
       for (int i = 0; i < live; ++i) nt = std::max(nt, h[i].nt);
-      if (nt == 1) break;  // a single tile is done
-      k_sw_panel<<<dim3(nt, live), 256, 0, st>>>(d, k, tiles, b.pan, b.minv);
+      if (nt > 1) k_sw_panel<<<dim3(nt, live), 256, 0, st>>>(d, k, tiles, b.pan, b.minv);
       k_sw_trail<<<dim3((unsigned)(tile_at(nt, 0) + 1), live), 256, 0, st>>>(d, k, tiles, b.pan, b.minv, b.info);
     }
   }

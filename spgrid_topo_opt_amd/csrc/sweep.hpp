@@ -25,7 +25,7 @@ __host__ __device__ inline int64_t tile_at(int I, int J) { return (int64_t)I * (
 struct SweepBatch {
   std::vector<SweepMat> h;  // by decreasing np
   SweepMat* d = nullptr;    // device copy of h
-  double *pan = nullptr, *minv = nullptr;  // panels, inverse factors of the diagonal tiles
+  double *pan = nullptr, *minv = nullptr;  // panels; two inverse factors of diagonal tiles per id
   int* info = nullptr;      // per id: 0, or 1 + the first pivot that is not positive
 };
 
