@@ -3796,12 +3796,13 @@ void launch_gs0_boundary(hipStream_t st, const LevelDev& L, const T* E, T dx, T*
                          bool forward) {
   if (sweeps <= 0 || L.bnd_off[8] == 0) return;
   int path = boundary_path();
-  // Automatic choice beyond the dense map (solver.hip has that line), FP32 per phase of 3 sweeps on the 256^3 shell (3655
-  // boundary nodes): data flow over blocks 40 us, over node groups 47 us (the
-  // way for more blocks than FlowBlocks has), grid barriers between the steps
-  // 87 us, per-colour list launches 145 us, single workgroup 154 us (one CU's
-  // VALU work).  The lists remain for a refused cooperative launch and after a
-  // time-out.
+  // Automatic choice beyond the dense map (solver.hip has that line), FP32 per
+  // phase of 3 sweeps on the 256^3 shell (3655 boundary nodes): data flow over
+  // blocks 40 us, over node groups 47 us (the way for more blocks than FlowBlocks
+  // has, and beside other solvers), grid barriers between the steps 87 us,
+  // per-colour list launches 145 us, single workgroup 154 us (one CU's VALU
+  // work).  The lists remain where no data-flow kernel may run: without room
+  // beside other solvers, after a time-out, for a refused cooperative launch.
   if (path == 0 && launch_bnd_map<T>(st, L, u, b, sweeps, forward)) return;
   if (path == 0 || path == 5) {
     if (launch_gs0_bnd_flow<T>(st, L, E, dx, u, b, sweeps, forward, path == 5)) return;
@@ -3847,7 +3848,7 @@ void launch_st_boundary(hipStream_t st, const LevelDev& L, const T* ST, T* u, co
   if (sweeps <= 0 || L.bnd_off[8] == 0) return;
   const int path = boundary_path() == 5 ? 0 : boundary_path();  // 5 selects a level-0 phase only
   if (path == 0 && launch_bnd_map<T>(st, L, u, b, sweeps, forward)) return;
-  // sets too large for a dense map: data flow; after a time-out one workgroup
+  // sets without a dense map: data flow; where that may not run, one workgroup
   if (path == 0 && launch_bnd_flow<T>(st, L, u, b, sweeps, false, forward, false)) return;
   if (path == 0 && launch_bnd_phase<T>(st, L, u, b, sweeps, false, forward)) return;
   const ColourOrder ord = colour_order(false, forward);
