@@ -3590,22 +3590,24 @@ static int flow_fit(F kernel) {
   return n;
 }
 template <class T>
-static void add_flow_need_t(FlowNeed& need, const LevelDev& L, bool level0) {
+static void add_flow_need_t(FlowNeed& need, const LevelDev& L, bool level0, bool any) {
   static const int fit_bnd = flow_fit(k_bnd_flow<T>), fit_bnd0 = flow_fit(k_gs0_bnd_flow<T>),
                    fit_gs0 = flow_fit(k_gs0_flow<T>), fit_st = flow_fit(k_st_flow<T>);
-  need.add(bnd_flow_waves(L), fit_bnd);
-  if (level0) {
-    need.add(gs0_bnd_flow_waves<T>(L), fit_bnd0);
-    need.add(sweep_flow_waves(L, FlowBlocks<T>::gs0), fit_gs0);
-  } else {
-    need.add(sweep_flow_waves(L, FlowBlocks<T>::st), fit_st);
-  }
+  // a V-cycle's phases run as the map, else over blocks, else over node groups
+  // (in FP64 the largest waves: one a SIMD)
+  const int blocks = level0 ? gs0_bnd_flow_waves<T>(L) : 0;
+  if (any || L.bmap_sweeps == 0) need.add(blocks, fit_bnd0);
+  if (any || (L.bmap_sweeps == 0 && blocks == 0)) need.add(bnd_flow_waves(L), fit_bnd);
+  if (level0) need.add(sweep_flow_waves(L, FlowBlocks<T>::gs0), fit_gs0);
+  else need.add(sweep_flow_waves(L, FlowBlocks<T>::st), fit_st);
 }
-void add_flow_need(FlowNeed& need, const LevelDev& L, bool level0, bool fp64, FlowUse use) {
+void add_flow_need(FlowNeed& need, const LevelDev& L, bool level0, bool fp64, FlowUse use, bool any) {
   LevelDev l = L;
   l.flow = use;
-  if (fp64) add_flow_need_t<double>(need, l, level0);
-  else add_flow_need_t<float>(need, l, level0);
+  // SPG_BOUNDARY_PATH, SPG_COOP_WG: other kernels than the automatic ones
+  any = any || std::getenv("SPG_BOUNDARY_PATH") || std::getenv("SPG_COOP_WG");
+  if (fp64) add_flow_need_t<double>(need, l, level0, any);
+  else add_flow_need_t<float>(need, l, level0, any);
 }
 // boundary phase by data flow (k_bnd_flow); false if the level has no tables
 // for it or the launch is refused (the caller then runs another path).

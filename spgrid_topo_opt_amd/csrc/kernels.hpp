@@ -152,8 +152,9 @@ template <class T>
 int launch_apply_dot(hipStream_t st, const LevelDev& L, const T* E, T dx, const T* in, T* out, double* bpart,
                      double* part, double* dot, CgScalars* sc = nullptr, int stage = -1);
 // what the level's data-flow kernels take of the device at most, of one
-// precision, under `use`
-void add_flow_need(FlowNeed& need, const LevelDev& L, bool level0, bool fp64, FlowUse use);
+// precision, under `use`: those of a V-cycle, or with `any` all that a boundary
+// phase of any sweep count or a switch may choose
+void add_flow_need(FlowNeed& need, const LevelDev& L, bool level0, bool fp64, FlowUse use, bool any);
 // level-0 GS: one colour over all blocks; all boundary sweeps of one phase.
 // With `bcm` (b in colour-major order, launch_colour_major) and the level's
 // flags_cm, the colour kernel reads b and the flags of its colour only.

@@ -225,7 +225,7 @@ void Solver::set_flow(FlowUse use) {
 // All data-flow kernels if their waves fit beside those that other solvers have
 // on the device; else boundary phases by few waves; else none.  A cooperative
 // launch makes its own room.  SPG_DATA_FLOW=0: none.
-Solver::FlowLease::FlowLease(Solver& s, int precision) : s_(s) {
+Solver::FlowLease::FlowLease(Solver& s, int precision, bool any) : s_(s) {
   const char* sw = std::getenv("SPG_DATA_FLOW");
   const char* coop = std::getenv("SPG_COOP_LAUNCH");
   FlowUse use = kFlowNone;
@@ -238,8 +238,8 @@ Solver::FlowLease::FlowLease(Solver& s, int precision) : s_(s) {
     for (const FlowUse u : {kFlowAll, kFlowFew}) {
       need_ = FlowNeed();
       for (size_t l = 0; l < s.lv_.size(); ++l) {
-        if (precision != 1) add_flow_need(need_, s.lv_[l].d, l == 0, false, u);
-        if (precision == 1 || s.coarse64_) add_flow_need(need_, s.lv_[l].d, l == 0, true, u);
+        if (precision != 1) add_flow_need(need_, s.lv_[l].d, l == 0, false, u, any);
+        if (precision == 1 || s.coarse64_) add_flow_need(need_, s.lv_[l].d, l == 0, true, u, any);
       }
       held_ = need_.cus == 0.0 || flow_budget().take(s.cfg_.device, cus, need_);
       if (!held_) continue;
@@ -1407,7 +1407,7 @@ void Solver::run_kernel(int op, int level, int precision, int forward, const dou
                         double* out) {
   activate();
   if (level < 0 || level >= lay_.nlev) throw SpgError(SPG_E_INVALID, "level out of range");
-  const FlowLease lease(*this, precision);
+  const FlowLease lease(*this, precision, true);
   auto body = [&](auto tag) {
     using T = decltype(tag);
     auto put = [&](DBuf& d, const double* h, int64_t nb) {
@@ -1550,7 +1550,7 @@ double Solver::bench_kernel(int op, int level, int precision, int arg, int reps)
   activate();
   if (level < 0 || level >= lay_.nlev) throw SpgError(SPG_E_INVALID, "level out of range");
   const int B = lay_.nlev - 1;
-  const FlowLease lease(*this, precision);
+  const FlowLease lease(*this, precision, true);
   hipEvent_t e0, e1;
   HIPCHK(hipEventCreate(&e0));
   HIPCHK(hipEventCreate(&e1));

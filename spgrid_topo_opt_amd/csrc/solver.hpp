@@ -153,7 +153,8 @@ class Solver {
   // use meanwhile.
   class FlowLease {
    public:
-    FlowLease(Solver& s, int precision);
+    // a solve's V-cycles, or with `any` every operator
+    FlowLease(Solver& s, int precision, bool any = false);
     ~FlowLease();
     FlowLease(const FlowLease&) = delete;
     FlowLease& operator=(const FlowLease&) = delete;
